@@ -299,6 +299,13 @@ typedef struct {
 
 int mh_kda_chunk_scan_fwd(const mh_kda_args* a, void* stream);
 
+/* The same with a workspace, which lets a scan of few heads split its sequence
+ * over the compute units: mh_kda_workspace_bytes gives the bytes (0 where these
+ * sizes gain nothing; workspace NULL walks each sequence at once, as
+ * mh_kda_chunk_scan_fwd does). */
+int mh_kda_workspace_bytes(const mh_kda_args* a, size_t* bytes);
+int mh_kda_chunk_scan_fwd_ws(const mh_kda_args* a, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Backward of the reference-mode scan (fwd.mode == MH_KDA_REFERENCE): the
  *   gradient PyTorch autograd forms through LinearDiffAttention._linear_attention_scan
  *   (mamformer/layers/kda_diff.py:357-478) when the layer is trained.

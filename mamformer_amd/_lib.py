@@ -186,7 +186,7 @@ EXPORTS = (
     "mh_ssd_ref_scan_bwd_workspace_bytes", "mh_ssd_ref_scan_bwd",
     "mh_silu_gate_fwd", "mh_silu_gate_bwd",
     "mh_ssd_state_update",
-    "mh_kda_chunk_scan_fwd", "mh_kda_bwd_workspace_bytes", "mh_kda_chunk_scan_bwd",
+    "mh_kda_chunk_scan_fwd", "mh_kda_workspace_bytes", "mh_kda_chunk_scan_fwd_ws", "mh_kda_bwd_workspace_bytes", "mh_kda_chunk_scan_bwd",
     "mh_kda_recurrent_step",
     "mh_causal_conv1d_fwd",
     "mh_conv1d_bwd_workspace_bytes", "mh_causal_conv1d_bwd",
@@ -236,6 +236,8 @@ def lib():
             h.mh_silu_gate_fwd.argtypes = [ct.POINTER(GateArgs), _vp]
             h.mh_silu_gate_bwd.argtypes = [ct.POINTER(GateArgs), _vp]
             h.mh_kda_chunk_scan_fwd.argtypes = [ct.POINTER(KdaArgs), _vp]
+            h.mh_kda_workspace_bytes.argtypes = [ct.POINTER(KdaArgs), ct.POINTER(_sz)]
+            h.mh_kda_chunk_scan_fwd_ws.argtypes = [ct.POINTER(KdaArgs), _vp, _sz, _vp]
             h.mh_kda_recurrent_step.argtypes = [ct.POINTER(KdaStepArgs), _vp]
             h.mh_kda_bwd_workspace_bytes.argtypes = [ct.POINTER(KdaBwdArgs), ct.POINTER(_sz)]
             h.mh_kda_chunk_scan_bwd.argtypes = [ct.POINTER(KdaBwdArgs), _vp]
@@ -244,7 +246,8 @@ def lib():
             h.mh_causal_conv1d_bwd.argtypes = [ct.POINTER(Conv1dBwdArgs), _vp]
             for name in ("mh_ssd_workspace_bytes", "mh_ssd_chunk_len", "mh_ssd_chunk_scan_fwd",
                          "mh_ssd_chunk_scan_fwd_noalloc",
-                         "mh_ssd_state_update", "mh_kda_chunk_scan_fwd", "mh_kda_recurrent_step",
+                         "mh_ssd_state_update", "mh_kda_chunk_scan_fwd", "mh_kda_workspace_bytes",
+                         "mh_kda_chunk_scan_fwd_ws", "mh_kda_recurrent_step",
                          "mh_causal_conv1d_fwd", "mh_conv1d_bwd_workspace_bytes", "mh_causal_conv1d_bwd",
                          "mh_ssd_bwd_workspace_bytes", "mh_ssd_chunk_scan_bwd",
                          "mh_kda_bwd_workspace_bytes", "mh_kda_chunk_scan_bwd",

@@ -1053,10 +1053,31 @@ int mh_ssd_state_update(const mh_ssu_args* a, void* stream) {
 }
 
 int mh_kda_chunk_scan_fwd(const mh_kda_args* a, void* stream) {
+  return mh_kda_chunk_scan_fwd_ws(a, nullptr, 0, stream);
+}
+
+int mh_kda_workspace_bytes(const mh_kda_args* a, size_t* bytes) {
+  if (!bytes) return fail(MH_ERR_NULL, "kda: bytes output is NULL");
   int rc = kda_validate(a);
   if (rc) return rc;
   mh::KdaParams p;
   kda_fill(a, p);
+  *bytes = mh::kda_plan_segments(p);
+  return MH_OK;
+}
+
+int mh_kda_chunk_scan_fwd_ws(const mh_kda_args* a, void* workspace, size_t workspace_bytes, void* stream) {
+  int rc = kda_validate(a);
+  if (rc) return rc;
+  mh::KdaParams p;
+  kda_fill(a, p);
+  if (workspace) {
+    const size_t need = mh::kda_plan_segments(p);
+    if (need > 0 && (workspace_bytes < need || !aligned16(workspace)))
+      return fail(MH_ERR_WORKSPACE, "kda: workspace of %zu bytes (16-byte aligned) required, got %zu", need,
+                  workspace_bytes);
+    p.seg_sum = reinterpret_cast<float*>(workspace);
+  }
   return hip_status(mh::launch_kda(p, reinterpret_cast<hipStream_t>(stream)), "kda_chunk_scan_fwd");
 }
 

@@ -18,8 +18,9 @@
 // with dS, dz the adjoint of the state after the chunk (zero, or the final-state gradient, at the end).
 // dq = dphi(q) * phi'(q) and phi'(x) = min(phi(x), 1) (e^x below 0, 1 above).
 //
-// kda_ref_bwd_q_kernel   grid (B*H, nq): one query stream per workgroup, forward walk: dq, and n, dn per
-//                        token into the workspace (plus sum(dout . o_i) for the lambda gradient).
+// kda_ref_bwd_q_kernel   grid (B*H, nq, segments): one query stream per workgroup, forward walk: dq, and n, dn per
+//                        token into the workspace (plus sum(dout . o_i) for the lambda gradient).  With few heads
+//                        the sequence is split (kda_split) and kda_sum_kernel forms the segments' states first.
 // kda_ref_bwd_segsum_kernel grid (nseg - 1, B*H): per sequence segment, its sum of adjoint-state
 //                        contributions, so that the segments' reverse walks run side by side.
 // kda_ref_bwd_kv_kernel  grid (nseg, B*H): reverse walk of one segment over the query streams (one combined
@@ -147,6 +148,8 @@ __device__ __forceinline__ float phic_f(float x) { return x > 0.f ? x : __expf(x
 
 }  // namespace
 
+// SPLIT: the workgroup walks segment blockIdx.z from the sums of the earlier segments (kda_sum_kernel, centered).
+template <bool SPLIT>
 __global__ __launch_bounds__(NT) void kda_ref_bwd_q_kernel(KdaBwdParams q) {
   __shared__ QSmem sm;
   const KdaParams& p = q.f;
@@ -157,6 +160,8 @@ __global__ __launch_bounds__(NT) void kda_ref_bwd_q_kernel(KdaBwdParams q) {
   const int tid = threadIdx.x;
   const int S = p.seqlen, kd = p.kernel_dim;
   const int64_t rowbase = (int64_t)bh * S;
+  const int seg = SPLIT ? blockIdx.z : 0;
+  const int p0 = SPLIT ? seg * p.seg_chunks * BC : 0, p1 = SPLIT ? min(S, p0 + p.seg_chunks * BC) : S;
   const bf16* qp = reinterpret_cast<const bf16*>(qi == 0 ? p.q1 : p.q2);
   const bf16* kp = reinterpret_cast<const bf16*>(p.k);
   const bf16* vp = reinterpret_cast<const bf16*>(p.v);
@@ -181,12 +186,30 @@ __global__ __launch_bounds__(NT) void kda_ref_bwd_q_kernel(KdaBwdParams q) {
   }
   if (tid < BD) {
     // an initial state enters S' and z' (Vsum = cnt = 0)
-    sm.z[0][tid] = p.init_z ? p.init_z[(int64_t)bh * BD + tid] : 0.f;
-    sm.vs[0][tid] = 0.f;
-    float c = 0.f;
+    float z = p.init_z ? p.init_z[(int64_t)bh * BD + tid] : 0.f, vs = 0.f, c = 0.f;
     if (p.init_state)
       for (int k = 0; k < kd; ++k) c += p.init_state[(int64_t)bh * BD * BD + k * BD + tid];
+    for (int j = 0; j < seg; ++j) {
+      const float* rec = p.seg_sum + ((int64_t)j * nbh + bh) * KDA_BWD_REC + BD * BD + tid;
+      z += rec[0];
+      vs += rec[BD];
+      c += rec[2 * BD];
+    }
+    sm.z[0][tid] = z;
+    sm.vs[0][tid] = vs;
     sm.cs[0][tid] = c;
+  }
+  for (int j = 0; j < seg; ++j) {
+    const float* rec = p.seg_sum + ((int64_t)j * nbh + bh) * KDA_BWD_REC;
+    float sv[2][16];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) sv[i][r] = rec[(32 * (2 * tt + i) + acc_row(half, r)) * BD + 32 * dt + l32];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) Sacc[i][r] += sv[i][r];
   }
   // lambda gradient pieces: sum dout . (o - Vsum / cnt) (cancellation-free: -R~_t / (n_t cnt_t)) and, once,
   // sum dout . Vsum / cnt (the same for both queries)
@@ -207,9 +230,9 @@ __global__ __launch_bounds__(NT) void kda_ref_bwd_q_kernel(KdaBwdParams q) {
       if (dop) td[i] = ld8(dop + r);
     }
   };
-  if (S > 0) load_tiles(0);
+  if (p0 < p1) load_tiles(p0);
 
-  for (int pos = 0, ci = 0; pos < S; pos += BC, ++ci) {
+  for (int pos = p0, ci = 0; pos < p1; pos += BC, ++ci) {
     const int len = min(BC, S - pos);
     const int zc = ci & 1;
     if (ci > 0 && tid < BD) {      // z', Vsum, column sums past the previous chunk (fixed-order sums)
@@ -282,7 +305,7 @@ __global__ __launch_bounds__(NT) void kda_ref_bwd_q_kernel(KdaBwdParams q) {
         *reinterpret_cast<bf16x4*>(&sm.SB[(32 * dt + l32) * P128 + 32 * (2 * tt + i) + 8 * g + 4 * half]) = v;
       }
     lds_barrier();
-    if (pos + BC < S) load_tiles(pos + BC);          // the staged registers are free: the next chunk flies all chunk
+    if (pos + BC < p1) load_tiles(pos + BC);          // the staged registers are free: the next chunk flies all chunk
 
     // ---- phase 1: A' tiles (t-block, s-block) = (0,0), (1,0), (1,1) by waves 0..2, computed transposed so
     // the row sums are lane-local; in-chunk prefix sums of K1 by wave 3; phi(q_t) . z' by waves 4..7.
@@ -511,8 +534,9 @@ __global__ __launch_bounds__(NT) void kda_ref_bwd_q_kernel(KdaBwdParams q) {
         s_ += sm.red[0][i];
         b_ += sm.red[1][i];
       }
-      q.lam_part[(int64_t)qi * nbh + bh] = s_;
-      if (qi == 0) q.lam_part[(int64_t)q.nq * nbh + bh] = b_;
+      const int64_t ns = SPLIT ? p.nseg : 1;
+      q.lam_part[(qi * ns + seg) * nbh + bh] = s_;
+      if (qi == 0) q.lam_part[(q.nq * ns + seg) * nbh + bh] = b_;
     }
   }
 }
@@ -894,6 +918,7 @@ __global__ __launch_bounds__(NT) void kda_ref_bwd_kv_kernel(KdaBwdParams q) {
 __global__ __launch_bounds__(256) void kda_ref_bwd_lam_kernel(KdaBwdParams q) {
   const KdaParams& p = q.f;
   const int nbh = p.batch * p.nheads;
+  const int64_t ns = p.nseg;                 // partials of each sum per (b, h)
   for (int h = threadIdx.x; h < p.nheads; h += 256) {
     const float lam = p.lam_h ? p.lam_h[h] : p.lam;
     const float c = 1.f / (1.f - lam + 1e-8f);
@@ -901,7 +926,11 @@ __global__ __launch_bounds__(256) void kda_ref_bwd_lam_kernel(KdaBwdParams q) {
     if (p.seqlen > 0)
       for (int b = 0; b < p.batch; ++b) {
         const int bh = b * p.nheads + h;
-        s += q.lam_part[bh] - (1.f + 1e-8f) * q.lam_part[nbh + bh] - 1e-8f * q.lam_part[2 * nbh + bh];
+        float t[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+          for (int j = 0; j < ns; ++j) t[i] += q.lam_part[(i * ns + j) * nbh + bh];
+        s += t[0] - (1.f + 1e-8f) * t[1] - 1e-8f * t[2];
       }
     q.dlam[h] = c * c * s;
   }
@@ -937,9 +966,23 @@ void kda_bwd_workspace_layout(KdaBwdParams& q, void* workspace) {
   q.segsum = q.lam_part + (size_t)(q.nq + 1) * nbh;
   q.nseg = kda_bwd_segments(q.f.batch, q.f.nheads, q.f.seqlen);
   const int nch = (q.f.seqlen + BC - 1) / BC;
+  // The query gradient's walk, grid B H x queries of one workgroup per CU, split where that leaves CUs idle (the fp32
+  // kernels walk each sequence at once).  Its records share the adjoint sums' space, which the key / value pass
+  // writes after it: 2 nseg - 1 of them fit behind the split lambda partials, and those lie in segment 0's own
+  // record, which is never formed.
+  q.f.nseg = 1;
+  q.f.seg_chunks = nch;
+  if (nch > 0 && !kda_precise_path(q.f))
+    kda_split((int64_t)nbh * q.nq, nch, min(16, 2 * q.nseg), q.f.nseg, q.f.seg_chunks);
+  if (q.f.nseg > 1) {
+    q.lam_part = q.segsum;
+    q.f.seg_sum = q.segsum + ((size_t)(q.nq + 1) * q.f.nseg * nbh + 3) / 4 * 4;
+  }
   q.seg_chunks = (nch + q.nseg - 1) / q.nseg;
   q.nseg = (nch + q.seg_chunks - 1) / q.seg_chunks;   // no empty trailing segment
 }
+static_assert(SEG_PARTS == 2 && 2 * 8 * (BD * BD + BD) >= (2 * 8 - 1) * KDA_BWD_REC + 3 * 16 + 3 &&
+              2 * (BD * BD + BD) >= KDA_BWD_REC + 3 * 2 + 3, "the walk's records fit the adjoint sums' space");
 
 hipError_t launch_kda_bwd(const KdaBwdParams& q, hipStream_t st) {
   const KdaParams& p = q.f;
@@ -951,8 +994,16 @@ hipError_t launch_kda_bwd(const KdaBwdParams& q, hipStream_t st) {
     hipError_t e = launch_kda_bwd_precise(q, st);
     if (e != hipSuccess) return e;
   } else {
-    hipLaunchKernelGGL(kda_ref_bwd_q_kernel, dim3((unsigned)nbh, (unsigned)q.nq), dim3(NT), 0, st, q);
-    hipError_t e = hipGetLastError();
+    hipError_t e = hipSuccess;
+    if (p.nseg > 1) {
+      e = launch_kda_centered_sums(p, st);
+      if (e != hipSuccess) return e;
+      hipLaunchKernelGGL(kda_ref_bwd_q_kernel<true>, dim3((unsigned)nbh, (unsigned)q.nq, (unsigned)p.nseg), dim3(NT), 0,
+                         st, q);
+    } else {
+      hipLaunchKernelGGL(kda_ref_bwd_q_kernel<false>, dim3((unsigned)nbh, (unsigned)q.nq), dim3(NT), 0, st, q);
+    }
+    e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (q.nseg > 1) {
       hipLaunchKernelGGL(kda_ref_bwd_segsum_kernel, dim3((unsigned)((q.nseg - 1) * SEG_PARTS), (unsigned)nbh),

@@ -66,6 +66,9 @@ struct KdaStage {
 
 }  // namespace
 
+// SPLIT: the workgroup walks segment blockIdx.y from the earlier segments' sums; without it the whole sequence (a
+// template, as the run-time bounds and the entering sums made the unsplit walk 0.7% slower).
+template <bool SPLIT>
 __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
   __shared__ KdaGatedSmem sm;
   using TQ = Tile<bf16, DK>;
@@ -88,6 +91,8 @@ __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
   const int S = p.seqlen;
   const float lam = p.lam_h ? p.lam_h[h] : p.lam;
   const int64_t rowbase = (int64_t)bh * S;          // token row index base in (B,H,S,*) tensors
+  const int seg = SPLIT ? blockIdx.y : 0;           // this workgroup's segment: tokens [p0, p1)
+  const int p0 = SPLIT ? seg * p.seg_chunks * SEG : 0, p1 = SPLIT ? min(S, p0 + p.seg_chunks * SEG) : S;
   const bf16* q1g = reinterpret_cast<const bf16*>(p.q1);
   const bf16* q2g = reinterpret_cast<const bf16*>(p.q2);
   const bf16* kg = reinterpret_cast<const bf16*>(p.k);
@@ -111,6 +116,22 @@ __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
         const int kr = 32 * (2 * kh + i) + acc_row(half, r);
         St[i][r] = s0[kr * 128 + v0 + 32 * vt + l32];
       }
+    }
+  }
+  // the state entering the segment: S <- e^{log-decay of segment j} S + (segment j's own sum), j in order
+  for (int j = 0; j < seg; ++j) {
+    const float* rec = p.seg_sum + ((int64_t)j * nbh + bh) * KDA_REC;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      float sv[16], ev[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int kr = 32 * (2 * kh + i) + acc_row(half, r);
+        sv[r] = rec[kr * 128 + v0 + 32 * vt + l32];
+        ev[r] = rec[128 * 128 + kr];
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) St[i][r] = St[i][r] * __expf(ev[r]) + sv[r];
     }
   }
 
@@ -140,10 +161,10 @@ __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
       }
     }
   };
-  load_gv(0);
-  load_qk(0);
+  load_gv(p0);
+  load_qk(p0);
 
-  for (int pos = 0; pos < S; pos += SEG) {
+  for (int pos = p0; pos < p1; pos += SEG) {
     const int len = min(SEG, S - pos);
     wait_vmem();                                         // this tile's registers
     *reinterpret_cast<uint4*>(&sm.V[TV::chunk(tid >> 3, tid & 7)]) = stg.v;
@@ -270,7 +291,7 @@ __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
         *reinterpret_cast<bf16x8*>(&sm.Kt[TQ::chunk(r, c8)]) = ko;
       }
       lds_barrier();                                     // Qt, Kt ready; G no longer read
-      const bool prefetch = last_window && pos + SEG < S;
+      const bool prefetch = last_window && pos + SEG < p1;
       if (prefetch) load_gv(pos + SEG);                  // the next tile streams in behind the MFMAs
 
       // ---- phase 1: A^T tiles (waves 5..7), the 12 operand transposes (waves 0..4), read-out partials
@@ -385,7 +406,7 @@ __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
     }
   }
 
-  if (p.final_state && tt == 0) {
+  if (p.final_state && tt == 0 && p1 == S) {
     float* sf_out = p.final_state + (int64_t)bh * DK * 128;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -506,6 +527,8 @@ __global__ __launch_bounds__(256 * NQ) void kda_ref_kernel(KdaParams p) {
   const float lam = p.lam_h ? p.lam_h[h] : p.lam;
   const float inv_1ml = 1.f / (1.f - lam + 1e-8f);
   const int64_t rowbase = (int64_t)bh * S;
+  const int seg = blockIdx.y;                       // this workgroup's segment: tokens [p0, p1)
+  const int p0 = seg * p.seg_chunks * SEGK, p1 = min(S, p0 + p.seg_chunks * SEGK);
   const bf16* const qp[2] = {reinterpret_cast<const bf16*>(p.q1), reinterpret_cast<const bf16*>(p.q2)};
   const bf16* kk = reinterpret_cast<const bf16*>(p.k);
   const bf16* vv = reinterpret_cast<const bf16*>(p.v);
@@ -525,12 +548,29 @@ __global__ __launch_bounds__(256 * NQ) void kda_ref_kernel(KdaParams p) {
       }
     }
   }
-  if (tid < DK) sm.z[tid] = p.init_z ? p.init_z[(int64_t)bh * DK + tid] : 0.f;
+  // the state and normaliser entering the segment: plus the earlier segments' sums, in order
+  for (int j = 0; j < seg; ++j) {
+    const float* rec = p.seg_sum + ((int64_t)j * nbh + bh) * KDA_REC;
+    float sv[2][16];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) sv[i][r] = rec[(32 * (2 * kh + i) + acc_row(half, r)) * 128 + v0 + 32 * vt + l32];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) St[i][r] += sv[i][r];
+  }
+  if (tid < DK) {
+    float z = p.init_z ? p.init_z[(int64_t)bh * DK + tid] : 0.f;
+    for (int j = 0; j < seg; ++j) z += p.seg_sum[((int64_t)j * nbh + bh) * KDA_REC + 128 * 128 + tid];
+    sm.z[tid] = z;
+  }
 
   static_assert(SEGK * (DK / 8) == KC * NT && SEGK * (DVH / 8) == VC * NT, "staging covers a segment");
   KdaRefStage<NQ> stg;
-  if (S > 0) kda_ref_load<NQ>(stg, qp, kk, vv, rowbase, 0, min(SEGK, S), v0, tid);
-  for (int pos = 0; pos < S; pos += SEGK) {
+  if (p0 < p1) kda_ref_load<NQ>(stg, qp, kk, vv, rowbase, p0, min(SEGK, S - p0), v0, tid);
+  for (int pos = p0; pos < p1; pos += SEGK) {
     const int len = min(SEGK, S - pos);
     // ---- phase B: phi(q_i), phi(k), v tiles from the staged rows; then stage the next segment's rows
     auto stage = [&](auto MASKc) {     // MASK: zero tokens past the segment end and channels past kernel_dim
@@ -569,7 +609,7 @@ __global__ __launch_bounds__(256 * NQ) void kda_ref_kernel(KdaParams p) {
       const int t = e >> 3, c0 = (e & 7) * 8;
       *reinterpret_cast<uint4*>(&sm.V[t * SM::PV + c0]) = stg.v[ie];
     }
-    if (pos + SEGK < S) kda_ref_load<NQ>(stg, qp, kk, vv, rowbase, pos + SEGK, min(SEGK, S - pos - SEGK), v0, tid);
+    if (pos + SEGK < p1) kda_ref_load<NQ>(stg, qp, kk, vv, rowbase, pos + SEGK, min(SEGK, S - pos - SEGK), v0, tid);
     __syncthreads();
 
     // ---- phase B2: phi(q_i,t) . z_prev  (4 adjacent lanes per (query, token), 32 channels each: one item
@@ -736,7 +776,7 @@ __global__ __launch_bounds__(256 * NQ) void kda_ref_kernel(KdaParams p) {
     }
   }
 
-  if (p.final_state && qw == 0) {
+  if (p.final_state && qw == 0 && p1 == S) {
     float* sf_out = p.final_state + (int64_t)bh * DK * 128;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -746,10 +786,254 @@ __global__ __launch_bounds__(256 * NQ) void kda_ref_kernel(KdaParams p) {
         sf_out[kr * 128 + v0 + 32 * vt + l32] = St[i][r];
       }
   }
-  if (p.final_z && vh == 0 && tid < DK) p.final_z[(int64_t)bh * DK + tid] = sm.z[tid];
+  if (p.final_z && vh == 0 && tid < DK && p1 == S) p.final_z[(int64_t)bh * DK + tid] = sm.z[tid];
 }
 
-hipError_t launch_kda(const KdaParams& p, hipStream_t st) {
+// ---------------------------------------------------------------------------
+// Sequence split.  A scan of B H heads is 2 B H workgroups of one per CU (LDS), so fewer than 128 heads leave CUs
+// idle for the whole serial walk.  The sequence of each (b, h) is then cut into segments of whole chunks that walk
+// side by side; kda_sum_kernel first forms each segment's own contribution to the state, and a segment starts from
+// the sum of the earlier ones (gated: S <- e^{sum g} S + S_j).  The sums cost one product per chunk where the walk
+// has the staging of the queries, the masked tiles, the read-out and the output besides.
+// ---------------------------------------------------------------------------
+namespace {
+
+enum { SUM_GATED = 0, SUM_PHI = 1, SUM_CENTERED = 2 };
+
+template <int MODE>
+struct KdaSumSmem {
+  static constexpr int NB = MODE == SUM_GATED ? 1 : 2;    // buffers
+  static constexpr int PK = DK + 24, PV = DVH + 32;       // pitches of KdaRefSmem
+  bf16 K[NB][SEGK * PK];        // phi(k), phi'(k) or e^{G_end - G_s} k_s
+  bf16 V[NB][SEGK * PV];
+  alignas(16) float W[MODE == SUM_GATED ? SEGK : 1][DK];   // e^{G_end - G_s}
+  float qtot[4][DK], eg[DK];    // gated: token-quarter sums of g, e^{sum of the chunk}
+  float k1[2][SEGK];            // centered: sum_k phi'(k_s)
+  float red[3][8][DK];          // per-wave partials of the vector sums
+};
+
+// grid (2 nbh, nseg - 1): segment blockIdx.y of (b, h, V-half).  8 waves, one 32x32 state tile each (k-tile w & 3,
+// v-tile w >> 2).  Every segment but the last is whole chunks, so no row is masked.
+template <int MODE>
+__global__ __launch_bounds__(512) void kda_sum_kernel(KdaParams p) {
+  using SM = KdaSumSmem<MODE>;
+  __shared__ SM sm;
+  const int nbh = p.batch * p.nheads;
+  int bh, vh;
+  const int L = blockIdx.x;
+  if ((nbh & 7) == 0) {               // both V-halves of a (b, h) on one XCD, as the scan kernels
+    bh = (L & 7) | ((L >> 4) << 3);
+    vh = (L >> 3) & 1;
+  } else {
+    bh = L >> 1;
+    vh = L & 1;
+  }
+  const int w = wave_id(), l = lane_id(), half = l >> 5, l32 = l & 31, tid = threadIdx.x;
+  const int kt = w & 3, vt = w >> 2;
+  const int seg = blockIdx.y;
+  const int64_t row0 = (int64_t)bh * p.seqlen + (int64_t)seg * p.seg_chunks * SEGK;
+  const int nch = p.seg_chunks, kd = p.kernel_dim;
+  const int c8 = tid & 15, kr = tid >> 4;                // k rows kr, kr + 32, columns 8 c8 ..
+  const int v8 = tid & 7, vr = tid >> 3;                 // v row vr, columns 8 v8 .. of the half
+  const int kc = tid & (DK - 1), qq = tid >> 7;          // gated: channel, token quarter
+  const bf16* kp = reinterpret_cast<const bf16*>(p.k) + (row0 + kr) * DK + 8 * c8;
+  const bf16* vp = reinterpret_cast<const bf16*>(p.v) + (row0 + vr) * 128 + vh * DVH + 8 * v8;
+  const float* gp = MODE == SUM_GATED && p.g ? p.g + (row0 + 16 * qq) * DK + kc : nullptr;
+
+  bf16x8 ks[2], vs;
+  float gs[16];
+  auto load = [&](int c) {
+    const int64_t o = (int64_t)c * SEGK * DK;
+    ks[0] = *reinterpret_cast<const bf16x8*>(kp + o);
+    ks[1] = *reinterpret_cast<const bf16x8*>(kp + o + 32 * DK);
+    vs = *reinterpret_cast<const bf16x8*>(vp + o);
+    if constexpr (MODE == SUM_GATED) {
+      if (gp) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) gs[i] = gp[o + i * DK];
+      }
+    }
+  };
+  if constexpr (MODE == SUM_GATED) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) gs[i] = 0.f;
+  }
+  load(0);
+  f32x16 acc = zero16();
+  float z8[8], s8[8], t8[8];          // sums of phi(k) (this thread's channels), of v and K1 v (its columns)
+#pragma unroll
+  for (int j = 0; j < 8; ++j) z8[j] = s8[j] = t8[j] = 0.f;
+  float gtot = 0.f;
+
+  for (int c = 0; c < nch; ++c) {
+    const int b = MODE == SUM_GATED ? 0 : c & 1;
+    bf16x8 vcur = vs;
+    if constexpr (MODE == SUM_GATED) {
+      float suf[16], run = 0.f;                          // sum of the later tokens' g within the quarter
+#pragma unroll
+      for (int i = 15; i >= 0; --i) {
+        suf[i] = run;
+        run += gs[i];
+      }
+      sm.qtot[qq][kc] = run;
+      lds_barrier();                                     // also: the previous chunk's tiles are read
+      float off = 0.f, tot = 0.f;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float t = sm.qtot[q][kc];
+        if (q > qq) off += t;
+        tot += t;
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sm.W[16 * qq + i][kc] = __expf(suf[i] + off);
+      if (qq == 0) {
+        sm.eg[kc] = __expf(tot);
+        gtot += tot;
+      }
+      lds_barrier();                                     // W
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const f32x4 w0 = *reinterpret_cast<const f32x4*>(&sm.W[kr + 32 * u][8 * c8]);
+        const f32x4 w1 = *reinterpret_cast<const f32x4*>(&sm.W[kr + 32 * u][8 * c8 + 4]);
+        bf16x8 ko;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) ko[j] = (bf16)((float)ks[u][j] * (j < 4 ? w0[j] : w1[j - 4]));
+        *reinterpret_cast<bf16x8*>(&sm.K[b][(kr + 32 * u) * SM::PK + 8 * c8]) = ko;
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        bf16x8 ko;
+        float ksum = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float x = (float)ks[u][j];
+          const float e = __expf(x);
+          float f = MODE == SUM_CENTERED ? (x > 0.f ? x : e - 1.f) : (x > 0.f ? x + 1.f : e);
+          f = 8 * c8 + j < kd ? f : 0.f;
+          ko[j] = (bf16)f;
+          z8[j] += (float)ko[j];
+          ksum += f;
+        }
+        *reinterpret_cast<bf16x8*>(&sm.K[b][(kr + 32 * u) * SM::PK + 8 * c8]) = ko;
+        if constexpr (MODE == SUM_CENTERED) {
+          // the token's 16 chunks are one 16-lane row: prefix sums on the DPP crossbar, the total in its last lane
+          ksum += dppf<0x111>(ksum);
+          ksum += dppf<0x112>(ksum);
+          ksum += dppf<0x114>(ksum);
+          ksum += dppf<0x118>(ksum);
+          if (c8 == 15) sm.k1[b][kr + 32 * u] = ksum;
+        }
+      }
+    }
+    *reinterpret_cast<bf16x8*>(&sm.V[b][vr * SM::PV + 8 * v8]) = vcur;
+    if (c + 1 < nch) load(c + 1);
+    lds_barrier();                                       // the chunk's tiles
+    if constexpr (MODE == SUM_CENTERED) {
+      const float k1 = sm.k1[b][vr];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float v = (float)vcur[j];
+        s8[j] += v;
+        t8[j] += k1 * v;
+      }
+    }
+    if constexpr (MODE == SUM_GATED) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const f32x4 e4 = *reinterpret_cast<const f32x4*>(&sm.eg[32 * kt + 8 * q + 4 * half]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[4 * q + j] *= e4[j];
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < SEGK / 16; ++s)
+      acc = mma(col_frag_tr(sm.K[b], SM::PK, 32 * kt, 16 * s), col_frag_tr(sm.V[b], SM::PV, 32 * vt, 16 * s), acc);
+  }
+
+  constexpr int REC = MODE == SUM_CENTERED ? KDA_BWD_REC : KDA_REC;
+  float* rec = p.seg_sum + ((int64_t)seg * nbh + bh) * REC;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) rec[(32 * kt + acc_row(half, r)) * 128 + vh * DVH + 32 * vt + l32] = acc[r];
+  if constexpr (MODE == SUM_GATED) {
+    if (vh == 0 && qq == 0) rec[128 * 128 + kc] = gtot;
+  } else {
+    // the vector sums: over a wave's token rows by shuffles, over the waves through LDS in wave order
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      z8[j] += __shfl_xor(z8[j], 16, 64);
+      z8[j] = sum_halves(z8[j]);
+      if constexpr (MODE == SUM_CENTERED) {
+        s8[j] += __shfl_xor(s8[j], 8, 64);
+        s8[j] += __shfl_xor(s8[j], 16, 64);
+        s8[j] = sum_halves(s8[j]);
+        t8[j] += __shfl_xor(t8[j], 8, 64);
+        t8[j] += __shfl_xor(t8[j], 16, 64);
+        t8[j] = sum_halves(t8[j]);
+      }
+      if (l < 16) sm.red[0][w][8 * c8 + j] = z8[j];
+      if (MODE == SUM_CENTERED && l < 8) {
+        sm.red[1][w][8 * v8 + j] = s8[j];
+        sm.red[2][w][8 * v8 + j] = t8[j];
+      }
+    }
+    lds_barrier();
+    auto total = [&](int m, int i) {
+      float a = 0.f;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) a += sm.red[m][q][i];
+      return a;
+    };
+    if (vh == 0 && tid < DK) rec[128 * 128 + tid] = total(0, tid);
+    if (MODE == SUM_CENTERED && tid >= 128 && tid < 128 + 2 * DVH) {
+      const int m = 1 + (tid - 128) / DVH, i = tid & (DVH - 1);
+      rec[128 * 128 + 128 * m + vh * DVH + i] = total(m, i);
+    }
+  }
+}
+
+}  // namespace
+
+void kda_split(int64_t units, int nch, int most, int& nseg, int& seg_chunks) {
+  // In chunk times of the walk (about 5 us), fitted to both scans at 16 to 192 workgroups and 200 to 8192 tokens: a
+  // round of 256 workgroups takes its segments' chunks plus two (the first loads, the entering sums, the drain); the
+  // sums, two workgroups per CU, a third of that; the second launch one.  B1 H16 S1500 (reference mode): 8 segments
+  // 29 us, unsplit 114; B1 H16 S200: 4 segments 13.5, unsplit 21.9; B2 H32 S4096: 4 segments 212, unsplit 324;
+  // B2 H48 S2048, unsplit by this rule: 157, 8 segments 184.
+  float best = 1e30f;
+  nseg = 1;
+  seg_chunks = nch;
+  for (int s = 1; s <= most && s <= nch; ++s) {
+    const int per = (nch + s - 1) / s;
+    if ((nch + per - 1) / per != s) continue;            // the same segments as a smaller s
+    float t = (float)((units * s + 255) / 256) * (per + 2);
+    if (s > 1) t += 0.35f * (float)((units * (s - 1) + 511) / 512) * (per + 2) + 1.f;
+    if (t < best) {
+      best = t;
+      nseg = s;
+      seg_chunks = per;
+    }
+  }
+}
+
+size_t kda_plan_segments(KdaParams& p) {
+  const int nch = (p.seqlen + SEGK - 1) / SEGK;
+  const int64_t nbh = (int64_t)p.batch * p.nheads;
+  p.nseg = 1;
+  p.seg_chunks = nch;
+  if (nch == 0 || kda_precise_path(p)) return 0;
+  kda_split(2 * nbh, nch, 16, p.nseg, p.seg_chunks);
+  return p.nseg > 1 ? (size_t)(p.nseg - 1) * nbh * KDA_REC * sizeof(float) : 0;
+}
+
+hipError_t launch_kda_centered_sums(const KdaParams& p, hipStream_t st) {
+  hipLaunchKernelGGL(kda_sum_kernel<SUM_CENTERED>, dim3((unsigned)(2 * p.batch * p.nheads), (unsigned)(p.nseg - 1)),
+                     dim3(512), 0, st, p);
+  return hipGetLastError();
+}
+
+hipError_t launch_kda(const KdaParams& p_, hipStream_t st) {
+  KdaParams p = p_;
   const int nbh = p.batch * p.nheads;
   if (p.seqlen == 0) {
     const size_t ns = p.final_state ? (size_t)nbh * p.dk * p.dv : 0, nz = p.final_z ? (size_t)nbh * p.dk : 0;
@@ -759,9 +1043,20 @@ hipError_t launch_kda(const KdaParams& p, hipStream_t st) {
     return hipGetLastError();
   }
   if (kda_precise_path(p)) return launch_kda_precise(p, st);
-  const dim3 grid((unsigned)(2 * nbh));
+  if (!p.seg_sum || p.nseg <= 1) {
+    p.nseg = 1;
+    p.seg_chunks = (p.seqlen + SEGK - 1) / SEGK;
+  } else {
+    const dim3 sgrid((unsigned)(2 * nbh), (unsigned)(p.nseg - 1));
+    if (p.mode == 0) hipLaunchKernelGGL(kda_sum_kernel<SUM_GATED>, sgrid, dim3(512), 0, st, p);
+    else hipLaunchKernelGGL(kda_sum_kernel<SUM_PHI>, sgrid, dim3(512), 0, st, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  const dim3 grid((unsigned)(2 * nbh), (unsigned)p.nseg);
   if (p.mode == 0) {
-    hipLaunchKernelGGL(kda_gated_kernel, grid, dim3(64 * KW), 0, st, p);
+    if (p.nseg > 1) hipLaunchKernelGGL(kda_gated_kernel<true>, grid, dim3(64 * KW), 0, st, p);
+    else hipLaunchKernelGGL(kda_gated_kernel<false>, grid, dim3(64 * KW), 0, st, p);
   } else if (p.q2) {
     hipLaunchKernelGGL(kda_ref_kernel<2>, grid, dim3(kda_ref_threads<2>), 0, st, p);
   } else {

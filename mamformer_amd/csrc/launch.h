@@ -184,8 +184,22 @@ struct KdaParams {
   float* final_z;            // reference mode: (B,H,dk) or null
   void* o;                   // gated: o; reference: o1
   void* o2;                  // reference: o2
+  // sequence split (kda_scan.hip): nseg segments of seg_chunks 64-token chunks walk side by side, each from the
+  // sums of the segments before it (seg_sum, nseg - 1 records per (b, h)); nseg <= 1 walks the sequence at once
+  int nseg, seg_chunks;
+  float* seg_sum;
 };
 hipError_t launch_kda(const KdaParams& p, hipStream_t st);
+// Segments and workspace of a split scan for p's sizes: sets p.nseg and p.seg_chunks, returns the workspace's bytes
+// (0: the scan is not split).
+size_t kda_plan_segments(KdaParams& p);
+// Segment count (at most `most`) and chunks per segment for `units` workgroups (one per CU) that each walk nch chunks.
+void kda_split(int64_t units, int nch, int most, int& nseg, int& seg_chunks);
+// Sums of phi'(k)^T v, phi'(k), v and K1 v over each of segments 0 .. nseg - 2 (the query gradient's walk), records
+// of KDA_BWD_REC floats per (segment, b, h).
+constexpr int KDA_REC = 128 * 128 + 128;          // a forward segment's record: state sum, then z sum or log-decay
+constexpr int KDA_BWD_REC = 128 * 128 + 3 * 128;  // S', z', Vsum, column sums of S'
+hipError_t launch_kda_centered_sums(const KdaParams& p, hipStream_t st);
 
 // Backward of the reference-mode scan (kda_backward.hip).
 struct KdaBwdParams {
@@ -203,6 +217,7 @@ struct KdaBwdParams {
   float* lam_part;           // workspace: sum dout . o_i per (query, b, h)
   float* segsum;             // workspace: per (segment, b, h) adjoint-state sums (dk*dv + dk floats)
   int nseg, seg_chunks;      // kv-walk segments per (b, h) and 64-token chunks per segment
+                             // (f.nseg, f.seg_chunks, f.seg_sum: the query gradient's walk)
 };
 hipError_t launch_kda_bwd(const KdaBwdParams& q, hipStream_t st);
 // fp32-arithmetic kernels (kda_precise.hip) for everything but bf16 with dk = dv = 128; launch_kda and

@@ -1184,6 +1184,20 @@ def plan_selective_scan_reference(*args, **kw):
     return selective_scan_reference(*args, _plan_only=True, **kw)
 
 
+class _KdaPlan(Plan):
+    """``Plan`` of ``mh_kda_chunk_scan_fwd_ws``, whose workspace (None: the sequence is not split) is an argument of
+    its own."""
+
+    def __init__(self, args, ws, device, keep=(), **outputs):
+        super().__init__("mh_kda_chunk_scan_fwd_ws", args, device, keep, **outputs)
+        self._ws, self._ws_bytes = ws, 0 if ws is None else ws.numel()
+
+    def __call__(self, stream=None):
+        s = _stream(self._device) if stream is None else ct.c_void_p(stream)
+        _lib.call(self._fn, ct.byref(self._args), _ptr(self._ws), self._ws_bytes, s)
+        return self
+
+
 def plan_linear_attn_scan(*args, **kw):
     """``Plan`` of ``linear_attn_scan`` on fixed buffers (outputs ``o``, ``o2``, ``final_state``, ``final_z``)."""
     return linear_attn_scan(*args, _plan_only=True, **kw)
@@ -1276,8 +1290,11 @@ def linear_attn_scan(q1, q2, k, v, *, g=None, lam=0.8, mode="gated", kernel_dim=
     a.initial_state, a.final_state = _ptr(s0), _ptr(fin)
     a.initial_z, a.final_z = _ptr(z0), _ptr(finz)
     a.o, a.o2 = _ptr(o), _ptr(o2)
-    plan = Plan("mh_kda_chunk_scan_fwd", a, q1.device, keep=(q1c, q2c, kc, vc, gc, lam_h, s0, z0),
-                o=o, o2=o2, final_state=fin, final_z=finz)
+    n = ct.c_size_t()
+    _lib.call("mh_kda_workspace_bytes", ct.byref(a), ct.byref(n))
+    ws = torch.empty(n.value, device=q1.device, dtype=torch.uint8) if n.value else None
+    plan = _KdaPlan(a, ws, q1.device, keep=(q1c, q2c, kc, vc, gc, lam_h, s0, z0),
+                    o=o, o2=o2, final_state=fin, final_z=finz)
     if _plan_only:
         return plan
     plan()
