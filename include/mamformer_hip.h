@@ -299,12 +299,20 @@ typedef struct {
 
 int mh_kda_chunk_scan_fwd(const mh_kda_args* a, void* stream);
 
-/* The same with a workspace, which lets a scan of few heads split its sequence
+/* lam_per_head holds lambda_raw: lambda = min(sigmoid(lambda_raw), 0.99), the
+ * reference's parameterisation (mamformer/layers/kda_diff.py:473-474; reference mode
+ * only).  A flag of
+ * mh_kda_chunk_scan_fwd_ws, mh_kda_bwd_args (d_lam is then w.r.t. lambda_raw) and
+ * mh_kda_step_args. */
+enum { MH_KDA_LAM_RAW = 2 };
+
+/* The same with flags (MH_KDA_LAM_RAW or 0) and a workspace, which lets a scan of few heads split its sequence
  * over the compute units: mh_kda_workspace_bytes gives the bytes (0 where these
  * sizes gain nothing; workspace NULL walks each sequence at once, as
  * mh_kda_chunk_scan_fwd does). */
 int mh_kda_workspace_bytes(const mh_kda_args* a, size_t* bytes);
-int mh_kda_chunk_scan_fwd_ws(const mh_kda_args* a, void* workspace, size_t workspace_bytes, void* stream);
+int mh_kda_chunk_scan_fwd_ws(const mh_kda_args* a, int32_t flags, void* workspace, size_t workspace_bytes,
+                             void* stream);
 
 /* Backward of the reference-mode scan (fwd.mode == MH_KDA_REFERENCE): the
  *   gradient PyTorch autograd forms through LinearDiffAttention._linear_attention_scan
@@ -367,6 +375,10 @@ typedef struct {
 } mh_kda_step_args;
 
 int mh_kda_recurrent_step(const mh_kda_step_args* a, void* stream);
+
+/* The same into other buffers: a->state and a->z are read only, the updated state
+ * and z go to state_out and z_out (each NULL: not kept; the input itself: in place). */
+int mh_kda_recurrent_step_to(const mh_kda_step_args* a, float* state_out, float* z_out, void* stream);
 
 /* ------------------------------------------------------------------------
  * Causal depthwise conv1d (+ optional SiLU), the Mamba layer prologue.

@@ -21,6 +21,7 @@ MH_F32, MH_BF16 = 0, 1
 MH_DT_SOFTPLUS, MH_DT_LIMIT, MH_D_PER_CHANNEL, MH_A_PER_STATE, MH_DT_PER_CHANNEL = 1, 2, 4, 8, 16
 MH_KDA_GATED, MH_KDA_REFERENCE = 0, 1
 MH_KDA_PHI = 1
+MH_KDA_LAM_RAW = 2
 
 ERRORS = {
     -1: "MH_ERR_NULL", -2: "MH_ERR_SHAPE", -3: "MH_ERR_DTYPE", -4: "MH_ERR_STRIDE",
@@ -187,7 +188,7 @@ EXPORTS = (
     "mh_silu_gate_fwd", "mh_silu_gate_bwd",
     "mh_ssd_state_update",
     "mh_kda_chunk_scan_fwd", "mh_kda_workspace_bytes", "mh_kda_chunk_scan_fwd_ws", "mh_kda_bwd_workspace_bytes", "mh_kda_chunk_scan_bwd",
-    "mh_kda_recurrent_step",
+    "mh_kda_recurrent_step", "mh_kda_recurrent_step_to",
     "mh_causal_conv1d_fwd",
     "mh_conv1d_bwd_workspace_bytes", "mh_causal_conv1d_bwd",
 )
@@ -237,7 +238,8 @@ def lib():
             h.mh_silu_gate_bwd.argtypes = [ct.POINTER(GateArgs), _vp]
             h.mh_kda_chunk_scan_fwd.argtypes = [ct.POINTER(KdaArgs), _vp]
             h.mh_kda_workspace_bytes.argtypes = [ct.POINTER(KdaArgs), ct.POINTER(_sz)]
-            h.mh_kda_chunk_scan_fwd_ws.argtypes = [ct.POINTER(KdaArgs), _vp, _sz, _vp]
+            h.mh_kda_chunk_scan_fwd_ws.argtypes = [ct.POINTER(KdaArgs), _i32, _vp, _sz, _vp]
+            h.mh_kda_recurrent_step_to.argtypes = [ct.POINTER(KdaStepArgs), _vp, _vp, _vp]
             h.mh_kda_recurrent_step.argtypes = [ct.POINTER(KdaStepArgs), _vp]
             h.mh_kda_bwd_workspace_bytes.argtypes = [ct.POINTER(KdaBwdArgs), ct.POINTER(_sz)]
             h.mh_kda_chunk_scan_bwd.argtypes = [ct.POINTER(KdaBwdArgs), _vp]
@@ -247,7 +249,7 @@ def lib():
             for name in ("mh_ssd_workspace_bytes", "mh_ssd_chunk_len", "mh_ssd_chunk_scan_fwd",
                          "mh_ssd_chunk_scan_fwd_noalloc",
                          "mh_ssd_state_update", "mh_kda_chunk_scan_fwd", "mh_kda_workspace_bytes",
-                         "mh_kda_chunk_scan_fwd_ws", "mh_kda_recurrent_step",
+                         "mh_kda_chunk_scan_fwd_ws", "mh_kda_recurrent_step", "mh_kda_recurrent_step_to",
                          "mh_causal_conv1d_fwd", "mh_conv1d_bwd_workspace_bytes", "mh_causal_conv1d_bwd",
                          "mh_ssd_bwd_workspace_bytes", "mh_ssd_chunk_scan_bwd",
                          "mh_kda_bwd_workspace_bytes", "mh_kda_chunk_scan_bwd",

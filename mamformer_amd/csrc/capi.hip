@@ -675,7 +675,7 @@ int kda_bwd_validate(const mh_kda_bwd_args* a) {
   if (f.mode != MH_KDA_REFERENCE)
     return fail(MH_ERR_UNSUPPORTED, "kda_bwd: only the reference mode has a backward (the gated operator has no "
                                     "reference training path)");
-  if (a->flags & ~MH_KDA_BWD_DIFF) return fail(MH_ERR_UNSUPPORTED, "kda_bwd: unknown flags 0x%x", a->flags);
+  if (a->flags & ~(MH_KDA_BWD_DIFF | MH_KDA_LAM_RAW)) return fail(MH_ERR_UNSUPPORTED, "kda_bwd: unknown flags 0x%x", a->flags);
   const bool diff = (a->flags & MH_KDA_BWD_DIFF) != 0;
   if (diff && !f.q2 && f.seqlen > 0) return fail(MH_ERR_NULL, "kda_bwd: the differential output needs q2");
   if (diff && a->do2) return fail(MH_ERR_SHAPE, "kda_bwd: do2 is not used with the differential output");
@@ -1053,7 +1053,7 @@ int mh_ssd_state_update(const mh_ssu_args* a, void* stream) {
 }
 
 int mh_kda_chunk_scan_fwd(const mh_kda_args* a, void* stream) {
-  return mh_kda_chunk_scan_fwd_ws(a, nullptr, 0, stream);
+  return mh_kda_chunk_scan_fwd_ws(a, 0, nullptr, 0, stream);
 }
 
 int mh_kda_workspace_bytes(const mh_kda_args* a, size_t* bytes) {
@@ -1066,11 +1066,16 @@ int mh_kda_workspace_bytes(const mh_kda_args* a, size_t* bytes) {
   return MH_OK;
 }
 
-int mh_kda_chunk_scan_fwd_ws(const mh_kda_args* a, void* workspace, size_t workspace_bytes, void* stream) {
+int mh_kda_chunk_scan_fwd_ws(const mh_kda_args* a, int32_t flags, void* workspace, size_t workspace_bytes,
+                             void* stream) {
   int rc = kda_validate(a);
   if (rc) return rc;
+  if (flags & ~MH_KDA_LAM_RAW) return fail(MH_ERR_UNSUPPORTED, "kda: unknown flags 0x%x", flags);
+  if (flags && a->mode != MH_KDA_REFERENCE)
+    return fail(MH_ERR_UNSUPPORTED, "kda: MH_KDA_LAM_RAW belongs to the reference mode");
   mh::KdaParams p;
   kda_fill(a, p);
+  p.lam_raw = (flags & MH_KDA_LAM_RAW) != 0;
   if (workspace) {
     const size_t need = mh::kda_plan_segments(p);
     if (need > 0 && (workspace_bytes < need || !aligned16(workspace)))
@@ -1102,6 +1107,7 @@ int mh_kda_chunk_scan_bwd(const mh_kda_bwd_args* a, void* stream) {
   mh::KdaBwdParams q;
   memset(&q, 0, sizeof(q));
   kda_fill(f, q.f);
+  q.f.lam_raw = (a->flags & MH_KDA_LAM_RAW) != 0;
   q.f.o = nullptr; q.f.o2 = nullptr; q.f.final_state = nullptr; q.f.final_z = nullptr;
   q.nq = nq;
   q.diff = (a->flags & MH_KDA_BWD_DIFF) != 0;
@@ -1115,16 +1121,21 @@ int mh_kda_chunk_scan_bwd(const mh_kda_bwd_args* a, void* stream) {
 }
 
 int mh_kda_recurrent_step(const mh_kda_step_args* a, void* stream) {
+  return mh_kda_recurrent_step_to(a, a ? a->state : nullptr, a ? a->z : nullptr, stream);
+}
+
+int mh_kda_recurrent_step_to(const mh_kda_step_args* a, float* state_out, float* z_out, void* stream) {
   int rc = kda_step_validate(a);
   if (rc) return rc;
+  if (state_out && !aligned16(state_out)) return fail(MH_ERR_ALIGN, "kda_step: state_out must be 16-byte aligned");
   mh::KdaStepParams p;
   memset(&p, 0, sizeof(p));
   p.batch = (int)a->batch; p.nheads = (int)a->nheads; p.dk = (int)a->dk; p.dv = (int)a->dv; p.dtype = a->dtype;
   p.apply_phi = (a->flags & MH_KDA_PHI) != 0;
   p.kernel_dim = p.apply_phi ? (a->kernel_dim < (int32_t)a->dk ? a->kernel_dim : (int32_t)a->dk) : (int)a->dk;
-  p.lam = a->lam; p.lam_h = a->lam_per_head;
+  p.lam = a->lam; p.lam_h = a->lam_per_head; p.lam_raw = (a->flags & MH_KDA_LAM_RAW) != 0;
   p.q1 = a->q1; p.q2 = a->q2; p.k = a->k; p.v = a->v;
-  p.state = a->state; p.z = a->z; p.o = a->o; p.o2 = a->o2;
+  p.state_in = a->state; p.z_in = a->z; p.state = state_out; p.z = z_out; p.o = a->o; p.o2 = a->o2;
   return hip_status(mh::launch_kda_step(p, reinterpret_cast<hipStream_t>(stream)), "kda_recurrent_step");
 }
 

@@ -238,4 +238,14 @@ __device__ __forceinline__ float silu_f(float x) { return x * __builtin_amdgcn_r
 // sigmoid(x) = 1 / (1 + e^{-x}) through the same reciprocal (0 for e^{-x} = +inf).
 __device__ __forceinline__ float sigmoid_f(float x) { return __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
 
+// The differential combination's lambda of head h: a scalar, a value per head, or (raw) min(sigmoid(x), 0.99) of a
+// per-head x, the reference's parameterisation (mamformer/layers/kda_diff.py:473-474); a NaN stays one.
+__device__ __forceinline__ float kda_lambda(const float* lam_h, float lam, int raw, int h) {
+  if (!lam_h) return lam;
+  const float x = lam_h[h];
+  if (!raw) return x;
+  const float s = 1.f / (1.f + expf(-x));
+  return s > 0.99f ? 0.99f : s;
+}
+
 }  // namespace mh

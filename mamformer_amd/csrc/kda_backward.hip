@@ -136,7 +136,7 @@ struct KVSmem {
 __device__ __forceinline__ void query_coef(const KdaBwdParams& q, int h, int qi, float& coef) {
   coef = 1.f;
   if (q.diff) {
-    const float lam = q.f.lam_h ? q.f.lam_h[h] : q.f.lam;
+    const float lam = kda_lambda(q.f.lam_h, q.f.lam, q.f.lam_raw, h);
     const float c = 1.f / (1.f - lam + 1e-8f);
     coef = qi == 0 ? c : -lam * c;
   }
@@ -914,13 +914,14 @@ __global__ __launch_bounds__(NT) void kda_ref_bwd_kv_kernel(KdaBwdParams q) {
 
 // d lambda_h = sum_b c^2 (sum dout . o1 - (1 + 1e-8) sum dout . o2),  c = 1 / (1 - lambda_h + 1e-8):
 // the derivative of (o1 - lam o2) / (1 - lam + 1e-8) (kda_diff.py:473-478), summed in a fixed order from
-// P_i = sum dout . (o_i - Vsum / cnt) and B = sum dout . Vsum / cnt:  P1 - (1 + 1e-8) P2 - 1e-8 B.
+// P_i = sum dout . (o_i - Vsum / cnt) and B = sum dout . Vsum / cnt:  P1 - (1 + 1e-8) P2 - 1e-8 B.  With lam_raw
+// the gradient of lambda_raw.
 __global__ __launch_bounds__(256) void kda_ref_bwd_lam_kernel(KdaBwdParams q) {
   const KdaParams& p = q.f;
   const int nbh = p.batch * p.nheads;
   const int64_t ns = p.nseg;                 // partials of each sum per (b, h)
   for (int h = threadIdx.x; h < p.nheads; h += 256) {
-    const float lam = p.lam_h ? p.lam_h[h] : p.lam;
+    const float lam = kda_lambda(p.lam_h, p.lam, p.lam_raw, h);
     const float c = 1.f / (1.f - lam + 1e-8f);
     float s = 0.f;
     if (p.seqlen > 0)
@@ -932,7 +933,12 @@ __global__ __launch_bounds__(256) void kda_ref_bwd_lam_kernel(KdaBwdParams q) {
           for (int j = 0; j < ns; ++j) t[i] += q.lam_part[(i * ns + j) * nbh + bh];
         s += t[0] - (1.f + 1e-8f) * t[1] - 1e-8f * t[2];
       }
-    q.dlam[h] = c * c * s;
+    float g = c * c * s;
+    if (p.lam_raw && p.lam_h) {                // through the sigmoid and the clamp (which passes 0.99 itself)
+      const float sg = 1.f / (1.f + expf(-p.lam_h[h]));
+      g = sg > 0.99f ? 0.f : g * sg * (1.f - sg);
+    }
+    q.dlam[h] = g;
   }
 }
 

@@ -135,7 +135,7 @@ __global__ __launch_bounds__(64 * FW) void kda_precise_fwd_kernel(KdaParams p) {
   const int w = wave_id(), l = lane_id(), half = l >> 5, l32 = l & 31;
   const int tid = threadIdx.x;
   const int S = p.seqlen, kd = GATED ? DK : p.kernel_dim;
-  const float lam = p.lam_h ? p.lam_h[h] : p.lam;
+  const float lam = kda_lambda(p.lam_h, p.lam, p.lam_raw, h);
   const int64_t rowbase = (int64_t)bh * S;
   const T* q1 = reinterpret_cast<const T*>(p.q1);
   const T* q2 = reinterpret_cast<const T*>(p.q2);
@@ -354,7 +354,7 @@ struct PBwdSmem {
 // Output-gradient pointer and coefficient of query stream qi (see KdaBwdParams).
 __device__ __forceinline__ float stream_coef(const KdaBwdParams& q, int h, int qi) {
   if (!q.diff) return 1.f;
-  const float lam = q.f.lam_h ? q.f.lam_h[h] : q.f.lam;
+  const float lam = kda_lambda(q.f.lam_h, q.f.lam, q.f.lam_raw, h);
   const float c = 1.f / (1.f - lam + 1e-8f);
   return qi == 0 ? c : -lam * c;
 }

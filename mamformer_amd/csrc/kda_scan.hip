@@ -524,7 +524,7 @@ __global__ __launch_bounds__(256 * NQ) void kda_ref_kernel(KdaParams p) {
   const int S = p.seqlen;
   const int kd = p.kernel_dim;
   const bool fuse_diff = (NQ == 2) && (p.o2 == nullptr);
-  const float lam = p.lam_h ? p.lam_h[h] : p.lam;
+  const float lam = kda_lambda(p.lam_h, p.lam, p.lam_raw, h);
   const float inv_1ml = 1.f / (1.f - lam + 1e-8f);
   const int64_t rowbase = (int64_t)bh * S;
   const int seg = blockIdx.y;                       // this workgroup's segment: tokens [p0, p1)

@@ -3,8 +3,8 @@
 // Per (b, h), with phi(x) = elu(x) + 1 on the first kernel_dim channels and 0
 // beyond (kda_diff.py:67-89; applied here when MH_KDA_PHI is set, otherwise
 // q/k arrive already feature-mapped as in the reference's call, kda_diff.py:302-304):
-//     S <- S + phi(k)^T v            (dk x dv, fp32, in place)
-//     z <- z + phi(k)                (dk, fp32, in place)
+//     S <- S + phi(k)^T v            (dk x dv, fp32, in place or into another buffer)
+//     z <- z + phi(k)                (dk, fp32, likewise)
 //     o_i = phi(q_i) S / (phi(q_i) z + 1e-8),   i = 1, 2
 //     o   = (o_1 - lam o_2) / (1 - lam + 1e-8)  (or o_1, o_2 separately; or o_1 alone)
 // Semantics of LinearDiffAttention._linear_attention_recurrent
@@ -41,11 +41,11 @@ __global__ __launch_bounds__(1024) void kda_step_kernel(KdaStepParams p) {
   const int dk = p.dk;
   const int nq = p.q2 ? 2 : 1;
 
-  float* Sb = p.state + (int64_t)bh * dk * DV;
-  f32x4* S4 = reinterpret_cast<f32x4*>(Sb);
+  const f32x4* Si = reinterpret_cast<const f32x4*>(p.state_in + (int64_t)bh * dk * DV);
+  f32x4* S4 = p.state ? reinterpret_cast<f32x4*>(p.state + (int64_t)bh * dk * DV) : nullptr;
   f32x4 s[KSTEP_ROWS];
 #pragma unroll
-  for (int i = 0; i < KSTEP_ROWS; ++i) s[i] = __builtin_nontemporal_load(&S4[min(r0 + i * rg, dk - 1) * TPC + c]);
+  for (int i = 0; i < KSTEP_ROWS; ++i) s[i] = __builtin_nontemporal_load(&Si[min(r0 + i * rg, dk - 1) * TPC + c]);
 
   const T* vrow = reinterpret_cast<const T*>(p.v) + (int64_t)bh * DV;
   float vv[4];
@@ -72,8 +72,8 @@ __global__ __launch_bounds__(1024) void kda_step_kernel(KdaStepParams p) {
   if (tid < 64) {
     float d0 = 0.f, d1 = 0.f;
     for (int k = tid; k < dk; k += 64) {
-      const float zn = p.z[(int64_t)bh * dk + k] + fk[k];
-      p.z[(int64_t)bh * dk + k] = zn;
+      const float zn = p.z_in[(int64_t)bh * dk + k] + fk[k];
+      if (p.z) p.z[(int64_t)bh * dk + k] = zn;
       d0 += fq[0][k] * zn;
       d1 += fq[1][k] * zn;
     }
@@ -95,7 +95,7 @@ __global__ __launch_bounds__(1024) void kda_step_kernel(KdaStepParams p) {
       const float kr = fk[r];
 #pragma unroll
       for (int j = 0; j < 4; ++j) v[j] += kr * vv[j];
-      __builtin_nontemporal_store(v, &S4[r * TPC + c]);
+      if (S4) __builtin_nontemporal_store(v, &S4[r * TPC + c]);
       const float a0 = fq[0][r], a1 = fq[1][r];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -120,7 +120,7 @@ __global__ __launch_bounds__(1024) void kda_step_kernel(KdaStepParams p) {
     o[1] /= den[1];
     T* o1p = reinterpret_cast<T*>(p.o) + (int64_t)bh * DV;
     if (nq == 2 && !p.o2) {
-      const float lam = p.lam_h ? p.lam_h[h] : p.lam;
+      const float lam = kda_lambda(p.lam_h, p.lam, p.lam_raw, h);
       o1p[tid] = from_f32<T>((o[0] - lam * o[1]) / (1.f - lam + 1e-8f));
     } else {
       o1p[tid] = from_f32<T>(o[0]);

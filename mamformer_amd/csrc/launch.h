@@ -188,6 +188,7 @@ struct KdaParams {
   // sums of the segments before it (seg_sum, nseg - 1 records per (b, h)); nseg <= 1 walks the sequence at once
   int nseg, seg_chunks;
   float* seg_sum;
+  int lam_raw;               // reference mode: lam_h holds lambda_raw, lambda = min(sigmoid(lambda_raw), 0.99)
 };
 hipError_t launch_kda(const KdaParams& p, hipStream_t st);
 // Segments and workspace of a split scan for p's sizes: sets p.nseg and p.seg_chunks, returns the workspace's bytes
@@ -235,9 +236,12 @@ struct KdaStepParams {
   int apply_phi;             // 1: q/k are raw, apply phi in the kernel; 0: already feature-mapped
   float lam;
   const float* lam_h;
+  int lam_raw;               // as in KdaParams
   const void* q1; const void* q2; const void* k; const void* v;   // (B,H,dk) / (B,H,dv) contiguous
-  float* state;              // (B,H,dk,dv) fp32, in place
-  float* z;                  // (B,H,dk) fp32, in place
+  const float* state_in;     // (B,H,dk,dv) fp32
+  const float* z_in;         // (B,H,dk) fp32
+  float* state;              // the updated state: state_in itself, another buffer, or null (not kept)
+  float* z;                  // the updated z, likewise
   void* o;                   // (B,H,dv): fused diff output, or o1
   void* o2;                  // optional o2 (pair)
 };

@@ -135,25 +135,34 @@ def kda_linear_attention(q1, q2, k, v, lambda_raw, kernel_dim, use_cache=False, 
     """
     Bb, H, S, Dh = q1.shape
     K = min(int(kernel_dim), Dh)
-    if use_cache and cache is not None and cache.get("attn_type") == "linear":
-        S_prev = cache["S"].to(torch.float32)
-        z_prev = cache["z"].to(torch.float32)
-    else:
-        S_prev = torch.zeros((Bb, H, K, Dh), device=q1.device, dtype=torch.float32)
-        z_prev = torch.zeros((Bb, H, K, 1), device=q1.device, dtype=torch.float32)
-    lam = ops.diff_lambda(lambda_raw)
-    if S == 1 and use_cache:
-        # one in-place step (dk = K) on fp32 copies of the cache, which become the new cache (the reference
-        # returns new tensors): the state has K rows, so only the first K channels of q and k enter
-        St = S_prev.clone(memory_format=torch.contiguous_format)
-        zt = z_prev.clone(memory_format=torch.contiguous_format)
-        out = ops.linear_attn_step(St, zt, q1[..., :K], q2[..., :K], k[..., :K], v, lam=lam, kernel_dim=K,
-                                   apply_phi=True)
-        out = out.reshape(Bb, H, 1, Dh)
-        return out, {"S": St, "z": zt, "attn_type": "linear"}
     if not use_cache:
         return ops.linear_attention_scan(q1, q2, k, v, K, lambda_raw), None
-    out, S_new, z_new = ops.linear_attn_scan(q1, q2, k, v, mode="reference", kernel_dim=K, lam=lam,
-                                             return_final_state=True)
-    new_cache = {"S": S_prev + S_new[:, :, :K], "z": z_prev + z_new[:, :, :K, None], "attn_type": "linear"}
-    return out, new_cache
+    S_prev = z_prev = None
+    if cache is not None and cache.get("attn_type") == "linear":
+        S_prev = cache["S"].to(torch.float32)
+        z_prev = cache["z"].to(torch.float32)
+    if S == 1:
+        if S_prev is None:
+            S_prev = torch.zeros((Bb, H, K, Dh), device=q1.device, dtype=torch.float32)
+            z_prev = torch.zeros((Bb, H, K, 1), device=q1.device, dtype=torch.float32)
+        # one step (dk = K) from the cache into new tensors, as the reference returns: the state has K rows, so
+        # only the first K channels of q and k enter
+        args = (q1[..., :K], q2[..., :K], k[..., :K], v)
+        if torch.is_grad_enabled() and (S_prev.requires_grad or z_prev.requires_grad):
+            # a cache that autograd tracks: its identity gradient goes through the copies that the step updates
+            St = S_prev.clone(memory_format=torch.contiguous_format)
+            zt = z_prev.clone(memory_format=torch.contiguous_format)
+            out = ops.linear_attn_step(St, zt, *args, lam=lambda_raw, kernel_dim=K, apply_phi=True, _lam_raw=True)
+        else:
+            St = torch.empty(S_prev.shape, device=S_prev.device, dtype=torch.float32)
+            zt = torch.empty(z_prev.shape, device=z_prev.device, dtype=torch.float32)
+            out = ops.linear_attn_step(ops._step_input(S_prev), ops._step_input(z_prev), *args, lam=lambda_raw,
+                                       kernel_dim=K, apply_phi=True, _out=(St, zt), _lam_raw=True)
+        out = out.reshape(Bb, H, 1, Dh)
+        return out, {"S": St, "z": zt, "attn_type": "linear"}
+    out, S_new, z_new = ops.linear_attn_scan(q1, q2, k, v, mode="reference", kernel_dim=K, lam=lambda_raw,
+                                             return_final_state=True, _lam_raw=True)
+    S_new, z_new = S_new[:, :, :K], z_new[:, :, :K, None]
+    if S_prev is not None:
+        S_new, z_new = S_prev + S_new, z_prev + z_new
+    return out, {"S": S_new.contiguous(), "z": z_new.contiguous(), "attn_type": "linear"}

@@ -1185,16 +1185,16 @@ def plan_selective_scan_reference(*args, **kw):
 
 
 class _KdaPlan(Plan):
-    """``Plan`` of ``mh_kda_chunk_scan_fwd_ws``, whose workspace (None: the sequence is not split) is an argument of
-    its own."""
+    """``Plan`` of ``mh_kda_chunk_scan_fwd_ws``, whose flags and workspace (None: the sequence is not split) are
+    arguments of their own."""
 
-    def __init__(self, args, ws, device, keep=(), **outputs):
+    def __init__(self, args, flags, ws, device, keep=(), **outputs):
         super().__init__("mh_kda_chunk_scan_fwd_ws", args, device, keep, **outputs)
-        self._ws, self._ws_bytes = ws, 0 if ws is None else ws.numel()
+        self._flags, self._ws, self._ws_bytes = flags, ws, 0 if ws is None else ws.numel()
 
     def __call__(self, stream=None):
         s = _stream(self._device) if stream is None else ct.c_void_p(stream)
-        _lib.call(self._fn, ct.byref(self._args), _ptr(self._ws), self._ws_bytes, s)
+        _lib.call(self._fn, ct.byref(self._args), self._flags, _ptr(self._ws), self._ws_bytes, s)
         return self
 
 
@@ -1209,7 +1209,8 @@ def diff_lambda(lambda_raw):
 
 
 def linear_attn_scan(q1, q2, k, v, *, g=None, lam=0.8, mode="gated", kernel_dim=None, initial_state=None,
-                     initial_z=None, return_final_state=False, pair=False, chunk_size=64, _plan_only=False):
+                     initial_z=None, return_final_state=False, pair=False, chunk_size=64, _plan_only=False,
+                     _lam_raw=False):
     """KDA linear-attention chunked scan on the GPU, layout (B, H, S, D) as the reference (kda_diff.py:270-273).
 
     mode="gated" (benchmark operator, no reference function):
@@ -1250,6 +1251,8 @@ def linear_attn_scan(q1, q2, k, v, *, g=None, lam=0.8, mode="gated", kernel_dim=
             raise ValueError("linear_attn_scan: g must be (B, H, S, dk)")
         gc = g.to(torch.float32).contiguous()
     lam_h = None
+    if _lam_raw and not torch.is_tensor(lam):
+        raise TypeError("linear_attn_scan: lambda_raw must be a tensor (H,)")
     if torch.is_tensor(lam):
         lam_h = lam.to(device=q1.device, dtype=torch.float32).reshape(-1).contiguous()
         if lam_h.numel() != H:
@@ -1271,7 +1274,7 @@ def linear_attn_scan(q1, q2, k, v, *, g=None, lam=0.8, mode="gated", kernel_dim=
         if not ref_mode:
             raise RuntimeError("linear_attn_scan: the gated operator has no backward (it has no reference "
                                "training path); use mode='reference' or call it under torch.no_grad()")
-        cfg = (a_kernel_dim(kernel_dim, dk), pair, return_final_state, lam_f)
+        cfg = (a_kernel_dim(kernel_dim, dk), pair, return_final_state, lam_f, _lam_raw)
         outs = _KdaRefFn.apply(q1c, q2c, kc, vc, lam_h, s0, z0, cfg)
         return outs if len(outs) > 1 else outs[0]
     o = torch.empty((Bb, H, S, dv), device=q1.device, dtype=q1.dtype)
@@ -1293,7 +1296,7 @@ def linear_attn_scan(q1, q2, k, v, *, g=None, lam=0.8, mode="gated", kernel_dim=
     n = ct.c_size_t()
     _lib.call("mh_kda_workspace_bytes", ct.byref(a), ct.byref(n))
     ws = torch.empty(n.value, device=q1.device, dtype=torch.uint8) if n.value else None
-    plan = _KdaPlan(a, ws, q1.device, keep=(q1c, q2c, kc, vc, gc, lam_h, s0, z0),
+    plan = _KdaPlan(a, _lib.MH_KDA_LAM_RAW if _lam_raw else 0, ws, q1.device, keep=(q1c, q2c, kc, vc, gc, lam_h, s0, z0),
                     o=o, o2=o2, final_state=fin, final_z=finz)
     if _plan_only:
         return plan
@@ -1314,9 +1317,10 @@ class _KdaRefFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q1, q2, k, v, lam_h, s0, z0, cfg):
-        kd, pair, ret_fin, lam_f = cfg
+        kd, pair, ret_fin, lam_f, lam_raw = cfg
         res = linear_attn_scan(q1, q2, k, v, mode="reference", kernel_dim=kd, lam=lam_h if lam_h is not None
-                               else lam_f, initial_state=s0, initial_z=z0, return_final_state=ret_fin, pair=pair)
+                               else lam_f, initial_state=s0, initial_z=z0, return_final_state=ret_fin, pair=pair,
+                               _lam_raw=lam_raw)
         res = res if isinstance(res, tuple) else (res,)
         ctx.save_for_backward(q1, q2, k, v, lam_h, s0, z0)
         ctx.cfg = cfg
@@ -1325,14 +1329,15 @@ class _KdaRefFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, *grads):
         q1, q2, k, v, lam_h, s0, z0 = ctx.saved_tensors
-        kd, pair, ret_fin, lam_f = ctx.cfg
+        kd, pair, ret_fin, lam_f, lam_raw = ctx.cfg
         n_o = 2 if pair else 1
         g_o = list(grads[:n_o])
         g_fin, g_finz = (grads[n_o], grads[n_o + 1]) if ret_fin else (None, None)
         r = linear_attn_scan_bwd(q1, q2, k, v, kernel_dim=kd, lam=lam_h if lam_h is not None else lam_f,
                                  do1=g_o[0], do2=g_o[1] if pair else None, pair=pair, initial_state=s0,
                                  initial_z=z0, d_final_state=g_fin, d_final_z=g_finz,
-                                 need_initial=(ctx.needs_input_grad[5] or ctx.needs_input_grad[6]))
+                                 need_initial=(ctx.needs_input_grad[5] or ctx.needs_input_grad[6]),
+                                 _lam_raw=lam_raw)
         dlam = r.get("d_lam") if (lam_h is not None and ctx.needs_input_grad[4]) else None
         return (r["dq1"], r.get("dq2"), r["dk"], r["dv"], dlam,
                 r.get("d_initial_state") if ctx.needs_input_grad[5] else None,
@@ -1340,7 +1345,8 @@ class _KdaRefFn(torch.autograd.Function):
 
 
 def linear_attn_scan_bwd(q1, q2, k, v, *, kernel_dim=None, lam=0.8, do1=None, do2=None, pair=False,
-                         initial_state=None, initial_z=None, d_final_state=None, d_final_z=None, need_initial=True):
+                         initial_state=None, initial_z=None, d_final_state=None, d_final_z=None, need_initial=True,
+                         _lam_raw=False):
     """Gradients of the reference-mode scan (``linear_attn_scan(..., mode="reference")``) on the GPU.
 
     Loss = <do1, o1> + <do2, o2> (``pair=True``), <do1, out> for the fused differential output
@@ -1397,7 +1403,7 @@ def linear_attn_scan_bwd(q1, q2, k, v, *, kernel_dim=None, lam=0.8, do1=None, do
     f.lam, f.lam_per_head = lam_f, _ptr(lam_h)
     f.q1, f.q2, f.k, f.v = _ptr(q1c), _ptr(q2c), _ptr(kc), _ptr(vc)
     f.initial_state, f.initial_z = _ptr(s0), _ptr(z0)
-    a.flags = _lib.MH_KDA_BWD_DIFF if diff else 0
+    a.flags = (_lib.MH_KDA_BWD_DIFF if diff else 0) | (_lib.MH_KDA_LAM_RAW if _lam_raw else 0)
     a.do1, a.do2 = _ptr(do1c), _ptr(do2c)
     a.d_final_state, a.d_final_z = _ptr(dfs), _ptr(dfz)
     a.dq1, a.dq2, a.dk, a.dv = _ptr(dq1), _ptr(dq2), _ptr(dkk), _ptr(dvv)
@@ -1432,9 +1438,9 @@ def linear_attn_scan_single(q, k, v, kernel_dim, block_k=128, block_d=128):
 def linear_attention_scan(q1, q2, k, v, kernel_dim, lambda_raw):
     """``LinearDiffAttention._linear_attention_scan`` counterpart (R/mamformer/layers/kda_diff.py:357-478):
     the normalised scan of both queries with the differential combination
-    (o1 - lam o2) / (1 - lam + 1e-8), lam = min(sigmoid(lambda_raw), 0.99) per head, fused into the kernel.
+    (o1 - lam o2) / (1 - lam + 1e-8), lam = min(sigmoid(lambda_raw), 0.99) per head, both in the kernel.
     Starts from a zero state, as the reference does."""
-    return linear_attn_scan(q1, q2, k, v, mode="reference", kernel_dim=kernel_dim, lam=diff_lambda(lambda_raw))
+    return linear_attn_scan(q1, q2, k, v, mode="reference", kernel_dim=kernel_dim, lam=lambda_raw, _lam_raw=True)
 
 
 def plan_linear_attn_step(*args, **kw):
@@ -1443,7 +1449,7 @@ def plan_linear_attn_step(*args, **kw):
 
 
 def linear_attn_step(state, z, q1, q2, k, v, *, lam=0.8, kernel_dim=None, apply_phi=True, pair=False,
-                     _plan_only=False):
+                     _plan_only=False, _out=None, _lam_raw=False):
     """One-token step of the reference-mode scan, updating ``state`` and ``z`` in place (KDA decode).
 
     state (B, H, dk, dv) fp32 contiguous; z (B, H, dk) or (B, H, dk, 1) fp32 contiguous; q1, q2, k
@@ -1452,6 +1458,8 @@ def linear_attn_step(state, z, q1, q2, k, v, *, lam=0.8, kernel_dim=None, apply_
     feature-mapped).  Returns the differential output (o1 - lam o2) / (1 - lam + 1e-8) shaped like v
     (q2=None: o1; ``pair=True``: (o1, o2)).  Semantics of ``_linear_attention_recurrent``
     (R/mamformer/layers/kda_diff.py:564-605) with the cache update of kda_diff.py:329-338.
+    (``_out``: (state, z) buffers that receive the update instead, each None: not kept.  ``_lam_raw``: lam holds
+    lambda_raw.)
     """
     _require_cuda("linear_attn_step", state, z, q1, q2, k, v)
     if state.dim() != 4 or state.dtype != torch.float32 or not state.is_contiguous():
@@ -1473,6 +1481,8 @@ def linear_attn_step(state, z, q1, q2, k, v, *, lam=0.8, kernel_dim=None, apply_
 
     q1c, q2c, kc, vc = rows(q1, dk, "q1"), rows(q2, dk, "q2"), rows(k, dk, "k"), rows(v, dv, "v")
     lam_h = None
+    if _lam_raw and not torch.is_tensor(lam):
+        raise TypeError("linear_attn_step: lambda_raw must be a tensor (H,)")
     if torch.is_tensor(lam):
         lam_h = lam.to(device=state.device, dtype=torch.float32).reshape(-1).contiguous()
         if lam_h.numel() != H:
@@ -1485,17 +1495,20 @@ def linear_attn_step(state, z, q1, q2, k, v, *, lam=0.8, kernel_dim=None, apply_
     a = _lib.KdaStepArgs()
     a.batch, a.nheads, a.dk, a.dv = Bb, H, dk, dv
     a.dtype = _DT[q1.dtype]
-    a.flags = _lib.MH_KDA_PHI if apply_phi else 0
+    a.flags = (_lib.MH_KDA_PHI if apply_phi else 0) | (_lib.MH_KDA_LAM_RAW if _lam_raw else 0)
     a.kernel_dim = int(kernel_dim) if kernel_dim is not None else dk
     a.lam = lam_f
     a.lam_per_head = _ptr(lam_h)
     a.q1, a.q2, a.k, a.v = _ptr(q1c), _ptr(q2c), _ptr(kc), _ptr(vc)
     a.state, a.z = _ptr(state), _ptr(z)
     a.o, a.o2 = _ptr(o), _ptr(o2)
-    plan = Plan("mh_kda_recurrent_step", a, state.device, keep=(state, z, q1c, q2c, kc, vc, lam_h), o=o, o2=o2)
-    if _plan_only:
-        return plan
-    plan()
+    if _out is not None:
+        _lib.call("mh_kda_recurrent_step_to", ct.byref(a), _ptr(_out[0]), _ptr(_out[1]), _stream(state.device))
+    else:
+        plan = Plan("mh_kda_recurrent_step", a, state.device, keep=(state, z, q1c, q2c, kc, vc, lam_h), o=o, o2=o2)
+        if _plan_only:
+            return plan
+        plan()
     shape = v.shape
     return (o.view(shape), o2.view(shape)) if pair else o.view(shape)
 
@@ -1504,9 +1517,14 @@ def linear_attention_recurrent(q1_phi, q2_phi, k_phi, v, S, z, lambda_raw):
     """``LinearDiffAttention._linear_attention_recurrent`` counterpart (R/mamformer/layers/kda_diff.py:564-605).
 
     q1_phi, q2_phi, k_phi (B, H, 1, K) already feature-mapped; v (B, H, 1, D); S (B, H, K, D); z (B, H, K, 1).
-    Returns the differential output (B, H, 1, D).  As in the reference, S and z are not modified (the step
-    runs on float32 copies); ``linear_attn_step`` is the in-place form for a float32 cache.
+    Returns the differential output (B, H, 1, D).  As in the reference, S and z are not modified (the updated ones
+    are not kept); ``linear_attn_step`` is the in-place form for a float32 cache.
     """
-    S32 = S.to(torch.float32).clone(memory_format=torch.contiguous_format)
-    z32 = z.to(torch.float32).clone(memory_format=torch.contiguous_format)
-    return linear_attn_step(S32, z32, q1_phi, q2_phi, k_phi, v, lam=diff_lambda(lambda_raw), apply_phi=False)
+    return linear_attn_step(_step_input(S), _step_input(z), q1_phi, q2_phi, k_phi, v, lam=lambda_raw, apply_phi=False,
+                            _out=(None, None), _lam_raw=True)
+
+
+def _step_input(t):
+    """A cached state or z as the step's kernel reads it: float32, contiguous, 16-byte aligned (a copy if needed)."""
+    t = t.detach().to(torch.float32).contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()

@@ -125,6 +125,6 @@ def test_workspace_of_a_split_scan():
     a.dtype = _lib.MH_F32                              # the fp32 kernels walk each sequence at once
     assert _lib.lib().mh_kda_workspace_bytes(ct.byref(a), ct.byref(n)) == 0 and n.value == 0
     a = _args(1, 16, 1500)
-    assert _lib.lib().mh_kda_chunk_scan_fwd_ws(ct.byref(a), 8192, 64, None) == -7
+    assert _lib.lib().mh_kda_chunk_scan_fwd_ws(ct.byref(a), 0, 8192, 64, None) == -7
     a.v = None
     assert _lib.lib().mh_kda_workspace_bytes(ct.byref(a), ct.byref(n)) == -1
