@@ -381,6 +381,37 @@ int mh_kda_recurrent_step(const mh_kda_step_args* a, void* stream);
 int mh_kda_recurrent_step_to(const mh_kda_step_args* a, float* state_out, float* z_out, void* stream);
 
 /* ------------------------------------------------------------------------
+ * One token through a whole Mamba-2 layer from its cache (bf16): in_proj, causal
+ *   conv + SiLU, the dt / B / C projections, the state update with the gate, out_proj.
+ * Replaces the incremental path of Mamba2Block.forward
+ *   (mamformer/layers/mamba2.py:272-296, 337-364) in the per-head form.
+ *   u (batch, d_model); weights (out, in) contiguous bf16, 16-byte aligned; biases bf16 or NULL;
+ *   conv_w (d_inner, width); A_log, dt_bias, D (nheads,) fp32; conv_state (batch, conv_state_len,
+ *   d_inner) bf16 with a contiguous last dimension, conv_state_len <= width - 1;
+ *   state_in / state_out (batch, nheads, headdim, dstate) fp32, distinct or identical.
+ *   Outputs: out (batch, d_model), conv_out (batch, min(conv_state_len + 1, width - 1), d_inner).
+ *   Supported: batch <= 64, d_model and d_inner multiples of 32, 2 <= width <= 8, dstate as
+ *   mh_ssd_state_update.
+ * ---------------------------------------------------------------------- */
+typedef struct {
+  int64_t batch, d_model, nheads, headdim, dstate, ngroups, dt_rank, width;
+  const void* u; int64_t u_stride_b;
+  const void* in_w; const void* in_b;
+  const void* conv_w; const void* conv_b;
+  const void* dt_w0; const void* dt_b0; const void* dt_w1; const void* dt_b1;
+  const void* B_w; const void* B_b; const void* C_w; const void* C_b;
+  const void* out_w; const void* out_b;
+  const float* A_log; const float* dt_bias; const float* D;
+  const void* conv_state; int64_t conv_state_len, conv_state_stride_b, conv_state_stride_l;
+  const float* state_in; float* state_out;
+  void* conv_out; void* out;
+  void* workspace; size_t workspace_bytes;
+} mh_layer_step_args;
+
+int mh_mamba2_layer_step_workspace_bytes(const mh_layer_step_args* a, size_t* bytes);
+int mh_mamba2_layer_step(const mh_layer_step_args* a, void* stream);
+
+/* ------------------------------------------------------------------------
  * Causal depthwise conv1d (+ optional SiLU), the Mamba layer prologue.
  * Replaces Mamba2Block._causal_conv1d (mamformer/layers/mamba2.py:370-405)
  *   and the SiLU that follows it (mamba2.py:282-283):

@@ -176,6 +176,21 @@ class GateArgs(ct.Structure):
     ]
 
 
+class LayerStepArgs(ct.Structure):
+    _fields_ = [
+        ("batch", _i64), ("d_model", _i64), ("nheads", _i64), ("headdim", _i64), ("dstate", _i64), ("ngroups", _i64),
+        ("dt_rank", _i64), ("width", _i64),
+        ("u", _vp), ("u_stride_b", _i64),
+        ("in_w", _vp), ("in_b", _vp), ("conv_w", _vp), ("conv_b", _vp),
+        ("dt_w0", _vp), ("dt_b0", _vp), ("dt_w1", _vp), ("dt_b1", _vp),
+        ("B_w", _vp), ("B_b", _vp), ("C_w", _vp), ("C_b", _vp), ("out_w", _vp), ("out_b", _vp),
+        ("A_log", _vp), ("dt_bias", _vp), ("D", _vp),
+        ("conv_state", _vp), ("conv_state_len", _i64), ("conv_state_stride_b", _i64), ("conv_state_stride_l", _i64),
+        ("state_in", _vp), ("state_out", _vp), ("conv_out", _vp), ("out", _vp),
+        ("workspace", _vp), ("workspace_bytes", _sz),
+    ]
+
+
 # every symbol include/mamformer_hip.h declares
 EXPORTS = (
     "mh_abi_version", "mh_last_error",
@@ -189,6 +204,7 @@ EXPORTS = (
     "mh_ssd_state_update",
     "mh_kda_chunk_scan_fwd", "mh_kda_workspace_bytes", "mh_kda_chunk_scan_fwd_ws", "mh_kda_bwd_workspace_bytes", "mh_kda_chunk_scan_bwd",
     "mh_kda_recurrent_step", "mh_kda_recurrent_step_to",
+    "mh_mamba2_layer_step_workspace_bytes", "mh_mamba2_layer_step",
     "mh_causal_conv1d_fwd",
     "mh_conv1d_bwd_workspace_bytes", "mh_causal_conv1d_bwd",
 )
@@ -243,6 +259,8 @@ def lib():
             h.mh_kda_recurrent_step.argtypes = [ct.POINTER(KdaStepArgs), _vp]
             h.mh_kda_bwd_workspace_bytes.argtypes = [ct.POINTER(KdaBwdArgs), ct.POINTER(_sz)]
             h.mh_kda_chunk_scan_bwd.argtypes = [ct.POINTER(KdaBwdArgs), _vp]
+            h.mh_mamba2_layer_step_workspace_bytes.argtypes = [ct.POINTER(LayerStepArgs), ct.POINTER(_sz)]
+            h.mh_mamba2_layer_step.argtypes = [ct.POINTER(LayerStepArgs), _vp]
             h.mh_causal_conv1d_fwd.argtypes = [ct.POINTER(Conv1dArgs), _vp]
             h.mh_conv1d_bwd_workspace_bytes.argtypes = [ct.POINTER(Conv1dBwdArgs), ct.POINTER(_sz)]
             h.mh_causal_conv1d_bwd.argtypes = [ct.POINTER(Conv1dBwdArgs), _vp]
@@ -250,6 +268,7 @@ def lib():
                          "mh_ssd_chunk_scan_fwd_noalloc",
                          "mh_ssd_state_update", "mh_kda_chunk_scan_fwd", "mh_kda_workspace_bytes",
                          "mh_kda_chunk_scan_fwd_ws", "mh_kda_recurrent_step", "mh_kda_recurrent_step_to",
+                         "mh_mamba2_layer_step_workspace_bytes", "mh_mamba2_layer_step",
                          "mh_causal_conv1d_fwd", "mh_conv1d_bwd_workspace_bytes", "mh_causal_conv1d_bwd",
                          "mh_ssd_bwd_workspace_bytes", "mh_ssd_chunk_scan_bwd",
                          "mh_kda_bwd_workspace_bytes", "mh_kda_chunk_scan_bwd",

@@ -665,6 +665,58 @@ void kda_fill(const mh_kda_args* a, mh::KdaParams& p) {
   p.o = a->o; p.o2 = a->o2;
 }
 
+int layer_step_validate(const mh_layer_step_args* a) {
+  if (!a) return fail(MH_ERR_NULL, "layer_step: args is NULL");
+  if (a->batch <= 0 || a->d_model <= 0 || a->nheads <= 0 || a->headdim <= 0 || a->dstate <= 0 || a->ngroups <= 0 ||
+      a->dt_rank <= 0)
+    return fail(MH_ERR_SHAPE, "layer_step: sizes must be positive");
+  if (a->nheads > kMaxDim || a->headdim > 4096 || a->d_model > (1 << 20) || a->nheads * a->headdim > (1 << 20) ||
+      a->dt_rank > (1 << 20) || a->ngroups * a->dstate > (1 << 20))
+    return fail(MH_ERR_SHAPE, "layer_step: sizes out of range");
+  if (a->batch > 64) return fail(MH_ERR_UNSUPPORTED, "layer_step: batch %lld > 64", (long long)a->batch);
+  if (a->nheads % a->ngroups) return fail(MH_ERR_SHAPE, "layer_step: nheads must be a multiple of ngroups");
+  if (a->d_model % 32 || (a->nheads * a->headdim) % 32)
+    return fail(MH_ERR_UNSUPPORTED, "layer_step: d_model and d_inner must be multiples of 32");
+  switch (a->dstate) {
+    case 8: case 16: case 32: case 64: case 128: case 256: break;
+    default: return fail(MH_ERR_UNSUPPORTED, "layer_step: dstate %lld not supported (8..256, power of two)",
+                         (long long)a->dstate);
+  }
+  if (a->width < 2 || a->width > 8) return fail(MH_ERR_UNSUPPORTED, "layer_step: conv width %lld not in 2..8", (long long)a->width);
+  if (a->conv_state_len < 0 || a->conv_state_len > a->width - 1)
+    return fail(MH_ERR_SHAPE, "layer_step: conv_state_len must be 0 .. width - 1");
+  if (!a->u || !a->in_w || !a->conv_w || !a->dt_w0 || !a->dt_w1 || !a->B_w || !a->C_w || !a->out_w || !a->A_log ||
+      !a->dt_bias || !a->D || (a->conv_state_len > 0 && !a->conv_state) || !a->state_in || !a->state_out ||
+      !a->conv_out || !a->out)
+    return fail(MH_ERR_NULL, "layer_step: a required pointer is NULL");
+  if (a->u_stride_b < 0 || a->u_stride_b % 8 || a->conv_state_stride_b < 0 || a->conv_state_stride_l < 0)
+    return fail(MH_ERR_STRIDE, "layer_step: bad stride");
+  if (!aligned16(a->u) || !aligned16(a->in_w) || !aligned16(a->dt_w0) || !aligned16(a->B_w) || !aligned16(a->C_w) ||
+      !aligned16(a->out_w) || !aligned16(a->state_in) || !aligned16(a->state_out))
+    return fail(MH_ERR_ALIGN, "layer_step: u, the weight matrices and the states must be 16-byte aligned");
+  if (a->state_in != a->state_out) {
+    const uintptr_t bytes = (uintptr_t)(a->batch * a->nheads * a->headdim * a->dstate * 4);
+    const uintptr_t i0 = (uintptr_t)a->state_in, o0 = (uintptr_t)a->state_out;
+    if (i0 < o0 + bytes && o0 < i0 + bytes)
+      return fail(MH_ERR_STRIDE, "layer_step: state_in and state_out overlap without being identical");
+  }
+  return MH_OK;
+}
+
+void layer_step_fill(const mh_layer_step_args* a, mh::LayerStepParams& p) {
+  memset(&p, 0, sizeof(p));
+  p.batch = (int)a->batch; p.d_model = (int)a->d_model; p.nheads = (int)a->nheads; p.headdim = (int)a->headdim;
+  p.d_inner = p.nheads * p.headdim; p.dstate = (int)a->dstate; p.ngroups = (int)a->ngroups;
+  p.dt_rank = (int)a->dt_rank; p.width = (int)a->width; p.cs_len = (int)a->conv_state_len;
+  p.u = a->u; p.u_sb = a->u_stride_b;
+  p.in_w = a->in_w; p.in_b = a->in_b; p.conv_w = a->conv_w; p.conv_b = a->conv_b;
+  p.dt_w0 = a->dt_w0; p.dt_b0 = a->dt_b0; p.dt_w1 = a->dt_w1; p.dt_b1 = a->dt_b1;
+  p.B_w = a->B_w; p.B_b = a->B_b; p.C_w = a->C_w; p.C_b = a->C_b; p.out_w = a->out_w; p.out_b = a->out_b;
+  p.A_log = a->A_log; p.dt_bias = a->dt_bias; p.D = a->D;
+  p.conv_state = a->conv_state; p.cs_sb = a->conv_state_stride_b; p.cs_sl = a->conv_state_stride_l;
+  p.state_in = a->state_in; p.state_out = a->state_out; p.conv_out = a->conv_out; p.out = a->out;
+}
+
 int kda_bwd_validate(const mh_kda_bwd_args* a) {
   if (!a) return fail(MH_ERR_NULL, "kda_bwd: args is NULL");
   mh_kda_args f = a->fwd;
@@ -1137,6 +1189,28 @@ int mh_kda_recurrent_step_to(const mh_kda_step_args* a, float* state_out, float*
   p.q1 = a->q1; p.q2 = a->q2; p.k = a->k; p.v = a->v;
   p.state_in = a->state; p.z_in = a->z; p.state = state_out; p.z = z_out; p.o = a->o; p.o2 = a->o2;
   return hip_status(mh::launch_kda_step(p, reinterpret_cast<hipStream_t>(stream)), "kda_recurrent_step");
+}
+
+int mh_mamba2_layer_step_workspace_bytes(const mh_layer_step_args* a, size_t* bytes) {
+  if (!bytes) return fail(MH_ERR_NULL, "layer_step: bytes output is NULL");
+  int rc = layer_step_validate(a);
+  if (rc) return rc;
+  mh::LayerStepParams p;
+  layer_step_fill(a, p);
+  *bytes = mh::layer_step_workspace_bytes(p);
+  return MH_OK;
+}
+
+int mh_mamba2_layer_step(const mh_layer_step_args* a, void* stream) {
+  int rc = layer_step_validate(a);
+  if (rc) return rc;
+  mh::LayerStepParams p;
+  layer_step_fill(a, p);
+  const size_t need = mh::layer_step_workspace_bytes(p);
+  if (!a->workspace || a->workspace_bytes < need || !aligned16(a->workspace))
+    return fail(MH_ERR_WORKSPACE, "layer_step: workspace of %zu bytes (16-byte aligned) required, got %zu", need,
+                a->workspace_bytes);
+  return hip_status(mh::launch_layer_step(p, a->workspace, reinterpret_cast<hipStream_t>(stream)), "mamba2_layer_step");
 }
 
 int mh_causal_conv1d_fwd(const mh_conv1d_args* a, void* stream) {

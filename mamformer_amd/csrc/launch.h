@@ -26,8 +26,45 @@ struct SsuParams {
   const float* dt_bias;
   void* y; int64_t y_stride_b;
   const void* z; int64_t z_stride_b;       // optional gate: y <- y * silu(z)
+  // dt from its low-rank row (the layer step, bf16 with a gate): dt[b, h] = bf16(dt_low[b] . dt_w[h] + dt_wb[h]) in
+  // place of p.dt, and A = -exp(p.A); null otherwise
+  const void* dt_low;                      // (b, dt_rank) contiguous
+  const void* dt_w;                        // (H, dt_rank) contiguous
+  const void* dt_wb;                       // (H,) or null
+  int dt_rank;
 };
 hipError_t launch_ssu(const SsuParams& p, hipStream_t st);
+
+// ------------------------------------------------------------- one token through a layer (layer_step.hip)
+struct StepSeg {
+  const void* W; const void* bias;         // (rows, K) bf16 contiguous, (rows,) bf16 or null
+  int rows;
+  void* out;                               // (batch, rows) bf16
+};
+struct StepGemm {
+  int batch, K, nseg;
+  int tiles[3];                            // 16-row tiles of each segment
+  const void* X; int64_t x_stride;         // (batch, K) bf16
+  StepSeg seg[3];
+  // in_proj's epilogue
+  int d_inner, width, cs_len;
+  const void* conv_w; const void* conv_b;  // (d_inner, width), (d_inner,) or null, bf16
+  const void* conv_state; int64_t cs_sb, cs_sl;
+  void* conv_out; void* x_act; void* z;
+};
+struct LayerStepParams {
+  int batch, d_model, d_inner, nheads, headdim, dstate, ngroups, dt_rank, width, cs_len;
+  const void* u; int64_t u_sb;
+  const void *in_w, *in_b, *conv_w, *conv_b, *dt_w0, *dt_b0, *dt_w1, *dt_b1, *B_w, *B_b, *C_w, *C_b, *out_w, *out_b;
+  const float *A_log, *dt_bias, *D;
+  const void* conv_state; int64_t cs_sb, cs_sl;
+  const float* state_in;
+  float* state_out;
+  void* conv_out;                          // (batch, min(cs_len + 1, width - 1), d_inner) bf16
+  void* out;                               // (batch, d_model) bf16
+};
+size_t layer_step_workspace_bytes(const LayerStepParams& p);
+hipError_t launch_layer_step(const LayerStepParams& p, void* workspace, hipStream_t st);
 
 // ------------------------------------------------------------- SSD prefill
 struct SsdParams {

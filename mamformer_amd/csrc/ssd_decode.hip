@@ -24,8 +24,9 @@ constexpr int SSU_ROWS = 2;   // state rows per thread per pass
 
 // GEN: the general form, with the decay rate per state column (p.A_per_state) and/or the step per channel
 // (p.dt_per_channel); without it one decay factor per head.  GATE: p.z is given (its rows are loaded with x's,
-// not under a branch of their own, which would wait for them alone).
-template <int N, typename T, bool GEN, bool GATE>
+// not under a branch of their own, which would wait for them alone).  LOW: dt is formed from its low-rank row and A from
+// A_log (SsuParams::dt_low).
+template <int N, typename T, bool GEN, bool GATE, bool LOW = false>
 __global__ __launch_bounds__(1024) void ssu_kernel(SsuParams p) {
   constexpr int TPR = N / 4;        // threads per state row
   const int rp = blockDim.x / TPR;  // rows per pass
@@ -77,7 +78,18 @@ __global__ __launch_bounds__(1024) void ssu_kernel(SsuParams p) {
   };
   load(row0);
 
-  float dt = dtc ? 0.f : p.dt[(int64_t)b * p.dt_stride_b + h];
+  float dt;
+  if constexpr (LOW) {                               // every wave for itself; rounded as a bf16 projection is
+    const T* lo = reinterpret_cast<const T*>(p.dt_low) + (int64_t)b * p.dt_rank;
+    const T* lw = reinterpret_cast<const T*>(p.dt_w) + (int64_t)h * p.dt_rank;
+    float acc = 0.f;
+    for (int i = threadIdx.x & 63; i < p.dt_rank; i += 64) acc += to_f32(lo[i]) * to_f32(lw[i]);
+    acc = wave_sum(acc);
+    if (p.dt_wb) acc += to_f32(reinterpret_cast<const T*>(p.dt_wb)[h]);
+    dt = to_f32(from_f32<T>(acc));
+  } else {
+    dt = dtc ? 0.f : p.dt[(int64_t)b * p.dt_stride_b + h];
+  }
   const T* Bp = reinterpret_cast<const T*>(p.B) + (int64_t)b * p.B_stride_b + (int64_t)g * N + ln * 4;
   const T* Cp = reinterpret_cast<const T*>(p.C) + (int64_t)b * p.C_stride_b + (int64_t)g * N + ln * 4;
   float Bv[4], Cv[4];
@@ -91,7 +103,7 @@ __global__ __launch_bounds__(1024) void ssu_kernel(SsuParams p) {
     if (p.dt_softplus) dt = softplus_f(dt);
     if (p.has_dt_limit) dt = fminf(fmaxf(dt, p.dt_min), p.dt_max);
   }
-  const float a = GEN ? 0.f : __expf(p.A[h] * dt);
+  const float a = GEN ? 0.f : __expf((LOW ? -expf(p.A[h]) : p.A[h]) * dt);
   float Av[4];                                       // general form: the decay rate of each state column
 #pragma unroll
   for (int i = 0; i < 4; ++i) Av[i] = (GEN && p.A_per_state) ? p.A[ln * 4 + i] : p.A[h];
@@ -138,6 +150,10 @@ static hipError_t launch_ssu_n(const SsuParams& p, hipStream_t st) {
   if (rows * TPR > 1024) rows = 1024 / TPR;
   const int threads = ((rows * TPR + 63) / 64) * 64;   // whole waves; extra lanes fall past P
   dim3 grid((unsigned)(p.batch * p.nheads)), block((unsigned)threads);
+  if (p.dt_low) {
+    hipLaunchKernelGGL((ssu_kernel<N, bf16, false, true, true>), grid, block, 0, st, p);
+    return hipGetLastError();
+  }
   const bool gen = p.A_per_state || p.dt_per_channel, gate = p.z != nullptr;
 #define SSU_LAUNCH(T)                                                                              \
   do {                                                                                             \

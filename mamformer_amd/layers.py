@@ -6,7 +6,8 @@ prefill, or the one-token recurrent step when a cache holds an SSM state) -> SiL
 -> out_proj, with the reference's cache dict ``{"conv_state", "ssm_state"}``.  The conv,
 SiLU, scan, z-gate and decode step run the HIP kernels of ``mamformer_amd.ops`` (conv and
 SiLU fused; the gate applied by the scan / step kernels as y is stored); the projections are
-plain library GEMMs.
+plain library GEMMs, except that one bf16 token of up to 64 sequences runs the whole layer in its own
+kernels (``Mamba2Layer._step``).
 
 Recorded deviation (per-head SSD convention): the reference parameterises dt per channel
 (``dt_proj: d_inner -> d_inner``) and A per state (``A_log (d_state,)``), which is a
@@ -83,6 +84,10 @@ class Mamba2Layer(nn.Module):
         chunked scan.  The cache is ``{"conv_state": last d_conv-1 raw x rows, "ssm_state": (b, d_inner, N)
         fp32}`` (:343-364).
         """
+        if use_cache and cache is not None and not return_h_states:
+            step = self._step(u, cache)
+            if step is not None:
+                return step
         b, L, _ = u.shape
         x, z = self.in_proj(u).chunk(2, dim=-1)                 # mamba2.py:272-273
         raw_x = x
@@ -120,6 +125,80 @@ class Mamba2Layer(nn.Module):
         if return_h_states:
             return out, new_cache, h_states
         return out, new_cache
+
+    def _step(self, u, cache):
+        """One token from the cache by ``mh_mamba2_layer_step`` (four launches; the composition below takes about
+        twenty): (out, new cache), or None where the call is not that kernel's -- more than one token or 64 sequences,
+        another dtype or layout, gradients wanted, or projections that are more than plain ``nn.Linear`` calls (hooks,
+        parametrisations, autocast, tracing, function or dispatch modes) -- and the general path runs."""
+        h0, cs = cache.get("ssm_state"), cache.get("conv_state")
+        if not (type(u) is type(h0) is type(cs) is torch.Tensor and u.dtype is cs.dtype is torch.bfloat16
+                and h0.dtype is torch.float32 and u.is_cuda and u.dim() == 3 and cs.dim() == 3):
+            return None
+        b, L, D = u.shape
+        di, N, K = self.d_inner, self.d_state, self.d_conv
+        if L != 1 or not 1 <= b <= 64 or D != self.d_model or D % 32 or di % 32 or N not in (8, 16, 32, 64, 128, 256) \
+                or not 2 <= K <= 8 or not _plain_calls():
+            return None
+        S = cs.shape[1]
+        if not 1 <= S < K or cs.shape[0] != b or cs.shape[2] != di or cs.stride(2) != 1 \
+                or h0.numel() != b * di * N or not h0.is_contiguous() or u.stride(2) != 1 or u.stride(0) % 8:
+            return None
+        mods, par = self._modules, self._parameters
+        dtp = mods["dt_proj"]
+        if type(dtp) is not nn.Sequential or len(dtp._modules) != 2 or not _unhooked(dtp):
+            return None
+        lin = [mods["in_proj"], *dtp._modules.values(), mods["B_proj"], mods["C_proj"], mods["out_proj"]]
+        w = []
+        for m in lin:
+            if type(m) is not nn.Linear or not _unhooked(m):
+                return None
+            w += (m._parameters["weight"], m._parameters["bias"])
+        cw, cb = par["conv_weight"], self.conv_bias
+        f32 = (par["A_log"], par["dt_bias"], par["D"])
+        if any(t is not None and type(t) is not nn.Parameter for t in (*w, cw, cb, *f32)):
+            return None
+        r = w[2].shape[0]
+        G = self.ngroups
+        if [t.shape for t in w[::2]] != [(2 * di, D), (r, di), (self.nheads, r), (G * N, di), (G * N, di), (D, di)] \
+                or cw.shape != (di, 1, K) or any(t.shape != (self.nheads,) for t in f32):
+            return None
+        bf16, dev = torch.bfloat16, u.device
+        track = torch.is_grad_enabled()
+        for t in (u, h0, cs, *w, cw, cb, *f32):
+            if t is not None and (t.device != dev or not t.is_contiguous() and t is not u and t is not cs
+                                  or track and t.requires_grad):
+                return None
+        if any(t is not None and t.dtype is not bf16 for t in (*w, cw, cb)) or any(t.dtype is not torch.float32
+                                                                                   for t in f32):
+            return None
+        p = [None if t is None else t.data_ptr() for t in (u, h0, *w, cw, cb, *f32, cs)]
+        if (p[0] | p[1] | p[2] | p[4] | p[8] | p[10] | p[12]) % 16:
+            return None
+        out = torch.empty((b, 1, D), device=dev, dtype=bf16)
+        conv = torch.empty((b, min(S + 1, K - 1), di), device=dev, dtype=bf16)
+        state = torch.empty((b, di, N), device=dev, dtype=torch.float32)
+        ops.mamba2_layer_step(
+            b, D, self.nheads, self.headdim, N, G, r, K, p[0], u.stride(0), p[2], p[3], p[14], p[15], *p[4:14],
+            *p[16:19], p[19], S, cs.stride(0), cs.stride(1), p[1], state.data_ptr(), conv.data_ptr(), out.data_ptr(),
+            device=dev)
+        return out, {"conv_state": conv, "ssm_state": state}
+
+
+def _plain_calls():
+    """Whether a call runs eagerly as written: no autocast, tracing, functorch transform, function or dispatch mode,
+    and no hooks on every module."""
+    from torch.nn.modules import module as m
+    return not (torch.is_autocast_enabled() or torch.jit.is_tracing() or torch.compiler.is_compiling()
+                or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch._C._len_torch_function_stack() or torch._C._len_torch_dispatch_stack()
+                or m._global_forward_hooks or m._global_forward_pre_hooks or m._global_backward_hooks
+                or m._global_backward_pre_hooks)
+
+
+def _unhooked(m):
+    return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                or "forward" in m.__dict__)
 
 
 def kda_linear_attention(q1, q2, k, v, lambda_raw, kernel_dim, use_cache=False, cache=None):

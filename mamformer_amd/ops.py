@@ -969,6 +969,17 @@ def selective_state_update(state, x, dt, A, B, C, D=None, *, dt_bias=None, dt_so
     return y
 
 
+def mamba2_layer_step(*fields, device):
+    """``mh_mamba2_layer_step`` on the current stream: the fields of ``LayerStepArgs`` in order, up to the workspace,
+    which is allocated here (``layers.Mamba2Layer`` checks the tensors behind the pointers)."""
+    a = _lib.LayerStepArgs(*fields)
+    n = ct.c_size_t()
+    _lib.call("mh_mamba2_layer_step_workspace_bytes", ct.byref(a), ct.byref(n))
+    ws = torch.empty(n.value, device=device, dtype=torch.uint8)
+    a.workspace, a.workspace_bytes = ws.data_ptr(), n.value
+    _lib.call("mh_mamba2_layer_step", ct.byref(a), _stream(device))
+
+
 def recurrent_step(x, dt, B, C, h_prev, A, D, *, dt_bias=None, dt_softplus=False, dt_limit=None, z=None):
     """``Mamba2Block._recurrent_step`` counterpart (R/mamformer/layers/mamba2.py:407-458), per-head form.
 
