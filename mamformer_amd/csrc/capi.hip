@@ -47,7 +47,8 @@ int ssd_heads_per_wg(const mh_ssd_args* a) {
   return hg;
 }
 
-int64_t ssd_auto_chunk(const mh_ssd_args* a) {
+// The chunk that gives every CU one workgroup (of at least 256 tokens): few chunks, so a small workspace.
+int64_t ssd_one_round_chunk(const mh_ssd_args* a) {
   const int64_t hg = ssd_heads_per_wg(a);
   const int64_t units = a->batch * (a->nheads / hg);           // workgroups per chunk index
   const int64_t target = 256;                                   // one 8-wave workgroup per CU on 256 CUs
@@ -56,6 +57,58 @@ int64_t ssd_auto_chunk(const mh_ssd_args* a) {
   if (want < 256) want = 256;
   if (want > 16384) want = 16384;
   return want;
+}
+
+size_t ssd_chunk_workspace(const mh_ssd_args* a, int64_t chunk) {
+  return mh::ssd_workspace_bytes((int)a->batch, (int)a->seqlen, (int)((a->seqlen + chunk - 1) / chunk), (int)a->nheads,
+                                 (int)a->headdim, (int)a->dstate, (int)a->ngroups, a->dtype);
+}
+
+// The state-passing chunk with the shortest time by a model of both kernels: a workgroup takes f + s us per 64-token
+// segment, 256 run at a time, and the states' pass between the kernels d per chunk (bf16: only beyond the look-back's
+// 8 chunks).  f, s and d are fitted to 64 .. 2048-token chunks of 15 sizes from b1 L64 H32 to b3 L2600 H64 and b1 L6000
+// H128; of both dtypes, the model's choice is within 8% of the best measured chunk there, where the one-round chunk was
+// up to 1.7 times slower (bf16 b1 L1000 H32 N128: 192 tokens 24.1 us, 256: 30.9; fp32: 128 tokens 69, 256: 102; fp32
+// b3 L2600 H64 G8: 192 tokens 812, one round of 1984: 1365).  bf16 chunks are no shorter than 192 tokens: a chunk's state
+// is rounded to bf16, and at 128 and 64 the outputs' error against float64 grows by 1 and 4%.  Sizes whose one-round chunk
+// fits the static scratch of the no-allocation entry point keep fitting it.
+int64_t ssd_auto_chunk(const mh_ssd_args* a) {
+  const int64_t hg = ssd_heads_per_wg(a), nseg = (a->seqlen + 63) / 64;
+  const int64_t units = a->batch * (a->nheads / hg);
+  const bool f32 = a->dtype == MH_F32, wide = a->dstate > 64;
+  const double s = f32 ? (wide ? 19.5 : 8.0 + 5.0 * hg) : (wide ? 4.6 : 3.6);
+  const double f = f32 ? 24.0 : (wide ? 14.0 : 12.0), d = f32 ? 0.2 : (wide ? 0.45 : 0.3);
+  // at most what one round takes, and twice that where partial rounds could be filled better
+  const int64_t one = ssd_one_round_chunk(a) / 64;
+  const int64_t lo = f32 ? 1 : 3, hi = std::min<int64_t>(256, std::max<int64_t>(lo, 2 * one));
+  const bool fits = ssd_chunk_workspace(a, 64 * one) <= MH_NOALLOC_SCRATCH_BYTES;
+  auto time_of = [&](int64_t c) {
+    const int64_t full = nseg / c, rem = nseg % c, chunks = full + (rem ? 1 : 0);
+    if (f32) {
+      // two workgroups can share a CU: beyond one round every workgroup takes a slot of a full one
+      const int64_t wgs = units * chunks;
+      const double per = (double)std::min(c, nseg);
+      return (wgs <= 256 ? f + s * per : (double)((wgs + 255) / 256) * (8.0 + 1.18 * s * per) + 16.0) + d * (double)chunks;
+    }
+    const int64_t rounds = (units * full + 255) / 256, left = rounds * 256 - units * full;
+    const double tr = rem ? f + s * (double)rem : 0.0;   // the short last chunk's workgroups, in slots left over or after
+    double t = (double)rounds * (f + s * (double)c);
+    if (full == 1 && rounds == 1) t -= 6.0;              // the first chunk looks back at nothing
+    if (rem && units > left) t += (double)((units - left + 255) / 256) * tr;
+    else t = std::max(t, tr);
+    return chunks > 8 ? t + d * (double)(chunks - 4) : t;
+  };
+  int64_t pick = std::max(one, lo);
+  double best = time_of(pick);
+  for (int64_t c = hi; c >= lo; c -= std::max<int64_t>(1, c / 32)) {
+    if (fits && c < one && ssd_chunk_workspace(a, 64 * c) > MH_NOALLOC_SCRATCH_BYTES) break;
+    const double t = time_of(c);
+    if (t < 0.98 * best) {                               // the longer chunk where it makes little difference
+      best = t;
+      pick = c;
+    }
+  }
+  return 64 * pick;
 }
 
 int ssd_validate(const mh_ssd_args* a, int64_t* chunk_len_out) {
@@ -781,8 +834,7 @@ int mh_ssd_chunk_scan_fwd_noalloc(const mh_ssd_args* a, void* stream) {
     return fail(MH_ERR_UNSUPPORTED, "ssd_noalloc: dstate %lld runs as a composition of 64/128-column scans that needs "
                 "a caller workspace (call mh_ssd_chunk_scan_fwd)", (long long)a->dstate);
   const int64_t nchunks = (a->seqlen + cl - 1) / cl;
-  const size_t need = mh::ssd_workspace_bytes((int)a->batch, (int)a->seqlen, (int)nchunks, (int)a->nheads,
-                                              (int)a->headdim, (int)a->dstate, (int)a->ngroups, a->dtype);
+  const size_t need = ssd_chunk_workspace(a, cl);
   if (need > MH_NOALLOC_SCRATCH_BYTES)
     return fail(MH_ERR_WORKSPACE, "ssd_noalloc: these sizes need %zu bytes of workspace, more than the %zu-byte static "
                 "scratch (call mh_ssd_chunk_scan_fwd with a caller workspace)", need, (size_t)MH_NOALLOC_SCRATCH_BYTES);
