@@ -292,5 +292,6 @@ def check(fn: str, rc: int):
 
 
 def call(fn: str, *args):
-    rc = getattr(lib(), fn)(*args)
-    check(fn, rc)
+    rc = getattr(_lib or lib(), fn)(*args)
+    if rc:
+        check(fn, rc)

@@ -106,66 +106,73 @@ class _Heads64:
         return dD.reshape(self.H, self.Pp)[:, :self.P].reshape(D.shape)
 
 
+# What a small call costs is this module's Python (25-45 us against 10-25 of GPU time): pointers and streams are passed
+# as the plain integers that ctypes takes, argument blocks are filled in one constructor call, and each tensor's strides
+# are asked for once.
+
 def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None else ct.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _stream(dev: torch.device):
-    return ct.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(dev.index)
 
 
 def _require_cuda(name, *ts):
+    dev = None
     for t in ts:
-        if t is not None and not t.is_cuda:
+        if t is None:
+            continue
+        if not t.is_cuda:
             raise RuntimeError(f"{name}: HIP op needs device tensors (got {t.device}); no CPU path exists")
-    devs = {t.device for t in ts if t is not None}
-    if len(devs) > 1:
-        raise RuntimeError(f"{name}: tensors on different devices {devs}")
+        if dev is None:
+            dev = t.device
+        elif t.device != dev:
+            raise RuntimeError(f"{name}: tensors on different devices {({u.device for u in ts if u is not None})}")
 
 
 def _f32c(t: Optional[torch.Tensor]):
-    if t is None:
-        return None
+    if t is None or (t.dtype is torch.float32 and t.is_contiguous()):
+        return t
     return t.to(torch.float32).contiguous()
 
 
 def _inner_contig(t: torch.Tensor, ndim_inner: int = 1) -> torch.Tensor:
     """Make the innermost `ndim_inner` dims contiguous and 16-byte aligned rows (copy if needed)."""
+    st = t.stride()
+    if st[-1] != 1 or (ndim_inner != 1 and st[-2] != t.shape[-1]) or t.data_ptr() % 16:
+        return t.contiguous()
     es = t.element_size()
-    ok = t.stride(-1) == 1 and (ndim_inner == 1 or t.stride(-2) == t.shape[-1])
-    ok = ok and t.data_ptr() % 16 == 0 and all((s * es) % 16 == 0 for s in t.stride()[:-ndim_inner])
-    return t if ok else t.contiguous()
+    for s in st[:-ndim_inner]:
+        if (s * es) % 16:
+            return t.contiguous()
+    return t
 
 
 def _ssd_args(x4, dt, A, B4, C4, D, dt_bias, dt_softplus, dt_limit, initial_state, y4, final_state, chunk_size,
               z4=None, xsum=None):
     b, L, H, P = x4.shape
-    G, N = B4.shape[2], B4.shape[3]
-    a = SsdArgs()
-    a.batch, a.seqlen, a.nheads, a.headdim, a.dstate, a.ngroups = b, L, H, P, N, G
-    a.chunk_len = int(chunk_size or 0)
-    a.dtype = _DT[x4.dtype]
-    flags = 0
+    G, N = B4.shape[2:4]
+    flags, dt_min, dt_max = 0, 0.0, 0.0
     if dt_softplus:
         flags |= _lib.MH_DT_SOFTPLUS
     if dt_limit is not None:
         flags |= _lib.MH_DT_LIMIT
-        a.dt_min, a.dt_max = float(dt_limit[0]), float(dt_limit[1])
+        dt_min, dt_max = float(dt_limit[0]), float(dt_limit[1])
     if D is not None and D.numel() == H * P and H * P != H:
         flags |= _lib.MH_D_PER_CHANNEL
-    a.flags = flags
-    a.x, a.x_stride_b, a.x_stride_l, a.x_stride_h = _ptr(x4), x4.stride(0), x4.stride(1), x4.stride(2)
-    a.dt, a.dt_stride_b, a.dt_stride_l = _ptr(dt), dt.stride(0), dt.stride(1)
-    a.A = _ptr(A)
-    a.B, a.B_stride_b, a.B_stride_l = _ptr(B4), B4.stride(0), B4.stride(1)
-    a.C, a.C_stride_b, a.C_stride_l = _ptr(C4), C4.stride(0), C4.stride(1)
-    a.D, a.dt_bias, a.initial_state = _ptr(D), _ptr(dt_bias), _ptr(initial_state)
-    a.y, a.y_stride_b, a.y_stride_l, a.y_stride_h = _ptr(y4), y4.stride(0), y4.stride(1), y4.stride(2)
-    a.final_state = _ptr(final_state)
-    if z4 is not None:
-        a.z, a.z_stride_b, a.z_stride_l, a.z_stride_h = _ptr(z4), z4.stride(0), z4.stride(1), z4.stride(2)
-    a.xsum = _ptr(xsum)
-    return a
+    return SsdArgs(
+        b, L, H, P, N, G, int(chunk_size or 0), _DT[x4.dtype], flags, dt_min, dt_max, x4.data_ptr(), *x4.stride()[:3],
+        dt.data_ptr(), *dt.stride()[:2], A.data_ptr(), B4.data_ptr(), *B4.stride()[:2], C4.data_ptr(),
+        *C4.stride()[:2], _ptr(D), _ptr(dt_bias), _ptr(initial_state), y4.data_ptr(), *y4.stride()[:3],
+        _ptr(final_state), None, 0, *((None, 0, 0, 0) if z4 is None else (z4.data_ptr(), *z4.stride()[:3])), _ptr(xsum))
+
+
+def _workspace(query, a, dev):
+    """The workspace that ``query`` asks for (at least 16 bytes), and the bytes it asked for."""
+    n = ct.c_size_t()
+    _lib.call(query, ct.byref(a), ct.byref(n))
+    return torch.empty(max(n.value, 16), device=dev, dtype=torch.uint8), n.value
 
 
 def ssd_chunk_len(batch, seqlen, nheads, headdim, dstate, ngroups, dtype=torch.bfloat16, chunk_size=None):
@@ -202,7 +209,7 @@ class Plan:
         self.__dict__.update(outputs)
 
     def __call__(self, stream=None):
-        s = _stream(self._device) if stream is None else ct.c_void_p(stream)
+        s = _stream(self._device) if stream is None else stream
         _lib.call(self._fn, ct.byref(self._args), s)
         return self
 
@@ -334,20 +341,17 @@ def selective_scan(x, dt, A, B, C, D, return_h_states=False, return_final_state=
     fin = torch.empty((b, H, P, N), device=x.device, dtype=torch.float32) if return_final_state else None
     args = _ssd_args(x4, dt32, A32, B4, C4, D32, bias32, dt_softplus, dt_limit, h0, y4, fin, chunk_size, z4,
                      None if _plan_only else xsum)
-    nbytes = ct.c_size_t()
-    _lib.call("mh_ssd_workspace_bytes", ct.byref(args), ct.byref(nbytes))
-    ws = torch.empty(max(int(nbytes.value), 16), device=x.device, dtype=torch.uint8)
-    args.workspace, args.workspace_bytes = _ptr(ws), nbytes.value
+    ws, args.workspace_bytes = _workspace("mh_ssd_workspace_bytes", args, x.device)
+    args.workspace = ws.data_ptr()
     y = y4.view(x.shape) if x.dim() == 3 else y4
     if fin is not None and x.dim() == 3:
         fin_out = fin.view(b, H * P, N)
     else:
         fin_out = fin
-    plan = Plan("mh_ssd_chunk_scan_fwd", args, x.device,
-                keep=(x4, dt32, A32, B4, C4, D32, bias32, h0, y4, fin, ws, z4), y=y, final_state=fin_out)
     if _plan_only:
-        return plan
-    plan()
+        return Plan("mh_ssd_chunk_scan_fwd", args, x.device,
+                    keep=(x4, dt32, A32, B4, C4, D32, bias32, h0, y4, fin, ws, z4), y=y, final_state=fin_out)
+    _lib.call("mh_ssd_chunk_scan_fwd", ct.byref(args), _stream(x.device))
     out = [y]
     if return_h_states:
         out.append(_h_states(x4, dt32, A32, B4, h0, bias32, dt_softplus, dt_limit, chunk_size, xsum=xsum))
@@ -365,10 +369,8 @@ def _scan_fwd(x4, dt32, A32, B4, C4, D32, h0, bias32, cfg):
     fin = torch.empty((b, H, P, N), device=x4.device, dtype=torch.float32)
     args = _ssd_args(x4, dt32, A32, B4, C4, D32, bias32, dt_softplus, dt_limit, h0, y4, fin, chunk_size, None,
                      xsum)
-    nbytes = ct.c_size_t()
-    _lib.call("mh_ssd_workspace_bytes", ct.byref(args), ct.byref(nbytes))
-    ws = torch.empty(max(int(nbytes.value), 16), device=x4.device, dtype=torch.uint8)
-    args.workspace, args.workspace_bytes = _ptr(ws), nbytes.value
+    ws, args.workspace_bytes = _workspace("mh_ssd_workspace_bytes", args, x4.device)
+    args.workspace = ws.data_ptr()
     _lib.call("mh_ssd_chunk_scan_fwd", ct.byref(args), _stream(x4.device))
     return y4, fin
 
@@ -392,22 +394,13 @@ def _scan_bwd(x4, dt32, A32, B4, C4, D32, h0, bias32, cfg, dy4, dfin, need_dh0, 
     dD = torch.empty_like(D32) if D32 is not None else None
     dbias = torch.empty((H,), device=dev, dtype=torch.float32) if bias32 is not None else None
     dh0 = torch.empty((b, H, P, N), device=dev, dtype=torch.float32) if need_dh0 else None
-    a = SsdBwdArgs()
-    a.fwd = _ssd_args(x4, dt32, A32, B4, C4, D32, bias32, dt_softplus, dt_limit, h0, x4, None, 64)
-    a.fwd.y = None
-    a.dy, a.dy_stride_b, a.dy_stride_l, a.dy_stride_h = _ptr(dy4), dy4.stride(0), dy4.stride(1), dy4.stride(2)
-    a.d_final_state = _ptr(dfin)
-    a.dx, a.dx_stride_b, a.dx_stride_l, a.dx_stride_h = _ptr(dx), dx.stride(0), dx.stride(1), dx.stride(2)
-    a.ddt, a.ddt_stride_b, a.ddt_stride_l = _ptr(ddt), ddt.stride(0), ddt.stride(1)
-    a.dA = _ptr(dA)
-    a.dB, a.dB_stride_b, a.dB_stride_l = _ptr(dB), dB.stride(0), dB.stride(1)
-    a.dC, a.dC_stride_b, a.dC_stride_l = _ptr(dC), dC.stride(0), dC.stride(1)
-    a.dD, a.d_dt_bias, a.d_initial_state = _ptr(dD), _ptr(dbias), _ptr(dh0)
-    a.dx_rows = _ptr(dx_rows)
-    nbytes = ct.c_size_t()
-    _lib.call("mh_ssd_bwd_workspace_bytes", ct.byref(a), ct.byref(nbytes))
-    ws = torch.empty(max(int(nbytes.value), 16), device=dev, dtype=torch.uint8)
-    a.workspace, a.workspace_bytes = _ptr(ws), nbytes.value
+    fwd = _ssd_args(x4, dt32, A32, B4, C4, D32, bias32, dt_softplus, dt_limit, h0, x4, None, 64)
+    fwd.y = None
+    a = SsdBwdArgs(fwd, dy4.data_ptr(), *dy4.stride()[:3], _ptr(dfin), dx.data_ptr(), *dx.stride()[:3], ddt.data_ptr(),
+                   *ddt.stride()[:2], dA.data_ptr(), dB.data_ptr(), *dB.stride()[:2], dC.data_ptr(), *dC.stride()[:2],
+                   _ptr(dD), _ptr(dbias), _ptr(dh0), None, 0, _ptr(dx_rows))
+    ws, a.workspace_bytes = _workspace("mh_ssd_bwd_workspace_bytes", a, dev)
+    a.workspace = ws.data_ptr()
     if plan_only:
         return Plan("mh_ssd_chunk_scan_bwd", a, dev,
                     keep=(x4, dt32, A32, B4, C4, D32, h0, bias32, dy4, dfin, ws),
@@ -477,17 +470,10 @@ class _SelectiveScanHsFn(torch.autograd.Function):
 
 
 def _gate_args(y4, z4, out, g=None, dz=None):
-    b, L, H, P = y4.shape
-    a = _lib.GateArgs()
-    a.batch, a.seqlen, a.nheads, a.headdim = b, L, H, P
-    a.dtype = _DT[y4.dtype]
-    for name, t in (("y", y4), ("z", z4), ("out", out), ("g", g), ("dz", dz)):
-        if t is not None:
-            setattr(a, name, _ptr(t))
-            setattr(a, name + "_stride_b", t.stride(0))
-            setattr(a, name + "_stride_l", t.stride(1))
-            setattr(a, name + "_stride_h", t.stride(2))
-    return a
+    def part(t):
+        return (None, 0, 0, 0) if t is None else (t.data_ptr(), *t.stride()[:3])
+
+    return _lib.GateArgs(*y4.shape, _DT[y4.dtype], 0, *part(y4), *part(z4), *part(g), *part(out), *part(dz))
 
 
 class _GateFn(torch.autograd.Function):
@@ -788,16 +774,9 @@ def _h_states_swap(x4, dt32, A32, B4, h0, bias32, dt_softplus, dt_limit, chunk_s
 
 def _conv_args(x, w, bc, cs, silu):
     b, L, Dm = x.shape
-    a = Conv1dArgs()
-    a.batch, a.seqlen, a.dim, a.width = b, L, Dm, w.shape[1]
-    a.dtype = _DT[x.dtype]
-    a.flags = _lib.MH_CONV_SILU if silu else 0
-    a.x, a.x_stride_b, a.x_stride_l = _ptr(x), x.stride(0), x.stride(1)
-    a.weight, a.bias = _ptr(w), _ptr(bc)
-    if cs is not None and cs.shape[1] > 0:
-        a.conv_state, a.conv_state_len = _ptr(cs), cs.shape[1]
-        a.conv_state_stride_b, a.conv_state_stride_l = cs.stride(0), cs.stride(1)
-    return a
+    cached = (None, 0, 0, 0) if cs is None or cs.shape[1] == 0 else (cs.data_ptr(), cs.shape[1], *cs.stride()[:2])
+    return Conv1dArgs(b, L, Dm, w.shape[1], _DT[x.dtype], _lib.MH_CONV_SILU if silu else 0, x.data_ptr(),
+                      *x.stride()[:2], w.data_ptr(), _ptr(bc), *cached)
 
 
 def _conv_fwd(xc, w, bc, cs, silu):
@@ -938,34 +917,23 @@ def selective_state_update(state, x, dt, A, B, C, D=None, *, dt_bias=None, dt_so
             raise ValueError(f"selective_state_update: z must be {(b, H, P)} in the dtype of x")
         zs = z if (z.stride(-1) == 1 and z.stride(-2) == P) else z.contiguous()
     y = torch.empty((b, H, P), device=x.device, dtype=x.dtype)
-    a = SsuArgs()
-    a.batch, a.nheads, a.headdim, a.dstate, a.ngroups = b, H, P, N, G
-    a.dtype = _DT[x.dtype]
-    flags = _lib.MH_DT_SOFTPLUS if dt_softplus else 0
+    flags, dt_min, dt_max = _lib.MH_DT_SOFTPLUS if dt_softplus else 0, 0.0, 0.0
     if dt_limit is not None:
         flags |= _lib.MH_DT_LIMIT
-        a.dt_min, a.dt_max = float(dt_limit[0]), float(dt_limit[1])
+        dt_min, dt_max = float(dt_limit[0]), float(dt_limit[1])
     if D32 is not None and D32.numel() == H * P and P != 1:
         flags |= _lib.MH_D_PER_CHANNEL
     if A_per_state:
         flags |= _lib.MH_A_PER_STATE
     if dt_chan:
         flags |= _lib.MH_DT_PER_CHANNEL
-    a.flags = flags
-    a.state_in, a.state_out = _ptr(state), _ptr(dst)
-    a.x, a.x_stride_b = _ptr(xs), xs.stride(0)
-    a.dt, a.dt_stride_b = _ptr(dt32), dt32.stride(0)
-    a.A = _ptr(A32)
-    a.B, a.B_stride_b = _ptr(Bs), Bs.stride(0)
-    a.C, a.C_stride_b = _ptr(Cs), Cs.stride(0)
-    a.D, a.dt_bias = _ptr(D32), _ptr(bias32)
-    a.y, a.y_stride_b = _ptr(y), y.stride(0)
-    if zs is not None:
-        a.z, a.z_stride_b = _ptr(zs), zs.stride(0)
-    plan = Plan("mh_ssd_state_update", a, x.device, keep=(state, dst, xs, dt32, A32, Bs, Cs, D32, bias32, zs), y=y)
+    a = SsuArgs(b, H, P, N, G, _DT[x.dtype], flags, dt_min, dt_max, state.data_ptr(), dst.data_ptr(), xs.data_ptr(),
+                xs.stride(0), dt32.data_ptr(), dt32.stride(0), A32.data_ptr(), Bs.data_ptr(), Bs.stride(0),
+                Cs.data_ptr(), Cs.stride(0), _ptr(D32), _ptr(bias32), y.data_ptr(), y.stride(0), _ptr(zs),
+                0 if zs is None else zs.stride(0))
     if _plan_only:
-        return plan
-    plan()
+        return Plan("mh_ssd_state_update", a, x.device, keep=(state, dst, xs, dt32, A32, Bs, Cs, D32, bias32, zs), y=y)
+    _lib.call("mh_ssd_state_update", ct.byref(a), _stream(x.device))
     return y
 
 
@@ -1185,7 +1153,7 @@ class _RefScanPlan(Plan):
         self._hs = hs_ptr
 
     def __call__(self, stream=None):
-        s = _stream(self._device) if stream is None else ct.c_void_p(stream)
+        s = _stream(self._device) if stream is None else stream
         _lib.call(self._fn, ct.byref(self._args), self._hs, s)
         return self
 
@@ -1204,7 +1172,7 @@ class _KdaPlan(Plan):
         self._flags, self._ws, self._ws_bytes = flags, ws, 0 if ws is None else ws.numel()
 
     def __call__(self, stream=None):
-        s = _stream(self._device) if stream is None else ct.c_void_p(stream)
+        s = _stream(self._device) if stream is None else stream
         _lib.call(self._fn, ct.byref(self._args), self._flags, _ptr(self._ws), self._ws_bytes, s)
         return self
 
@@ -1293,25 +1261,18 @@ def linear_attn_scan(q1, q2, k, v, *, g=None, lam=0.8, mode="gated", kernel_dim=
     fin = torch.empty((Bb, H, dk, dv), device=q1.device, dtype=torch.float32) if return_final_state else None
     finz = (torch.empty((Bb, H, dk), device=q1.device, dtype=torch.float32)
             if (return_final_state and ref_mode) else None)
-    a = KdaArgs()
-    a.batch, a.nheads, a.seqlen, a.dk, a.dv = Bb, H, S, dk, dv
-    a.dtype = _DT[q1.dtype]
-    a.mode = _lib.MH_KDA_REFERENCE if ref_mode else _lib.MH_KDA_GATED
-    a.kernel_dim = int(kernel_dim) if (ref_mode and kernel_dim is not None) else dk
-    a.lam = lam_f
-    a.lam_per_head = _ptr(lam_h)
-    a.q1, a.q2, a.k, a.v, a.g = _ptr(q1c), _ptr(q2c), _ptr(kc), _ptr(vc), _ptr(gc)
-    a.initial_state, a.final_state = _ptr(s0), _ptr(fin)
-    a.initial_z, a.final_z = _ptr(z0), _ptr(finz)
-    a.o, a.o2 = _ptr(o), _ptr(o2)
+    a = KdaArgs(Bb, H, S, dk, dv, _DT[q1.dtype], _lib.MH_KDA_REFERENCE if ref_mode else _lib.MH_KDA_GATED,
+                int(kernel_dim) if (ref_mode and kernel_dim is not None) else dk, lam_f, _ptr(lam_h), q1c.data_ptr(),
+                _ptr(q2c), kc.data_ptr(), vc.data_ptr(), _ptr(gc), _ptr(s0), _ptr(z0), _ptr(fin), _ptr(finz),
+                o.data_ptr(), _ptr(o2))
     n = ct.c_size_t()
     _lib.call("mh_kda_workspace_bytes", ct.byref(a), ct.byref(n))
     ws = torch.empty(n.value, device=q1.device, dtype=torch.uint8) if n.value else None
-    plan = _KdaPlan(a, _lib.MH_KDA_LAM_RAW if _lam_raw else 0, ws, q1.device, keep=(q1c, q2c, kc, vc, gc, lam_h, s0, z0),
-                    o=o, o2=o2, final_state=fin, final_z=finz)
+    flags = _lib.MH_KDA_LAM_RAW if _lam_raw else 0
     if _plan_only:
-        return plan
-    plan()
+        return _KdaPlan(a, flags, ws, q1.device, keep=(q1c, q2c, kc, vc, gc, lam_h, s0, z0), o=o, o2=o2,
+                        final_state=fin, final_z=finz)
+    _lib.call("mh_kda_chunk_scan_fwd_ws", ct.byref(a), flags, _ptr(ws), n.value, _stream(q1.device))
     out = (o, o2) if pair else (o,)
     if return_final_state:
         out = out + ((fin, finz) if ref_mode else (fin,))
@@ -1405,24 +1366,14 @@ def linear_attn_scan_bwd(q1, q2, k, v, *, kernel_dim=None, lam=0.8, do1=None, do
     dS0 = torch.empty((Bb, H, dk, dv), device=q1.device, dtype=torch.float32) if need_initial else None
     dz0 = torch.empty((Bb, H, dk), device=q1.device, dtype=torch.float32) if need_initial else None
     dlam = torch.empty(H, device=q1.device, dtype=torch.float32) if diff else None
-    a = _lib.KdaBwdArgs()
-    f = a.fwd
-    f.batch, f.nheads, f.seqlen, f.dk, f.dv = Bb, H, S, dk, dv
-    f.dtype = _DT[q1.dtype]
-    f.mode = _lib.MH_KDA_REFERENCE
-    f.kernel_dim = a_kernel_dim(kernel_dim, dk)
-    f.lam, f.lam_per_head = lam_f, _ptr(lam_h)
-    f.q1, f.q2, f.k, f.v = _ptr(q1c), _ptr(q2c), _ptr(kc), _ptr(vc)
-    f.initial_state, f.initial_z = _ptr(s0), _ptr(z0)
-    a.flags = (_lib.MH_KDA_BWD_DIFF if diff else 0) | (_lib.MH_KDA_LAM_RAW if _lam_raw else 0)
-    a.do1, a.do2 = _ptr(do1c), _ptr(do2c)
-    a.d_final_state, a.d_final_z = _ptr(dfs), _ptr(dfz)
-    a.dq1, a.dq2, a.dk, a.dv = _ptr(dq1), _ptr(dq2), _ptr(dkk), _ptr(dvv)
-    a.d_initial_state, a.d_initial_z, a.d_lam = _ptr(dS0), _ptr(dz0), _ptr(dlam)
-    n = ct.c_size_t()
-    _lib.call("mh_kda_bwd_workspace_bytes", ct.byref(a), ct.byref(n))
-    ws = torch.empty(max(n.value, 16), device=q1.device, dtype=torch.uint8)
-    a.workspace, a.workspace_bytes = _ptr(ws), ws.numel()
+    f = KdaArgs(Bb, H, S, dk, dv, _DT[q1.dtype], _lib.MH_KDA_REFERENCE, a_kernel_dim(kernel_dim, dk), lam_f,
+                _ptr(lam_h), q1c.data_ptr(), _ptr(q2c), kc.data_ptr(), vc.data_ptr(), None, _ptr(s0), _ptr(z0))
+    a = _lib.KdaBwdArgs(
+        f, (_lib.MH_KDA_BWD_DIFF if diff else 0) | (_lib.MH_KDA_LAM_RAW if _lam_raw else 0), _ptr(do1c), _ptr(do2c),
+        _ptr(dfs), _ptr(dfz), dq1.data_ptr(), _ptr(dq2), dkk.data_ptr(), dvv.data_ptr(), _ptr(dS0), _ptr(dz0),
+        _ptr(dlam))
+    ws, _ = _workspace("mh_kda_bwd_workspace_bytes", a, q1.device)
+    a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
     _lib.call("mh_kda_chunk_scan_bwd", ct.byref(a), _stream(q1.device))
     res = {"dq1": dq1, "dk": dkk, "dv": dvv}
     if dq2 is not None:
@@ -1503,23 +1454,16 @@ def linear_attn_step(state, z, q1, q2, k, v, *, lam=0.8, kernel_dim=None, apply_
         lam_f = float(lam)
     o = torch.empty((Bb, H, dv), device=state.device, dtype=q1.dtype)
     o2 = torch.empty((Bb, H, dv), device=state.device, dtype=q1.dtype) if pair else None
-    a = _lib.KdaStepArgs()
-    a.batch, a.nheads, a.dk, a.dv = Bb, H, dk, dv
-    a.dtype = _DT[q1.dtype]
-    a.flags = (_lib.MH_KDA_PHI if apply_phi else 0) | (_lib.MH_KDA_LAM_RAW if _lam_raw else 0)
-    a.kernel_dim = int(kernel_dim) if kernel_dim is not None else dk
-    a.lam = lam_f
-    a.lam_per_head = _ptr(lam_h)
-    a.q1, a.q2, a.k, a.v = _ptr(q1c), _ptr(q2c), _ptr(kc), _ptr(vc)
-    a.state, a.z = _ptr(state), _ptr(z)
-    a.o, a.o2 = _ptr(o), _ptr(o2)
+    a = _lib.KdaStepArgs(
+        Bb, H, dk, dv, _DT[q1.dtype], (_lib.MH_KDA_PHI if apply_phi else 0) | (_lib.MH_KDA_LAM_RAW if _lam_raw else 0),
+        int(kernel_dim) if kernel_dim is not None else dk, lam_f, _ptr(lam_h), q1c.data_ptr(), _ptr(q2c),
+        kc.data_ptr(), vc.data_ptr(), state.data_ptr(), z.data_ptr(), o.data_ptr(), _ptr(o2))
     if _out is not None:
         _lib.call("mh_kda_recurrent_step_to", ct.byref(a), _ptr(_out[0]), _ptr(_out[1]), _stream(state.device))
     else:
-        plan = Plan("mh_kda_recurrent_step", a, state.device, keep=(state, z, q1c, q2c, kc, vc, lam_h), o=o, o2=o2)
         if _plan_only:
-            return plan
-        plan()
+            return Plan("mh_kda_recurrent_step", a, state.device, keep=(state, z, q1c, q2c, kc, vc, lam_h), o=o, o2=o2)
+        _lib.call("mh_kda_recurrent_step", ct.byref(a), _stream(state.device))
     shape = v.shape
     return (o.view(shape), o2.view(shape)) if pair else o.view(shape)
 
