@@ -992,17 +992,16 @@ __global__ __launch_bounds__(128 * (N / 32)) void ssd_bwd_grad_kernel(SsdBwdPara
   }
 }
 
-// ------------------------------------------------------------------ kernel 3: partials -> dB, dC
+// ------------------------------------------------------------------ kernel 3: partials -> dB, dC, dA, dD, d_dt_bias
 
 // out[b, t, g, n] = sum over the nparts head-block partials (fixed order), in the I/O dtype and the caller's strides.
 template <typename T>
-__global__ __launch_bounds__(256) void ssd_bwd_reduce_kernel(const float* __restrict__ part, int nparts,
-                                                             void* out, int64_t sb, int64_t sl, int L, int GN,
-                                                             int64_t n4) {
-  const int64_t i4 = (int64_t)blockIdx.x * 256 + threadIdx.x;
+__device__ __forceinline__ void bwd_reduce_rows(const float* __restrict__ part, int nparts, void* out, int64_t sb,
+                                                int64_t sl, int L, int GN, int64_t n4, int64_t i4) {
   if (i4 >= n4) return;
   const int64_t e = i4 * 4;
   f32x4 v = *reinterpret_cast<const f32x4*>(part + e);
+#pragma unroll 8
   for (int k = 1; k < nparts; ++k) {
     const f32x4 u = *reinterpret_cast<const f32x4*>(part + (int64_t)k * n4 * 4 + e);
 #pragma unroll
@@ -1025,9 +1024,8 @@ __global__ __launch_bounds__(256) void ssd_bwd_reduce_kernel(const float* __rest
 // dA, d_dt_bias and dD from the per-(batch, segment, head) partials, summed in a fixed order (deterministic):
 // one wave per output, lane k taking partials k, k + 64, ... in order, then a fixed shuffle tree.  Output o < H:
 // dA, d_dt_bias, dD (per head) of head o; o = H + h * P + c: dD[h, c] (per channel, both token halves).
-__global__ __launch_bounds__(256) void ssd_bwd_param_reduce_kernel(SsdBwdParams q) {
+__device__ __forceinline__ void bwd_reduce_params(const SsdBwdParams& q, int o, int l) {
   const SsdParams& p = q.f;
-  const int o = blockIdx.x * 4 + wave_id(), l = lane_id();
   const int H = p.nheads, nbs = p.batch * p.nseg;
   if (o < H) {
     float a = 0.f, bi = 0.f, d = 0.f;
@@ -1052,6 +1050,24 @@ __global__ __launch_bounds__(256) void ssd_bwd_param_reduce_kernel(SsdBwdParams 
     d = wave_sum(d);
     if (l == 0) q.dD[h * HD + c] = d;
   }
+}
+
+// Every reduction of the gradient kernel's partials in one launch (three, and one that cleared outputs these write,
+// were 14 us of a backward at b2 L4096 H64, each bound by its own launch and drain): the first npar workgroups the
+// parameters, then nblk of dB and nblk of dC.
+template <typename T>
+__global__ __launch_bounds__(256) void ssd_bwd_reduce_kernel(SsdBwdParams q, int npar, int nblk, int nparts, int GN,
+                                                             int64_t n4) {
+  int i = blockIdx.x;
+  if (i < npar) {
+    bwd_reduce_params(q, i * 4 + wave_id(), lane_id());
+    return;
+  }
+  i -= npar;
+  const bool c = i >= nblk;
+  const int64_t i4 = (int64_t)(c ? i - nblk : i) * 256 + threadIdx.x;
+  bwd_reduce_rows<T>(c ? q.dC_part : q.dB_part, nparts, c ? q.dC : q.dB, c ? q.dC_sb : q.dB_sb, c ? q.dC_sl : q.dB_sl,
+                     q.f.seqlen, GN, n4, i4);
 }
 
 // ------------------------------------------------------------------ host side
@@ -1111,31 +1127,24 @@ static hipError_t launch_bwd_t(const SsdBwdParams& q, hipStream_t st) {
   const int GN = p.ngroups * N;
   const int nparts = (p.nheads / p.ngroups) / q.heads_per_wg;
   const int64_t n4 = (int64_t)p.batch * p.seqlen * GN / 4;
-  const unsigned nblk = (unsigned)((n4 + 255) / 256);
-  hipLaunchKernelGGL((ssd_bwd_reduce_kernel<T>), dim3(nblk), dim3(256), 0, st, q.dB_part, nparts, q.dB, q.dB_sb,
-                     q.dB_sl, p.seqlen, GN, n4);
-  e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((ssd_bwd_reduce_kernel<T>), dim3(nblk), dim3(256), 0, st, q.dC_part, nparts, q.dC, q.dC_sb,
-                     q.dC_sl, p.seqlen, GN, n4);
-  e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const int nout = p.nheads * (1 + (p.D_per_channel && q.dD ? HD : 0));
-  hipLaunchKernelGGL(ssd_bwd_param_reduce_kernel, dim3((unsigned)((nout + 3) / 4)), dim3(256), 0, st, q);
+  const int nblk = (int)((n4 + 255) / 256);
+  const int nout = p.nheads * (1 + (p.D_per_channel && q.dD ? HD : 0)), npar = (nout + 3) / 4;
+  hipLaunchKernelGGL((ssd_bwd_reduce_kernel<T>), dim3((unsigned)(npar + 2 * nblk)), dim3(256), 0, st, q, npar, nblk,
+                     nparts, GN, n4);
   return hipGetLastError();
 }
 
 hipError_t launch_ssd_bwd(const SsdBwdParams& q, hipStream_t st) {
   const SsdParams& p = q.f;
-  ZeroRanges z;
-  for (int i = 0; i < 5; ++i) { z.p[i] = nullptr; z.n[i] = 0; }
-  z.p[0] = q.dA;      z.n[0] = p.nheads;
-  z.p[1] = q.dD;      z.n[1] = p.D_per_channel ? (int64_t)p.nheads * HD : p.nheads;
-  z.p[2] = q.dbias;   z.n[2] = p.nheads;
-  hipLaunchKernelGGL(ssd_bwd_zero_kernel, dim3(1, 3), dim3(256), 0, st, z);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
   if (p.nseg == 0) {
+    ZeroRanges z;
+    for (int i = 0; i < 5; ++i) { z.p[i] = nullptr; z.n[i] = 0; }
+    z.p[0] = q.dA;      z.n[0] = p.nheads;
+    z.p[1] = q.dD;      z.n[1] = p.D_per_channel ? (int64_t)p.nheads * HD : p.nheads;
+    z.p[2] = q.dbias;   z.n[2] = p.nheads;
+    hipLaunchKernelGGL(ssd_bwd_zero_kernel, dim3(1, 3), dim3(256), 0, st, z);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
     if (!q.dh0) return hipSuccess;
     const size_t n = (size_t)p.batch * p.nheads * HD * p.dstate;
     hipLaunchKernelGGL(ssd_bwd_copy_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, q.d_final, q.dh0, n);
