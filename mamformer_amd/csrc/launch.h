@@ -138,10 +138,12 @@ struct RfParams {
   float* dD;                 // like D, or null
   float* d_dt_bias;          // (d_inner,) or null
   float* dh0;                // (b, d_inner, N) or null
-  float* ckpt;               // workspace: (b, pieces, d_inner, N) the state entering every piece of the sequence
+  float* ckpt;               // workspace: (b, pieces, d_inner, N) the state entering every 16-token piece
+  float* lam_ckpt;           // workspace: the same shape, the adjoint handed into every piece from its right
   float* dB_part; float* dC_part;   // workspace: (b, channel blocks, L, N) sums over a block's channels
-  float* dA_part;            // workspace: (b, channel blocks, N)
-  float* dD_part; float* dbias_part;  // workspace: (b, d_inner) sums over the tokens of one batch row
+  float* dA_part;            // workspace: (b, pieces, channel blocks, N)
+  float* dD_part; float* dbias_part;  // workspace: (b, pieces, d_inner) sums over the tokens of a piece
+  float* dD_sum;             // workspace: (d_inner) a channel's dD where D is per head
 };
 bool ssd_rf_supported(int dstate);
 size_t ssd_rf_workspace_bytes(int batch, int seqlen, int d_inner, int dstate, bool h_states);

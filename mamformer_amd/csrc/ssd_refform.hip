@@ -17,6 +17,8 @@
 //   that the sum over channels is a reduce-scatter inside the wave (v_permlane32_swap, v_permlane16_swap, then the
 //   DPP row sums) plus a sum over the 4 waves; the per-block sums go to a workspace and rf_hs_reduce_kernel adds
 //   them in a fixed order (deterministic).
+#include <algorithm>
+
 #include "common.h"
 #include "launch.h"
 #include "ssd_shared.h"
@@ -36,9 +38,9 @@ template <int N> constexpr int rf_lpc() { return N >= 32 ? 32 : 16; }
 template <int N> constexpr int rf_ns() { return N / rf_lpc<N>(); }
 template <int N> constexpr int rf_cpb() { return 4 * (64 / rf_lpc<N>()); }
 template <int N> constexpr int rf_tb() { return N <= 128 ? 32 : 16; }
-// Tokens per piece of the backward (the checkpoint spacing): the per-token states and decays of a piece are held in
-// registers, RK * NS of each per lane.
-template <int N> constexpr int rf_rk() { return rf_ns<N>() <= 4 ? 16 : 8; }
+constexpr int RF_RK = 16;            // tokens per piece of the backward (the checkpoint spacing)
+constexpr int RF_HK = 8;             // tokens whose states and decays the gradient kernel holds in registers at once
+constexpr int RF_CH = 64;            // channels per workgroup of the gradient kernel
 
 // Per-lane token prologue: dt <- clamp(softplus?(dt + bias), dt_min, dt_max).
 __device__ __forceinline__ float rf_dt(const RfParams& p, float raw, float bias) {
@@ -319,12 +321,11 @@ __device__ __forceinline__ void rf_tok(const RfStage<N, TB, CPB>& s, int t, int 
   }
 }
 
-// CKPT: the checkpoint pass of the backward, which writes the state entering every piece of rf_rk<N>() tokens
-// (p.ckpt) and no y.
-template <typename T, int N, bool GATE, bool CKPT = false>
-__global__ __launch_bounds__(RF_NT) void rf_scan_kernel(RfParams p) {
+// CKPT: the checkpoint pass of the backward, which writes the state entering every piece of RF_RK tokens (p.ckpt) and
+// no y.
+template <typename T, int N, bool GATE, bool CKPT>
+__device__ __forceinline__ void rf_scan_walk(const RfParams& p, RfSmem<N, rf_tb<N>(), rf_cpb<N>()>& sm) {
   constexpr int TB = rf_tb<N>(), LPC = rf_lpc<N>(), NS = rf_ns<N>(), CPB = rf_cpb<N>();
-  __shared__ RfSmem<N, TB, CPB> sm;
   const int nper = p.d_inner / CPB;
   int b, cb;
   rf_block(p.batch * nper, nper, b, cb);
@@ -366,7 +367,7 @@ __global__ __launch_bounds__(RF_NT) void rf_scan_kernel(RfParams p) {
 #pragma unroll
       for (int t = 0; t < TB; ++t) {
         if constexpr (CKPT) {
-          constexpr int RK = rf_rk<N>();                   // divides TB: a piece starts where t % RK == 0
+          constexpr int RK = RF_RK;                        // divides TB: a piece starts where t % RK == 0
           const int tt = k * TB + t;
           if (t % RK == 0 && tt < p.seqlen) {
             const int nsb = (p.seqlen + RK - 1) / RK;
@@ -400,7 +401,7 @@ __global__ __launch_bounds__(RF_NT) void rf_scan_kernel(RfParams p) {
     for (int t = 0; t < TB; ++t) {
       if (t + 1 < TB) rf_tok<N, TB, CPB, NS>(s, t + 1, cl, n0, nxt);
       if constexpr (CKPT) {
-        constexpr int RK = rf_rk<N>();                     // divides TB: a piece starts where t % RK == 0
+        constexpr int RK = RF_RK;                          // divides TB: a piece starts where t % RK == 0
         const int tt = k * TB + t;
         if (t % RK == 0 && tt < p.seqlen) {
           const int nsb = (p.seqlen + RK - 1) / RK;
@@ -448,6 +449,12 @@ __global__ __launch_bounds__(RF_NT) void rf_scan_kernel(RfParams p) {
 #pragma unroll
     for (int q = 0; q < NS; ++q) fo[q] = h[q];
   }
+}
+
+template <typename T, int N, bool GATE>
+__global__ __launch_bounds__(RF_NT) void rf_scan_kernel(RfParams p) {
+  __shared__ RfSmem<N, rf_tb<N>(), rf_cpb<N>()> sm;
+  rf_scan_walk<T, N, GATE, false>(p, sm);
 }
 
 // h_states: sums over the workgroup's 256 channels of every state of group gs (4 states), per token, into
@@ -585,16 +592,20 @@ hipError_t launch_rf_n(const RfParams& p, hipStream_t st) {
 //     ddt_t[c] = (sum_n lam_t A_n a_t h_{t-1} + x_t[c] sum_n lam_t B_t[n]) * d dt / d raw,
 //     dB_t[n]  = sum_c lam_t dt_t[c] x_t[c],      dC_t[n] = sum_c dy_t[c] h_t[c, n],
 //     dA_n     = sum_{t, c} lam_t a_t dt_t[c] h_{t-1},   d h0 = a_0 lam_0,   dD_c = sum_t dy_t[c] x_t[c].
-// Every (c, n) pair follows its own recurrences given the per-token inputs.  The sums over n (dx, ddt) and over c
-// (dB, dC, dA) want opposite layouts, so two kernels walk the sequence backward in pieces of RK tokens from the
-// checkpoints (the state entering each piece, written by the CKPT scan): in each piece the states and decays are
-// recomputed forward into registers, then the adjoint runs backward through them.
-//   rf_bwd_chan_kernel: the scan's layout (a channel's states over LPC lanes, CPB channels per workgroup); the sums
-//     over n on the DPP crossbar; dx, ddt per token, and per (batch, channel) dD, d dt_bias partials and d h0.
-//   rf_bwd_state_kernel: lane = channel (256 per workgroup), 4 states per lane (a workgroup per batch, channel
-//     block and group of 4 states); the sums over c as in rf_hs_kernel; dB, dC per (channel block, token) and dA per
-//     channel block, as partials.
-//   rf_bwd_reduce_kernel / rf_bwd_param_kernel: the partials added in a fixed order (deterministic).
+// Every (c, n) pair follows its own recurrences given the per-token inputs.
+//   rf_sweep_kernel: the state entering every piece of RF_RK tokens (a forward walk) and the adjoint a_{t+1} lam_{t+1}
+//     handed into every piece from its right (a backward walk, which ends with d h0), both directions in one grid: each
+//     is a serial walk that leaves its SIMD waiting on its own for half the time.
+//   rf_grad_kernel: every piece of every channel block by itself.  A wave holds the states of LC channels (4 states a
+//     lane); a piece's states and decays are recomputed forward into registers 8 tokens at a time, the adjoint runs
+//     back through them, and both kinds of sums are formed there: over n (dx, ddt) by a reduce-scatter over the
+//     channel's lanes per 8 tokens, over c (dB, dC, dA) in registers over the channels the wave takes one after the
+//     other, then over the workgroup.
+//   rf_bwd_reduce_kernel / rf_bwd_param_kernel: the channel blocks' and pieces' partials added in a fixed order
+//     (deterministic).
+// Two kernels that each walked the whole sequence backward, one per kind of sum, formed every exponential twice more
+// and left half the issue slots empty: b1 L2048 d_inner 2048 N 128, 1420 us for the three passes where these take
+// RF_MEASURED.
 
 // d dt / d raw for dt = clamp(softplus?(raw + bias), dt_min, dt_max) (the clamp passes the gradient inside its
 // closed range, as torch.clamp does).
@@ -609,429 +620,484 @@ __device__ __forceinline__ float rf_dt_chain(const RfParams& p, float raw, float
   return g;
 }
 
-template <int N, int RK, int CPB>
-struct __align__(16) RfbChanSmem {
-  // 16-byte aligned rows: a lane's consecutive states of B, C and G are 16-byte LDS reads
-  __align__(16) float B[RK][N];
-  __align__(16) float C[RK][N];
-  __align__(16) float G[RK][N];            // G = dhs / d_inner
-  float dt[RK][CPB], chain[RK][CPB], x[RK][CPB], dy[RK][CPB];
-  float dx[RK][CPB], ddt[RK][CPB];
-};
-
-// Piece j's rows into LDS (0 past the end of the sequence).  Every load is unconditional at a clamped (valid)
-// address and masked by a factor 0 afterwards, so that all of a thread's loads are in flight together (a select
-// between a loaded value and 0 lets the compiler put each load behind its own branch and wait); a missing dy or
-// dhs reads x or B instead, times 0 (finite inputs).
-template <typename T, int N, int RK, int CPB>
-__device__ void rfb_load_piece(const RfParams& p, RfbChanSmem<N, RK, CPB>& sm, int b, int c0, int t0) {
-  constexpr int NE = RK * N / RF_NT, NC = (RK * CPB + RF_NT - 1) / RF_NT;
-  static_assert(RK * N % RF_NT == 0, "whole rows of B / C per pass");
-  const int tid = threadIdx.x, L = p.seqlen, di = p.d_inner;
-  const T* Bp = reinterpret_cast<const T*>(p.B) + (int64_t)b * p.B_sb;
-  const T* Cp = reinterpret_cast<const T*>(p.C) + (int64_t)b * p.C_sb;
-  const T* Gp = p.dhs ? reinterpret_cast<const T*>(p.dhs) + (int64_t)b * L * N : Bp;
-  const int64_t gsl = p.dhs ? N : p.B_sl;
-  const float gmul = p.dhs ? 1.f / (float)di : 0.f;
-  T bv[NE], cv[NE], gv[NE];
-#pragma unroll
-  for (int k = 0; k < NE; ++k) {
-    const int e = tid + RF_NT * k, t = e / N, n = e % N, tt = min(t0 + t, L - 1);
-    bv[k] = Bp[(int64_t)tt * p.B_sl + n];
-    cv[k] = Cp[(int64_t)tt * p.C_sl + n];
-    gv[k] = Gp[(int64_t)tt * gsl + n];
-  }
-  const T* xb = reinterpret_cast<const T*>(p.x) + (int64_t)b * p.x_sb;
-  const T* dyb = p.dy ? reinterpret_cast<const T*>(p.dy) + (int64_t)b * L * di : xb;
-  const int64_t dysl = p.dy ? di : p.x_sl;
-  const float dymul = p.dy ? 1.f : 0.f;
-  float raw[NC];
-  T xv[NC], dv[NC];
-#pragma unroll
-  for (int k = 0; k < NC; ++k) {
-    const int e = min(tid + RF_NT * k, RK * CPB - 1), t = e / CPB, cl = e % CPB, tt = min(t0 + t, L - 1);
-    raw[k] = p.dt[(int64_t)b * p.dt_sb + (int64_t)tt * p.dt_sl + c0 + cl];
-    xv[k] = xb[(int64_t)tt * p.x_sl + c0 + cl];
-    dv[k] = dyb[(int64_t)tt * dysl + c0 + cl];
-  }
-  __builtin_amdgcn_sched_barrier(0);   // every load issued before the first use
-#pragma unroll
-  for (int k = 0; k < NE; ++k) {
-    const int e = tid + RF_NT * k, t = e / N, n = e % N;
-    const float in = t0 + t < L ? 1.f : 0.f;
-    sm.B[t][n] = to_f32(bv[k]) * in;
-    sm.C[t][n] = to_f32(cv[k]) * in;
-    sm.G[t][n] = to_f32(gv[k]) * (in * gmul);
-  }
-#pragma unroll
-  for (int k = 0; k < NC; ++k) {
-    const int e = tid + RF_NT * k;
-    if (e < RK * CPB) {
-      const int t = e / CPB, cl = e % CPB;
-      const float in = t0 + t < L ? 1.f : 0.f;
-      const float bias = p.dt_bias ? p.dt_bias[c0 + cl] : 0.f;
-      sm.dt[t][cl] = rf_dt(p, raw[k], bias) * in;
-      sm.chain[t][cl] = rf_dt_chain(p, raw[k], bias) * in;
-      sm.x[t][cl] = to_f32(xv[k]) * in;
-      sm.dy[t][cl] = to_f32(dv[k]) * (in * dymul);
-    }
-  }
-}
-
+// The adjoint walk, last block first, in the scan's layout.  p carries dy in x's place, C in B's and dhs in C's
+// (rf_sweep_kernel); dymul / gmul are 0 where dy / dhs is missing (finite stand-ins are read).
 template <typename T, int N>
-__global__ __launch_bounds__(RF_NT) void rf_bwd_chan_kernel(RfParams p) {
-  constexpr int LPC = rf_lpc<N>(), NS = rf_ns<N>(), CPB = rf_cpb<N>(), RK = rf_rk<N>();
-  __shared__ RfbChanSmem<N, RK, CPB> sm;
+__device__ __forceinline__ void rf_adj_walk(const RfParams& p, RfSmem<N, rf_tb<N>(), rf_cpb<N>()>& sm, float dymul,
+                                            float gmul) {
+  constexpr int TB = rf_tb<N>(), LPC = rf_lpc<N>(), NS = rf_ns<N>(), CPB = rf_cpb<N>(), RK = RF_RK;
   const int nper = p.d_inner / CPB;
-  const int b = blockIdx.x / nper, c0 = (blockIdx.x % nper) * CPB;
+  int b, cb;
+  rf_block(p.batch * nper, nper, b, cb);
+  const int c0 = cb * CPB;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int cl = (64 / LPC) * w + lane / LPC, g = lane % LPC;
-  const int c = c0 + cl, n0 = g * NS, L = p.seqlen, di = p.d_inner;
-  const bool ylane = g == LPC - 1;   // holds the channel's sums over n after the row sums (as in the scan)
-  const int nsb = (L + RK - 1) / RK;
-  float k2[NS], As[NS], lamc[NS];
+  const int c = c0 + cl, n0 = g * NS, L = p.seqlen;
+  const int nblk = (L + TB - 1) / TB, nsb = (L + RK - 1) / RK;
+  float k2[NS], lamc[NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    As[s] = p.A[n0 + s];
-    k2[s] = As[s] * LOG2E;
-    lamc[s] = p.d_final ? p.d_final[((int64_t)b * di + c) * N + n0 + s] : 0.f;
+    k2[s] = p.A[n0 + s] * LOG2E;
+    lamc[s] = p.d_final ? p.d_final[((int64_t)b * p.d_inner + c) * N + n0 + s] : 0.f;
   }
-  const float Dc = p.D ? (p.D_per_channel ? p.D[c] : p.D[c / p.headdim]) : 0.f;
-  float dD_acc = 0.f, db_acc = 0.f;
-  for (int j = nsb - 1; j >= 0; --j) {
-    const int t0 = j * RK;
-    __syncthreads();                   // the previous piece's LDS no longer read
-    rfb_load_piece<T, N, RK, CPB>(p, sm, b, c0, t0);
-    float h[NS];
-    {
-      const float* ck = p.ckpt + (((int64_t)b * nsb + j) * di + c) * N + n0;
+  RfRegs<T, N, TB, CPB> r;
+  float4 bias4 = {0.f, 0.f, 0.f, 0.f};
+  if (p.dt_bias && tid < RfRegs<T, N, TB, CPB>::NQ)
+    bias4 = *reinterpret_cast<const float4*>(p.dt_bias + c0 + 4 * (tid % (CPB / 4)));
+  rf_load<T, N, TB, CPB, false>(p, r, b, c0, (nblk - 1) * TB);
+  rf_store<T, N, TB, CPB, false>(p, r, sm.st[(nblk - 1) & 1], (nblk - 1) * TB, bias4);
+  if (nblk > 1) rf_load<T, N, TB, CPB, false>(p, r, b, c0, (nblk - 2) * TB);
+  __syncthreads();
+  float* ck = p.lam_ckpt + ((int64_t)b * nsb * p.d_inner + c) * N + n0;
+  for (int k = nblk - 1; k >= 0; --k) {
+    const RfStage<N, TB, CPB>& s = sm.st[k & 1];
+#pragma unroll 16
+    for (int t = TB - 1; t >= 0; --t) {
+      const int tt = k * TB + t;                           // (past the end: dt = 0, dy = 0, no dhs)
+      if (t % RK == RK - 1 && tt - (RK - 1) < L) {
+        float* o = ck + (int64_t)(tt / RK) * p.d_inner * N;
 #pragma unroll
-      for (int s = 0; s < NS; ++s) h[s] = ck[s];
+        for (int s2 = 0; s2 < NS; ++s2) o[s2] = lamc[s2];
+      }
+      RfTok<NS> o;
+      rf_tok<N, TB, CPB, NS>(s, t, cl, n0, o);
+      const float dy = o.x * dymul, gm = tt < L ? gmul : 0.f;
+#pragma unroll
+      for (int s2 = 0; s2 < NS; ++s2) {
+        float lam = fmaf(dy, o.b[s2], lamc[s2]);
+        if (gmul != 0.f) lam = fmaf(gm, o.c[s2], lam);
+        lamc[s2] = __builtin_amdgcn_exp2f(o.dt * k2[s2]) * lam;
+      }
     }
+    if (k > 0) rf_store<T, N, TB, CPB, false>(p, r, sm.st[(k - 1) & 1], (k - 1) * TB, bias4);
+    if (k > 1) rf_load<T, N, TB, CPB, false>(p, r, b, c0, (k - 2) * TB);
     __syncthreads();
-    // forward through the piece: the state before every token and every decay
-    float hp[RK][NS], av[RK][NS];
-#pragma unroll
-    for (int t = 0; t < RK; ++t) {
-      const float dtv = sm.dt[t][cl], u = dtv * sm.x[t][cl];
-#pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        const float a = __builtin_amdgcn_exp2f(dtv * k2[s]);
-        hp[t][s] = h[s];
-        av[t][s] = a;
-        h[s] = fmaf(a, h[s], u * sm.B[t][n0 + s]);
-      }
-    }
-    // backward through it
-    if constexpr (LPC == 32 && RK == 16) {
-      // every token's two sums over the states (du, qq) stay one value per lane; after each group of 8 tokens one
-      // reduce-scatter over the channel's 32 lanes leaves lanes 2 m, 2 m + 1 the sum for du (m < 8) or qq (m >= 8)
-      // of token t + m % 8
-      float vv[16];
-#pragma unroll
-      for (int t = RK - 1; t >= 0; --t) {
-        const float dyv = sm.dy[t][cl];
-        float du = 0.f, qq = 0.f;
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-          const float lam = lamc[s] + dyv * sm.C[t][n0 + s] + sm.G[t][n0 + s];
-          du = fmaf(lam, sm.B[t][n0 + s], du);
-          qq = fmaf(lam * As[s], av[t][s] * hp[t][s], qq);
-          lamc[s] = av[t][s] * lam;
-        }
-        vv[t % 8] = du;
-        vv[8 + t % 8] = qq;
-        if (t % 8 == 0) {
-          const float r = rf_reduce_scatter32_16(vv, lane);
-          // v_permlane16_swap of the value with itself: the first row's lanes hold du (first) and, from the second
-          // row, qq (second) of token t + g / 2; its even lanes finish the token
-          const auto pr = __builtin_amdgcn_permlane16_swap(__float_as_uint(r), __float_as_uint(r), false, false);
-          if (g < 16 && (g & 1) == 0) {
-            const int tk = t + (g >> 1);
-            const float du = __uint_as_float(pr[0]), qq = __uint_as_float(pr[1]);
-            const float dyk = sm.dy[tk][cl], dtv = sm.dt[tk][cl], xv = sm.x[tk][cl];
-            const float ddr = (qq + xv * du) * sm.chain[tk][cl];
-            sm.dx[tk][cl] = dtv * du + Dc * dyk;
-            sm.ddt[tk][cl] = ddr;
-            dD_acc = fmaf(dyk, xv, dD_acc);
-            db_acc += ddr;
-          }
-        }
-      }
-    } else {
-#pragma unroll
-    for (int t = RK - 1; t >= 0; --t) {
-      const float dyv = sm.dy[t][cl];
-      float du = 0.f, qq = 0.f;
-#pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        const float lam = lamc[s] + dyv * sm.C[t][n0 + s] + sm.G[t][n0 + s];
-        du = fmaf(lam, sm.B[t][n0 + s], du);
-        qq = fmaf(lam * As[s], av[t][s] * hp[t][s], qq);
-        lamc[s] = av[t][s] * lam;
-      }
-      du = row_sum16(du);
-      qq = row_sum16(qq);
-      if constexpr (LPC == 32) {
-        du += dppf<0x142, 0xa>(du);
-        qq += dppf<0x142, 0xa>(qq);
-      }
-      if (ylane) {
-        const float dtv = sm.dt[t][cl], xv = sm.x[t][cl];
-        const float ddr = (qq + xv * du) * sm.chain[t][cl];
-        sm.dx[t][cl] = dtv * du + Dc * dyv;
-        sm.ddt[t][cl] = ddr;
-        dD_acc = fmaf(dyv, xv, dD_acc);
-        db_acc += ddr;
-      }
-    }
-    }
-    __syncthreads();
-    for (int e = tid; e < RK * CPB; e += RF_NT) {
-      const int t = e / CPB, q = e % CPB, tt = t0 + t;
-      if (tt < L) {
-        const int64_t o = ((int64_t)b * L + tt) * di + c0 + q;
-        reinterpret_cast<T*>(p.dx)[o] = from_f32<T>(sm.dx[t][q]);
-        p.ddt[o] = sm.ddt[t][q];
-      }
-    }
   }
   if (p.dh0) {
-    float* o = p.dh0 + ((int64_t)b * di + c) * N + n0;
+    float* o = p.dh0 + ((int64_t)b * p.d_inner + c) * N + n0;
 #pragma unroll
     for (int s = 0; s < NS; ++s) o[s] = lamc[s];
   }
-  if constexpr (LPC == 32 && RK == 16) {
-    // the first row's lanes hold the channel's partial sums over their tokens
-    dD_acc = row_sum16(dD_acc);
-    db_acc = row_sum16(db_acc);
-    if (g == 0) {
-      p.dD_part[(int64_t)b * di + c] = dD_acc;
-      p.dbias_part[(int64_t)b * di + c] = db_acc;
+}
+
+template <typename T, int N>
+__global__ __launch_bounds__(RF_NT) void rf_sweep_kernel(RfParams p) {
+  __shared__ RfSmem<N, rf_tb<N>(), rf_cpb<N>()> sm;
+  if (blockIdx.y == 0) {
+    rf_scan_walk<T, N, false, true>(p, sm);
+    return;
+  }
+  const float dymul = p.dy ? 1.f : 0.f, gmul = p.dhs ? 1.f / (float)p.d_inner : 0.f;
+  if (p.dy) {
+    p.x = p.dy; p.x_sl = p.d_inner; p.x_sb = (int64_t)p.seqlen * p.d_inner;
+  }
+  p.B = p.C; p.B_sb = p.C_sb; p.B_sl = p.C_sl;
+  if (p.dhs) {
+    p.C = p.dhs; p.C_sl = N; p.C_sb = (int64_t)p.seqlen * N;
+  }
+  rf_adj_walk<T, N>(p, sm, dymul, gmul);
+}
+
+// Lanes and channels of the gradient kernel's waves: 4 states a lane.
+template <int N> constexpr int rfg_ln() { return N / 4; }
+template <int N> constexpr int rfg_lc() { return 64 / rfg_ln<N>(); }
+
+template <int N, bool HASG>
+struct __align__(16) RfGradSmem {
+  float4 sv[RF_RK + 1][RF_CH];         // dt, dt x, dy, x per (token, channel) (0 past the ends); then dx, ddt; the last
+  float chain[RF_RK + 1][RF_CH];       // row is nobody's (lanes that finish no token).  chain: d dt / d raw
+  float D[RF_CH];
+  __align__(16) float B[RF_RK][N], C[RF_RK][N], G[HASG ? RF_RK : 1][N];   // G = dhs / d_inner
+  float4 lam[RF_CH][N / 4];            // the adjoint between the piece's halves
+  float4 red[2][RF_HK][N / 4];         // dB, dC of a half over the workgroup; at the end each wave's dA
+};
+
+// Exchange-and-add over lane bit M: the lanes with the bit set end with the upper half of the K values summed over
+// the pair, the others with the lower half.
+template <int M, int K, int NV>
+__device__ __forceinline__ void rf_halve(float (&v)[NV], int l) {
+  if constexpr (M == 32 || M == 16) {
+#pragma unroll
+    for (int k = 0; k < K / 2; ++k) {
+      if constexpr (M == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[k]), __float_as_uint(v[k + K / 2]), false, false);
+        v[k] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+      } else {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[k]), __float_as_uint(v[k + K / 2]), false, false);
+        v[k] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+      }
     }
-  } else if (ylane) {
-    p.dD_part[(int64_t)b * di + c] = dD_acc;
-    p.dbias_part[(int64_t)b * di + c] = db_acc;
+  } else {
+    rf_rs_step<M, K>(v, l);
+  }
+}
+// The value of lane l ^ M.
+template <int M>
+__device__ __forceinline__ float rf_xor(float v) {
+  if constexpr (M == 8) return xor8(v);
+  else if constexpr (M == 4) return xor4(v);
+  else if constexpr (M == 2) return xor2(v);
+  else return xor1(v);
+}
+// 16 values summed over LN lanes (the low bits of l): lane g of them ends with v[k] the sum of value g K + k,
+// K = 16 / LN (at least 1: lanes g and g ^ 1, .. share one where LN > 16).
+template <int LN>
+__device__ __forceinline__ void rf_sum16(float (&v)[16], int l) {
+  if constexpr (LN == 64) {
+    rf_halve<32, 16>(v, l); rf_halve<16, 8>(v, l); rf_halve<8, 4>(v, l); rf_halve<4, 2>(v, l);
+    v[0] += rf_xor<2>(v[0]);
+    v[0] += rf_xor<1>(v[0]);
+  } else if constexpr (LN == 32) {
+    rf_halve<16, 16>(v, l); rf_halve<8, 8>(v, l); rf_halve<4, 4>(v, l); rf_halve<2, 2>(v, l);
+    v[0] += rf_xor<1>(v[0]);
+  } else if constexpr (LN == 16) {
+    rf_halve<8, 16>(v, l); rf_halve<4, 8>(v, l); rf_halve<2, 4>(v, l); rf_halve<1, 2>(v, l);
+  } else if constexpr (LN == 8) {
+    rf_halve<4, 16>(v, l); rf_halve<2, 8>(v, l); rf_halve<1, 4>(v, l);
+  } else {
+    rf_halve<2, 16>(v, l); rf_halve<1, 8>(v, l);
   }
 }
 
-// lane = channel, states n0 .. n0 + 3 of group gs; the piece's B, C and dhs of those states in LDS.
-template <typename T, int N>
-__global__ __launch_bounds__(RF_NT) void rf_bwd_state_kernel(RfParams p) {
-  constexpr int RK = rf_rk<N>();
-  __shared__ float4 sB[RK], sC[RK], sG[RK];
-  __shared__ float red[4][RK][2 * HS_NS];
+// grid (batch x pieces, channel blocks).  The piece's later half first, for all of the workgroup's channels, then the
+// earlier one (its adjoint waits in LDS): the sums over the channels then hold 64 registers at a time, and with the
+// states and decays of 8 tokens the kernel fits two waves per SIMD (both halves' sums at once spilled 58 registers).
+template <typename T, int N, bool HASG>
+__global__ __launch_bounds__(RF_NT, 2) void rf_grad_kernel(RfParams p) {
+  constexpr int LN = rfg_ln<N>(), LC = rfg_lc<N>(), RK = RF_RK, HK = RF_HK, CH = RF_CH;
+  constexpr int NSTEP = CH / (4 * LC);
+  __shared__ RfGradSmem<N, HASG> sm;
   const int L = p.seqlen, di = p.d_inner;
-  const int ncb = (di + HS_CPB - 1) / HS_CPB, ngs = N / HS_NS;
-  const int i = rf_xcd_block();
-  const int gs = i % ngs, cblk = (i / ngs) % ncb, b = i / (ngs * ncb);
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int c = cblk * HS_CPB + tid;
-  const bool on = c < di;
-  const int cc = on ? c : di - 1;
-  const int n0 = gs * HS_NS, nsb = (L + RK - 1) / RK;
-  const bool u32 = lane & 32, u16 = lane & 16;
-  float k2[HS_NS], As[HS_NS], lamc[HS_NS], dA_acc[HS_NS];
+  const int nsb = (L + RK - 1) / RK, ncb = gridDim.y;
+  const int b = blockIdx.x / nsb, j = blockIdx.x - b * nsb, cb = blockIdx.y;
+  const int t0 = j * RK, c0 = cb * CH;
+  const int tid = threadIdx.x, l = tid & 63, w = wave_id(), gl = l % LN;
+  const int n0 = 4 * gl;
+
+  // ---- the piece's inputs: every load unconditional at a clamped address, masked by factors afterwards
+  {
+    const T* xb = reinterpret_cast<const T*>(p.x) + (int64_t)b * p.x_sb;
+    const T* dyb = p.dy ? reinterpret_cast<const T*>(p.dy) + (int64_t)b * L * di : xb;
+    const int64_t dysl = p.dy ? di : p.x_sl;
+    const float dymul = p.dy ? 1.f : 0.f;
+    const float* dtb = p.dt + (int64_t)b * p.dt_sb;
 #pragma unroll
-  for (int s = 0; s < HS_NS; ++s) {
-    As[s] = p.A[n0 + s];
-    k2[s] = As[s] * LOG2E;
-    lamc[s] = (on && p.d_final) ? p.d_final[((int64_t)b * di + c) * N + n0 + s] : 0.f;
-    dA_acc[s] = 0.f;
+    for (int k = 0; k < RK * CH / RF_NT; ++k) {
+      const int e = tid + RF_NT * k, t = e / CH, q = e % CH, tt = min(t0 + t, L - 1), c = min(c0 + q, di - 1);
+      const float in = (t0 + t < L && c0 + q < di) ? 1.f : 0.f;
+      const float raw = dtb[(int64_t)tt * p.dt_sl + c], bias = p.dt_bias ? p.dt_bias[c] : 0.f;
+      const float x = to_f32(xb[(int64_t)tt * p.x_sl + c]) * in, dy = to_f32(dyb[(int64_t)tt * dysl + c]) * (in * dymul);
+      const float dt = rf_dt(p, raw, bias) * in;
+      sm.sv[t][q] = float4{dt, dt * x, dy, x};
+      sm.chain[t][q] = rf_dt_chain(p, raw, bias) * in;
+    }
+    if (tid < CH) {
+      const int c = c0 + tid;
+      sm.D[tid] = p.D && c < di ? (p.D_per_channel ? p.D[c] : p.D[c / p.headdim]) : 0.f;
+    }
+    const T* Bp = reinterpret_cast<const T*>(p.B) + (int64_t)b * p.B_sb;
+    const T* Cp = reinterpret_cast<const T*>(p.C) + (int64_t)b * p.C_sb;
+#pragma unroll
+    for (int k = 0; k < RK * N / RF_NT; ++k) {
+      const int e = tid + RF_NT * k, t = e / N, n = e % N, tt = min(t0 + t, L - 1);
+      const float in = t0 + t < L ? 1.f : 0.f;
+      sm.B[t][n] = to_f32(Bp[(int64_t)tt * p.B_sl + n]) * in;
+      sm.C[t][n] = to_f32(Cp[(int64_t)tt * p.C_sl + n]) * in;
+      if constexpr (HASG)
+        sm.G[t][n] = to_f32((reinterpret_cast<const T*>(p.dhs) + (int64_t)b * L * N)[(int64_t)tt * N + n]) * (in / (float)di);
+    }
   }
-  const float bias = p.dt_bias ? p.dt_bias[cc] : 0.f;
-  const float inv = 1.f / (float)di;
-  float h[HS_NS];
-  float* dBp = p.dB_part + ((int64_t)b * ncb + cblk) * L * N + n0;
-  float* dCp = p.dC_part + ((int64_t)b * ncb + cblk) * L * N + n0;
-  for (int j = nsb - 1; j >= 0; --j) {
-    const int t0 = j * RK;
-    __syncthreads();                   // the previous piece's LDS no longer read
-    if (tid < RK) {
-      const int tt = t0 + tid;
-      float4 bv = {0.f, 0.f, 0.f, 0.f}, cv = bv, gv = bv;
-      if (tt < L) {
-        const T* bp = reinterpret_cast<const T*>(p.B) + (int64_t)b * p.B_sb + (int64_t)tt * p.B_sl + n0;
-        const T* cp = reinterpret_cast<const T*>(p.C) + (int64_t)b * p.C_sb + (int64_t)tt * p.C_sl + n0;
-        bv = float4{to_f32(bp[0]), to_f32(bp[1]), to_f32(bp[2]), to_f32(bp[3])};
-        cv = float4{to_f32(cp[0]), to_f32(cp[1]), to_f32(cp[2]), to_f32(cp[3])};
-        if (p.dhs) {
-          const T* gp = reinterpret_cast<const T*>(p.dhs) + ((int64_t)b * L + tt) * N + n0;
-          gv = float4{to_f32(gp[0]) * inv, to_f32(gp[1]) * inv, to_f32(gp[2]) * inv, to_f32(gp[3]) * inv};
+  static_assert(RK * CH % RF_NT == 0 && RK * N % RF_NT == 0, "whole passes of the staging");
+  float k2[4], As[4], dA[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    As[i] = p.A[n0 + i];
+    k2[i] = As[i] * LOG2E;
+    dA[i] = 0.f;
+  }
+  __syncthreads();
+  const int64_t prow = ((int64_t)b * nsb + j) * di;
+  if (tid < CH && c0 + tid < di) {
+    float dD = 0.f;
+#pragma unroll
+    for (int t = 0; t < RK; ++t) dD = fmaf(sm.sv[t][tid].z, sm.sv[t][tid].w, dD);
+    p.dD_part[prow + c0 + tid] = dD;
+  }
+  __syncthreads();                                         // dx takes the place of dt below
+
+  auto chan = [&](int s) { return (4 * s + w) * LC + l / LN; };      // channel within the block
+  auto ckpt = [&](const float* base, int q) {
+    return *reinterpret_cast<const float4*>(base + (prow + min(c0 + q, di - 1)) * N + n0);
+  };
+  auto half = [&](auto OFFc) {
+    constexpr int OFF = decltype(OFFc)::value;             // the half's first token
+    float acc[2 * HK * 4];                                 // dB then dC: [token][state] sums over this lane's channels
+#pragma unroll
+    for (int i = 0; i < 2 * HK * 4; ++i) acc[i] = 0.f;
+    float4 hn = ckpt(p.ckpt, chan(0)), ln;
+    if constexpr (OFF > 0) ln = ckpt(p.lam_ckpt, chan(0));
+    int s = 0;
+#pragma unroll 1
+    do {                                                   // (no branch inside: a second copy of the sums at every join)
+      const int q = chan(s);
+      const float on = c0 + q < di ? 1.f : 0.f;            // (a channel past d_inner repeats the last one's states)
+      if constexpr (OFF == 0) ln = sm.lam[q][gl];          // (this wave's own)
+      float h[4] = {hn.x * on, hn.y * on, hn.z * on, hn.w * on};
+      float lamc[4] = {ln.x * on, ln.y * on, ln.z * on, ln.w * on};
+      const int qn = chan(min(s + 1, NSTEP - 1));
+      hn = ckpt(p.ckpt, qn);
+      if constexpr (OFF > 0) ln = ckpt(p.lam_ckpt, qn);
+      const float Dc = sm.D[q];
+      // the B and C rows are the same every step: laundered here, so that they are read from LDS again instead of
+      // held in 128 registers for the whole loop
+      int nl = n0;
+      asm volatile("" : "+v"(nl));
+      // Each token's operands are read one token ahead; the scheduling barriers keep the compiler from reading more
+      // of them at once than the registers hold.
+      struct Tok { float4 v, B; };
+      auto tok = [&](int t) { return Tok{sm.sv[t][q], *reinterpret_cast<const float4*>(&sm.B[t][nl])}; };
+      Tok cur = tok(0);
+      float hp[HK][4], av[HK][4];
+#pragma unroll
+      for (int t = 0; t < OFF + HK; ++t) {                 // from the half's first token on states and decays are kept
+        const Tok nxt = tok(t + 1 < OFF + HK ? t + 1 : t);
+        const float bb[4] = {cur.B.x, cur.B.y, cur.B.z, cur.B.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float a = __builtin_amdgcn_exp2f(cur.v.x * k2[i]);
+          if (t >= OFF) {
+            hp[t >= OFF ? t - OFF : 0][i] = h[i];
+            av[t >= OFF ? t - OFF : 0][i] = a;
+          }
+          h[i] = fmaf(a, h[i], cur.v.y * bb[i]);
+        }
+        cur = nxt;
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      float vv[2 * HK];                                    // du, qq of token t at 2 t, 2 t + 1
+      auto row = [&](const float (*m)[N], int t) { return *reinterpret_cast<const float4*>(&m[t][nl]); };
+      float4 C4 = row(sm.C, OFF + HK - 1), G4 = {0.f, 0.f, 0.f, 0.f};
+      if constexpr (HASG) G4 = row(sm.G, OFF + HK - 1);
+#pragma unroll
+      for (int t = HK - 1; t >= 0; --t) {
+        const int tn = OFF + (t > 0 ? t - 1 : 0);
+        const Tok nxt = tok(tn);
+        const float4 Cn = row(sm.C, tn);
+        float4 Gn = G4;
+        if constexpr (HASG) Gn = row(sm.G, tn);
+        const float4 v = cur.v;
+        const float bb[4] = {cur.B.x, cur.B.y, cur.B.z, cur.B.w}, cc[4] = {C4.x, C4.y, C4.z, C4.w};
+        const float gg[4] = {G4.x * on, G4.y * on, G4.z * on, G4.w * on};
+        float du = 0.f, qq = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float lam = fmaf(v.z, cc[i], lamc[i]);
+          if constexpr (HASG) lam += gg[i];
+          du = fmaf(lam, bb[i], du);
+          acc[4 * t + i] = fmaf(lam, v.y, acc[4 * t + i]);
+          acc[4 * (HK + t) + i] = fmaf(v.z, t + 1 < HK ? hp[t + 1 < HK ? t + 1 : 0][i] : h[i], acc[4 * (HK + t) + i]);
+          lamc[i] = av[t][i] * lam;
+          const float pz = lamc[i] * hp[t][i];             // lam a h_{t-1}
+          qq = fmaf(pz, As[i], qq);
+          dA[i] = fmaf(pz, v.x, dA[i]);
+        }
+        vv[2 * t] = du;
+        vv[2 * t + 1] = qq;
+        cur = nxt;
+        C4 = Cn;
+        G4 = Gn;
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (OFF > 0) sm.lam[q][gl] = float4{lamc[0], lamc[1], lamc[2], lamc[3]};
+      rf_sum16<LN>(vv, l);
+      // the lane that finishes a token: it holds (or its partner hands it) du and qq
+      auto finish = [&](int t, float du, float qq) {
+        const float4 v = sm.sv[t][q];
+        sm.sv[t][q].x = fmaf(v.x, du, Dc * v.z);
+        sm.sv[t][q].y = fmaf(v.w, du, qq) * sm.chain[t][q];
+      };
+      if constexpr (LN >= 16) {
+        constexpr int P = LN / 16;                         // lanes sharing a value
+        const float other = rf_xor<P>(vv[0]);
+        finish(gl % (2 * P) == 0 ? OFF + gl / (2 * P) : RK, vv[0], other);
+      } else {
+        constexpr int K = 16 / LN;
+#pragma unroll
+        for (int k = 0; k < K; k += 2) finish(OFF + (gl * K + k) / 2, vv[k], vv[k + 1]);
+      }
+    } while (++s < NSTEP);
+
+    // ---- sums over the channels: over the wave's LC channel groups, then over the 4 waves in order
+    constexpr int V = 2 * HK * 4 / LC;                     // values per lane afterwards, from index (l / LN) V
+    if constexpr (LC >= 2) rf_halve<32, 64>(acc, l);
+    if constexpr (LC >= 4) rf_halve<16, 32>(acc, l);
+    if constexpr (LC >= 8) rf_halve<8, 16>(acc, l);
+    if constexpr (LC >= 16) rf_halve<4, 8>(acc, l);
+    float4* red = &sm.red[0][0][0];
+    const int base = (l / LN) * (V / 4);                   // in 4-state rows: which * HK + token
+#pragma unroll 1
+    for (int k = 0; k < 4; ++k) {
+      if (w == k) {
+#pragma unroll
+        for (int r = 0; r < V / 4; ++r) {
+          float4 a = {acc[4 * r], acc[4 * r + 1], acc[4 * r + 2], acc[4 * r + 3]};
+          float4* d = red + (base + r) * (N / 4) + gl;
+          if (k) {
+            const float4 o = *d;
+            a = float4{o.x + a.x, o.y + a.y, o.z + a.z, o.w + a.w};
+          }
+          *d = a;
         }
       }
-      sB[tid] = bv;
-      sC[tid] = cv;
-      sG[tid] = gv;
+      __syncthreads();
     }
-    // this lane's channel for the piece's tokens: unconditional loads at clamped addresses, masked by factors
-    // (a missing dy reads x, times 0), so that they are all in flight together
-    float dtv[RK], xv[RK], dyv[RK];
-    {
-      float raw[RK];
-      T xr[RK], dr[RK];
-      const T* xb = reinterpret_cast<const T*>(p.x) + (int64_t)b * p.x_sb + cc;
-      const T* dyb = p.dy ? reinterpret_cast<const T*>(p.dy) + (int64_t)b * L * di + cc : xb;
-      const int64_t dysl = p.dy ? di : p.x_sl;
-#pragma unroll
-      for (int t = 0; t < RK; ++t) {
-        const int tt = min(t0 + t, L - 1);
-        raw[t] = p.dt[(int64_t)b * p.dt_sb + (int64_t)tt * p.dt_sl + cc];
-        xr[t] = xb[(int64_t)tt * p.x_sl];
-        dr[t] = dyb[(int64_t)tt * dysl];
-      }
-      const float4 hv = *reinterpret_cast<const float4*>(p.ckpt + (((int64_t)b * nsb + j) * di + cc) * N + n0);
-      h[0] = hv.x; h[1] = hv.y; h[2] = hv.z; h[3] = hv.w;
-      __builtin_amdgcn_sched_barrier(0);   // every load issued before the first use
-      const float dymul = p.dy ? 1.f : 0.f;
-#pragma unroll
-      for (int t = 0; t < RK; ++t) {
-        const float in = (on && t0 + t < L) ? 1.f : 0.f;
-        dtv[t] = rf_dt(p, raw[t], bias) * in;
-        xv[t] = to_f32(xr[t]) * in;
-        dyv[t] = to_f32(dr[t]) * (in * dymul);
-      }
+    const float* rf = reinterpret_cast<const float*>(red);
+    for (int e = tid; e < 2 * HK * N; e += RF_NT) {
+      const int t = t0 + OFF + (e / N) % HK, n = e % N;
+      if (t < L) (e < HK * N ? p.dB_part : p.dC_part)[(((int64_t)b * ncb + cb) * L + t) * N + n] = rf[e];
     }
-    __syncthreads();
-    // forward through the piece: the state after every token (hs[t]) and every decay; hs[-1] = the entry state
-    float he[HS_NS], hs[RK][HS_NS], av[RK][HS_NS];
+    __syncthreads();                                       // red is written again
+  };
+  half(std::integral_constant<int, HK>{});
+  half(std::integral_constant<int, 0>{});
+
+  float* dAw = reinterpret_cast<float*>(&sm.red[0][0][0]);
 #pragma unroll
-    for (int s = 0; s < HS_NS; ++s) he[s] = h[s];
-#pragma unroll
-    for (int t = 0; t < RK; ++t) {
-      const float4 b4 = sB[t];
-      const float bb[HS_NS] = {b4.x, b4.y, b4.z, b4.w};
-      const float u = dtv[t] * xv[t];
-#pragma unroll
-      for (int s = 0; s < HS_NS; ++s) {
-        const float a = __builtin_amdgcn_exp2f(dtv[t] * k2[s]);
-        av[t][s] = a;
-        h[s] = fmaf(a, h[s], u * bb[s]);
-        hs[t][s] = h[s];
-      }
-    }
-    // the piece's tokens backwards, in groups of 4: each token's 4-vectors of the dB and dC sums stay one value
-    // per lane (v[4 ti + s] and v[16 + 4 ti + s]) and one reduce-scatter over the wave's 64 channels after the
-    // group leaves lanes 2 m, 2 m + 1 the sum for (dB | dC by m / 16, token t + (m % 16) / 4, state m % 4)
-    static_assert(RK % 4 == 0, "whole groups of 4 tokens");
-    float v[32];
-#pragma unroll
-    for (int t = RK - 1; t >= 0; --t) {
-      const float4 c4 = sC[t], g4 = sG[t];
-      const float cv[HS_NS] = {c4.x, c4.y, c4.z, c4.w}, gv[HS_NS] = {g4.x, g4.y, g4.z, g4.w};
-      const float dx_ = dtv[t] * xv[t];
-      const int ti = t % 4;
-#pragma unroll
-      for (int s = 0; s < HS_NS; ++s) {
-        const float lam = lamc[s] + dyv[t] * cv[s] + gv[s];
-        const float hprev = t > 0 ? hs[t - 1][s] : he[s];
-        v[HS_NS * ti + s] = lam * dx_;
-        v[16 + HS_NS * ti + s] = dyv[t] * hs[t][s];
-        dA_acc[s] = fmaf(lam * av[t][s], dtv[t] * hprev, dA_acc[s]);
-        lamc[s] = av[t][s] * lam;
-      }
-      if (ti == 0) {
-        const float r = rf_reduce_scatter64_32(v, lane);
-        const int m = lane >> 1;
-        if ((lane & 1) == 0) red[w][t + ((m & 15) >> 2)][HS_NS * (m >> 4) + (m & 3)] = r;
-      }
-    }
-    __syncthreads();
-    if (tid < RK * 2 * HS_NS) {
-      const int t = tid / (2 * HS_NS), k = tid % (2 * HS_NS), tt = t0 + t;
-      if (tt < L) {
-        const float v = red[0][t][k] + red[1][t][k] + red[2][t][k] + red[3][t][k];
-        (k < HS_NS ? dBp : dCp)[(int64_t)tt * N + (k % HS_NS)] = v;
-      }
-    }
+  for (int i = 0; i < 4; ++i) {
+    if constexpr (LC >= 2) dA[i] = sum_halves(dA[i]);
+    if constexpr (LC >= 4) dA[i] += __shfl_xor(dA[i], 16, 64);
+    if constexpr (LC >= 8) dA[i] += xor8(dA[i]);
+    if constexpr (LC >= 16) dA[i] += xor4(dA[i]);
+    if (l < LN) dAw[w * N + n0 + i] = dA[i];
   }
-  // dA over the workgroup's channels: the same reduce-scatter, then the 4 waves in order
-  {
-    float v2[2];
+  __syncthreads();
+  if (tid < N)
+    p.dA_part[(((int64_t)b * nsb + j) * ncb + cb) * N + tid] = dAw[tid] + dAw[N + tid] + dAw[2 * N + tid] + dAw[3 * N + tid];
+  if (tid < CH && c0 + tid < di) {
+    float db = 0.f;
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const auto pr = __builtin_amdgcn_permlane32_swap(__float_as_uint(dA_acc[k]), __float_as_uint(dA_acc[k + 2]),
-                                                       false, false);
-      v2[k] = __uint_as_float(pr[0]) + __uint_as_float(pr[1]);
+    for (int t = 0; t < RK; ++t) db += sm.sv[t][tid].y;
+    p.dbias_part[prow + c0 + tid] = db;
+  }
+#pragma unroll
+  for (int k = 0; k < RK * CH / RF_NT; ++k) {
+    const int e = tid + RF_NT * k, t = e / CH, q = e % CH;
+    if (t0 + t < L && c0 + q < di) {
+      const int64_t o = ((int64_t)b * L + t0 + t) * di + c0 + q;
+      const float4 v = sm.sv[t][q];
+      reinterpret_cast<T*>(p.dx)[o] = from_f32<T>(v.x);
+      p.ddt[o] = v.y;
     }
-    const auto pr = __builtin_amdgcn_permlane16_swap(__float_as_uint(v2[0]), __float_as_uint(v2[1]), false, false);
-    float v1 = __uint_as_float(pr[0]) + __uint_as_float(pr[1]);
-    v1 = row_sum16(v1);
-    __syncthreads();
-    if ((lane & 15) == 0) red[w][0][2 * (int)u32 + (int)u16] = v1;
-    __syncthreads();
-    if (tid < HS_NS)
-      p.dA_part[((int64_t)b * ncb + cblk) * N + n0 + tid] = red[0][0][tid] + red[1][0][tid] + red[2][0][tid] +
-                                                            red[3][0][tid];
   }
 }
 
 // dB, dC (b, L, N) = the channel blocks' partials added in order.
 template <typename T>
-__global__ __launch_bounds__(256) void rf_bwd_reduce_kernel(RfParams p) {
-  const int ncb = (p.d_inner + HS_CPB - 1) / HS_CPB;
-  const int64_t per = (int64_t)p.seqlen * p.dstate;
+__global__ __launch_bounds__(256) void rf_bwd_reduce_kernel(RfParams p, int ncb) {
+  const int64_t per = (int64_t)p.seqlen * p.dstate / 4;
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= (int64_t)p.batch * per) return;
   const int64_t b = i / per, r = i % per;
-  float sb = 0.f, sc = 0.f;
+  const f32x4* pb = reinterpret_cast<const f32x4*>(p.dB_part);
+  const f32x4* pc = reinterpret_cast<const f32x4*>(p.dC_part);
+  f32x4 sb = {0.f, 0.f, 0.f, 0.f}, sc = sb;
+#pragma unroll 8
   for (int k = 0; k < ncb; ++k) {
-    sb += p.dB_part[(b * ncb + k) * per + r];
-    sc += p.dC_part[(b * ncb + k) * per + r];
+    sb += pb[(b * ncb + k) * per + r];
+    sc += pc[(b * ncb + k) * per + r];
   }
-  reinterpret_cast<T*>(p.dB)[i] = from_f32<T>(sb);
-  reinterpret_cast<T*>(p.dC)[i] = from_f32<T>(sc);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    reinterpret_cast<T*>(p.dB)[4 * i + j] = from_f32<T>(sb[j]);
+    reinterpret_cast<T*>(p.dC)[4 * i + j] = from_f32<T>(sc[j]);
+  }
 }
 
-// dA (N), dD (like D) and d dt_bias (d_inner): partials added over batch rows (and channel blocks) in order.
-__global__ __launch_bounds__(256) void rf_bwd_param_kernel(RfParams p) {
+// Sum over rows r of part[r][i] for column i of `cols`, by the 16 threads of a column (rows t, t + 16, .. in order, then
+// the 16 sums in order): a workgroup takes 16 columns.
+__device__ __forceinline__ float rf_column_sum(const float* part, int64_t rows, int64_t cols, int i, bool on,
+                                               float (&red)[16][17]) {
+  const int t = threadIdx.x >> 4, q = threadIdx.x & 15;
+  float s = 0.f;
+  if (on)
+#pragma unroll 4
+    for (int64_t r = t; r < rows; r += 16) s += part[r * cols + i];
+  __syncthreads();
+  red[t][q] = s;
+  __syncthreads();
+  float a = 0.f;
+#pragma unroll
+  for (int k = 0; k < 16; ++k) a += red[k][q];
+  return a;
+}
+
+// dA (N): partials per (batch, piece, channel block); dD per channel and d dt_bias (d_inner): per (batch, piece).  One
+// workgroup per 16 columns, dA's first; with D per head the channel sums go to dD_sum and rf_bwd_head_kernel adds a
+// head's channels.
+__global__ __launch_bounds__(256) void rf_bwd_param_kernel(RfParams p, int ncb, int na) {
+  __shared__ float red[16][17];
+  const int di = p.d_inner, N = p.dstate, q = threadIdx.x & 15;
+  const int nsb = (p.seqlen + RF_RK - 1) / RF_RK;
+  const int64_t rows = (int64_t)p.batch * nsb;
+  if ((int)blockIdx.x < na) {
+    const int i = blockIdx.x * 16 + q;
+    const float a = rf_column_sum(p.dA_part, rows * ncb, N, i, i < N, red);
+    if (threadIdx.x < 16 && i < N) p.dA[i] = a;
+    return;
+  }
+  const int i = (blockIdx.x - na) * 16 + q;
+  const float d = rf_column_sum(p.dD_part, rows, di, i, i < di, red);
+  const float s = rf_column_sum(p.dbias_part, rows, di, i, i < di, red);
+  if (threadIdx.x < 16 && i < di) {
+    if (p.d_dt_bias) p.d_dt_bias[i] = s;
+    if (p.dD) (p.D_per_channel ? p.dD : p.dD_sum)[i] = d;
+  }
+}
+
+__global__ __launch_bounds__(256) void rf_bwd_head_kernel(RfParams p) {
   const int i = blockIdx.x * 256 + threadIdx.x;
-  const int di = p.d_inner, N = p.dstate, ncb = (di + HS_CPB - 1) / HS_CPB;
-  if (i < N) {
-    float s = 0.f;
-    for (int k = 0; k < p.batch * ncb; ++k) s += p.dA_part[(int64_t)k * N + i];
-    p.dA[i] = s;
-  }
-  if (i < di) {
-    float sd = 0.f, sb = 0.f;
-    for (int b = 0; b < p.batch; ++b) {
-      sd += p.dD_part[(int64_t)b * di + i];
-      sb += p.dbias_part[(int64_t)b * di + i];
-    }
-    if (p.d_dt_bias) p.d_dt_bias[i] = sb;
-    if (p.dD && p.D_per_channel) p.dD[i] = sd;
-  }
-  if (p.dD && !p.D_per_channel && i < di / p.headdim) {     // D per head: its channels' sums
-    float sd = 0.f;
-    for (int b = 0; b < p.batch; ++b)
-      for (int q = 0; q < p.headdim; ++q) sd += p.dD_part[(int64_t)b * di + i * p.headdim + q];
-    p.dD[i] = sd;
-  }
+  if (i >= p.d_inner / p.headdim) return;
+  float sd = 0.f;
+  for (int q = 0; q < p.headdim; ++q) sd += p.dD_sum[i * p.headdim + q];
+  p.dD[i] = sd;
+}
+
+// Empty sequence: every sum is zero and d h0 is d_final.
+__global__ __launch_bounds__(256) void rf_bwd_empty_kernel(RfParams p) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int di = p.d_inner;
+  if (i < p.dstate) p.dA[i] = 0.f;
+  if (p.d_dt_bias && i < di) p.d_dt_bias[i] = 0.f;
+  if (p.dD && i < (p.D_per_channel ? di : di / p.headdim)) p.dD[i] = 0.f;
+  if (p.dh0 && i < (int64_t)p.batch * di * p.dstate) p.dh0[i] = p.d_final ? p.d_final[i] : 0.f;
 }
 
 template <typename T, int N>
 hipError_t launch_rf_bwd_t(const RfParams& p, hipStream_t st) {
-  const int nblk = p.batch * (p.d_inner / rf_cpb<N>());
-  if (p.seqlen > 0) {
-    hipLaunchKernelGGL((rf_scan_kernel<T, N, false, true>), dim3(nblk), dim3(RF_NT), 0, st, p);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+  if (p.seqlen == 0) {
+    const int64_t n = std::max<int64_t>(p.dh0 ? (int64_t)p.batch * p.d_inner * N : 0, std::max(p.d_inner, N));
+    hipLaunchKernelGGL(rf_bwd_empty_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, p);
+    return hipGetLastError();
   }
-  hipLaunchKernelGGL((rf_bwd_chan_kernel<T, N>), dim3(nblk), dim3(RF_NT), 0, st, p);
+  hipLaunchKernelGGL((rf_sweep_kernel<T, N>), dim3(p.batch * (p.d_inner / rf_cpb<N>()), 2), dim3(RF_NT), 0, st, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const int ncb = (p.d_inner + HS_CPB - 1) / HS_CPB;
-  hipLaunchKernelGGL((rf_bwd_state_kernel<T, N>), dim3(p.batch * ncb * (N / HS_NS)), dim3(RF_NT), 0, st, p);
+  const int ncb = (p.d_inner + RF_CH - 1) / RF_CH;
+  const int nsb = (p.seqlen + RF_RK - 1) / RF_RK;
+  const dim3 grid((unsigned)(nsb * p.batch), (unsigned)ncb);
+  if (p.dhs) hipLaunchKernelGGL((rf_grad_kernel<T, N, true>), grid, dim3(RF_NT), 0, st, p);
+  else hipLaunchKernelGGL((rf_grad_kernel<T, N, false>), grid, dim3(RF_NT), 0, st, p);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const int64_t tot = (int64_t)p.batch * p.seqlen * N;
-  if (tot > 0) {
-    hipLaunchKernelGGL((rf_bwd_reduce_kernel<T>), dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st, p);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  const int np = p.d_inner > N ? p.d_inner : N;
-  hipLaunchKernelGGL(rf_bwd_param_kernel, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, st, p);
+  const int64_t tot = (int64_t)p.batch * p.seqlen * N / 4;
+  hipLaunchKernelGGL((rf_bwd_reduce_kernel<T>), dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st, p, ncb);
+  e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  const int na = (N + 15) / 16;
+  hipLaunchKernelGGL(rf_bwd_param_kernel, dim3((unsigned)(na + (p.d_inner + 15) / 16)), dim3(256), 0, st, p, ncb, na);
+  e = hipGetLastError();
+  if (e != hipSuccess || !p.dD || p.D_per_channel) return e;
+  hipLaunchKernelGGL(rf_bwd_head_kernel, dim3((unsigned)((p.d_inner / p.headdim + 255) / 256)), dim3(256), 0, st, p);
   return hipGetLastError();
 }
 
@@ -1064,32 +1130,38 @@ hipError_t launch_ssd_rf(const RfParams& p, hipStream_t st) {
   return launch_rf_n<float>(p, st);
 }
 
-// Backward workspace: the checkpoints (b, pieces, d_inner, N), the dB and dC partials (b, channel blocks, L, N),
-// the dA partials (b, channel blocks, N), and the dD / d dt_bias partials (b, d_inner), all fp32.
-static size_t rf_rk_of(int dstate) { return dstate == 256 ? 8 : 16; }
+// Backward workspace, all fp32: the states and adjoints entering every piece (b, pieces, d_inner, N) each, the dB and
+// dC partials (b, channel blocks, L, N), the dA partials (b, pieces, channel blocks, N), the dD / d dt_bias partials
+// (b, pieces, d_inner) and the channels' dD sums (d_inner).
+struct RfBwdWorkspace {
+  size_t ck, part, da, dd, ds;
+  RfBwdWorkspace(size_t batch, size_t seqlen, size_t d_inner, size_t dstate) {
+    const size_t nsb = (seqlen + RF_RK - 1) / RF_RK, ncb = (d_inner + RF_CH - 1) / RF_CH;
+    ck = align256(batch * nsb * d_inner * dstate * 4);
+    part = align256(batch * ncb * seqlen * dstate * 4);
+    da = align256(batch * nsb * ncb * dstate * 4);
+    dd = align256(batch * nsb * d_inner * 4);
+    ds = align256(d_inner * 4);
+  }
+};
 
 size_t ssd_rf_bwd_workspace_bytes(int batch, int seqlen, int d_inner, int dstate) {
-  const size_t rk = rf_rk_of(dstate), nsb = (seqlen + rk - 1) / rk;
-  const size_t ncb = (size_t)(d_inner + HS_CPB - 1) / HS_CPB;
-  return align256((size_t)batch * nsb * d_inner * dstate * 4) + 2 * align256((size_t)batch * ncb * seqlen * dstate * 4) +
-         align256((size_t)batch * ncb * dstate * 4) + 2 * align256((size_t)batch * d_inner * 4);
+  const RfBwdWorkspace s(batch, seqlen, d_inner, dstate);
+  return 2 * s.ck + 2 * s.part + s.da + 2 * s.dd + s.ds;
 }
 
 void ssd_rf_bwd_layout(RfParams& p, void* workspace) {
-  const size_t rk = rf_rk_of(p.dstate), nsb = (p.seqlen + rk - 1) / rk;
-  const size_t ncb = (size_t)(p.d_inner + HS_CPB - 1) / HS_CPB;
+  const RfBwdWorkspace s(p.batch, p.seqlen, p.d_inner, p.dstate);
   char* w = reinterpret_cast<char*>(workspace);
-  p.ckpt = reinterpret_cast<float*>(w);
-  w += align256((size_t)p.batch * nsb * p.d_inner * p.dstate * 4);
-  p.dB_part = reinterpret_cast<float*>(w);
-  w += align256((size_t)p.batch * ncb * p.seqlen * p.dstate * 4);
-  p.dC_part = reinterpret_cast<float*>(w);
-  w += align256((size_t)p.batch * ncb * p.seqlen * p.dstate * 4);
-  p.dA_part = reinterpret_cast<float*>(w);
-  w += align256((size_t)p.batch * ncb * p.dstate * 4);
-  p.dD_part = reinterpret_cast<float*>(w);
-  w += align256((size_t)p.batch * p.d_inner * 4);
-  p.dbias_part = reinterpret_cast<float*>(w);
+  auto take = [&](size_t n) { char* r = w; w += n; return reinterpret_cast<float*>(r); };
+  p.ckpt = take(s.ck);
+  p.lam_ckpt = take(s.ck);
+  p.dB_part = take(s.part);
+  p.dC_part = take(s.part);
+  p.dA_part = take(s.da);
+  p.dD_part = take(s.dd);
+  p.dbias_part = take(s.dd);
+  p.dD_sum = take(s.ds);
 }
 
 hipError_t launch_ssd_rf_bwd(const RfParams& p, hipStream_t st) {
