@@ -1,7 +1,7 @@
 // The reference's own selective scan (mamformer/layers/mamba2.py:70-130) for gfx950: a decay rate per state
 // column and a step size per channel,
 //     h_t[c, n] = exp(A_n dt_t[c]) h_{t-1}[c, n] + dt_t[c] x_t[c] B_t[n],   y_t[c] = sum_n C_t[n] h_t[c, n] + D_c x_t[c]
-// with A_n = -exp(clamp(A_log_n, -5, 5)) formed by the caller.  The decay differs per (channel, state), so the
+// with A_n = -exp(clamp(A_log_n, -5, 5)), formed by the caller.  The decay differs per (channel, state), so the
 // recurrence has no matrix-unit factorisation (the per-head SSD form does): every (token, channel, state) costs
 // one exponential and a few fused multiply-adds, and the kernels are bound by that VALU work.
 //
@@ -10,8 +10,10 @@
 //   that forms y runs on the DPP crossbar (quad permutes, the row mirrors, then the row-15 broadcast that adds
 //   the two rows of a channel); a wave holds 2 channels, a workgroup of 4 waves 8.  Blocks of TB tokens of B, C
 //   (fp32), dt, x and the gate are staged in LDS (two stages; the next block's rows are loaded into registers
-//   while the current block computes, and each token's LDS values are read one token ahead), y is collected per
-//   block in LDS and stored as rows of the workgroup's channels.
+//   while the current block computes, and each token's LDS values are read two tokens ahead), y is collected per
+//   block in LDS and stored as rows of the workgroup's channels.  A wave has its SIMD to itself, so what it waits
+//   for nobody fills: with the reads one token ahead and softplus on one wave of four, b1 L2048 d_inner 2048 N 128
+//   took 231 us, now 171.
 // rf_hs_kernel (h_states, the per-token mean of the state over all channels, mamba2.py:114-116):
 //   lane = channel (256 channels per workgroup), a workgroup per (batch, channel block, group of 4 states), so
 //   that the sum over channels is a reduce-scatter inside the wave (v_permlane32_swap, v_permlane16_swap, then the
@@ -205,15 +207,18 @@ struct RfSmem {
 };
 
 // The rows of one token block held in registers between its load and its LDS store: thread i owns the 8-element
-// pieces i, i + 256, .. of B and of C (TB rows of N), and, for i < TB * CPB / 4, one 4-element piece of dt, x, z.
+// pieces i, i + 256, .. of B and of C (TB rows of N), and the elements i, i + 256, .. of dt, x and z (one element per
+// thread rather than 4 of a quarter of them: the softplus of dt then runs on every wave, not on one while three wait).
 template <typename T, int N, int TB, int CPB>
 struct RfRegs {
   static constexpr int NP = TB * N / 8;                     // 8-element pieces of B (and of C) per block
   static constexpr int PB = (NP + RF_NT - 1) / RF_NT;      // per thread
-  static constexpr int NQ = TB * CPB / 4;                  // 4-element pieces of dt (x, z) per block
+  static constexpr int NQ = TB * CPB;                      // elements of dt (x, z) per block
+  static constexpr int PQ = (NQ + RF_NT - 1) / RF_NT;      // per thread
+  static_assert(RF_NT % CPB == 0, "a thread's elements are of one channel");
   Row8<T> b[PB], c[PB];
-  float4 dt;                   // raw dt; processed (bias, softplus, clamp, 0 past the end) by rf_store
-  T xv[4], zv[4];              // raw x and gate
+  float dt[PQ];                // raw dt; processed (bias, softplus, clamp, 0 past the end) by rf_store
+  T xv[PQ], zv[PQ];            // raw x and gate
 };
 
 // Workgroup -> (batch, channel block): runs of 4 consecutive blocks go to the same XCD (workgroups are dealt to
@@ -238,7 +243,8 @@ __device__ __forceinline__ int rf_xcd_block() {
 
 // Loads only (every one unconditional at a clamped row), so that they stay in flight while the current block
 // computes: the values are converted, masked and stored to LDS by rf_store a block later.
-template <typename T, int N, int TB, int CPB, bool GATE>
+// ANYC: C's rows are read element by element (the backward's dhs in its place is aligned to its elements only).
+template <typename T, int N, int TB, int CPB, bool GATE, bool ANYC = false>
 __device__ __forceinline__ void rf_load(const RfParams& p, RfRegs<T, N, TB, CPB>& r, int b, int c0, int t0) {
   using R = RfRegs<T, N, TB, CPB>;
   const int tid = threadIdx.x;
@@ -250,28 +256,31 @@ __device__ __forceinline__ void rf_load(const RfParams& p, RfRegs<T, N, TB, CPB>
     const int e = min(tid + q * RF_NT, R::NP - 1);        // piece: row e / (N / 8), columns 8 (e % (N / 8))
     const int row = min(t0 + e / (N / 8), last), col = 8 * (e % (N / 8));
     r.b[q].load(Bp + (int64_t)row * p.B_sl + col);
-    r.c[q].load(Cp + (int64_t)row * p.C_sl + col);
-  }
-  if (tid < R::NQ) {
-    const int row = t0 + tid / (CPB / 4), col = 4 * (tid % (CPB / 4));
-    const int rr = min(row, last);
-    r.dt = *reinterpret_cast<const float4*>(p.dt + (int64_t)b * p.dt_sb + (int64_t)rr * p.dt_sl + c0 + col);
-    const T* xp = reinterpret_cast<const T*>(p.x) + (int64_t)b * p.x_sb + (int64_t)rr * p.x_sl + c0 + col;
+    const T* cp = Cp + (int64_t)row * p.C_sl + col;
+    if constexpr (ANYC) {
+      float v[8];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) r.xv[j] = xp[j];
-    if constexpr (GATE) {
-      const T* zp = reinterpret_cast<const T*>(p.z) + (int64_t)b * p.z_sb + (int64_t)rr * p.z_sl + c0 + col;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) r.zv[j] = zp[j];
+      for (int j = 0; j < 8; ++j) v[j] = to_f32(cp[j]);
+      r.c[q].set(v);
+    } else {
+      r.c[q].load(cp);
     }
+  }
+#pragma unroll
+  for (int q = 0; q < R::PQ; ++q) {
+    const int e = min(tid + q * RF_NT, R::NQ - 1);        // element: row e / CPB, channel e % CPB
+    const int rr = min(t0 + e / CPB, last), col = c0 + e % CPB;
+    r.dt[q] = p.dt[(int64_t)b * p.dt_sb + (int64_t)rr * p.dt_sl + col];
+    r.xv[q] = (reinterpret_cast<const T*>(p.x) + (int64_t)b * p.x_sb)[(int64_t)rr * p.x_sl + col];
+    if constexpr (GATE) r.zv[q] = (reinterpret_cast<const T*>(p.z) + (int64_t)b * p.z_sb)[(int64_t)rr * p.z_sl + col];
   }
 }
 
-// The block at t0 into LDS: B and C as fp32; dt processed with the thread's 4 channels' bias (bias4), dt and x 0
+// The block at t0 into LDS: B and C as fp32; dt processed with the thread's channel's bias, dt and x 0
 // past the end of the sequence.
 template <typename T, int N, int TB, int CPB, bool GATE>
 __device__ __forceinline__ void rf_store(const RfParams& p, const RfRegs<T, N, TB, CPB>& r, RfStage<N, TB, CPB>& s,
-                                         int t0, const float4& bias4) {
+                                         int t0, float bias) {
   using R = RfRegs<T, N, TB, CPB>;
   const int tid = threadIdx.x;
 #pragma unroll
@@ -281,17 +290,15 @@ __device__ __forceinline__ void rf_store(const RfParams& p, const RfRegs<T, N, T
     r.b[q].store_f32(&s.B[e / (N / 8)][8 * (e % (N / 8))]);
     r.c[q].store_f32(&s.C[e / (N / 8)][8 * (e % (N / 8))]);
   }
-  if (tid < R::NQ) {
-    const int row = tid / (CPB / 4), col = 4 * (tid % (CPB / 4));
+#pragma unroll
+  for (int q = 0; q < R::PQ; ++q) {
+    const int e = tid + q * RF_NT;
+    if (R::NQ % RF_NT != 0 && e >= R::NQ) break;
+    const int row = e / CPB, col = e % CPB;
     const float in = t0 + row < p.seqlen ? 1.f : 0.f;
-    *reinterpret_cast<float4*>(&s.dt[row][col]) =
-        float4{rf_dt(p, r.dt.x, bias4.x) * in, rf_dt(p, r.dt.y, bias4.y) * in, rf_dt(p, r.dt.z, bias4.z) * in,
-               rf_dt(p, r.dt.w, bias4.w) * in};
-    *reinterpret_cast<float4*>(&s.x[row][col]) =
-        float4{to_f32(r.xv[0]) * in, to_f32(r.xv[1]) * in, to_f32(r.xv[2]) * in, to_f32(r.xv[3]) * in};
-    if constexpr (GATE)
-      *reinterpret_cast<float4*>(&s.z[row][col]) =
-          float4{to_f32(r.zv[0]), to_f32(r.zv[1]), to_f32(r.zv[2]), to_f32(r.zv[3])};
+    s.dt[row][col] = rf_dt(p, r.dt[q], bias) * in;
+    s.x[row][col] = to_f32(r.xv[q]) * in;
+    if constexpr (GATE) s.z[row][col] = to_f32(r.zv[q]);
   }
 }
 
@@ -346,12 +353,10 @@ __device__ __forceinline__ void rf_scan_walk(const RfParams& p, RfSmem<N, rf_tb<
   const float Dc = p.D ? (p.D_per_channel ? p.D[c] : p.D[c / p.headdim]) : 0.f;
   const int nblk = (p.seqlen + TB - 1) / TB;
   RfRegs<T, N, TB, CPB> r;
-  float4 bias4 = {0.f, 0.f, 0.f, 0.f};      // this thread's 4 channels of dt_bias (the same rows every block)
-  if (p.dt_bias && tid < RfRegs<T, N, TB, CPB>::NQ)
-    bias4 = *reinterpret_cast<const float4*>(p.dt_bias + c0 + 4 * (tid % (CPB / 4)));
+  const float bias = p.dt_bias ? p.dt_bias[c0 + tid % CPB] : 0.f;   // of this thread's elements' channel
   if (nblk > 0) {
     rf_load<T, N, TB, CPB, GATE>(p, r, b, c0, 0);
-    rf_store<T, N, TB, CPB, GATE>(p, r, sm.st[0], 0, bias4);
+    rf_store<T, N, TB, CPB, GATE>(p, r, sm.st[0], 0, bias);
   }
   if (nblk > 1) rf_load<T, N, TB, CPB, GATE>(p, r, b, c0, TB);
   __syncthreads();
@@ -364,8 +369,16 @@ __device__ __forceinline__ void rf_scan_walk(const RfParams& p, RfSmem<N, rf_tb<
       // over the channel's 32 lanes after the block hands lane g the sum for token g (CKPT: no y; the state
       // entering every piece is stored)
       float yacc[32];
+      // operands two tokens ahead of their use, held there by the scheduling barriers: left to itself the compiler
+      // read a token's operands and waited for them, with one wave per SIMD nothing else to run
+      RfTok<NS> q0, q1;
+      rf_tok<N, TB, CPB, NS>(s, 0, cl, n0, q0);
+      rf_tok<N, TB, CPB, NS>(s, 1, cl, n0, q1);
 #pragma unroll
       for (int t = 0; t < TB; ++t) {
+        RfTok<NS> o = q0;
+        q0 = q1;
+        if (t + 2 < TB) rf_tok<N, TB, CPB, NS>(s, t + 2, cl, n0, q1);
         if constexpr (CKPT) {
           constexpr int RK = RF_RK;                        // divides TB: a piece starts where t % RK == 0
           const int tt = k * TB + t;
@@ -376,8 +389,6 @@ __device__ __forceinline__ void rf_scan_walk(const RfParams& p, RfSmem<N, rf_tb<
             for (int s2 = 0; s2 < NS; ++s2) o[s2] = h[s2];
           }
         }
-        RfTok<NS> o;
-        rf_tok<N, TB, CPB, NS>(s, t, cl, n0, o);
         const float u = o.dt * o.x;
         float yp = 0.f;
 #pragma unroll
@@ -387,6 +398,7 @@ __device__ __forceinline__ void rf_scan_walk(const RfParams& p, RfSmem<N, rf_tb<
           yp = fmaf(o.c[s2], h[s2], yp);
         }
         yacc[t] = yp;
+        __builtin_amdgcn_sched_barrier(0);
       }
       if constexpr (!CKPT) {
         float yv = rf_reduce_scatter32(yacc, lane);
@@ -430,9 +442,9 @@ __device__ __forceinline__ void rf_scan_walk(const RfParams& p, RfSmem<N, rf_tb<
       cur = nxt;
     }
     }
-    if (k + 1 < nblk) rf_store<T, N, TB, CPB, GATE>(p, r, sm.st[(k + 1) & 1], (k + 1) * TB, bias4);
+    if (k + 1 < nblk) rf_store<T, N, TB, CPB, GATE>(p, r, sm.st[(k + 1) & 1], (k + 1) * TB, bias);
     if (k + 2 < nblk) rf_load<T, N, TB, CPB, GATE>(p, r, b, c0, (k + 2) * TB);
-    __syncthreads();
+    lds_barrier();                       // (not __syncthreads, which would wait for the loads just issued)
     // y rows of this block: CPB channels = CPB / 8 pieces of 8 per token
     if (!CKPT && tid < TB * (CPB / 8)) {
       const int t = tid / (CPB / 8), piece = tid % (CPB / 8);
@@ -605,7 +617,7 @@ hipError_t launch_rf_n(const RfParams& p, hipStream_t st) {
 //     (deterministic).
 // Two kernels that each walked the whole sequence backward, one per kind of sum, formed every exponential twice more
 // and left half the issue slots empty: b1 L2048 d_inner 2048 N 128, 1420 us for the three passes where these take
-// RF_MEASURED.
+// 650 (226 for the sweep, 424 for the gradients), and 20 for the sums of the partials.
 
 // d dt / d raw for dt = clamp(softplus?(raw + bias), dt_min, dt_max) (the clamp passes the gradient inside its
 // closed range, as torch.clamp does).
@@ -621,8 +633,8 @@ __device__ __forceinline__ float rf_dt_chain(const RfParams& p, float raw, float
 }
 
 // The adjoint walk, last block first, in the scan's layout.  p carries dy in x's place, C in B's and dhs in C's
-// (rf_sweep_kernel); dymul / gmul are 0 where dy / dhs is missing (finite stand-ins are read).
-template <typename T, int N>
+// (rf_sweep_kernel); dymul is 0 where dy is missing (a finite stand-in is read); HASG: dhs is given, times gmul.
+template <typename T, int N, bool HASG>
 __device__ __forceinline__ void rf_adj_walk(const RfParams& p, RfSmem<N, rf_tb<N>(), rf_cpb<N>()>& sm, float dymul,
                                             float gmul) {
   constexpr int TB = rf_tb<N>(), LPC = rf_lpc<N>(), NS = rf_ns<N>(), CPB = rf_cpb<N>(), RK = RF_RK;
@@ -641,12 +653,10 @@ __device__ __forceinline__ void rf_adj_walk(const RfParams& p, RfSmem<N, rf_tb<N
     lamc[s] = p.d_final ? p.d_final[((int64_t)b * p.d_inner + c) * N + n0 + s] : 0.f;
   }
   RfRegs<T, N, TB, CPB> r;
-  float4 bias4 = {0.f, 0.f, 0.f, 0.f};
-  if (p.dt_bias && tid < RfRegs<T, N, TB, CPB>::NQ)
-    bias4 = *reinterpret_cast<const float4*>(p.dt_bias + c0 + 4 * (tid % (CPB / 4)));
-  rf_load<T, N, TB, CPB, false>(p, r, b, c0, (nblk - 1) * TB);
-  rf_store<T, N, TB, CPB, false>(p, r, sm.st[(nblk - 1) & 1], (nblk - 1) * TB, bias4);
-  if (nblk > 1) rf_load<T, N, TB, CPB, false>(p, r, b, c0, (nblk - 2) * TB);
+  const float bias = p.dt_bias ? p.dt_bias[c0 + tid % CPB] : 0.f;
+  rf_load<T, N, TB, CPB, false, HASG>(p, r, b, c0, (nblk - 1) * TB);
+  rf_store<T, N, TB, CPB, false>(p, r, sm.st[(nblk - 1) & 1], (nblk - 1) * TB, bias);
+  if (nblk > 1) rf_load<T, N, TB, CPB, false, HASG>(p, r, b, c0, (nblk - 2) * TB);
   __syncthreads();
   float* ck = p.lam_ckpt + ((int64_t)b * nsb * p.d_inner + c) * N + n0;
   for (int k = nblk - 1; k >= 0; --k) {
@@ -665,13 +675,13 @@ __device__ __forceinline__ void rf_adj_walk(const RfParams& p, RfSmem<N, rf_tb<N
 #pragma unroll
       for (int s2 = 0; s2 < NS; ++s2) {
         float lam = fmaf(dy, o.b[s2], lamc[s2]);
-        if (gmul != 0.f) lam = fmaf(gm, o.c[s2], lam);
+        if constexpr (HASG) lam = fmaf(gm, o.c[s2], lam);
         lamc[s2] = __builtin_amdgcn_exp2f(o.dt * k2[s2]) * lam;
       }
     }
-    if (k > 0) rf_store<T, N, TB, CPB, false>(p, r, sm.st[(k - 1) & 1], (k - 1) * TB, bias4);
-    if (k > 1) rf_load<T, N, TB, CPB, false>(p, r, b, c0, (k - 2) * TB);
-    __syncthreads();
+    if (k > 0) rf_store<T, N, TB, CPB, false>(p, r, sm.st[(k - 1) & 1], (k - 1) * TB, bias);
+    if (k > 1) rf_load<T, N, TB, CPB, false, HASG>(p, r, b, c0, (k - 2) * TB);
+    lds_barrier();
   }
   if (p.dh0) {
     float* o = p.dh0 + ((int64_t)b * p.d_inner + c) * N + n0;
@@ -680,22 +690,22 @@ __device__ __forceinline__ void rf_adj_walk(const RfParams& p, RfSmem<N, rf_tb<N
   }
 }
 
-template <typename T, int N>
+template <typename T, int N, bool HASG>
 __global__ __launch_bounds__(RF_NT) void rf_sweep_kernel(RfParams p) {
   __shared__ RfSmem<N, rf_tb<N>(), rf_cpb<N>()> sm;
   if (blockIdx.y == 0) {
     rf_scan_walk<T, N, false, true>(p, sm);
     return;
   }
-  const float dymul = p.dy ? 1.f : 0.f, gmul = p.dhs ? 1.f / (float)p.d_inner : 0.f;
+  const float dymul = p.dy ? 1.f : 0.f, gmul = HASG ? 1.f / (float)p.d_inner : 0.f;
   if (p.dy) {
     p.x = p.dy; p.x_sl = p.d_inner; p.x_sb = (int64_t)p.seqlen * p.d_inner;
   }
   p.B = p.C; p.B_sb = p.C_sb; p.B_sl = p.C_sl;
-  if (p.dhs) {
+  if constexpr (HASG) {
     p.C = p.dhs; p.C_sl = N; p.C_sb = (int64_t)p.seqlen * N;
   }
-  rf_adj_walk<T, N>(p, sm, dymul, gmul);
+  rf_adj_walk<T, N, HASG>(p, sm, dymul, gmul);
 }
 
 // Lanes and channels of the gradient kernel's waves: 4 states a lane.
@@ -759,8 +769,8 @@ __device__ __forceinline__ void rf_sum16(float (&v)[16], int l) {
   }
 }
 
-// grid (batch x pieces, channel blocks).  The piece's later half first, for all of the workgroup's channels, then the
-// earlier one (its adjoint waits in LDS): the sums over the channels then hold 64 registers at a time, and with the
+// grid batch x pieces x channel blocks (a piece's blocks read the same B and C rows).  The piece's later half first, for
+// all of the workgroup's channels, then the earlier one (its adjoint waits in LDS): the sums over the channels then hold 64 registers at a time, and with the
 // states and decays of 8 tokens the kernel fits two waves per SIMD (both halves' sums at once spilled 58 registers).
 template <typename T, int N, bool HASG>
 __global__ __launch_bounds__(RF_NT, 2) void rf_grad_kernel(RfParams p) {
@@ -768,8 +778,9 @@ __global__ __launch_bounds__(RF_NT, 2) void rf_grad_kernel(RfParams p) {
   constexpr int NSTEP = CH / (4 * LC);
   __shared__ RfGradSmem<N, HASG> sm;
   const int L = p.seqlen, di = p.d_inner;
-  const int nsb = (L + RK - 1) / RK, ncb = gridDim.y;
-  const int b = blockIdx.x / nsb, j = blockIdx.x - b * nsb, cb = blockIdx.y;
+  const int nsb = (L + RK - 1) / RK, ncb = (di + CH - 1) / CH;
+  const int bj = blockIdx.x / ncb, cb = blockIdx.x - bj * ncb;
+  const int b = bj / nsb, j = bj - b * nsb;
   const int t0 = j * RK, c0 = cb * CH;
   const int tid = threadIdx.x, l = tid & 63, w = wave_id(), gl = l % LN;
   const int n0 = 4 * gl;
@@ -1013,29 +1024,29 @@ __global__ __launch_bounds__(256) void rf_bwd_reduce_kernel(RfParams p, int ncb)
   }
 }
 
-// Sum over rows r of part[r][i] for column i of `cols`, by the 16 threads of a column (rows t, t + 16, .. in order, then
-// the 16 sums in order): a workgroup takes 16 columns.
+// Sum over rows r of part[r][i] for column i of `cols`, by the 64 threads of a column (rows t, t + 64, .. in order, then
+// the 64 sums in order): a workgroup of 1024 takes 16 columns (with 16 threads a column, 4096 rows took 32 us, now 8).
 __device__ __forceinline__ float rf_column_sum(const float* part, int64_t rows, int64_t cols, int i, bool on,
-                                               float (&red)[16][17]) {
+                                               float (&red)[64][17]) {
   const int t = threadIdx.x >> 4, q = threadIdx.x & 15;
   float s = 0.f;
   if (on)
-#pragma unroll 4
-    for (int64_t r = t; r < rows; r += 16) s += part[r * cols + i];
+#pragma unroll 8
+    for (int64_t r = t; r < rows; r += 64) s += part[r * cols + i];
   __syncthreads();
   red[t][q] = s;
   __syncthreads();
   float a = 0.f;
 #pragma unroll
-  for (int k = 0; k < 16; ++k) a += red[k][q];
+  for (int k = 0; k < 64; ++k) a += red[k][q];
   return a;
 }
 
 // dA (N): partials per (batch, piece, channel block); dD per channel and d dt_bias (d_inner): per (batch, piece).  One
 // workgroup per 16 columns, dA's first; with D per head the channel sums go to dD_sum and rf_bwd_head_kernel adds a
 // head's channels.
-__global__ __launch_bounds__(256) void rf_bwd_param_kernel(RfParams p, int ncb, int na) {
-  __shared__ float red[16][17];
+__global__ __launch_bounds__(1024) void rf_bwd_param_kernel(RfParams p, int ncb, int na) {
+  __shared__ float red[64][17];
   const int di = p.d_inner, N = p.dstate, q = threadIdx.x & 15;
   const int nsb = (p.seqlen + RF_RK - 1) / RF_RK;
   const int64_t rows = (int64_t)p.batch * nsb;
@@ -1079,12 +1090,14 @@ hipError_t launch_rf_bwd_t(const RfParams& p, hipStream_t st) {
     hipLaunchKernelGGL(rf_bwd_empty_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, p);
     return hipGetLastError();
   }
-  hipLaunchKernelGGL((rf_sweep_kernel<T, N>), dim3(p.batch * (p.d_inner / rf_cpb<N>()), 2), dim3(RF_NT), 0, st, p);
+  const dim3 sgrid((unsigned)(p.batch * (p.d_inner / rf_cpb<N>())), 2);
+  if (p.dhs) hipLaunchKernelGGL((rf_sweep_kernel<T, N, true>), sgrid, dim3(RF_NT), 0, st, p);
+  else hipLaunchKernelGGL((rf_sweep_kernel<T, N, false>), sgrid, dim3(RF_NT), 0, st, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const int ncb = (p.d_inner + RF_CH - 1) / RF_CH;
   const int nsb = (p.seqlen + RF_RK - 1) / RF_RK;
-  const dim3 grid((unsigned)(nsb * p.batch), (unsigned)ncb);
+  const dim3 grid((unsigned)((int64_t)p.batch * nsb * ncb));
   if (p.dhs) hipLaunchKernelGGL((rf_grad_kernel<T, N, true>), grid, dim3(RF_NT), 0, st, p);
   else hipLaunchKernelGGL((rf_grad_kernel<T, N, false>), grid, dim3(RF_NT), 0, st, p);
   e = hipGetLastError();
@@ -1094,7 +1107,7 @@ hipError_t launch_rf_bwd_t(const RfParams& p, hipStream_t st) {
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   const int na = (N + 15) / 16;
-  hipLaunchKernelGGL(rf_bwd_param_kernel, dim3((unsigned)(na + (p.d_inner + 15) / 16)), dim3(256), 0, st, p, ncb, na);
+  hipLaunchKernelGGL(rf_bwd_param_kernel, dim3((unsigned)(na + (p.d_inner + 15) / 16)), dim3(1024), 0, st, p, ncb, na);
   e = hipGetLastError();
   if (e != hipSuccess || !p.dD || p.D_per_channel) return e;
   hipLaunchKernelGGL(rf_bwd_head_kernel, dim3((unsigned)((p.d_inner / p.headdim + 255) / 256)), dim3(256), 0, st, p);
