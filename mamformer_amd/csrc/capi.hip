@@ -960,6 +960,7 @@ static void rf_fill(const mh_ssd_args* a, mh::RfParams& p) {
   p.y = a->y; p.y_sb = a->y_stride_b; p.y_sl = a->y_stride_l;
   p.z = a->z; p.z_sb = a->z_stride_b; p.z_sl = a->z_stride_l;
   p.final_state = a->final_state;
+  p.A_log = (a->flags & MH_A_LOG) != 0;
 }
 
 static int hs_bwd_validate(const mh_ssd_hs_bwd_args* a) {

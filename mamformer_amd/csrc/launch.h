@@ -144,6 +144,7 @@ struct RfParams {
   float* dA_part;            // workspace: (b, pieces, channel blocks, N)
   float* dD_part; float* dbias_part;  // workspace: (b, pieces, d_inner) sums over the tokens of a piece
   float* dD_sum;             // workspace: (d_inner) a channel's dD where D is per head
+  int A_log;                 // A holds log-rates: the rates are -exp(clamp(A, -5, 5)), dA the gradient of A itself
 };
 bool ssd_rf_supported(int dstate);
 size_t ssd_rf_workspace_bytes(int batch, int seqlen, int d_inner, int dstate, bool h_states);

@@ -1,7 +1,7 @@
 // The reference's own selective scan (mamformer/layers/mamba2.py:70-130) for gfx950: a decay rate per state
 // column and a step size per channel,
 //     h_t[c, n] = exp(A_n dt_t[c]) h_{t-1}[c, n] + dt_t[c] x_t[c] B_t[n],   y_t[c] = sum_n C_t[n] h_t[c, n] + D_c x_t[c]
-// with A_n = -exp(clamp(A_log_n, -5, 5)), formed by the caller.  The decay differs per (channel, state), so the
+// with A_n = -exp(clamp(A_log_n, -5, 5)), formed here or by the caller.  The decay differs per (channel, state), so the
 // recurrence has no matrix-unit factorisation (the per-head SSD form does): every (token, channel, state) costs
 // one exponential and a few fused multiply-adds, and the kernels are bound by that VALU work.
 //
@@ -43,6 +43,13 @@ template <int N> constexpr int rf_tb() { return N <= 128 ? 32 : 16; }
 constexpr int RF_RK = 16;            // tokens per piece of the backward (the checkpoint spacing)
 constexpr int RF_HK = 8;             // tokens whose states and decays the gradient kernel holds in registers at once
 constexpr int RF_CH = 64;            // channels per workgroup of the gradient kernel
+
+// The decay rate of state n: A as given, or -exp(clamp(A_log, -5, 5)) (mamba2.py:87-88; a NaN stays one).
+__device__ __forceinline__ float rf_rate(const RfParams& p, int n) {
+  const float a = p.A[n];
+  if (!p.A_log) return a;
+  return -expf(a < -5.f ? -5.f : a > 5.f ? 5.f : a);
+}
 
 // Per-lane token prologue: dt <- clamp(softplus?(dt + bias), dt_min, dt_max).
 __device__ __forceinline__ float rf_dt(const RfParams& p, float raw, float bias) {
@@ -347,7 +354,7 @@ __device__ __forceinline__ void rf_scan_walk(const RfParams& p, RfSmem<N, rf_tb<
   float k2[NS], h[NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    k2[s] = p.A[n0 + s] * LOG2E;                           // exp(A dt) = 2^(A log2(e) dt)
+    k2[s] = rf_rate(p, n0 + s) * LOG2E;                           // exp(A dt) = 2^(A log2(e) dt)
     h[s] = p.init_state ? p.init_state[((int64_t)b * p.d_inner + c) * N + n0 + s] : 0.f;
   }
   const float Dc = p.D ? (p.D_per_channel ? p.D[c] : p.D[c / p.headdim]) : 0.f;
@@ -486,7 +493,7 @@ __global__ __launch_bounds__(RF_NT) void rf_hs_kernel(RfParams p) {
   float k2[HS_NS], h[HS_NS];
 #pragma unroll
   for (int s = 0; s < HS_NS; ++s) {
-    k2[s] = p.A[n0 + s] * LOG2E;
+    k2[s] = rf_rate(p, n0 + s) * LOG2E;
     h[s] = (on && p.init_state) ? p.init_state[((int64_t)b * p.d_inner + c) * N + n0 + s] : 0.f;
   }
   const float bias = p.dt_bias ? p.dt_bias[cc] : 0.f;
@@ -649,7 +656,7 @@ __device__ __forceinline__ void rf_adj_walk(const RfParams& p, RfSmem<N, rf_tb<N
   float k2[NS], lamc[NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    k2[s] = p.A[n0 + s] * LOG2E;
+    k2[s] = rf_rate(p, n0 + s) * LOG2E;
     lamc[s] = p.d_final ? p.d_final[((int64_t)b * p.d_inner + c) * N + n0 + s] : 0.f;
   }
   RfRegs<T, N, TB, CPB> r;
@@ -822,7 +829,7 @@ __global__ __launch_bounds__(RF_NT, 2) void rf_grad_kernel(RfParams p) {
   float k2[4], As[4], dA[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    As[i] = p.A[n0 + i];
+    As[i] = rf_rate(p, n0 + i);
     k2[i] = As[i] * LOG2E;
     dA[i] = 0.f;
   }
@@ -1053,7 +1060,10 @@ __global__ __launch_bounds__(1024) void rf_bwd_param_kernel(RfParams p, int ncb,
   if ((int)blockIdx.x < na) {
     const int i = blockIdx.x * 16 + q;
     const float a = rf_column_sum(p.dA_part, rows * ncb, N, i, i < N, red);
-    if (threadIdx.x < 16 && i < N) p.dA[i] = a;
+    if (threadIdx.x < 16 && i < N) {
+      const float r = p.A[i];                              // A_log's gradient: through exp, inside the clamp
+      p.dA[i] = !p.A_log ? a : r >= -5.f && r <= 5.f ? a * rf_rate(p, i) : 0.f;
+    }
     return;
   }
   const int i = (blockIdx.x - na) * 16 + q;

@@ -1013,7 +1013,7 @@ def selective_scan_reference(x, dt, A, B, C, D, return_h_states=False, return_fi
     ``initial_state`` (b, d_inner, N) seeds the state (the reference starts at zero); ``z`` (b, L, d_inner) applies
     the block's gate y * silu(z) (mamba2.py:337-338), in the kernel without autograd.  x / B / C / z bf16 or fp32
     (y in that dtype), state and arithmetic fp32.  Differentiable: under autograd the backward is
-    ``mh_ssd_ref_scan_bwd`` (A_log's gradient passes through the clamp and the exponential in torch) and the gate's
+    ``mh_ssd_ref_scan_bwd`` and the gate's
     ``mh_silu_gate_bwd``."""
     _require_cuda("selective_scan_reference", x, dt, A, B, C, D, initial_state, dt_bias, z)
     if x.dim() != 3 or dt.shape != x.shape:
@@ -1035,7 +1035,9 @@ def selective_scan_reference(x, dt, A, B, C, D, return_h_states=False, return_fi
     dt32 = _inner_contig(dt.to(torch.float32))
     if dt32.stride(1) % 4 or dt32.stride(0) % 4:
         dt32 = dt32.contiguous()
-    rates = (-torch.exp(torch.clamp(A.to(torch.float32), min=-5.0, max=5.0))).contiguous()
+    logs = A.to(torch.float32).contiguous()              # the kernels form the rates -exp(clamp(A, -5, 5))
+    if _plan_only and logs is A:
+        logs = A.clone()                                  # a plan keeps the rates it was made with
     xc = _inner_contig(x)
     Bc = _inner_contig(B.to(x.dtype))
     Cc = _inner_contig(C.to(x.dtype))
@@ -1045,8 +1047,10 @@ def selective_scan_reference(x, dt, A, B, C, D, return_h_states=False, return_fi
     zc = None if z is None else _inner_contig(z.to(x.dtype))
     cfg = (dt_softplus, dt_limit, H, P)
     if not _plan_only and torch.is_grad_enabled() and any(
-            t is not None and t.requires_grad for t in (xc, dt32, rates, Bc, Cc, D32, h0, bias32, zc)):
-        y, hs, fin = _RefScanFn.apply(xc, dt32, rates, Bc, Cc, D32, h0, bias32, cfg, return_h_states)
+            t is not None and t.requires_grad for t in (xc, dt32, logs, Bc, Cc, D32, h0, bias32, zc)):
+        if logs is A and not A.requires_grad:
+            logs = A.clone()                              # a frozen A may be written before the backward reads it
+        y, hs, fin = _RefScanFn.apply(xc, dt32, logs, Bc, Cc, D32, h0, bias32, cfg, return_h_states)
         if zc is not None:
             y = _GateFn.apply(y.view(b, L, H, P), zc.view(b, L, H, P)).view(b, L, di)
         out = [y] + ([hs] if return_h_states else []) + ([fin] if return_final_state else [])
@@ -1054,13 +1058,13 @@ def selective_scan_reference(x, dt, A, B, C, D, return_h_states=False, return_fi
     y = torch.empty((b, L, di), device=x.device, dtype=x.dtype)
     fin = torch.empty((b, di, N), device=x.device, dtype=torch.float32) if return_final_state else None
     hs = torch.empty((b, L, N), device=x.device, dtype=x.dtype) if return_h_states else None
-    a = _ref_args(xc, dt32, rates, Bc, Cc, D32, h0, bias32, cfg, y, fin, zc)
+    a = _ref_args(xc, dt32, logs, Bc, Cc, D32, h0, bias32, cfg, y, fin, zc)
     n = ct.c_size_t()
     _lib.call("mh_ssd_ref_scan_workspace_bytes", ct.byref(a), int(return_h_states), ct.byref(n))
     ws = torch.empty(max(n.value, 1), device=x.device, dtype=torch.uint8) if n.value else None
     a.workspace, a.workspace_bytes = _ptr(ws), n.value
     if _plan_only:
-        return _RefScanPlan(a, _ptr(hs), x.device, keep=(xc, dt32, rates, Bc, Cc, D32, h0, bias32, zc, ws), y=y,
+        return _RefScanPlan(a, _ptr(hs), x.device, keep=(xc, dt32, logs, Bc, Cc, D32, h0, bias32, zc, ws), y=y,
                             h_states=hs, final_state=fin)
     _lib.call("mh_ssd_ref_scan_fwd", ct.byref(a), _ptr(hs), _stream(x.device))
     out = [y]
@@ -1071,15 +1075,15 @@ def selective_scan_reference(x, dt, A, B, C, D, return_h_states=False, return_fi
     return out[0] if len(out) == 1 else tuple(out)
 
 
-def _ref_args(xc, dt32, rates, Bc, Cc, D32, h0, bias32, cfg, y, fin, zc):
+def _ref_args(xc, dt32, logs, Bc, Cc, D32, h0, bias32, cfg, y, fin, zc):
     """``mh_ssd_args`` of the reference-form scan: (b, L, d_inner) rows seen as H heads of P channels."""
     dt_softplus, dt_limit, H, P = cfg
     b, L, di = xc.shape
-    N = rates.shape[0]
-    a = _ssd_args(xc.view(b, L, H, P), dt32, rates, Bc.view(b, L, 1, N), Cc.view(b, L, 1, N), None, bias32,
+    N = logs.shape[0]
+    a = _ssd_args(xc.view(b, L, H, P), dt32, logs, Bc.view(b, L, 1, N), Cc.view(b, L, 1, N), None, bias32,
                   dt_softplus, dt_limit, h0, (xc if y is None else y).view(b, L, H, P), fin, None,
                   None if zc is None else zc.view(b, L, H, P))
-    flags = a.flags | _lib.MH_A_PER_STATE | _lib.MH_DT_PER_CHANNEL
+    flags = a.flags | _lib.MH_A_PER_STATE | _lib.MH_DT_PER_CHANNEL | _lib.MH_A_LOG
     if D32 is not None:
         a.D = _ptr(D32)
         if D32.numel() == di:
@@ -1094,34 +1098,34 @@ def _ref_args(xc, dt32, rates, Bc, Cc, D32, h0, bias32, cfg, y, fin, zc):
 
 class _RefScanFn(torch.autograd.Function):
     """Autograd node of the reference-form scan: forward ``mh_ssd_ref_scan_fwd`` (y ungated, h_states when asked,
-    the final state), backward ``mh_ssd_ref_scan_bwd`` (every gradient, w.r.t. the rates A; torch chains A_log)."""
+    the final state), backward ``mh_ssd_ref_scan_bwd`` (every gradient, w.r.t. A_log itself)."""
 
     @staticmethod
-    def forward(ctx, xc, dt32, rates, Bc, Cc, D32, h0, bias32, cfg, want_hs):
+    def forward(ctx, xc, dt32, logs, Bc, Cc, D32, h0, bias32, cfg, want_hs):
         b, L, di = xc.shape
-        N = rates.shape[0]
+        N = logs.shape[0]
         y = torch.empty((b, L, di), device=xc.device, dtype=xc.dtype)
         fin = torch.empty((b, di, N), device=xc.device, dtype=torch.float32)
         hs = torch.empty((b, L, N), device=xc.device, dtype=xc.dtype) if want_hs else None
-        a = _ref_args(xc, dt32, rates, Bc, Cc, D32, h0, bias32, cfg, y, fin, None)
+        a = _ref_args(xc, dt32, logs, Bc, Cc, D32, h0, bias32, cfg, y, fin, None)
         n = ct.c_size_t()
         _lib.call("mh_ssd_ref_scan_workspace_bytes", ct.byref(a), int(want_hs), ct.byref(n))
         ws = torch.empty(max(n.value, 1), device=xc.device, dtype=torch.uint8) if n.value else None
         a.workspace, a.workspace_bytes = _ptr(ws), n.value
         _lib.call("mh_ssd_ref_scan_fwd", ct.byref(a), _ptr(hs), _stream(xc.device))
-        ctx.save_for_backward(xc, dt32, rates, Bc, Cc, D32, h0, bias32)
+        ctx.save_for_backward(xc, dt32, logs, Bc, Cc, D32, h0, bias32)
         ctx.cfg = cfg
         ctx.set_materialize_grads(False)
         return y, hs, fin
 
     @staticmethod
     def backward(ctx, dy, dhs, dfin):
-        xc, dt32, rates, Bc, Cc, D32, h0, bias32 = ctx.saved_tensors
+        xc, dt32, logs, Bc, Cc, D32, h0, bias32 = ctx.saved_tensors
         b, L, di = xc.shape
-        N = rates.shape[0]
+        N = logs.shape[0]
         dev = xc.device
         g = _lib.SsdRefBwdArgs()
-        g.fwd = _ref_args(xc, dt32, rates, Bc, Cc, D32, h0, bias32, ctx.cfg, None, None, None)
+        g.fwd = _ref_args(xc, dt32, logs, Bc, Cc, D32, h0, bias32, ctx.cfg, None, None, None)
         dy = None if dy is None else dy.to(xc.dtype).contiguous()
         dhs = None if dhs is None else dhs.to(xc.dtype).contiguous()
         dfin = None if dfin is None else dfin.to(torch.float32).contiguous()
