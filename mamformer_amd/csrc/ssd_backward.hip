@@ -114,6 +114,19 @@ __device__ __forceinline__ void blk_transpose(const StateBlk<T>& s, const Frag<T
   out[1] = acc_to_frag<T>(e, 1);
 }
 
+// The same fragments read transposed out of a bf16 state block in LDS: a lane's 8 bytes of it hold 4 consecutive rows
+// n of one column p, the piece a transposing read takes; rows n 16 g + 4 q .. + 3 lie at half q & 1, bytes 8 (q >> 1).
+__device__ __forceinline__ void state_tr_frags(const bf16* base, int nt, int pt, int l, Frag<bf16> (&out)[2]) {
+  const int half = l >> 5, i = l & 15;
+  const bf16* b = base + frag_off_bf(nt, pt, 4 * half + (i >> 2) + 32 * (i & 1), (l >> 4) & 1) + 4 * ((i >> 1) & 1);
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(b + 8 * (16 * c)));
+    const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(b + 8 * (16 * c + 8)));
+    out[c].v = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  }
+}
+
 // Row `row` of a swizzled Tile<T, W> at the 16 columns col0 + acc_row(half, i) -- the values an
 // accumulator tile whose lane column is `row` holds (col0 % 32 == 0).
 template <typename T, int W>
@@ -144,13 +157,6 @@ __device__ __forceinline__ void acc_rows(const float* a, int r0, int half, float
   }
 }
 
-template <typename T>
-__device__ __forceinline__ Frag<T> scaled(Frag<T> f, float s) {
-#pragma unroll
-  for (int j = 0; j < 8; ++j) f.set(j, f.get(j) * s);
-  return f;
-}
-
 // Operand fragments f[c] of the transposed 32x32 block of a Tile<T, W> at rows r0.., columns q0..: lane = column
 // q0 + lane % 32, k = row r0 + 16 c + KSET.  bf16: two transposing LDS reads each; fp32: the identity product.
 template <typename T, int W>
@@ -163,6 +169,37 @@ __device__ __forceinline__ void tr_frags(const T* tile, int r0, int q0, const Fr
     const f32x16 d = mfma_transpose<T, T, W>(tile, r0, q0, id, half, l32);
     f[0] = acc_to_frag<T>(d, 0);
     f[1] = acc_to_frag<T>(d, 1);
+  }
+}
+
+// tr_frags for a wave with direct-to-LDS loads in flight (into other bytes): the compiler cannot tell a transposing
+// read's bytes from theirs and waits for all of them before it, so the four reads and their own wait are written out.
+// (Rows 16 further down have the same chunk swizzle: an immediate offset.)
+template <typename T, int W>
+__device__ __forceinline__ void tr_frags_inflight(const T* tile, int r0, int q0, const Frag<T> (&id)[2], int half,
+                                                  int l32, Frag<T> (&f)[2]) {
+  if constexpr (sizeof(T) == 2) {
+    static_assert(W == 128 || W == 64, "chunk swizzle of period 16");
+    using TL = Tile<T, W>;
+    const int l = threadIdx.x & 63, i = l & 15;
+    const int r = r0 + 4 * half + (i >> 2), col = q0 + 16 * ((l >> 4) & 1) + 4 * (i & 3);
+    typedef __attribute__((address_space(3))) const T lds_t;
+    const uint32_t a0 = (uint32_t)(uintptr_t)(lds_t*)(tile + TL::chunk(r, col >> 3) + (col & 7));
+    const uint32_t a1 = (uint32_t)(uintptr_t)(lds_t*)(tile + TL::chunk(r + 8, col >> 3) + (col & 7));
+    i16x4_t v0, v1, v2, v3;
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %4\n\t"
+        "ds_read_b64_tr_b16 %1, %5\n\t"
+        "ds_read_b64_tr_b16 %2, %4 offset:%c6\n\t"
+        "ds_read_b64_tr_b16 %3, %5 offset:%c6\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(v0), "=&v"(v1), "=&v"(v2), "=&v"(v3)
+        : "v"(a0), "v"(a1), "n"(16 * W * 2)
+        : "memory");
+    f[0].v = __builtin_bit_cast(bf16x8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+    f[1].v = __builtin_bit_cast(bf16x8, __builtin_shufflevector(v2, v3, 0, 1, 2, 3, 4, 5, 6, 7));
+  } else {
+    tr_frags<T, W>(tile, r0, q0, id, half, l32, f);
   }
 }
 
@@ -361,6 +398,7 @@ struct GradStage {
   T X[SEG * HD];            // Tile<T, HD> of the head
   T DY[SEG * HD];
   float dtraw[SEG];
+  float D[HD];              // per channel (the head's own value in each, when it has one)
 };
 template <typename T, int N, bool SL> struct GradStates {};
 template <typename T, int N> struct GradStates<T, N, true> {
@@ -392,10 +430,10 @@ struct GradSmem {
   float dtp[2 * (N / 32)][SEG];  // per wave: processed dt
   float red[2][N / 32][SEG];     // per n-block partial dots: bint, u
   XdTiles<T> xds;                // bf16: the head's XD tiles, formed once and shared (fp32: per wave, none here)
-  float colg[3][32];             // per XD tile (t-block, s-block) = (0,0), (1,0), (1,1): sum_t (M o XD)[t][s]
-  float rowg[3][32];             // per XD^T tile (s-block, t-block) = (0,0), (0,1), (1,1): sum_s (M o XD)[t][s] dt_s
+  float colg[2][3][32];          // (by the head's parity, as rowg and dd) per XD tile (t-block, s-block) = (0,0), (1,0), (1,1): sum_t (M o XD)[t][s]
+  float rowg[2][3][32];          // per XD^T tile (s-block, t-block) = (0,0), (0,1), (1,1): sum_s (M o XD)[t][s] dt_s
   float lh[N / 32];              // <lam_out, h_in> per n-block
-  float dd[2];                   // trace of dy x^T per diagonal 32-block
+  float dd[2][2];                // trace of dy x^T per diagonal 32-block
   alignas(16) float cb[3][64 * 16];   // CB[t][s] tiles (t-block, s-block) = (0,0), (1,0), (1,1), accumulator
                                       // order (16-byte aligned: read and written as f32x4)
   float cbt[3][64 * 16];         // CB^T[s][t] tiles (s-block, t-block) = (0,0), (0,1), (1,1)
@@ -412,6 +450,12 @@ constexpr bool grad_sl = grad_fits<T, N, grad_nst<T, N>, true>;
 
 // Work split (NW = 2 N/32 waves): wave w owns n-block nb = w % (N/32) and token block r = w / (N/32) of the
 // dB^T [n][s] and dC^T [n][t] tiles; waves 0-3 also own the dx^T [p][s] tile (p-block w & 1, s-block w >> 1).
+// The LDS allows one workgroup per CU, two waves per SIMD, which hide neither each other's barriers nor a memory
+// latency: bf16 therefore takes two barriers per head and fetches a head ahead (its tiles, A, dt_bias and D; its states
+// over the current ones, which the waves read into registers first, transposed by the LDS).  b2 L4096 H64 N128 G1:
+// 283 us with the states fetched and waited for between heads, D read by 16 branches and three barriers, 258 with that,
+// 235 with decays applied to the products' sums instead of to their operands and no transposing products (VALU
+// instructions 83 M, 68 M).
 template <typename T, int N>
 __global__ __launch_bounds__(128 * (N / 32)) void ssd_bwd_grad_kernel(SsdBwdParams q) {
   constexpr int NB = N / 32, NW = 2 * NB;
@@ -419,6 +463,8 @@ __global__ __launch_bounds__(128 * (N / 32)) void ssd_bwd_grad_kernel(SsdBwdPara
   using TX = Tile<T, HD>;
   constexpr bool SL = grad_sl<T, N>;
   constexpr int NST = grad_nst<T, N>;
+  constexpr bool PIPE = sizeof(T) == 2 && NST == 2;   // two barriers per head, the next head's fetch between them
+  static_assert(!SL || PIPE, "states in LDS are fetched between the two barriers");
   __shared__ GradSmem<T, N, NST, SL> sm;
   const SsdParams& p = q.f;
   const int si = blockIdx.x, b = blockIdx.z;
@@ -461,6 +507,8 @@ __global__ __launch_bounds__(128 * (N / 32)) void ssd_bwd_grad_kernel(SsdBwdPara
     fetch_tile<T, HD>(sm.st[st].X, xb + (int64_t)h * p.x_sh, p.x_sl, tok0, last, w * nblk, nblk, l);
     fetch_tile<T, HD>(sm.st[st].DY, dyb + (int64_t)h * q.dy_sh, q.dy_sl, tok0, last, w * nblk, nblk, l);
     if (w == 0) fetch_dt(sm.st[st].dtraw, dtb + h, p.dt_sl, tok0, last, l);
+    if (w == NW - 1 && p.D)
+      fetch_dt(sm.st[st].D, p.D + (p.D_per_channel ? h * HD : h), p.D_per_channel ? 1 : 0, 0, HD - 1, l);
   };
   auto fetch_states = [&](int h) {
     if constexpr (SL) {
@@ -475,6 +523,7 @@ __global__ __launch_bounds__(128 * (N / 32)) void ssd_bwd_grad_kernel(SsdBwdPara
   fetch_head(hfirst, std::integral_constant<int, 0>());
   fetch_states(hfirst);
   f32x16 dBacc = zero16(), dCacc = zero16();
+  float A_nx = p.A[hfirst], bias_nx = p.dt_bias ? p.dt_bias[hfirst] : 0.f;   // of the head that comes next
 
   wait_vmem();                      // B / C tiles (and the first head's tiles) in LDS
   lds_barrier();
@@ -550,15 +599,20 @@ __global__ __launch_bounds__(128 * (N / 32)) void ssd_bwd_grad_kernel(SsdBwdPara
       if constexpr (SL) return sm.sts.Hin;
       else return reinterpret_cast<const T*>(hin_ws) + sidx;
     };
-    StateBlk<T> Lb[2], Hb[2];
+    StateBlk<T> Lb[2], Hb[2];            // states read from HBM: their blocks, transposed where they are used
+    Frag<T> lamT[2][2], hT[2][2];        // (states in LDS: read transposed)
 #pragma unroll
     for (int pt = 0; pt < 2; ++pt) {
-      Lb[pt] = load_state_blk<T>(lam_src(), nb, pt, l);
-      Hb[pt] = load_state_blk<T>(hin_src(), nb, pt, l);
+      if constexpr (SL) {
+        state_tr_frags(lam_src(), nb, pt, l, lamT[pt]);
+        state_tr_frags(hin_src(), nb, pt, l, hT[pt]);
+      } else {
+        Lb[pt] = load_state_blk<T>(lam_src(), nb, pt, l);
+        Hb[pt] = load_state_blk<T>(hin_src(), nb, pt, l);
+      }
     }
     // ---- decay of this head (lane = token), wave-private copies for per-row reads
-    const float Ah = p.A[h];
-    const float bias = p.dt_bias ? p.dt_bias[h] : 0.f;
+    const float Ah = A_nx, bias = bias_nx;
     const float raw = sg.dtraw[l];
     float dtv;
     const float cs = seg_decay(p, raw, bias, Ah, l, len, dtv);
@@ -567,7 +621,16 @@ __global__ __launch_bounds__(128 * (N / 32)) void ssd_bwd_grad_kernel(SsdBwdPara
     sm.dtp[w][l] = dtv;
     const float cs_l = from_half(cs, r), dt_l = from_half(dtv, r);
 
+    // the blocks of lam_out that the dx^T tile contracts (the second half of a split tile the upper ones): read here,
+    // so that after the next barrier the next head's states may land in the same LDS
     constexpr bool SHARE = sizeof(T) == 2;
+    constexpr int NT0 = SPLIT ? NB / 2 : NB;
+    const int nt0 = SPLIT && w >= 4 ? NT0 : 0;
+    StateBlk<T> Lx[NT0];
+    if constexpr (SL) {
+#pragma unroll
+      for (int k = 0; k < NT0; ++k) Lx[k] = load_state_blk<T>(lam_src(), nt0 + k, pb, l);
+    }
     Frag<T> XDf[2][2], XTf[2][2];        // per-wave tiles (fp32 only)
     if constexpr (SHARE) {
       // the six distinct XD tiles of the head, wave w forming tiles w, w + NW, ... (same masks, decays and sums
@@ -584,16 +647,17 @@ __global__ __launch_bounds__(128 * (N / 32)) void ssd_bwd_grad_kernel(SsdBwdPara
                   row_frag<T, T, HD>(sg.X, s_p, 16 * k + 8 * half), a);
         float ct[16];
         acc_rows(sm.cs[w], 32 * tb, half, ct);
-        float d = 0.f;
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
           const int t = 32 * tb + acc_row(half, i);
           a[i] = (t < len && t >= s_p) ? a[i] * __expf(ct[i] - cs_p) : 0.f;
-          d += (t == s_p) ? a[i] : 0.f;
         }
         if (tb == rr) {
+          float d = 0.f;                 // the diagonal element, in the half that holds it
+#pragma unroll
+          for (int i = 0; i < 16; ++i) d = acc_row(half, i) == l32 ? a[i] : d;
           d = wave_sum(d);
-          if (l == 0) sm.dd[rr] = d;
+          if (l == 0) sm.dd[st][rr] = d;
         }
         float cg = 0.f;
         const float* cbp = sm.cb[tix] + 16 * l;
@@ -604,7 +668,7 @@ __global__ __launch_bounds__(128 * (N / 32)) void ssd_bwd_grad_kernel(SsdBwdPara
           for (int k = 0; k < 4; ++k) cg += v[k] * a[4 * i + k];
         }
         cg = sum_halves(cg);
-        if (half == 0) sm.colg[tix][l32] = cg;
+        if (half == 0) sm.colg[st][tix][l32] = cg;
 #pragma unroll
         for (int c = 0; c < 2; ++c) sm.xds.xd[tix][c][l] = acc_to_frag<T>(a, c);
       } else {
@@ -633,12 +697,21 @@ __global__ __launch_bounds__(128 * (N / 32)) void ssd_bwd_grad_kernel(SsdBwdPara
           for (int k = 0; k < 4; ++k) rg += v[k] * a[4 * i + k];
         }
         rg = sum_halves(rg);
-        if (half == 0) sm.rowg[ti][l32] = rg;
+        if (half == 0) sm.rowg[st][ti][l32] = rg;
 #pragma unroll
         for (int c = 0; c < 2; ++c) sm.xds.xt[ti][c][l] = acc_to_frag<T>(a, c);
       }
       }
       lds_barrier();                     // the shared XD tiles are in LDS
+      if constexpr (PIPE) {
+        if (j + 1 < HB) {
+          // the next head's tiles into the other stage, its states over this head's (in registers by now)
+          fetch_head(h + 1, std::integral_constant<int, st ^ 1>());
+          fetch_states(h + 1);
+          A_nx = p.A[h + 1];
+          if (p.dt_bias) bias_nx = p.dt_bias[h + 1];
+        }
+      }
     } else {
       // ---- XD[t][s] = dy_t . x_s (tiles tb >= r, column block r), masked and decayed (L o XD), as
       //      B-operand fragments (column s, k = t)
@@ -667,7 +740,7 @@ __global__ __launch_bounds__(128 * (N / 32)) void ssd_bwd_grad_kernel(SsdBwdPara
             // trace of dy x^T (per-head D): the diagonal block (r, r)
             if (tb == r) {
               d = wave_sum(d);
-              if (l == 0) sm.dd[r] = d;
+              if (l == 0) sm.dd[st][r] = d;
             }
             const float* cbp = sm.cb[tb + r] + 16 * l;
   #pragma unroll
@@ -684,29 +757,30 @@ __global__ __launch_bounds__(128 * (N / 32)) void ssd_bwd_grad_kernel(SsdBwdPara
       if (nb == 0) {
         colg = sum_halves(colg);
         if (half == 0) {
-          sm.colg[r == 0 ? 0 : 2][l32] = colg;      // the s-block's sum over its t-blocks
-          if (r == 0) sm.colg[1][l32] = 0.f;
+          sm.colg[st][r == 0 ? 0 : 2][l32] = colg;      // the s-block's sum over its t-blocks
+          if (r == 0) sm.colg[st][1][l32] = 0.f;
         }
       }
     }
     __builtin_amdgcn_sched_barrier(0);   // keep the phases apart: bounded register lifetimes
     // ---- dB^T tile (n-block nb, s-block r): inter part from lam_out, intra part from C^T (L o XD)
     {
-      Frag<T> lamT[2][2];
+      if constexpr (!SL) {
 #pragma unroll
-      for (int pt = 0; pt < 2; ++pt) blk_transpose<T>(Lb[pt], idk, lamT[pt]);
-      const float wend_l = __expf(cend - cs_l);
+        for (int pt = 0; pt < 2; ++pt) blk_transpose<T>(Lb[pt], idk, lamT[pt]);
+      }
+      const float wend_l = __expf(cend - cs_l);   // of this lane's column: applied to the sums, not to the operands
       f32x16 ai = zero16(), aa = zero16();
 #pragma unroll
       for (int pt = 0; pt < 2; ++pt)
 #pragma unroll
         for (int c = 0; c < 2; ++c)
-          ai = mma(lamT[pt][c], scaled<T>(kset_frag<T, T, HD>(sg.X, s_l, 32 * pt + 16 * c, half), wend_l), ai);
+          ai = mma(lamT[pt][c], kset_frag<T, T, HD>(sg.X, s_l, 32 * pt + 16 * c, half), ai);
 #pragma unroll
       for (int tb = 0; tb < 2; ++tb) {
         if (tb >= r) {
           Frag<T> ct[2];
-          tr_frags<T, N>(sm.C, 32 * tb, 32 * nb, id, half, l32, ct);   // lane n, k = t
+          tr_frags_inflight<T, N>(sm.C, 32 * tb, 32 * nb, id, half, l32, ct);   // lane n, k = t
 #pragma unroll
           for (int c = 0; c < 2; ++c) {
             if constexpr (SHARE) aa = mma(ct[c], sm.xds.xd[r == 0 ? tb : 2][c][l], aa);
@@ -720,9 +794,9 @@ __global__ __launch_bounds__(128 * (N / 32)) void ssd_bwd_grad_kernel(SsdBwdPara
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         sI += ai[i] * Bv[i];
-        dBacc[i] += dt_l * (ai[i] + aa[i]);
+        dBacc[i] += dt_l * fmaf(wend_l, ai[i], aa[i]);
       }
-      sI = sum_halves(sI);
+      sI = sum_halves(sI) * wend_l;
       if (half == 0) sm.red[0][nb][s_l] = sI;
     }
     __builtin_amdgcn_sched_barrier(0);   // keep the phases apart: bounded register lifetimes
@@ -761,8 +835,8 @@ __global__ __launch_bounds__(128 * (N / 32)) void ssd_bwd_grad_kernel(SsdBwdPara
       if (nb == 0) {
         rowg = sum_halves(rowg);
         if (half == 0) {
-          sm.rowg[r == 0 ? 0 : 1][l32] = rowg;      // the t-block's sum over its s-blocks
-          if (r == 1) sm.rowg[2][l32] = 0.f;
+          sm.rowg[st][r == 0 ? 0 : 1][l32] = rowg;      // the t-block's sum over its s-blocks
+          if (r == 1) sm.rowg[st][2][l32] = 0.f;
         }
       }
 
@@ -774,28 +848,32 @@ __global__ __launch_bounds__(128 * (N / 32)) void ssd_bwd_grad_kernel(SsdBwdPara
 #pragma unroll
       for (int pt = 0; pt < 2; ++pt)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) d += Lb[pt].at(i) * Hb[pt].at(i);
+        for (int i = 0; i < 16; ++i) {
+          if constexpr (SL) d += lamT[pt][i >> 3].get(i & 7) * hT[pt][i >> 3].get(i & 7);
+          else d += Lb[pt].at(i) * Hb[pt].at(i);
+        }
       d = wave_sum(d);
       if (l == 0) sm.lh[nb] = d;
     }
 
     // ---- dC^T tile (n-block nb, t-block r): inter part from h_in, intra part from B^T (L o XD o dt)^T
     {
-      Frag<T> hT[2][2];
+      if constexpr (!SL) {
 #pragma unroll
-      for (int pt = 0; pt < 2; ++pt) blk_transpose<T>(Hb[pt], idk, hT[pt]);
+        for (int pt = 0; pt < 2; ++pt) blk_transpose<T>(Hb[pt], idk, hT[pt]);
+      }
       const float ec_l = __expf(cs_l);
       f32x16 ah = zero16(), ac = zero16();
 #pragma unroll
       for (int pt = 0; pt < 2; ++pt)
 #pragma unroll
         for (int c = 0; c < 2; ++c)
-          ah = mma(hT[pt][c], scaled<T>(kset_frag<T, T, HD>(sg.DY, s_l, 32 * pt + 16 * c, half), ec_l), ah);
+          ah = mma(hT[pt][c], kset_frag<T, T, HD>(sg.DY, s_l, 32 * pt + 16 * c, half), ah);
 #pragma unroll
       for (int sb = 0; sb < 2; ++sb) {
         if (sb <= r) {
           Frag<T> bt[2];
-          tr_frags<T, N>(sm.B, 32 * sb, 32 * nb, id, half, l32, bt);   // lane n, k = s
+          tr_frags_inflight<T, N>(sm.B, 32 * sb, 32 * nb, id, half, l32, bt);   // lane n, k = s
 #pragma unroll
           for (int c = 0; c < 2; ++c) {
             if constexpr (SHARE) ac = mma(bt[c], sm.xds.xt[r == 0 ? 0 : (sb == 0 ? 1 : 2)][c][l], ac);
@@ -809,9 +887,9 @@ __global__ __launch_bounds__(128 * (N / 32)) void ssd_bwd_grad_kernel(SsdBwdPara
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         sU += ah[i] * Cv[i];
-        dCacc[i] += ah[i] + ac[i];
+        dCacc[i] += fmaf(ec_l, ah[i], ac[i]);
       }
-      sU = sum_halves(sU);
+      sU = sum_halves(sU) * ec_l;
       if (half == 0) sm.red[1][nb][s_l] = sU;
     }
 
@@ -843,27 +921,33 @@ __global__ __launch_bounds__(128 * (N / 32)) void ssd_bwd_grad_kernel(SsdBwdPara
               m[i] = (t < len && t >= s_x) ? m[i] * __expf(ct[i] - csx) : 0.f;
             }
             Frag<T> dyt[2];
-            tr_frags<T, HD>(sg.DY, 32 * tb, 32 * pb, id, half, l32, dyt);   // lane p, k = t
+            tr_frags_inflight<T, HD>(sg.DY, 32 * tb, 32 * pb, id, half, l32, dyt);   // lane p, k = t
 #pragma unroll
             for (int c = 0; c < 2; ++c) ax = mma(dyt[c], acc_to_frag<T>(m, c), ax);
           }
         }
       }
-      constexpr int NT0 = SPLIT ? NB / 2 : NB;
-      const int nt0 = dxB ? NT0 : 0;
+      f32x16 as = zero16();              // lam_out B of this lane's column, scaled when it is whole
 #pragma unroll
       for (int k = 0; k < NT0; ++k) {
         const int nt = nt0 + k;
-        const StateBlk<T> lx = load_state_blk<T>(lam_src(), nt, pb, l);
+        StateBlk<T> lx;
+        if constexpr (SL) lx = Lx[k];
+        else lx = load_state_blk<T>(lam_src(), nt, pb, l);
 #pragma unroll
         for (int c = 0; c < 2; ++c)
-          ax = mma(lx.frag(c), scaled<T>(kset_frag<T, T, N>(sm.B, s_x, 32 * nt + 16 * c, half), wx), ax);
+          as = mma(lx.frag(c), kset_frag<T, T, N>(sm.B, s_x, 32 * nt + 16 * c, half), as);
       }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) ax[i] = fmaf(wx, as[i], ax[i]);
       if (!SPLIT || dxB) {
         acc_cols<T, HD>(sg.DY, s_x, 32 * pb, half, dyv);
+        if (p.D) {
+          acc_rows(sg.D, 32 * pb, half, Dv);
+        } else {
 #pragma unroll
-        for (int i = 0; i < 16; ++i)
-          Dv[i] = p.D ? (p.D_per_channel ? p.D[h * HD + 32 * pb + acc_row(half, i)] : p.D[h]) : 0.f;
+          for (int i = 0; i < 16; ++i) Dv[i] = 0.f;
+        }
         if (p.D_per_channel && q.dD) {
           // per-channel dD of this token half: sum over the lane-half's 32 tokens in a fixed shuffle order,
           // one partial per (segment, head, token half) in the workspace, summed in order by the reduce kernel
@@ -914,14 +998,20 @@ __global__ __launch_bounds__(128 * (N / 32)) void ssd_bwd_grad_kernel(SsdBwdPara
     };
     if (!SPLIT && dxw) store_dx();
 
-    // The next head's fetch: into the other stage (head j - 1's, read by nobody since the last barrier) before
-    // the barrier, or, with one stage, after it.  It is issued late on purpose: a spill reload in the work above
-    // would wait for it (the vector-memory counter is shared).
-    if (NST == 2 && j + 1 < HB) fetch_head(h + 1, std::integral_constant<int, st ^ 1>());
-    lds_barrier();                     // partial dots and dx partials complete; this head's states no longer read
-    if (j + 1 < HB) {
+    // The end of the head: partial dots and dx partials complete, the next head's tiles and states in LDS (fetched
+    // since the XD tiles' barrier).  What follows -- the split dx tile's sum and store, the decay gradient -- runs
+    // beside the next head's XD tiles: it reads what that head writes only after its own barrier, or by parity.
+    // fp32 has no such barrier and, at N = 128, one stage: the fetch follows, and is waited for, below (issued late:
+    // a spill reload in the work above would wait for it, the vector-memory counter is shared).
+    if (PIPE) wait_vmem();
+    if constexpr (!PIPE && NST == 2) {
+      if (j + 1 < HB) fetch_head(h + 1, std::integral_constant<int, st ^ 1>());
+    }
+    lds_barrier();
+    if (!PIPE && j + 1 < HB) {
       if (NST == 1) fetch_head(h + 1, std::integral_constant<int, 0>());
-      fetch_states(h + 1);
+      A_nx = p.A[h + 1];
+      if (p.dt_bias) bias_nx = p.dt_bias[h + 1];
     }
     if (dxB) {
       const float* ip = sm.dxp.v[w & 3] + 16 * l;
@@ -933,9 +1023,9 @@ __global__ __launch_bounds__(128 * (N / 32)) void ssd_bwd_grad_kernel(SsdBwdPara
       }
       store_dx();
     }
-    if (w == 0) {
-      const float colG = l < 32 ? sm.colg[0][l] + sm.colg[1][l] : sm.colg[2][l - 32];
-      const float rowG = l < 32 ? sm.rowg[0][l] : sm.rowg[1][l - 32] + sm.rowg[2][l - 32];
+    if (w == NW - 1) {                  // (a wave without an XD tile of the next head)
+      const float colG = l < 32 ? sm.colg[st][0][l] + sm.colg[st][1][l] : sm.colg[st][2][l - 32];
+      const float rowG = l < 32 ? sm.rowg[st][0][l] : sm.rowg[st][1][l - 32] + sm.rowg[st][2][l - 32];
       float bint = 0.f, u = 0.f, lh = 0.f;
 #pragma unroll
       for (int k = 0; k < NB; ++k) {
@@ -958,10 +1048,10 @@ __global__ __launch_bounds__(128 * (N / 32)) void ssd_bwd_grad_kernel(SsdBwdPara
         float* ps = q.part_s + (((int64_t)b * p.nseg + si) * p.nheads + h) * 3;
         ps[0] = sdA;
         ps[1] = sdb;
-        ps[2] = sm.dd[0] + sm.dd[1];
+        ps[2] = sm.dd[st][0] + sm.dd[st][1];
       }
     }
-    if (j + 1 < HB) {
+    if (!PIPE && j + 1 < HB) {
       wait_vmem();                     // the next head's stage (and this head's stores)
       lds_barrier();
     }
