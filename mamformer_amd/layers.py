@@ -27,6 +27,7 @@ from typing import Optional
 
 import torch
 import torch.nn as nn
+from torch.autograd import forward_ad as _forward_ad
 
 from . import ops
 
@@ -186,11 +187,11 @@ class Mamba2Layer(nn.Module):
 
 
 def _plain_calls():
-    """Whether a call runs eagerly as written: no autocast, tracing, functorch transform, function or dispatch mode,
-    and no hooks on every module."""
+    """Whether a call runs eagerly as written: no autocast, tracing, functorch transform, forward-mode level, function
+    or dispatch mode, and no hooks on every module."""
     from torch.nn.modules import module as m
     return not (torch.is_autocast_enabled() or torch.jit.is_tracing() or torch.compiler.is_compiling()
-                or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch._C._functorch.peek_interpreter_stack() is not None or _forward_ad._current_level >= 0
                 or torch._C._len_torch_function_stack() or torch._C._len_torch_dispatch_stack()
                 or m._global_forward_hooks or m._global_forward_pre_hooks or m._global_backward_hooks
                 or m._global_backward_pre_hooks)
@@ -227,7 +228,8 @@ def kda_linear_attention(q1, q2, k, v, lambda_raw, kernel_dim, use_cache=False, 
         # one step (dk = K) from the cache into new tensors, as the reference returns: the state has K rows, so
         # only the first K channels of q and k enter
         args = (q1[..., :K], q2[..., :K], k[..., :K], v)
-        if torch.is_grad_enabled() and (S_prev.requires_grad or z_prev.requires_grad):
+        if _forward_ad._current_level >= 0 or torch.is_grad_enabled() and (S_prev.requires_grad
+                                                                           or z_prev.requires_grad):
             # a cache that autograd tracks: its identity gradient goes through the copies that the step updates
             St = S_prev.clone(memory_format=torch.contiguous_format)
             zt = z_prev.clone(memory_format=torch.contiguous_format)

@@ -1298,7 +1298,8 @@ class _KdaRefFn(torch.autograd.Function):
                                else lam_f, initial_state=s0, initial_z=z0, return_final_state=ret_fin, pair=pair,
                                _lam_raw=lam_raw)
         res = res if isinstance(res, tuple) else (res,)
-        ctx.save_for_backward(q1, q2, k, v, lam_h, s0, z0)
+        # lambda_raw may be written before the backward reads it: the values of this pass are kept
+        ctx.save_for_backward(q1, q2, k, v, lam_h.clone() if lam_raw else lam_h, s0, z0)
         ctx.cfg = cfg
         return res
 

@@ -68,3 +68,17 @@ def test_lambda_raw_keeps_nan_and_rejects_a_float():
     assert torch.isnan(o[:, 1]).all() and torch.isfinite(o[:, [0, 2, 3, 4]]).all()
     with pytest.raises(TypeError):
         mh.linear_attention_scan(*a, 128, 0.5)
+
+
+@pytest.mark.parametrize("trains", [True, False])
+def test_lambda_raw_may_be_written_before_the_backward(trains):
+    (q1, q2, k, v), _, _ = inputs(2, 128, torch.bfloat16, 4)
+    a = [dev(t, torch.bfloat16).requires_grad_() for t in (q1, q2, k, v)]
+    raw = dev(RAW).requires_grad_(trains)
+    leaves = a + [raw] * trains
+    want = torch.autograd.grad(mh.linear_attention_scan(*a, 128, raw).float().sum(), leaves)
+    loss = mh.linear_attention_scan(*a, 128, raw).float().sum()
+    with torch.no_grad():
+        raw.add_(1.0)                                         # an optimizer's step on this parameter alone
+    got = torch.autograd.grad(loss, leaves)
+    assert all(torch.equal(x, y) for x, y in zip(got, want))

@@ -90,6 +90,8 @@ def test_other_calls_take_the_general_path(monkeypatch):
         assert not taken(monkeypatch, lay, big, cache_of(lay, 65, 3))[1]
         with torch.autocast("cuda", dtype=BF):
             assert not taken(monkeypatch, lay, u, cache)[1]
+        with torch.autograd.forward_ad.dual_level():
+            assert not taken(monkeypatch, lay, u, cache)[1]
     assert not taken(monkeypatch, lay, u, cache)[1]                                     # gradients wanted
     lay32 = Mamba2Layer(64, device="cuda")
     with torch.no_grad():
