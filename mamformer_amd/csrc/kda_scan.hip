@@ -11,11 +11,11 @@
 //
 // Per window of tokens (a 64-token tile, or a piece of one), with G the
 // in-tile inclusive cumsum of g (per channel k), base / end its values just
-// before / at the window's last token and m the midpoint of its range:
+// before / at the window's last token and m near the midpoint of its range:
 //     A^T[s][t] = sum_k (k_s e^{m-G_s})[k] (q_e,t e^{G_t-m})[k]   (s <= t)   MFMA, K = dk
 //     o^T[v][t] = sum_s v^T[v][s] A^T[s][t]                                    MFMA
 //               + sum_k (S[k][v] e^{m-base}) (q_e,t e^{G_t-m})[k]              MFMA (state read-out)
-//     S[k][v]  <- e^{end-base} S[k][v] + sum_s (e^{end-m} k_s e^{m-G_s})[k] v_s[v]   MFMA
+//     S[k][v]  <- e^{end-m} (e^{m-base} S[k][v] + sum_s (k_s e^{m-G_s})[k] v_s[v])   MFMA
 // Windows are cut so that the spread of G within one never exceeds KRANGE,
 // which keeps every factor finite.
 #include "common.h"
@@ -29,40 +29,65 @@ namespace {
 constexpr int SEGK = 64;          // tokens per segment (max)
 constexpr int DK = 128;
 constexpr int DVH = 64;           // v columns per workgroup
+constexpr float LOG2E = 1.44269504088896340736f;
 constexpr float KRANGE = 50.f;    // max spread of G per channel within a segment
 
 // ----------------------------------------------------------------- gated mode
 // One workgroup of 8 waves per (b, h, V-half) walks the sequence in 64-token
 // tiles.  The next tile's q1, q2, k, v and g are loaded into registers while
-// the current tile computes, so the walk streams at memory speed.  Wave w owns v-tile vt = w & 1, t-tile tt = (w >> 1) & 1 and
-// k-half kh = w >> 2: it keeps the state tiles S[kh][vt] (replicated over tt),
-// computes the read-out partial of (vt, tt) over its k-half, and the kh = 1
-// partials are summed through LDS.  Waves 5..7 also form the three masked
-// A^T tiles while waves 0..4 transpose the token-contracted operands (k^T,
-// v^T) on the MFMA unit, each transpose once per tile, shared through LDS.  A tile is one factorisation window unless the spread of G within it
-// exceeds KRANGE for some channel; it is then cut into shorter windows.
+// the current tile computes.  Wave w owns v-tile vt = w & 1, t-tile
+// tt = (w >> 1) & 1 and k-half kh = w >> 2: it keeps the state tiles S[kh][vt]
+// (replicated over tt) and computes the read-out partial of (vt, tt) over its
+// k-half; the kh = 1 partials are summed through LDS.  Waves 5..7 also form the
+// three masked A^T tiles.  A tile is one factorisation window unless the spread
+// of G within it exceeds KRANGE for some channel; it is then cut into shorter
+// windows.
+//
+// One workgroup per CU (the grid is 2 B H), so every barrier and LDS round trip
+// of a tile is exposed: a tile has three barriers.  Each thread keeps 4 tokens x
+// 4 channels of g, q and k in registers, so the cumsum is 4 additions, one
+// exchange between the wave's halves and the sum of the earlier waves' totals,
+// and G never passes through LDS; with base = 0 and m = end / 2 both window
+// factors are e^m.  The token-contracted operands are read transposed by the
+// LDS, and the state update S <- e^{end-m} (e^{m-base} S + K~^T v) starts from the
+// scaled state that the read-out multiplies, so it needs no barrier of its own.
 constexpr int KW = 8;                 // waves per workgroup
 
 struct KdaGatedSmem {
-  float G[SEG][DK];                   // raw g of the tile (direct loads), then its in-tile inclusive cumsum
-  bf16 Qt[SEG * DK];                  // q_e e^{G - m}   (Tile<bf16, DK>, zero rows outside the window)
-  bf16 Kt[SEG * DK];                  // k e^{m - G}     (zero rows outside the window)
-  bf16 V[SEG * DVH];                  // v[:, V-half]    (Tile<bf16, DVH>)
+  float G[SEG][DK];                   // in-tile inclusive cumsum of g (tiles that are cut only)
+  static constexpr int PK = DK + 24, PV = DVH + 32;   // pitches of KdaRefSmem (transposing and row reads spread over the banks)
+  bf16 Qt[SEG * PK];                  // q_e e^{G - m}, zero rows outside the window
+  bf16 Kt[SEG * PK];                  // k e^{m - G}, zero rows outside the window
+  bf16 V[SEG * PV];                   // v[:, V-half]
   Frag<bf16> A[3][2][64];             // masked A^T tiles (s0,t0), (s0,t1), (s1,t1) as B-operand fragments
-  Frag<bf16> VF[2][4][64];            // v^T fragments per v-tile (lane = v, k = token 16 c + KSET)
-  Frag<bf16> KF[4][4][64];            // e^{end - m}-scaled k^T fragments per k-tile (lane = channel)
-  f32x16 red[2][2][64];               // read-out partials of the kh = 1 waves: vt, tt, lane
+  AccPark red[2][2];                  // read-out partials of the kh = 1 waves: vt, tt
   bf16 O[4][32 * 32];                 // o blocks (vt, tt) staged for coalesced stores (XHalf rows 0..31)
-  float qtot[4][DK], qmin[4][DK], qmax[4][DK];   // per token-quarter cumsum statistics
-  float mm[DK], em[DK], ek[DK], eg[DK];          // window midpoint m, e^{m - base}, e^{end - m}, e^{end - base}
-  int wend, cut;
+  float wtot[KW][DK];                 // sums of g over each wave's 8 tokens
+  alignas(16) float mm[DK];           // window midpoint m (tiles that are cut)
+  alignas(16) float em[DK];           // e^{m - base + pl}
+  alignas(16) float pl[2][DK];        // by the tile's parity: end - m of the window before the tile
+  int wend, cut[2];                   // cut: by the tile's parity
 };
 
-// Register-staged q1, q2, k (two 16-byte chunks each per thread), v (one) and g (four) of a tile.
+// A tile's rows in registers: 4 tokens x 4 channels of q1, q2, k and g, one 16-byte chunk of v.
 struct KdaStage {
-  uint4 q1[2], q2[2], k[2], v;
+  bf16x4 q1[4], q2[4], k[4];
+  uint4 v;
   f32x4 g[4];
 };
+
+// 8 consecutive elements of a row, and the 4 + 4 (8 apart) that match an accumulator's row order, as fragments.
+__device__ __forceinline__ Frag<bf16> rows8(const bf16* p) {
+  Frag<bf16> f;
+  f.v = *reinterpret_cast<const bf16x8*>(p);
+  return f;
+}
+__device__ __forceinline__ Frag<bf16> kset8(const bf16* p) {
+  const bf16x4 lo = *reinterpret_cast<const bf16x4*>(p), hi = *reinterpret_cast<const bf16x4*>(p + 8);
+  Frag<bf16> f;
+  f.v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  return f;
+}
 
 }  // namespace
 
@@ -71,8 +96,7 @@ struct KdaStage {
 template <bool SPLIT>
 __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
   __shared__ KdaGatedSmem sm;
-  using TQ = Tile<bf16, DK>;
-  using TV = Tile<bf16, DVH>;
+  using SM = KdaGatedSmem;
   using XO = XHalf<bf16>;
   const int nbh = p.batch * p.nheads;
   int bh, vh;
@@ -100,10 +124,6 @@ __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
   bf16* og = reinterpret_cast<bf16*>(p.o);
   const int v0 = vh * DVH;
   const bool has_q2 = p.q2 != nullptr, has_g = p.g != nullptr;
-  Frag<bf16> id[2];
-  id[0] = ident_frag<bf16>(0, half, l32);
-  id[1] = ident_frag<bf16>(1, half, l32);
-
   // state tiles S[k][v] for k-tile 2 kh + i, v-tile vt of this V-half
   f32x16 St[2];
 #pragma unroll
@@ -136,99 +156,127 @@ __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
   }
 
   // tile loads into registers (plain loads: a direct-to-LDS load in flight would make every later LDS
-  // access of the tile wait for it): q1 / q2 / k chunks e = tid + 512 i -> row e >> 4, columns 8 (e & 15);
-  // v chunk tid -> row tid >> 3, columns v0 + 8 (tid & 7); g chunks e = tid + 512 i -> row e >> 5, columns 4 (e & 31)
+  // access of the tile wait for it): tokens 4 (tid >> 5) + i, channels 4 (tid & 31) .. of q1, q2, k and g;
+  // v chunk tid -> row tid >> 3, columns v0 + 8 (tid & 7)
+  const int r0 = 4 * (tid >> 5), c4 = 4 * (tid & 31);
   KdaStage stg;
-  auto load_qk = [&](int pos) {
-    const int last = S - 1;
+  auto load = [&](int pos) {
+    // uniform bases and 32-bit lane offsets, formed here (hoisted, they would hold 40 registers through the loop)
+    int th = tid;
+    asm volatile("" : "+v"(th));
+    const int last = S - 1 - pos;
+    const char* vb = reinterpret_cast<const char*>(vg + (rowbase + pos) * 128 + v0);
+    const int64_t o = (rowbase + pos) * DK;
+    const char *gb = reinterpret_cast<const char*>(p.g + o), *kb = reinterpret_cast<const char*>(kg + o),
+               *q1b = reinterpret_cast<const char*>(q1g + o), *q2b = reinterpret_cast<const char*>(q2g + o);
+    stg.v = *reinterpret_cast<const uint4*>(vb + (uint32_t)(min(th >> 3, last) * 256 + 16 * (th & 7)));
+    uint32_t off[4];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int e = tid + 512 * i;
-      const int64_t off = (rowbase + min(pos + (e >> 4), last)) * DK + 8 * (e & 15);
-      stg.q1[i] = *reinterpret_cast<const uint4*>(q1g + off);
-      if (has_q2) stg.q2[i] = *reinterpret_cast<const uint4*>(q2g + off);
-      stg.k[i] = *reinterpret_cast<const uint4*>(kg + off);
-    }
-  };
-  auto load_gv = [&](int pos) {
-    const int last = S - 1;
-    stg.v = *reinterpret_cast<const uint4*>(vg + (rowbase + min(pos + (tid >> 3), last)) * 128 + v0 + 8 * (tid & 7));
+    for (int i = 0; i < 4; ++i) off[i] = (uint32_t)(min(4 * (th >> 5) + i, last) * (2 * DK) + 8 * (th & 31));
     if (has_g) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int e = tid + 512 * i;                     // row e >> 5, columns 4 (e & 31)
-        stg.g[i] = *reinterpret_cast<const f32x4*>(p.g + (rowbase + min(pos + (e >> 5), last)) * DK + 4 * (e & 31));
-      }
+      for (int i = 0; i < 4; ++i) stg.g[i] = *reinterpret_cast<const f32x4*>(gb + 2 * off[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      stg.k[i] = *reinterpret_cast<const bf16x4*>(kb + off[i]);
+      stg.q1[i] = *reinterpret_cast<const bf16x4*>(q1b + off[i]);
+    }
+    if (has_q2) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) stg.q2[i] = *reinterpret_cast<const bf16x4*>(q2b + off[i]);
     }
   };
-  load_gv(p0);
-  load_qk(p0);
+  if (tid == 0) sm.cut[0] = sm.cut[1] = 0;
+  if (tid < DK) sm.pl[0][tid] = 0.f;
+  load(p0);
 
-  for (int pos = p0; pos < p1; pos += SEG) {
+  f32x4 G[4], low;                                       // sums of g over this thread's tokens, before them
+  // Qt = q_e e^{G - m}, Kt = k e^{m - G} on rows [a, b), zero elsewhere (FULL: every row, two queries); the largest |G - m|
+  // in units of ln 2
+  auto scale = [&](auto FULLc, const f32x4& m, int a, int b) {
+    constexpr bool FULL = decltype(FULLc)::value;
+    const f32x4 c = (low - m) * LOG2E;
+    float top = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = r0 + i;
+      bf16x4 qo, ko;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float d = __builtin_fmaf(G[i][j], LOG2E, c[j]);
+        const float qe = FULL || has_q2 ? __builtin_fmaf(-lam, (float)stg.q2[i][j], (float)stg.q1[i][j]) : (float)stg.q1[i][j];
+        top = fmaxf(top, fabsf(d));
+        qo[j] = (bf16)(qe * __builtin_amdgcn_exp2f(d));
+        ko[j] = (bf16)((float)stg.k[i][j] * __builtin_amdgcn_exp2f(-d));
+      }
+      uint2 qw = __builtin_bit_cast(uint2, qo), kw = __builtin_bit_cast(uint2, ko);
+      if (!FULL && !(r >= a && r < b)) qw = kw = uint2{0, 0};
+      *reinterpret_cast<uint2*>(&sm.Qt[r * SM::PK + c4]) = qw;
+      *reinterpret_cast<uint2*>(&sm.Kt[r * SM::PK + c4]) = kw;
+    }
+    return top;
+  };
+  // The whole tile as one window: base 0, end - m = m; every factor within e^{+-KRANGE / 2}, or the tile is cut.
+  auto stage = [&](auto FULLc, int len, int par) {
+    constexpr bool FULL = decltype(FULLc)::value;
+    *reinterpret_cast<uint4*>(&sm.V[(tid >> 3) * SM::PV + 8 * (tid & 7)]) = stg.v;
+    // the in-tile inclusive cumsum of g, g = 0 past the end (G stays flat)
+    f32x4 run = {0.f, 0.f, 0.f, 0.f}, both;              // both: the wave's eight tokens
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (FULL || (has_g && r0 + i < len)) run += stg.g[i];
+      G[i] = run;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float first = from_half(run[j], 0);          // every lane active: the swap reads both halves
+      low[j] = half ? first : 0.f;
+      both[j] = sum_halves(run[j]);
+    }
+    if (half == 0) *reinterpret_cast<f32x4*>(&sm.wtot[w][c4]) = both;
+    lds_barrier();                                       // B1: the waves' sums
+    f32x4 end = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < KW; ++j) {
+      if (j && j == w) {
+        low += end;
+        asm volatile("" : "+v"(low));                    // a scalar branch, not four selects
+      }
+      end += *reinterpret_cast<const f32x4*>(&sm.wtot[j][c4]);
+    }
+    const f32x4 m = 0.5f * end;
+    const float top = scale(FULLc, m, 0, len);
+    if (w == 0 && half == 0) {
+      const f32x4 pv = *reinterpret_cast<const f32x4*>(&sm.pl[par][c4]);
+      f32x4 e;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) e[j] = __expf(m[j] + pv[j]);
+      *reinterpret_cast<f32x4*>(&sm.em[c4]) = e;
+      *reinterpret_cast<f32x4*>(&sm.pl[par ^ 1][c4]) = m;
+    }
+    if (tid == 0) sm.cut[par ^ 1] = 0;                   // read a tile ago, set after the next tile's B1
+    if (top > 0.5f * KRANGE * LOG2E) sm.cut[par] = 1;    // benign race: every writer stores 1
+  };
+  const bool plain = has_g && has_q2;
+  int par = 0;
+  for (int pos = p0; pos < p1; pos += SEG, par ^= 1) {
     const int len = min(SEG, S - pos);
     wait_vmem();                                         // this tile's registers
-    *reinterpret_cast<uint4*>(&sm.V[TV::chunk(tid >> 3, tid & 7)]) = stg.v;
-    if (has_g) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int e = tid + 512 * i;
-        *reinterpret_cast<f32x4*>(&sm.G[e >> 5][4 * (e & 31)]) = stg.g[i];
-      }
-    }
-    lds_barrier();                                       // B1: g and v rows are in LDS
-
-    // ---- in-tile cumsum of g per channel: thread (channel kc, token quarter qq)
-    {
-      const int kc = tid & (DK - 1), qq = tid >> 7;
-      float loc[16];
-      float run = 0.f, lmin = INFINITY, lmax = -INFINITY;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int t = 16 * qq + i;
-        const float gv = (has_g && t < len) ? sm.G[t][kc] : 0.f;   // g = 0 past the end: G stays flat
-        run += gv;
-        loc[i] = run;
-        lmin = fminf(lmin, run);
-        lmax = fmaxf(lmax, run);
-      }
-      sm.qtot[qq][kc] = run;
-      sm.qmin[qq][kc] = lmin;
-      sm.qmax[qq][kc] = lmax;
-      if (tid == 0) sm.cut = 0;                          // set below (after B2), read after B3
-      lds_barrier();                                     // B2
-      float off = 0.f, end = 0.f, gmin = INFINITY, gmax = -INFINITY;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float tq = sm.qtot[q][kc];
-        gmin = fminf(gmin, end + sm.qmin[q][kc]);
-        gmax = fmaxf(gmax, end + sm.qmax[q][kc]);
-        if (q < qq) off += tq;
-        end += tq;
-      }
-#pragma unroll
-      for (int i = 0; i < 16; ++i) sm.G[16 * qq + i][kc] = loc[i] + off;
-      if (qq == 0) {
-        // window [0, len): base G_{-1} = 0, end = G_{len-1}, m = midpoint of the G range
-        const float m = 0.5f * (gmin + gmax);
-        sm.mm[kc] = m;
-        sm.em[kc] = __expf(m);
-        sm.ek[kc] = __expf(end - m);
-        sm.eg[kc] = __expf(end);
-        if (gmax - gmin > KRANGE) sm.cut = 1;            // benign race: every writer stores 1
-      }
-    }
-    lds_barrier();                                       // B3: G, window parameters, cut flag
-    const bool cut = sm.cut != 0;
+    if (plain && len == SEG) stage(std::true_type{}, len, par);
+    else stage(std::false_type{}, len, par);
+    lds_barrier();                                       // B2: Qt, Kt, V, window factors, cut flag
+    const bool cut = sm.cut[par] != 0;
 
     // ---- factorisation windows [a, b) of this tile
     for (int a = 0; a < len;) {
-      // lane-dependent LDS addresses are recomputed per window instead of hoisted (and spilled)
-      int lq = l;
-      asm volatile("" : "+v"(lq));
-      const int halfq = lq >> 5, l32q = lq & 31;
       int b = len;
       if (cut) {
         // longest window from a whose per-channel G spread stays within KRANGE (at least one token)
+        if (a == 0) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) *reinterpret_cast<f32x4*>(&sm.G[r0 + i][c4]) = G[i] + low;
+        }
         if (tid == 0) sm.wend = len;
         lds_barrier();
         if (tid < DK) {
@@ -254,78 +302,37 @@ __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
           const float base = a ? sm.G[a - 1][tid] : 0.f, end = sm.G[b - 1][tid];
           const float m = 0.5f * (mn + mx);
           sm.mm[tid] = m;
-          sm.em[tid] = __expf(m - base);
-          sm.ek[tid] = __expf(end - m);
-          sm.eg[tid] = __expf(end - base);
+          sm.em[tid] = __expf(m - base + sm.pl[a ? par ^ 1 : par][tid]);
+          sm.pl[par ^ 1][tid] = end - m;
         }
         lds_barrier();
+        scale(std::false_type{}, *reinterpret_cast<const f32x4*>(&sm.mm[c4]), a, b);
+        lds_barrier();
       }
-      const bool last_window = (b == len);
+      if (b == len && pos + SEG < p1) load(pos + SEG);   // the next tile streams in behind this one's products
 
-      // Qt = q_e e^{G - m}, Kt = k e^{m - G} on rows [a, b), zero elsewhere
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int e = tid + 512 * i;
-        const int r = e >> 4, c8 = e & 15;
-        bf16x8 qo, ko;
-        if (r >= a && r < b) {
-          const bf16x8 x1 = __builtin_bit_cast(bf16x8, stg.q1[i]);
-          const bf16x8 x2 = __builtin_bit_cast(bf16x8, stg.q2[i]);
-          const bf16x8 xk = __builtin_bit_cast(bf16x8, stg.k[i]);
-          const f32x4 g0 = *reinterpret_cast<const f32x4*>(&sm.G[r][8 * c8]);
-          const f32x4 g1 = *reinterpret_cast<const f32x4*>(&sm.G[r][8 * c8 + 4]);
-          const f32x4 m0 = *reinterpret_cast<const f32x4*>(&sm.mm[8 * c8]);
-          const f32x4 m1 = *reinterpret_cast<const f32x4*>(&sm.mm[8 * c8 + 4]);
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const float d = (j < 4 ? g0[j] : g1[j - 4]) - (j < 4 ? m0[j] : m1[j - 4]);   // G - m
-            const float qe = has_q2 ? (float)x1[j] - lam * (float)x2[j] : (float)x1[j];
-            qo[j] = (bf16)(qe * __expf(d));
-            ko[j] = (bf16)((float)xk[j] * __expf(-d));
-          }
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) qo[j] = ko[j] = (bf16)0.f;
-        }
-        *reinterpret_cast<bf16x8*>(&sm.Qt[TQ::chunk(r, c8)]) = qo;
-        *reinterpret_cast<bf16x8*>(&sm.Kt[TQ::chunk(r, c8)]) = ko;
-      }
-      lds_barrier();                                     // Qt, Kt ready; G no longer read
-      const bool prefetch = last_window && pos + SEG < p1;
-      if (prefetch) load_gv(pos + SEG);                  // the next tile streams in behind the MFMAs
-
-      // ---- phase 1: A^T tiles (waves 5..7), the 12 operand transposes (waves 0..4), read-out partials
-      if (w < 5) {
-        // jobs 0..3: v^T of (v-tile j >> 1, token tile j & 1); 4..11: k^T of (k-tile (j-4) >> 1, token tile)
-        for (int j = w; j < 12; j += 5) {
-          if (j < 4) {
-            const int vtj = j >> 1, st = j & 1;
-            const f32x16 d = mfma_transpose<bf16, bf16, DVH>(sm.V, 32 * st, 32 * vtj, id, halfq, l32q);
-            sm.VF[vtj][2 * st][lq] = acc_to_frag<bf16>(d, 0);
-            sm.VF[vtj][2 * st + 1][lq] = acc_to_frag<bf16>(d, 1);
-          } else {
-            const int kt = (j - 4) >> 1, st = (j - 4) & 1;
-            const float ekl = sm.ek[32 * kt + l32q];
-            const f32x16 d = mfma_transpose<bf16, bf16, DK>(sm.Kt, 32 * st, 32 * kt, id, halfq, l32q);
-            sm.KF[kt][2 * st][lq] = acc_to_frag_scaled<bf16>(d, 0, ekl);
-            sm.KF[kt][2 * st + 1][lq] = acc_to_frag_scaled<bf16>(d, 1, ekl);
-          }
-        }
-      } else {
+      // ---- phase 1: A^T tiles (waves 5..7), read-out partials, state update
+      if (w >= 5) {
         const int it = w - 5;
         const int st = (it == 2) ? 1 : 0, ttA = (it == 0) ? 0 : 1;
         f32x16 acc = zero16();
 #pragma unroll
         for (int c = 0; c < DK / 16; ++c)
-          acc = mma(row_frag<bf16, bf16, DK>(sm.Kt, 32 * st + l32q, 16 * c + 8 * halfq),
-                    row_frag<bf16, bf16, DK>(sm.Qt, 32 * ttA + l32q, 16 * c + 8 * halfq), acc);
+          acc = mma(rows8(sm.Kt + (32 * st + l32) * SM::PK + 8 * half + 16 * c),
+                    rows8(sm.Qt + (32 * ttA + l32) * SM::PK + 8 * half + 16 * c), acc);
+        if (st == ttA) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r)
-          if (32 * st + acc_row(halfq, r) > 32 * ttA + l32q) acc[r] = 0.f;
-        sm.A[it][0][lq] = acc_to_frag<bf16>(acc, 0);
-        sm.A[it][1][lq] = acc_to_frag<bf16>(acc, 1);
+          for (int r = 0; r < 16; ++r)
+            if (acc_row(half, r) > l32) acc[r] = 0.f;
+        }
+        sm.A[it][0][l] = acc_to_frag<bf16>(acc, 0);
+        sm.A[it][1][l] = acc_to_frag<bf16>(acc, 1);
       }
-      // o^T[v][t] = sum_k (S[k][v] e^{m_k - base_k}) Qt[t][k] over this wave's k-half, t-tile tt
+      // o^T[v][t] = sum_k (S[k][v] e^{m_k - base_k}) Qt[t][k] over this wave's k-half, t-tile tt, and
+      // St[k][v] <- S[k][v] e^{m_k - base_k} + sum_s Kt[s][k] v_s[v], with S = e^{pl} St of the window before
+      Frag<bf16> vf[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) vf[c] = col_frag_tr(sm.V, SM::PV, 32 * vt, 16 * c);
       f32x16 o = zero16();
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
@@ -333,68 +340,45 @@ __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
         f32x16 sv = St[i];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const f32x4 e4 = *reinterpret_cast<const f32x4*>(&sm.em[32 * kt + 8 * q + 4 * halfq]);
+          const f32x4 e4 = *reinterpret_cast<const f32x4*>(&sm.em[32 * kt + 8 * q + 4 * half]);
 #pragma unroll
           for (int j = 0; j < 4; ++j) sv[4 * q + j] *= e4[j];
         }
 #pragma unroll
         for (int c = 0; c < 2; ++c)
-          o = mma(acc_to_frag<bf16>(sv, c), kset_frag<bf16, bf16, DK>(sm.Qt, 32 * tt + l32q, 32 * kt + 16 * c, halfq), o);
-      }
-      lds_barrier();                                     // A^T, v^T, k^T fragments ready
-      if (prefetch) load_qk(pos + SEG);
-
-      // ---- phase 2: intra-window term (kh = 0), partial exchange, state update
-      Frag<bf16> vf[4];
+          o = mma(acc_to_frag<bf16>(sv, c), kset8(sm.Qt + (32 * tt + l32) * SM::PK + 4 * half + 32 * kt + 16 * c), o);
 #pragma unroll
-      for (int c = 0; c < 4; ++c) vf[c] = sm.VF[vt][c][lq];
+        for (int c = 0; c < 4; ++c) sv = mma(col_frag_tr(sm.Kt, SM::PK, 32 * kt, 16 * c), vf[c], sv);
+        St[i] = sv;
+      }
+      if (kh) park_acc(sm.red[vt][tt], o, l);
+      lds_barrier();                                     // B3: A^T tiles and partials; Qt, Kt and V have been read
+
+      // ---- phase 2 (the kh = 0 waves; the others go on to the next tile): intra-window term, then output rows
+      // [a, b) of block (vt, tt), staged for 16-byte stores
       if (kh == 0) {
         if (tt == 0) {
-          o = mma(vf[0], sm.A[0][0][lq], o);
-          o = mma(vf[1], sm.A[0][1][lq], o);
+          o = mma(vf[0], sm.A[0][0][l], o);
+          o = mma(vf[1], sm.A[0][1][l], o);
         } else {
-          o = mma(vf[0], sm.A[1][0][lq], o);
-          o = mma(vf[1], sm.A[1][1][lq], o);
-          o = mma(vf[2], sm.A[2][0][lq], o);
-          o = mma(vf[3], sm.A[2][1][lq], o);
+          o = mma(vf[0], sm.A[1][0][l], o);
+          o = mma(vf[1], sm.A[1][1][l], o);
+          o = mma(vf[2], sm.A[2][0][l], o);
+          o = mma(vf[3], sm.A[2][1][l], o);
         }
-      } else {
-        sm.red[vt][tt][lq] = o;
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int kt = 2 * kh + i;
-        Frag<bf16> kf[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) kf[c] = sm.KF[kt][c][lq];
-        f32x16 acc = St[i];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const f32x4 e4 = *reinterpret_cast<const f32x4*>(&sm.eg[32 * kt + 8 * q + 4 * halfq]);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) acc[4 * q + j] *= e4[j];
-        }
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc = mma(kf[c], vf[c], acc);
-        St[i] = acc;
-      }
-      lds_barrier();                                     // partials in LDS; tile fragments no longer read
-
-      // ---- output rows [a, b) of block (vt, tt): staged, then 16-byte stores
-      if (kh == 0) {
-        const f32x16 other = sm.red[vt][tt][lq];
+        const f32x16 other = unpark_acc(sm.red[vt][tt], l);
         bf16* ob = sm.O[2 * vt + tt];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const int c0 = 8 * q + 4 * halfq;              // 4 consecutive v columns inside one 16-byte chunk
+          const int c0 = 8 * q + 4 * half;              // 4 consecutive v columns inside one 16-byte chunk
           bf16x4 yv;
 #pragma unroll
           for (int j = 0; j < 4; ++j) yv[j] = (bf16)(o[4 * q + j] + other[4 * q + j]);
-          *reinterpret_cast<bf16x4*>(ob + XO::chunk(l32q, c0 >> 3) + (c0 & 7)) = yv;
+          *reinterpret_cast<bf16x4*>(ob + XO::chunk(l32, c0 >> 3) + (c0 & 7)) = yv;
         }
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-          const int e = lq + 64 * i;
+          const int e = l + 64 * i;
           const int r = e >> 2, c = e & 3;               // row t of the block, 16-byte chunk
           const uint4 val = *reinterpret_cast<const uint4*>(ob + XO::chunk(r, c));
           const int t = 32 * tt + r;
@@ -413,7 +397,7 @@ __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int kr = 32 * (2 * kh + i) + acc_row(half, r);
-        sf_out[kr * 128 + v0 + 32 * vt + l32] = St[i][r];
+        sf_out[kr * 128 + v0 + 32 * vt + l32] = St[i][r] * __expf(sm.pl[par][kr]);
       }
   }
 }
