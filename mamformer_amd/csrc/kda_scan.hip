@@ -34,46 +34,51 @@ constexpr float KRANGE = 50.f;    // max spread of G per channel within a segmen
 
 // ----------------------------------------------------------------- gated mode
 // One workgroup of 8 waves per (b, h, V-half) walks the sequence in 64-token
-// tiles.  The next tile's q1, q2, k, v and g are loaded into registers while
-// the current tile computes.  Wave w owns v-tile vt = w & 1, t-tile
-// tt = (w >> 1) & 1 and k-half kh = w >> 2: it keeps the state tiles S[kh][vt]
-// (replicated over tt) and computes the read-out partial of (vt, tt) over its
-// k-half; the kh = 1 partials are summed through LDS.  Waves 5..7 also form the
-// three masked A^T tiles.  A tile is one factorisation window unless the spread
-// of G within it exceeds KRANGE for some channel; it is then cut into shorter
-// windows.
+// tiles, as a pipeline of two roles.  Waves 4..7 prepare: they hold the next
+// tile's rows in registers, form the in-tile cumsum of g and write Qt, Kt and V
+// of tile n + 1 to LDS.  Waves 0..3 multiply: wave w owns v-tile vt = w & 1 and
+// k-half kh = w >> 1, keeps the state tiles S[kh][vt], forms the read-out of tile
+// n over its k-half and the state update; waves 1..3 also form the three masked
+// A^T tiles.  The k-halves' partials are exchanged through LDS and wave (vt, kh)
+// finishes token tile tt = kh.  A tile is one factorisation window unless the
+// spread of G within it exceeds KRANGE for some channel; it is then cut into
+// shorter windows, which both roles walk together.
 //
-// One workgroup per CU (the grid is 2 B H), so every barrier and LDS round trip
-// of a tile is exposed: a tile has three barriers.  Each thread keeps 4 tokens x
-// 4 channels of g, q and k in registers, so the cumsum is 4 additions, one
-// exchange between the wave's halves and the sum of the earlier waves' totals,
-// and G never passes through LDS; with base = 0 and m = end / 2 both window
-// factors are e^m.  The token-contracted operands are read transposed by the
-// LDS, and the state update S <- e^{end-m} (e^{m-base} S + K~^T v) starts from the
-// scaled state that the read-out multiplies, so it needs no barrier of its own.
+// One workgroup per CU (the grid is 2 B H), so what a tile costs is its chain of
+// barriers and LDS round trips, and with every wave in the same phase the
+// exponentials and conversions (VALU) never ran beside the products (MFMA, LDS):
+// 4.5 us a tile in that form.  Here one wave of each role shares each SIMD and a
+// step has two barriers: scaling of tile n + 1 beside the products of tile n,
+// then the cumsum of tile n + 2 beside the output of tile n.  With base = 0 and
+// m = end / 2 both window factors are e^m; the factor between two windows'
+// states is applied once, where the read-out needs it; the token-contracted
+// operands are read transposed by the LDS.
 constexpr int KW = 8;                 // waves per workgroup
 
-struct KdaGatedSmem {
-  float G[SEG][DK];                   // in-tile inclusive cumsum of g (tiles that are cut only)
+struct KdaGatedTile {
   static constexpr int PK = DK + 24, PV = DVH + 32;   // pitches of KdaRefSmem (transposing and row reads spread over the banks)
   bf16 Qt[SEG * PK];                  // q_e e^{G - m}, zero rows outside the window
   bf16 Kt[SEG * PK];                  // k e^{m - G}, zero rows outside the window
   bf16 V[SEG * PV];                   // v[:, V-half]
+};
+struct KdaGatedSmem {
+  alignas(16) KdaGatedTile t[2];      // by the tile's parity; a cut tile's G lies in the other one's Qt and Kt
   Frag<bf16> A[3][2][64];             // masked A^T tiles (s0,t0), (s0,t1), (s1,t1) as B-operand fragments
-  AccPark red[2][2];                  // read-out partials of the kh = 1 waves: vt, tt
-  bf16 O[4][32 * 32];                 // o blocks (vt, tt) staged for coalesced stores (XHalf rows 0..31)
-  float wtot[KW][DK];                 // sums of g over each wave's 8 tokens
+  AccPark red[2][2];                  // read-out partials for the wave of the other k-half: vt, tt
+  bf16 O[4][32 * 32];                 // o blocks staged for coalesced stores (XHalf rows 0..31)
+  alignas(16) float wtot[4][DK];      // sums of g over each preparing wave's 16 tokens
   alignas(16) float mm[DK];           // window midpoint m (tiles that are cut)
-  alignas(16) float em[DK];           // e^{m - base + pl}
+  alignas(16) float em[2][DK];        // by the tile's parity: e^{m - base + pl}
   alignas(16) float pl[2][DK];        // by the tile's parity: end - m of the window before the tile
   int wend, cut[2];                   // cut: by the tile's parity
 };
+static_assert(sizeof(bf16) * 2 * SEG * KdaGatedTile::PK >= sizeof(float) * SEG * DK, "G fits beside a tile");
 
-// A tile's rows in registers: 4 tokens x 4 channels of q1, q2, k and g, one 16-byte chunk of v.
+// A preparing thread's rows: 8 tokens x 4 channels of q1, q2, k and g, two 16-byte chunks of v.
 struct KdaStage {
-  bf16x4 q1[4], q2[4], k[4];
-  uint4 v;
-  f32x4 g[4];
+  bf16x4 q1[8], q2[8], k[8];
+  uint4 v[2];
+  f32x4 g[8];
 };
 
 // 8 consecutive elements of a row, and the 4 + 4 (8 apart) that match an accumulator's row order, as fragments.
@@ -96,7 +101,7 @@ __device__ __forceinline__ Frag<bf16> kset8(const bf16* p) {
 template <bool SPLIT>
 __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
   __shared__ KdaGatedSmem sm;
-  using SM = KdaGatedSmem;
+  using TL = KdaGatedTile;
   using XO = XHalf<bf16>;
   const int nbh = p.batch * p.nheads;
   int bh, vh;
@@ -110,21 +115,240 @@ __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
   }
   const int h = bh % p.nheads;
   const int w = wave_id(), l = lane_id(), half = l >> 5, l32 = l & 31;
-  const int vt = w & 1, tt = (w >> 1) & 1, kh = w >> 2;
-  const int tid = threadIdx.x;
   const int S = p.seqlen;
-  const float lam = p.lam_h ? p.lam_h[h] : p.lam;
   const int64_t rowbase = (int64_t)bh * S;          // token row index base in (B,H,S,*) tensors
   const int seg = SPLIT ? blockIdx.y : 0;           // this workgroup's segment: tokens [p0, p1)
   const int p0 = SPLIT ? seg * p.seg_chunks * SEG : 0, p1 = SPLIT ? min(S, p0 + p.seg_chunks * SEG) : S;
-  const bf16* q1g = reinterpret_cast<const bf16*>(p.q1);
-  const bf16* q2g = reinterpret_cast<const bf16*>(p.q2);
-  const bf16* kg = reinterpret_cast<const bf16*>(p.k);
-  const bf16* vg = reinterpret_cast<const bf16*>(p.v);
-  bf16* og = reinterpret_cast<bf16*>(p.o);
+  const int nt = (p1 - p0 + SEG - 1) / SEG;
   const int v0 = vh * DVH;
-  const bool has_q2 = p.q2 != nullptr, has_g = p.g != nullptr;
-  // state tiles S[k][v] for k-tile 2 kh + i, v-tile vt of this V-half
+  // Both roles run the same barriers: one after the first cumsum, then per step n (products of tile n) any of a cut
+  // tile's windows and two.
+
+  if (w >= 4) {
+    // ------------------------------------------------------------ preparing waves
+    const bool has_q2 = p.q2 != nullptr, has_g = p.g != nullptr, plain = has_g && has_q2;
+    const float lam = p.lam_h ? p.lam_h[h] : p.lam;
+    const int pt = threadIdx.x & 255, pw = w - 4;
+    const int r0 = 8 * (pt >> 5), c4 = 4 * (pt & 31);   // tokens r0 .., channels c4 ..
+    const bf16* q1g = reinterpret_cast<const bf16*>(p.q1) + rowbase * DK;
+    const bf16* q2g = reinterpret_cast<const bf16*>(p.q2) + rowbase * DK;
+    const bf16* kg = reinterpret_cast<const bf16*>(p.k) + rowbase * DK;
+    const bf16* vg = reinterpret_cast<const bf16*>(p.v) + rowbase * 128 + v0;
+    const float* gg = p.g + rowbase * DK;
+    KdaStage stg;
+    // Plain loads (a direct-to-LDS load in flight would make every later LDS access wait for it) from a uniform base
+    // and a 32-bit lane offset; rows past the sequence read its last one, a tile past it that row alone.
+    auto base_of = [&](int n) { return min(p0 + n * SEG, S - 1); };
+    auto off_of = [&](int pos, int i) { return (uint32_t)(min(r0 + i, S - 1 - pos) * DK + c4); };
+    auto load_g = [&](auto FULLc, int n) {
+      const int pos = base_of(n);
+      if (decltype(FULLc)::value || has_g) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          stg.g[i] = *reinterpret_cast<const f32x4*>(reinterpret_cast<const char*>(gg + (int64_t)pos * DK) + 4 * off_of(pos, i));
+      }
+    };
+    auto load_v = [&](int n) {
+      const int pos = base_of(n);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        stg.v[i] = *reinterpret_cast<const uint4*>(
+            reinterpret_cast<const char*>(vg + (int64_t)pos * 128) +
+            (uint32_t)(min((pt >> 3) + 32 * i, S - 1 - pos) * 256 + 16 * (pt & 7)));
+    };
+    auto load_row = [&](auto FULLc, int pos, int i) {
+      const uint32_t o = 2 * off_of(pos, i);
+      stg.q1[i] = *reinterpret_cast<const bf16x4*>(reinterpret_cast<const char*>(q1g + (int64_t)pos * DK) + o);
+      if (decltype(FULLc)::value || has_q2)
+        stg.q2[i] = *reinterpret_cast<const bf16x4*>(reinterpret_cast<const char*>(q2g + (int64_t)pos * DK) + o);
+      stg.k[i] = *reinterpret_cast<const bf16x4*>(reinterpret_cast<const char*>(kg + (int64_t)pos * DK) + o);
+    };
+    f32x4 G[8], low;                                     // sums of g over this thread's tokens, before them
+    // in-tile inclusive cumsum of g, g = 0 past the end (G stays flat); then the next tile's g
+    auto cumsum = [&](auto FULLc, int n) {
+      constexpr bool FULL = decltype(FULLc)::value;
+      const int len = min(SEG, S - (p0 + n * SEG));
+      f32x4 run = {0.f, 0.f, 0.f, 0.f}, both;            // both: the wave's 16 tokens
+      if (FULL && len == SEG) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          run += stg.g[i];
+          G[i] = run;
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          if ((FULL || has_g) && r0 + i < len) run += stg.g[i];
+          G[i] = run;
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float first = from_half(run[j], 0);        // every lane active: the swap reads both halves
+        low[j] = half ? first : 0.f;
+        both[j] = sum_halves(run[j]);
+      }
+      if (half == 0) *reinterpret_cast<f32x4*>(&sm.wtot[pw][c4]) = both;
+      load_g(FULLc, n + 1);
+    };
+    // Qt = q_e e^{G - m}, Kt = k e^{m - G}, zero rows past the end, of tile n as one window: base 0, end - m = m.  Every
+    // factor is then within e^{+-KRANGE / 2}, or the tile is cut.  Each row's registers take the next tile's row.
+    auto scale = [&](auto FULLc, int n) {
+      constexpr bool FULL = decltype(FULLc)::value;
+      const int par = n & 1, len = min(SEG, S - (p0 + n * SEG)), next = base_of(n + 1);
+      TL& T = sm.t[par];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        *reinterpret_cast<uint4*>(&T.V[((pt >> 3) + 32 * i) * TL::PV + 8 * (pt & 7)]) = stg.v[i];
+      f32x4 end = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (j && j == pw) {
+          low += end;
+          asm volatile("" : "+v"(low));                  // a scalar branch, not four selects
+        }
+        end += *reinterpret_cast<const f32x4*>(&sm.wtot[j][c4]);
+      }
+      const f32x4 m = 0.5f * end, c = (low - m) * LOG2E;
+      float top = 0.f;                                   // the largest |G - m|, in units of ln 2
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        bf16x4 qo, ko;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float d = __builtin_fmaf(G[i][j], LOG2E, c[j]);
+          const float qe = FULL || has_q2 ? __builtin_fmaf(-lam, (float)stg.q2[i][j], (float)stg.q1[i][j])
+                                          : (float)stg.q1[i][j];
+          top = fmaxf(top, fabsf(d));
+          qo[j] = (bf16)(qe * __builtin_amdgcn_exp2f(d));
+          ko[j] = (bf16)((float)stg.k[i][j] * __builtin_amdgcn_exp2f(-d));
+        }
+        uint2 qw = __builtin_bit_cast(uint2, qo), kw = __builtin_bit_cast(uint2, ko);
+        if (!FULL && r0 + i >= len) qw = kw = uint2{0, 0};
+        *reinterpret_cast<uint2*>(&T.Qt[(r0 + i) * TL::PK + c4]) = qw;
+        *reinterpret_cast<uint2*>(&T.Kt[(r0 + i) * TL::PK + c4]) = kw;
+        load_row(FULLc, next, i);
+        __builtin_amdgcn_sched_barrier(0);               // a row at a time: interleaved, the rows spill
+      }
+      load_v(n + 1);
+      if (pw == 0 && half == 0) {
+        const f32x4 pv = *reinterpret_cast<const f32x4*>(&sm.pl[par][c4]);
+        f32x4 e;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) e[j] = __expf(m[j] + pv[j]);
+        *reinterpret_cast<f32x4*>(&sm.em[par][c4]) = e;
+        *reinterpret_cast<f32x4*>(&sm.pl[par ^ 1][c4]) = m;
+      }
+      if (top > 0.5f * KRANGE * LOG2E) sm.cut[par] = 1;  // benign race: every writer stores 1
+    };
+    // The windows of a cut tile (rare): G to LDS, then per window its end, factors, and Qt and Kt from memory again.
+    auto windows = [&](int n) {
+      const int par = n & 1, pos = p0 + n * SEG, len = min(SEG, S - pos);
+      TL& T = sm.t[par];
+      float* Gs = reinterpret_cast<float*>(sm.t[par ^ 1].Qt);
+      int pt = threadIdx.x & 255;                        // formed here: nothing of this path is held by the others
+      asm volatile("" : "+v"(pt));
+      const int r0 = 8 * (pt >> 5), c4 = 4 * (pt & 31);
+      for (int a = 0; a < len;) {
+        if (pt == 0) sm.wend = len;
+        if (a == 0 && pt < DK) {
+          float run = 0.f;
+          for (int t = 0; t < len; ++t) {
+            if (has_g) run += gg[(int64_t)(pos + t) * DK + pt];
+            Gs[t * DK + pt] = run;
+          }
+        }
+        lds_barrier();                                   // W1
+        // longest window from a whose per-channel G spread stays within KRANGE (at least one token)
+        if (pt < DK) {
+          float mn = INFINITY, mx = -INFINITY;
+          int bad = len;
+          for (int t = a; t < len; ++t) {
+            const float gv = Gs[t * DK + pt];
+            mn = fminf(mn, gv);
+            mx = fmaxf(mx, gv);
+            if (mx - mn > KRANGE) { bad = t; break; }
+          }
+          atomicMin(&sm.wend, bad);
+        }
+        lds_barrier();                                   // W2
+        const int b = max(sm.wend, a + 1);
+        if (pt < DK) {
+          float mn = INFINITY, mx = -INFINITY;
+          for (int t = a; t < b; ++t) {
+            const float gv = Gs[t * DK + pt];
+            mn = fminf(mn, gv);
+            mx = fmaxf(mx, gv);
+          }
+          const float base = a ? Gs[(a - 1) * DK + pt] : 0.f, end = Gs[(b - 1) * DK + pt];
+          const float m = 0.5f * (mn + mx);
+          sm.mm[pt] = m;
+          sm.em[par][pt] = __expf(m - base + sm.pl[a ? par ^ 1 : par][pt]);
+          sm.pl[par ^ 1][pt] = end - m;
+        }
+        lds_barrier();                                   // W3
+        for (int i = 0; i < 8; ++i) {
+          const int r = r0 + i;
+          bf16x4 qo = {}, ko = {};
+          if (r >= a && r < b) {
+            const int64_t o = (int64_t)(pos + r) * DK + c4;
+            const bf16x4 x1 = *reinterpret_cast<const bf16x4*>(q1g + o), xk = *reinterpret_cast<const bf16x4*>(kg + o);
+            bf16x4 x2 = {};
+            if (has_q2) x2 = *reinterpret_cast<const bf16x4*>(q2g + o);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const float d = Gs[r * DK + c4 + j] - sm.mm[c4 + j];
+              const float qe = has_q2 ? (float)x1[j] - lam * (float)x2[j] : (float)x1[j];
+              qo[j] = (bf16)(qe * __expf(d));
+              ko[j] = (bf16)((float)xk[j] * __expf(-d));
+            }
+          }
+          *reinterpret_cast<bf16x4*>(&T.Qt[r * TL::PK + c4]) = qo;
+          *reinterpret_cast<bf16x4*>(&T.Kt[r * TL::PK + c4]) = ko;
+        }
+        lds_barrier();                                   // W4: the window's operands
+        lds_barrier();                                   // W5: they have been read
+        a = b;
+      }
+    };
+
+    if (pt == 0) sm.cut[0] = sm.cut[1] = 0;
+    if (pt < DK) sm.pl[0][pt] = 0.f;
+    using Any = std::false_type;
+    using Full = std::true_type;
+    load_g(Any{}, 0);
+    load_v(0);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) load_row(Any{}, p0, i);
+    cumsum(Any{}, 0);
+    lds_barrier();
+    for (int n = -1; n < nt; ++n) {
+      // Steps whose tile n + 1 is whole (a tile n + 2 follows) and whose tile n is not cut, in a loop without other
+      // paths: every wait for a row's registers then counts exactly the younger loads.  All loads have landed on entry.
+      if (plain) {
+        wait_vmem();
+        for (; n + 2 < nt && !(n >= 0 && sm.cut[n & 1]); ++n) {
+          scale(Full{}, n + 1);
+          lds_barrier();                                 // X
+          if (n >= 0 && pt == 0) sm.cut[n & 1] = 0;
+          cumsum(Full{}, n + 2);
+          lds_barrier();                                 // Y
+        }
+      }
+      if (n >= 0 && sm.cut[n & 1]) windows(n);
+      if (n + 1 < nt) scale(Any{}, n + 1);
+      lds_barrier();                                     // X: tile n + 1 is ready; tile n's partials and A^T tiles
+      if (n >= 0 && pt == 0) sm.cut[n & 1] = 0;          // read before X; set again for tile n + 2 after Y
+      if (n + 2 < nt) cumsum(Any{}, n + 2);
+      lds_barrier();                                     // Y
+    }
+    return;
+  }
+
+  // -------------------------------------------------------------- multiplying waves
+  const int vt = w & 1, kh = w >> 1;
+  bf16* og = reinterpret_cast<bf16*>(p.o);
+  // state tiles of k-tile 2 kh + i, v-tile vt of this V-half
   f32x16 St[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
@@ -155,249 +379,124 @@ __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
     }
   }
 
-  // tile loads into registers (plain loads: a direct-to-LDS load in flight would make every later LDS
-  // access of the tile wait for it): tokens 4 (tid >> 5) + i, channels 4 (tid & 31) .. of q1, q2, k and g;
-  // v chunk tid -> row tid >> 3, columns v0 + 8 (tid & 7)
-  const int r0 = 4 * (tid >> 5), c4 = 4 * (tid & 31);
-  KdaStage stg;
-  auto load = [&](int pos) {
-    // uniform bases and 32-bit lane offsets, formed here (hoisted, they would hold 40 registers through the loop)
-    int th = tid;
-    asm volatile("" : "+v"(th));
-    const int last = S - 1 - pos;
-    const char* vb = reinterpret_cast<const char*>(vg + (rowbase + pos) * 128 + v0);
-    const int64_t o = (rowbase + pos) * DK;
-    const char *gb = reinterpret_cast<const char*>(p.g + o), *kb = reinterpret_cast<const char*>(kg + o),
-               *q1b = reinterpret_cast<const char*>(q1g + o), *q2b = reinterpret_cast<const char*>(q2g + o);
-    stg.v = *reinterpret_cast<const uint4*>(vb + (uint32_t)(min(th >> 3, last) * 256 + 16 * (th & 7)));
-    uint32_t off[4];
+  Frag<bf16> vf[4];
+  f32x16 o;                                              // token tile tt = kh of the read-out
+  // o^T[v][t] = sum_k (S[k][v] e^{m_k - base_k}) Qt[t][k] over this wave's k-half, and
+  // St[k][v] <- S[k][v] e^{m_k - base_k} + sum_s Kt[s][k] v_s[v], with S = e^{pl} St of the window before
+  auto products = [&](int par) {
+    const TL& T = sm.t[par];
+    if (w) {
+      const int it = w - 1;
+      const int st = (it == 2) ? 1 : 0, ttA = (it == 0) ? 0 : 1;
+      f32x16 acc = zero16();
 #pragma unroll
-    for (int i = 0; i < 4; ++i) off[i] = (uint32_t)(min(4 * (th >> 5) + i, last) * (2 * DK) + 8 * (th & 31));
-    if (has_g) {
+      for (int c = 0; c < DK / 16; ++c)
+        acc = mma(rows8(T.Kt + (32 * st + l32) * TL::PK + 8 * half + 16 * c),
+                  rows8(T.Qt + (32 * ttA + l32) * TL::PK + 8 * half + 16 * c), acc);
+      if (st == ttA) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) stg.g[i] = *reinterpret_cast<const f32x4*>(gb + 2 * off[i]);
+        for (int r = 0; r < 16; ++r)
+          if (acc_row(half, r) > l32) acc[r] = 0.f;
+      }
+      sm.A[it][0][l] = acc_to_frag<bf16>(acc, 0);
+      sm.A[it][1][l] = acc_to_frag<bf16>(acc, 1);
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      stg.k[i] = *reinterpret_cast<const bf16x4*>(kb + off[i]);
-      stg.q1[i] = *reinterpret_cast<const bf16x4*>(q1b + off[i]);
-    }
-    if (has_q2) {
+    for (int c = 0; c < 4; ++c) vf[c] = col_frag_tr(T.V, TL::PV, 32 * vt, 16 * c);
+    f32x16 ot[2];
+    ot[0] = ot[1] = zero16();
 #pragma unroll
-      for (int i = 0; i < 4; ++i) stg.q2[i] = *reinterpret_cast<const bf16x4*>(q2b + off[i]);
+    for (int i = 0; i < 2; ++i) {
+      const int kt = 2 * kh + i;
+      f32x16 sv = St[i];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const f32x4 e4 = *reinterpret_cast<const f32x4*>(&sm.em[par][32 * kt + 8 * q + 4 * half]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sv[4 * q + j] *= e4[j];
+      }
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const Frag<bf16> sa = acc_to_frag<bf16>(sv, c);
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+          ot[tt] = mma(sa, kset8(T.Qt + (32 * tt + l32) * TL::PK + 4 * half + 32 * kt + 16 * c), ot[tt]);
+      }
+#pragma unroll
+      for (int c = 0; c < 4; ++c) sv = mma(col_frag_tr(T.Kt, TL::PK, 32 * kt, 16 * c), vf[c], sv);
+      St[i] = sv;
+    }
+    if (kh == 0) {
+      park_acc(sm.red[vt][1], ot[1], l);
+      o = ot[0];
+    } else {
+      park_acc(sm.red[vt][0], ot[0], l);
+      o = ot[1];
     }
   };
-  if (tid == 0) sm.cut[0] = sm.cut[1] = 0;
-  if (tid < DK) sm.pl[0][tid] = 0.f;
-  load(p0);
-
-  f32x4 G[4], low;                                       // sums of g over this thread's tokens, before them
-  // Qt = q_e e^{G - m}, Kt = k e^{m - G} on rows [a, b), zero elsewhere (FULL: every row, two queries); the largest |G - m|
-  // in units of ln 2
-  auto scale = [&](auto FULLc, const f32x4& m, int a, int b) {
-    constexpr bool FULL = decltype(FULLc)::value;
-    const f32x4 c = (low - m) * LOG2E;
-    float top = 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = r0 + i;
-      bf16x4 qo, ko;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float d = __builtin_fmaf(G[i][j], LOG2E, c[j]);
-        const float qe = FULL || has_q2 ? __builtin_fmaf(-lam, (float)stg.q2[i][j], (float)stg.q1[i][j]) : (float)stg.q1[i][j];
-        top = fmaxf(top, fabsf(d));
-        qo[j] = (bf16)(qe * __builtin_amdgcn_exp2f(d));
-        ko[j] = (bf16)((float)stg.k[i][j] * __builtin_amdgcn_exp2f(-d));
-      }
-      uint2 qw = __builtin_bit_cast(uint2, qo), kw = __builtin_bit_cast(uint2, ko);
-      if (!FULL && !(r >= a && r < b)) qw = kw = uint2{0, 0};
-      *reinterpret_cast<uint2*>(&sm.Qt[r * SM::PK + c4]) = qw;
-      *reinterpret_cast<uint2*>(&sm.Kt[r * SM::PK + c4]) = kw;
+  // intra-window term and the other k-half's partial, then output rows [a, b) of tile pos, staged for 16-byte stores
+  auto output = [&](int pos, int a, int b) {
+    if (kh == 0) {
+      o = mma(vf[0], sm.A[0][0][l], o);
+      o = mma(vf[1], sm.A[0][1][l], o);
+    } else {
+      o = mma(vf[0], sm.A[1][0][l], o);
+      o = mma(vf[1], sm.A[1][1][l], o);
+      o = mma(vf[2], sm.A[2][0][l], o);
+      o = mma(vf[3], sm.A[2][1][l], o);
     }
-    return top;
+    const f32x16 other = unpark_acc(sm.red[vt][kh], l);
+    bf16* ob = sm.O[w];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int c0 = 8 * q + 4 * half;                   // 4 consecutive v columns inside one 16-byte chunk
+      bf16x4 yv;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) yv[j] = (bf16)(o[4 * q + j] + other[4 * q + j]);
+      *reinterpret_cast<bf16x4*>(ob + XO::chunk(l32, c0 >> 3) + (c0 & 7)) = yv;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int e = l + 64 * i;
+      const int r = e >> 2, c = e & 3;                   // row t of the block, 16-byte chunk
+      const uint4 val = *reinterpret_cast<const uint4*>(ob + XO::chunk(r, c));
+      const int t = 32 * kh + r;
+      if (t >= a && t < b)
+        *reinterpret_cast<uint4*>(og + (rowbase + pos + t) * 128 + v0 + 32 * vt + 8 * c) = val;
+    }
   };
-  // The whole tile as one window: base 0, end - m = m; every factor within e^{+-KRANGE / 2}, or the tile is cut.
-  auto stage = [&](auto FULLc, int len, int par) {
-    constexpr bool FULL = decltype(FULLc)::value;
-    *reinterpret_cast<uint4*>(&sm.V[(tid >> 3) * SM::PV + 8 * (tid & 7)]) = stg.v;
-    // the in-tile inclusive cumsum of g, g = 0 past the end (G stays flat)
-    f32x4 run = {0.f, 0.f, 0.f, 0.f}, both;              // both: the wave's eight tokens
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (FULL || (has_g && r0 + i < len)) run += stg.g[i];
-      G[i] = run;
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float first = from_half(run[j], 0);          // every lane active: the swap reads both halves
-      low[j] = half ? first : 0.f;
-      both[j] = sum_halves(run[j]);
-    }
-    if (half == 0) *reinterpret_cast<f32x4*>(&sm.wtot[w][c4]) = both;
-    lds_barrier();                                       // B1: the waves' sums
-    f32x4 end = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int j = 0; j < KW; ++j) {
-      if (j && j == w) {
-        low += end;
-        asm volatile("" : "+v"(low));                    // a scalar branch, not four selects
-      }
-      end += *reinterpret_cast<const f32x4*>(&sm.wtot[j][c4]);
-    }
-    const f32x4 m = 0.5f * end;
-    const float top = scale(FULLc, m, 0, len);
-    if (w == 0 && half == 0) {
-      const f32x4 pv = *reinterpret_cast<const f32x4*>(&sm.pl[par][c4]);
-      f32x4 e;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) e[j] = __expf(m[j] + pv[j]);
-      *reinterpret_cast<f32x4*>(&sm.em[c4]) = e;
-      *reinterpret_cast<f32x4*>(&sm.pl[par ^ 1][c4]) = m;
-    }
-    if (tid == 0) sm.cut[par ^ 1] = 0;                   // read a tile ago, set after the next tile's B1
-    if (top > 0.5f * KRANGE * LOG2E) sm.cut[par] = 1;    // benign race: every writer stores 1
-  };
-  const bool plain = has_g && has_q2;
-  int par = 0;
-  for (int pos = p0; pos < p1; pos += SEG, par ^= 1) {
-    const int len = min(SEG, S - pos);
-    wait_vmem();                                         // this tile's registers
-    if (plain && len == SEG) stage(std::true_type{}, len, par);
-    else stage(std::false_type{}, len, par);
-    lds_barrier();                                       // B2: Qt, Kt, V, window factors, cut flag
-    const bool cut = sm.cut[par] != 0;
 
-    // ---- factorisation windows [a, b) of this tile
-    for (int a = 0; a < len;) {
-      int b = len;
-      if (cut) {
-        // longest window from a whose per-channel G spread stays within KRANGE (at least one token)
-        if (a == 0) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) *reinterpret_cast<f32x4*>(&sm.G[r0 + i][c4]) = G[i] + low;
-        }
-        if (tid == 0) sm.wend = len;
-        lds_barrier();
-        if (tid < DK) {
-          float mn = INFINITY, mx = -INFINITY;
-          int bad = len;
-          for (int t = a; t < len; ++t) {
-            const float gv = sm.G[t][tid];
-            mn = fminf(mn, gv);
-            mx = fmaxf(mx, gv);
-            if (mx - mn > KRANGE) { bad = t; break; }
-          }
-          atomicMin(&sm.wend, bad);
-        }
-        lds_barrier();
-        b = max(sm.wend, a + 1);
-        if (tid < DK) {
-          float mn = INFINITY, mx = -INFINITY;
-          for (int t = a; t < b; ++t) {
-            const float gv = sm.G[t][tid];
-            mn = fminf(mn, gv);
-            mx = fmaxf(mx, gv);
-          }
-          const float base = a ? sm.G[a - 1][tid] : 0.f, end = sm.G[b - 1][tid];
-          const float m = 0.5f * (mn + mx);
-          sm.mm[tid] = m;
-          sm.em[tid] = __expf(m - base + sm.pl[a ? par ^ 1 : par][tid]);
-          sm.pl[par ^ 1][tid] = end - m;
-        }
-        lds_barrier();
-        scale(std::false_type{}, *reinterpret_cast<const f32x4*>(&sm.mm[c4]), a, b);
-        lds_barrier();
+  lds_barrier();
+  for (int n = -1; n < nt; ++n) {
+    const int pos = p0 + n * SEG, len = min(SEG, S - pos);
+    const bool cut = n >= 0 && sm.cut[n & 1] != 0, whole = n >= 0 && !cut;
+    if (cut) {
+      for (int a = 0; a < len;) {
+        lds_barrier();                                   // W1
+        lds_barrier();                                   // W2
+        const int b = max(sm.wend, a + 1);
+        lds_barrier();                                   // W3
+        lds_barrier();                                   // W4
+        products(n & 1);
+        lds_barrier();                                   // W5
+        output(pos, a, b);
+        a = b;
       }
-      if (b == len && pos + SEG < p1) load(pos + SEG);   // the next tile streams in behind this one's products
-
-      // ---- phase 1: A^T tiles (waves 5..7), read-out partials, state update
-      if (w >= 5) {
-        const int it = w - 5;
-        const int st = (it == 2) ? 1 : 0, ttA = (it == 0) ? 0 : 1;
-        f32x16 acc = zero16();
-#pragma unroll
-        for (int c = 0; c < DK / 16; ++c)
-          acc = mma(rows8(sm.Kt + (32 * st + l32) * SM::PK + 8 * half + 16 * c),
-                    rows8(sm.Qt + (32 * ttA + l32) * SM::PK + 8 * half + 16 * c), acc);
-        if (st == ttA) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            if (acc_row(half, r) > l32) acc[r] = 0.f;
-        }
-        sm.A[it][0][l] = acc_to_frag<bf16>(acc, 0);
-        sm.A[it][1][l] = acc_to_frag<bf16>(acc, 1);
-      }
-      // o^T[v][t] = sum_k (S[k][v] e^{m_k - base_k}) Qt[t][k] over this wave's k-half, t-tile tt, and
-      // St[k][v] <- S[k][v] e^{m_k - base_k} + sum_s Kt[s][k] v_s[v], with S = e^{pl} St of the window before
-      Frag<bf16> vf[4];
-#pragma unroll
-      for (int c = 0; c < 4; ++c) vf[c] = col_frag_tr(sm.V, SM::PV, 32 * vt, 16 * c);
-      f32x16 o = zero16();
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int kt = 2 * kh + i;
-        f32x16 sv = St[i];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const f32x4 e4 = *reinterpret_cast<const f32x4*>(&sm.em[32 * kt + 8 * q + 4 * half]);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) sv[4 * q + j] *= e4[j];
-        }
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-          o = mma(acc_to_frag<bf16>(sv, c), kset8(sm.Qt + (32 * tt + l32) * SM::PK + 4 * half + 32 * kt + 16 * c), o);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) sv = mma(col_frag_tr(sm.Kt, SM::PK, 32 * kt, 16 * c), vf[c], sv);
-        St[i] = sv;
-      }
-      if (kh) park_acc(sm.red[vt][tt], o, l);
-      lds_barrier();                                     // B3: A^T tiles and partials; Qt, Kt and V have been read
-
-      // ---- phase 2 (the kh = 0 waves; the others go on to the next tile): intra-window term, then output rows
-      // [a, b) of block (vt, tt), staged for 16-byte stores
-      if (kh == 0) {
-        if (tt == 0) {
-          o = mma(vf[0], sm.A[0][0][l], o);
-          o = mma(vf[1], sm.A[0][1][l], o);
-        } else {
-          o = mma(vf[0], sm.A[1][0][l], o);
-          o = mma(vf[1], sm.A[1][1][l], o);
-          o = mma(vf[2], sm.A[2][0][l], o);
-          o = mma(vf[3], sm.A[2][1][l], o);
-        }
-        const f32x16 other = unpark_acc(sm.red[vt][tt], l);
-        bf16* ob = sm.O[2 * vt + tt];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int c0 = 8 * q + 4 * half;              // 4 consecutive v columns inside one 16-byte chunk
-          bf16x4 yv;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) yv[j] = (bf16)(o[4 * q + j] + other[4 * q + j]);
-          *reinterpret_cast<bf16x4*>(ob + XO::chunk(l32, c0 >> 3) + (c0 & 7)) = yv;
-        }
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const int e = l + 64 * i;
-          const int r = e >> 2, c = e & 3;               // row t of the block, 16-byte chunk
-          const uint4 val = *reinterpret_cast<const uint4*>(ob + XO::chunk(r, c));
-          const int t = 32 * tt + r;
-          if (t >= a && t < b)
-            *reinterpret_cast<uint4*>(og + (rowbase + pos + t) * 128 + v0 + 32 * vt + 8 * c) = val;
-        }
-      }
-      a = b;
     }
+    if (whole) products(n & 1);
+    lds_barrier();                                       // X
+    if (whole) output(pos, 0, len);
+    lds_barrier();                                       // Y
   }
 
-  if (p.final_state && tt == 0 && p1 == S) {
+  if (p.final_state && p1 == S) {
     float* sf_out = p.final_state + (int64_t)bh * DK * 128;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int kr = 32 * (2 * kh + i) + acc_row(half, r);
-        sf_out[kr * 128 + v0 + 32 * vt + l32] = St[i][r] * __expf(sm.pl[par][kr]);
+        sf_out[kr * 128 + v0 + 32 * vt + l32] = St[i][r] * __expf(sm.pl[nt & 1][kr]);
       }
   }
 }
