@@ -979,7 +979,7 @@ void kda_bwd_workspace_layout(KdaBwdParams& q, void* workspace) {
   q.f.nseg = 1;
   q.f.seg_chunks = nch;
   if (nch > 0 && !kda_precise_path(q.f))
-    kda_split((int64_t)nbh * q.nq, nch, min(16, 2 * q.nseg), q.f.nseg, q.f.seg_chunks);
+    kda_split((int64_t)nbh * q.nq, nch, min(16, 2 * q.nseg), KDA_COST_REF, q.f.nseg, q.f.seg_chunks);
   if (q.f.nseg > 1) {
     q.lam_part = q.segsum;
     q.f.seg_sum = q.segsum + ((size_t)(q.nq + 1) * q.f.nseg * nbh + 3) / 4 * 4;

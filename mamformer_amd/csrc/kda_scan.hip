@@ -1077,12 +1077,14 @@ __global__ __launch_bounds__(512) void kda_sum_kernel(KdaParams p) {
 
 }  // namespace
 
-void kda_split(int64_t units, int nch, int most, int& nseg, int& seg_chunks) {
-  // In chunk times of the walk (about 5 us), fitted to both scans at 16 to 192 workgroups and 200 to 8192 tokens: a
-  // round of 256 workgroups takes its segments' chunks plus two (the first loads, the entering sums, the drain); the
-  // sums, two workgroups per CU, a third of that; the second launch one.  B1 H16 S1500 (reference mode): 8 segments
-  // 29 us, unsplit 114; B1 H16 S200: 4 segments 13.5, unsplit 21.9; B2 H32 S4096: 4 segments 212, unsplit 324;
-  // B2 H48 S2048, unsplit by this rule: 157, 8 segments 184.
+void kda_split(int64_t units, int nch, int most, KdaSplitCost cost, int& nseg, int& seg_chunks) {
+  // In chunk times of the walk (reference mode about 5 us, gated 2.6), fitted at 16 to 192 workgroups and 200 to 8192
+  // tokens: a round of 256 workgroups takes its segments' chunks plus two (the first loads, the entering sums, the
+  // drain); the sums, two workgroups per CU, `sums` of that, or `alone` with one; the second launch `launch`.  Reference mode: B1 H16 S1500
+  // 8 segments 29 us, unsplit 114; B1 H16 S200 4 segments 13.5, unsplit 21.9; B2 H32 S4096 4 segments 212, unsplit
+  // 324; B2 H48 S2048, unsplit by this rule: 157, 8 segments 184.  Gated: B1 H8 S8192 16 segments 56, unsplit 283;
+  // B1 H16 S300 5 segments 15.1, unsplit 17.1; by this rule unsplit: B4 H24 S8192 333, 4 segments 476; B2 H32 S1000
+  // 42.4, 4 segments 49.2.
   float best = 1e30f;
   nseg = 1;
   seg_chunks = nch;
@@ -1090,7 +1092,8 @@ void kda_split(int64_t units, int nch, int most, int& nseg, int& seg_chunks) {
     const int per = (nch + s - 1) / s;
     if ((nch + per - 1) / per != s) continue;            // the same segments as a smaller s
     float t = (float)((units * s + 255) / 256) * (per + 2);
-    if (s > 1) t += 0.35f * (float)((units * (s - 1) + 511) / 512) * (per + 2) + 1.f;
+    const int64_t n = units * (s - 1);
+    if (s > 1) t += (n <= 256 ? cost.alone : cost.sums * (float)((n + 511) / 512)) * (per + 2) + cost.launch;
     if (t < best) {
       best = t;
       nseg = s;
@@ -1105,7 +1108,7 @@ size_t kda_plan_segments(KdaParams& p) {
   p.nseg = 1;
   p.seg_chunks = nch;
   if (nch == 0 || kda_precise_path(p)) return 0;
-  kda_split(2 * nbh, nch, 16, p.nseg, p.seg_chunks);
+  kda_split(2 * nbh, nch, 16, p.mode == 0 ? KDA_COST_GATED : KDA_COST_REF, p.nseg, p.seg_chunks);
   return p.nseg > 1 ? (size_t)(p.nseg - 1) * nbh * KDA_REC * sizeof(float) : 0;
 }
 

@@ -235,7 +235,10 @@ hipError_t launch_kda(const KdaParams& p, hipStream_t st);
 // (0: the scan is not split).
 size_t kda_plan_segments(KdaParams& p);
 // Segment count (at most `most`) and chunks per segment for `units` workgroups (one per CU) that each walk nch chunks.
-void kda_split(int64_t units, int nch, int most, int& nseg, int& seg_chunks);
+// cost: a chunk of the segments' sums (two workgroups on a CU, one alone), and their launch, in chunk times of the walk.
+struct KdaSplitCost { float sums, alone, launch; };
+constexpr KdaSplitCost KDA_COST_REF{0.35f, 0.35f, 1.f}, KDA_COST_GATED{0.8f, 0.49f, 1.5f};
+void kda_split(int64_t units, int nch, int most, KdaSplitCost cost, int& nseg, int& seg_chunks);
 // Sums of phi'(k)^T v, phi'(k), v and K1 v over each of segments 0 .. nseg - 2 (the query gradient's walk), records
 // of KDA_BWD_REC floats per (segment, b, h).
 constexpr int KDA_REC = 128 * 128 + 128;          // a forward segment's record: state sum, then z sum or log-decay
