@@ -20,7 +20,7 @@
 //     ddt_tau = colG_tau + bint_tau + A da_tau,    dA = sum_tau dt_tau da_tau,    dD = sum dy . x.
 //
 // Launches (caller's stream):
-//   0. ssd_bwd_zero      clears dA, dD, d_dt_bias (a kernel, not a memset node).
+//   0. ssd_bwd_zero      an empty sequence's dA, dD, d_dt_bias, and nothing else (a kernel, not a memset node).
 //   1. ssd_bwd_sweep     grid (2 directions, H, b): the forward direction walks the segments
 //      first to last and stores the entering state h_in of every 64-token segment; the adjoint direction walks
 //      them last to first, stores lam_out of every segment and finally dh0
@@ -28,7 +28,7 @@
 //   2. ssd_bwd_grad      grid (nseg, H / HB, b): one workgroup per (segment, block of HB heads of a group),
 //      fully parallel; dx and ddt stored directly, dB / dC summed over the block's heads in registers and
 //      stored as one fp32 partial per head block; dA / dD / dt_bias as per-segment partials.
-//   3. ssd_bwd_reduce    partials -> dB, dC (fixed summation order) in the I/O dtype and the caller's strides.
+//   3. ssd_bwd_reduce    partials -> dB, dC (the I/O dtype, the caller's strides), dA, dD, d_dt_bias, each in a fixed order.
 // Token-contracted products take their transposed operands from the MFMA unit (identity products), as in
 // the forward; all accumulation is fp32.
 #include <type_traits>

@@ -238,9 +238,9 @@ __device__ __forceinline__ void rf_block(int nblk, int nper, int& b, int& cb) {
   cb = j % nper;
 }
 
-// Workgroup index of the channel-major walks (rf_hs_kernel, rf_bwd_state_kernel: (batch, channel block, state
-// group), state group fastest), remapped so that each XCD runs a contiguous range of them: the state groups of a
-// channel block then read its rows of dt, x and dy through one L2 (workgroups are dealt to the 8 XCDs
+// Workgroup index of the channel-major walks (rf_hs_kernel: (batch, channel block, state group), state group
+// fastest), remapped so that each XCD runs a contiguous range of them: the state groups of a channel block then read
+// its rows of dt and x through one L2 (workgroups are dealt to the 8 XCDs
 // round-robin; dealt as they come, each row was fetched by all eight).
 __device__ __forceinline__ int rf_xcd_block() {
   const int i = blockIdx.x, n = gridDim.x;
