@@ -64,43 +64,33 @@ size_t ssd_chunk_workspace(const mh_ssd_args* a, int64_t chunk) {
                                  (int)a->headdim, (int)a->dstate, (int)a->ngroups, a->dtype);
 }
 
-// The state-passing chunk with the shortest time by a model of both kernels: a workgroup takes f + s us per 64-token
-// segment, 256 run at a time, and the states' pass between the kernels d per chunk (bf16: only beyond the look-back's
-// 8 chunks).  f, s and d are fitted to 64 .. 2048-token chunks of 15 sizes from b1 L64 H32 to b3 L2600 H64 and b1 L6000
-// H128; of both dtypes, the model's choice is within 8% of the best measured chunk there, where the one-round chunk was
-// up to 1.7 times slower (bf16 b1 L1000 H32 N128: 192 tokens 24.1 us, 256: 30.9; fp32: 128 tokens 69, 256: 102; fp32
-// b3 L2600 H64 G8: 192 tokens 812, one round of 1984: 1365).  bf16 chunks are no shorter than 192 tokens: a chunk's state
-// is rounded to bf16, and at 128 and 64 the outputs' error against float64 grows by 1 and 4%.  Sizes whose one-round chunk
-// fits the static scratch of the no-allocation entry point keep fitting it.
+// bf16: the chunk of one round.  A chunk's state is rounded to bf16, and beyond the look-back's 8 chunks the state entering
+// it once more, so shorter chunks are faster at small sizes (b1 L1000 H32 N128: 192 tokens 24.1 us, 256: 30.9) but not as
+// exact: at steps near 1e-3 the error of y grew by 4% and that of h by 18% (b1 L2000 H8 N128, 192 tokens against 256).
+// fp32 rounds no state: the chunk with the shortest time by a model of both kernels.  A workgroup takes f + s us per
+// 64-token segment, 256 run at a time, and the states' pass between the kernels d per chunk.  f, s and d are fitted to
+// 64 .. 2048-token chunks of 15 sizes from b1 L64 H32 to b3 L2600 H64 and b1 L6000 H128; the model's choice is within 8%
+// of the best measured chunk there, where the one-round chunk was up to 1.7 times slower (b1 L1000 H32 N128: 128 tokens 69
+// us, 256: 102; b3 L2600 H64 G8: 192 tokens 812, one round of 1984: 1365).  Sizes whose one-round chunk fits the static
+// scratch of the no-allocation entry point keep fitting it.
 int64_t ssd_auto_chunk(const mh_ssd_args* a) {
+  if (a->dtype != MH_F32) return ssd_one_round_chunk(a);
   const int64_t hg = ssd_heads_per_wg(a), nseg = (a->seqlen + 63) / 64;
   const int64_t units = a->batch * (a->nheads / hg);
-  const bool f32 = a->dtype == MH_F32, wide = a->dstate > 64;
-  const double s = f32 ? (wide ? 19.5 : 8.0 + 5.0 * hg) : (wide ? 4.6 : 3.6);
-  const double f = f32 ? 24.0 : (wide ? 14.0 : 12.0), d = f32 ? 0.2 : (wide ? 0.45 : 0.3);
+  const double s = a->dstate > 64 ? 19.5 : 8.0 + 5.0 * hg, f = 24.0, d = 0.2;
   // at most what one round takes, and twice that where partial rounds could be filled better
   const int64_t one = ssd_one_round_chunk(a) / 64;
-  const int64_t lo = f32 ? 1 : 3, hi = std::min<int64_t>(256, std::max<int64_t>(lo, 2 * one));
+  const int64_t hi = std::min<int64_t>(256, 2 * one);
   const bool fits = ssd_chunk_workspace(a, 64 * one) <= MH_NOALLOC_SCRATCH_BYTES;
   auto time_of = [&](int64_t c) {
-    const int64_t full = nseg / c, rem = nseg % c, chunks = full + (rem ? 1 : 0);
-    if (f32) {
-      // two workgroups can share a CU: beyond one round every workgroup takes a slot of a full one
-      const int64_t wgs = units * chunks;
-      const double per = (double)std::min(c, nseg);
-      return (wgs <= 256 ? f + s * per : (double)((wgs + 255) / 256) * (8.0 + 1.18 * s * per) + 16.0) + d * (double)chunks;
-    }
-    const int64_t rounds = (units * full + 255) / 256, left = rounds * 256 - units * full;
-    const double tr = rem ? f + s * (double)rem : 0.0;   // the short last chunk's workgroups, in slots left over or after
-    double t = (double)rounds * (f + s * (double)c);
-    if (full == 1 && rounds == 1) t -= 6.0;              // the first chunk looks back at nothing
-    if (rem && units > left) t += (double)((units - left + 255) / 256) * tr;
-    else t = std::max(t, tr);
-    return chunks > 8 ? t + d * (double)(chunks - 4) : t;
+    // two workgroups can share a CU: beyond one round every workgroup takes a slot of a full one
+    const int64_t chunks = (nseg + c - 1) / c, wgs = units * chunks;
+    const double per = (double)std::min(c, nseg);
+    return (wgs <= 256 ? f + s * per : (double)((wgs + 255) / 256) * (8.0 + 1.18 * s * per) + 16.0) + d * (double)chunks;
   };
-  int64_t pick = std::max(one, lo);
+  int64_t pick = one;
   double best = time_of(pick);
-  for (int64_t c = hi; c >= lo; c -= std::max<int64_t>(1, c / 32)) {
+  for (int64_t c = hi; c >= 1; c -= std::max<int64_t>(1, c / 32)) {
     if (fits && c < one && ssd_chunk_workspace(a, 64 * c) > MH_NOALLOC_SCRATCH_BYTES) break;
     const double t = time_of(c);
     if (t < 0.98 * best) {                               // the longer chunk where it makes little difference
