@@ -145,25 +145,16 @@ class Mamba2Layer(nn.Module):
         if not 1 <= S < K or cs.shape[0] != b or cs.shape[2] != di or cs.stride(2) != 1 \
                 or h0.numel() != b * di * N or not h0.is_contiguous() or u.stride(2) != 1 or u.stride(0) % 8:
             return None
-        mods, par = self._modules, self._parameters
-        dtp = mods["dt_proj"]
-        if type(dtp) is not nn.Sequential or len(dtp._modules) != 2 or not _unhooked(dtp):
+        par = self._step_parameters()
+        if par is None:
             return None
-        lin = [mods["in_proj"], *dtp._modules.values(), mods["B_proj"], mods["C_proj"], mods["out_proj"]]
-        w = []
-        for m in lin:
-            if type(m) is not nn.Linear or not _unhooked(m):
-                return None
-            w += (m._parameters["weight"], m._parameters["bias"])
-        cw, cb = par["conv_weight"], self.conv_bias
-        f32 = (par["A_log"], par["dt_bias"], par["D"])
-        if any(t is not None and type(t) is not nn.Parameter for t in (*w, cw, cb, *f32)):
-            return None
-        r = w[2].shape[0]
+        weights, biases, cb, cw, *f32 = par
+        r = weights[1].shape[0]
         G = self.ngroups
-        if [t.shape for t in w[::2]] != [(2 * di, D), (r, di), (self.nheads, r), (G * N, di), (G * N, di), (D, di)] \
+        if [t.shape for t in weights] != [(2 * di, D), (r, di), (self.nheads, r), (G * N, di), (G * N, di), (D, di)] \
                 or cw.shape != (di, 1, K) or any(t.shape != (self.nheads,) for t in f32):
             return None
+        w = [t for pair in zip(weights, biases) for t in pair]
         bf16, dev = torch.bfloat16, u.device
         track = torch.is_grad_enabled()
         for t in (u, h0, cs, *w, cw, cb, *f32):
@@ -184,6 +175,32 @@ class Mamba2Layer(nn.Module):
             *p[16:19], p[19], S, cs.stride(0), cs.stride(1), p[1], state.data_ptr(), conv.data_ptr(), out.data_ptr(),
             device=dev)
         return out, {"conv_state": conv, "ssm_state": state}
+
+    def _step_parameters(self):
+        """The parameters that ``mh_mamba2_layer_step`` reads -- weights and biases of the six projections, conv_bias,
+        conv_weight, A_log, dt_bias, D -- or None where one is not a plain ``nn.Parameter`` in its place (parametrised,
+        deleted, a buffer or tensor instead) or a projection is not a plain, unhooked ``nn.Linear``: what reading the
+        attribute or calling the module gives is then for the general path to find out."""
+        mods, par = self._modules, self._parameters
+        dtp = mods.get("dt_proj")
+        if type(dtp) is not nn.Sequential or len(dtp._modules) != 2 or not _unhooked(dtp):
+            return None
+        weights, biases = [], []
+        for m in (mods.get("in_proj"), *dtp._modules.values(), mods.get("B_proj"), mods.get("C_proj"),
+                  mods.get("out_proj")):
+            if type(m) is not nn.Linear or not _unhooked(m) or "bias" not in m._parameters:
+                return None
+            weights.append(m._parameters.get("weight"))
+            biases.append(m._parameters["bias"])
+        own = [par.get("conv_weight"), par.get("A_log"), par.get("dt_bias"), par.get("D")]
+        cb = self.conv_bias
+        for t in (*weights, *own):
+            if type(t) is not nn.Parameter:
+                return None
+        for t in (*biases, cb):
+            if t is not None and type(t) is not nn.Parameter:
+                return None
+        return weights, biases, cb, *own
 
 
 def _plain_calls():
