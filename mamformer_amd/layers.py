@@ -152,9 +152,14 @@ class Mamba2Layer(nn.Module):
         r = weights[1].shape[0]
         G = self.ngroups
         if [t.shape for t in weights] != [(2 * di, D), (r, di), (self.nheads, r), (G * N, di), (G * N, di), (D, di)] \
-                or cw.shape != (di, 1, K) or any(t.shape != (self.nheads,) for t in f32):
+                or cw.shape != (di, 1, K) or cb is not None and cb.shape != (di,) \
+                or any(t.shape != (self.nheads,) for t in f32):
             return None
-        w = [t for pair in zip(weights, biases) for t in pair]
+        w = []
+        for t, bias in zip(weights, biases):
+            if bias is not None and bias.shape != t.shape[:1]:
+                return None
+            w += (t, bias)
         bf16, dev = torch.bfloat16, u.device
         track = torch.is_grad_enabled()
         for t in (u, h0, cs, *w, cw, cb, *f32):

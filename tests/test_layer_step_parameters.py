@@ -70,3 +70,19 @@ def test_step_of_replaced_parameters(name, how):
         want, wnew = plain(u, use_cache=True, cache=cache)
     assert torch.equal(out, want)
     assert all(torch.equal(new[k], wnew[k]) for k in wnew)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["in_proj", "dt_proj.1", "C_proj", "out_proj"])
+def test_a_bias_of_another_size_is_left_to_the_general_path(name):
+    lay = Mamba2Layer(64, bias=True, device="cuda", dtype=BF)
+    u = torch.randn(2, 1, 64, device="cuda").to(BF)
+    cache = {"conv_state": torch.randn(2, 3, 64, device="cuda").to(BF), "ssm_state": torch.randn(2, 64, 128, device="cuda")}
+    lin = lay.get_submodule(name)
+    with torch.no_grad():
+        one = torch.full((1,), 0.5, device="cuda", dtype=BF)
+        lin.bias.copy_(one.expand_as(lin.bias))
+        want = lay(u, use_cache=True, cache=cache, return_h_states=True)[0]      # (the general path)
+        lin.bias = nn.Parameter(one)                       # broadcast there; the kernel reads a value per row
+        out = lay(u, use_cache=True, cache=cache)[0]
+    assert (out.float() - want.float()).norm() <= 1e-2 * want.float().norm()
