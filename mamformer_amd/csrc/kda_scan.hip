@@ -238,6 +238,9 @@ __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
         for (int j = 0; j < 4; ++j) e[j] = __expf(m[j] + pv[j]);
         *reinterpret_cast<f32x4*>(&sm.em[par][c4]) = e;
         *reinterpret_cast<f32x4*>(&sm.pl[par ^ 1][c4]) = m;
+        // A channel whose sum is not finite has no midpoint (and fmaxf drops a NaN): 0 m is then a NaN and the tile is
+        // cut, so that the windows before the first such token are as they would be without it.
+        if (0.f * (m[0] + m[1] + m[2] + m[3]) != 0.f) sm.cut[par] = 1;
       }
       if (top > 0.5f * KRANGE * LOG2E) sm.cut[par] = 1;  // benign race: every writer stores 1
     };
