@@ -30,7 +30,7 @@ constexpr int SEGK = 64;          // tokens per segment (max)
 constexpr int DK = 128;
 constexpr int DVH = 64;           // v columns per workgroup
 constexpr float LOG2E = 1.44269504088896340736f;
-constexpr float KRANGE = 50.f;    // max spread of G per channel within a segment
+constexpr float KRANGE = 80.f;    // max spread of G per channel within a segment
 
 // ----------------------------------------------------------------- gated mode
 // One workgroup of 8 waves per (b, h, V-half) walks the sequence in 64-token
@@ -40,19 +40,20 @@ constexpr float KRANGE = 50.f;    // max spread of G per channel within a segmen
 // k-half kh = w >> 1, keeps the state tiles S[kh][vt], forms the read-out of tile
 // n over its k-half and the state update; waves 1..3 also form the three masked
 // A^T tiles.  The k-halves' partials are exchanged through LDS and wave (vt, kh)
-// finishes token tile tt = kh.  A tile is one factorisation window unless the
-// spread of G within it exceeds KRANGE for some channel; it is then cut into
-// shorter windows, which both roles walk together.
+// finishes token tile tt = kh.  A tile is one factorisation window, with m the
+// midpoint of five of its G (its first token's and those at the end of each 16
+// tokens: the range's own for gates of one sign), unless some G lies further than
+// KRANGE / 2 from m; it is then cut into shorter windows, which both roles walk
+// together.
 //
 // One workgroup per CU (the grid is 2 B H), so what a tile costs is its chain of
 // barriers and LDS round trips, and with every wave in the same phase the
 // exponentials and conversions (VALU) never ran beside the products (MFMA, LDS):
 // 4.5 us a tile in that form.  Here one wave of each role shares each SIMD and a
 // step has two barriers: scaling of tile n + 1 beside the products of tile n,
-// then the cumsum of tile n + 2 beside the output of tile n.  With base = 0 and
-// m = end / 2 both window factors are e^m; the factor between two windows'
-// states is applied once, where the read-out needs it; the token-contracted
-// operands are read transposed by the LDS.
+// then the cumsum of tile n + 2 beside the output of tile n.  The factor between
+// two windows' states is applied once, where the read-out needs it; the
+// token-contracted operands are read transposed by the LDS.
 constexpr int KW = 8;                 // waves per workgroup
 
 struct KdaGatedTile {
@@ -67,7 +68,8 @@ struct KdaGatedSmem {
   AccPark red[2][2];                  // read-out partials for the wave of the other k-half: vt, tt
   bf16 O[4][32 * 32];                 // o blocks staged for coalesced stores (XHalf rows 0..31)
   alignas(16) float wtot[4][DK];      // sums of g over each preparing wave's 16 tokens
-  alignas(16) float mm[DK];           // window midpoint m (tiles that are cut)
+  alignas(16) float g1[DK];           // g of the tile's first token
+  alignas(16) float mm[4][DK];        // window midpoint m (tiles that are cut), a copy per preparing wave
   alignas(16) float em[2][DK];        // by the tile's parity: e^{m - base + pl}
   alignas(16) float pl[2][DK];        // by the tile's parity: end - m of the window before the tile
   int wend, cut[2];                   // cut: by the tile's parity
@@ -121,8 +123,9 @@ __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
   const int p0 = SPLIT ? seg * p.seg_chunks * SEG : 0, p1 = SPLIT ? min(S, p0 + p.seg_chunks * SEG) : S;
   const int nt = (p1 - p0 + SEG - 1) / SEG;
   const int v0 = vh * DVH;
-  // Both roles run the same barriers: one after the first cumsum, then per step n (products of tile n) any of a cut
-  // tile's windows and two.
+  auto is_cut = [&](int n) { return __builtin_amdgcn_readfirstlane(sm.cut[n & 1]) != 0; };
+  // Both roles run the same barriers: one after the first cumsum, then per step n (products of tile n) two for each
+  // window of a cut tile but the last, one for that, and two.
 
   if (w >= 4) {
     // ------------------------------------------------------------ preparing waves
@@ -130,6 +133,8 @@ __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
     const float lam = p.lam_h ? p.lam_h[h] : p.lam;
     const int pt = threadIdx.x & 255, pw = w - 4;
     const int r0 = 8 * (pt >> 5), c4 = 4 * (pt & 31);   // tokens r0 .., channels c4 ..
+    int to = r0 * TL::PK + c4;                           // its place in an operand tile; laundered, so that the rows lie
+    asm volatile("" : "+v"(to));                         // at immediate offsets and no address a row is held
     const bf16* q1g = reinterpret_cast<const bf16*>(p.q1) + rowbase * DK;
     const bf16* q2g = reinterpret_cast<const bf16*>(p.q2) + rowbase * DK;
     const bf16* kg = reinterpret_cast<const bf16*>(p.k) + rowbase * DK;
@@ -188,11 +193,17 @@ __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
         low[j] = half ? first : 0.f;
         both[j] = sum_halves(run[j]);
       }
-      if (half == 0) *reinterpret_cast<f32x4*>(&sm.wtot[pw][c4]) = both;
+      if (half == 0) {
+        *reinterpret_cast<f32x4*>(&sm.wtot[pw][c4]) = both;
+        if (pw == 0) *reinterpret_cast<f32x4*>(&sm.g1[c4]) = G[0];
+      }
       load_g(FULLc, n + 1);
     };
-    // Qt = q_e e^{G - m}, Kt = k e^{m - G}, zero rows past the end, of tile n as one window: base 0, end - m = m.  Every
-    // factor is then within e^{+-KRANGE / 2}, or the tile is cut.  Each row's registers take the next tile's row.
+    // Qt = q_e e^{G - m}, Kt = k e^{m - G}, zero rows past the end, of tile n as one window from base 0.  Every factor is
+    // then within e^{+-KRANGE / 2}, or the tile is cut.  m is a midpoint of sampled G and not half of end, for gates that
+    // rise and fall within a tile and for drops in its first token, which half of end would cut (b4 H32 S8192 with such
+    // gates 1113 us, 404 whole), and for a NaN, which minima and maxima drop: the tokens before it stay as they are.  The
+    // samples cost 0.8% of the kernel's time.  Each row's registers take the next tile's row.
     auto scale = [&](auto FULLc, int n) {
       constexpr bool FULL = decltype(FULLc)::value;
       const int par = n & 1, len = min(SEG, S - (p0 + n * SEG)), next = base_of(n + 1);
@@ -200,7 +211,7 @@ __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
 #pragma unroll
       for (int i = 0; i < 2; ++i)
         *reinterpret_cast<uint4*>(&T.V[((pt >> 3) + 32 * i) * TL::PV + 8 * (pt & 7)]) = stg.v[i];
-      f32x4 end = {0.f, 0.f, 0.f, 0.f};
+      f32x4 end = {0.f, 0.f, 0.f, 0.f}, mn = *reinterpret_cast<const f32x4*>(&sm.g1[c4]), mx = mn;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         if (j && j == pw) {
@@ -208,8 +219,13 @@ __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
           asm volatile("" : "+v"(low));                  // a scalar branch, not four selects
         }
         end += *reinterpret_cast<const f32x4*>(&sm.wtot[j][c4]);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          mn[k] = fminf(mn[k], end[k]);
+          mx[k] = fmaxf(mx[k], end[k]);
+        }
       }
-      const f32x4 m = 0.5f * end, c = (low - m) * LOG2E;
+      const f32x4 m = 0.5f * (mn + mx), c = (low - m) * LOG2E;
       float top = 0.f;                                   // the largest |G - m|, in units of ln 2
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
@@ -225,8 +241,8 @@ __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
         }
         uint2 qw = __builtin_bit_cast(uint2, qo), kw = __builtin_bit_cast(uint2, ko);
         if (!FULL && r0 + i >= len) qw = kw = uint2{0, 0};
-        *reinterpret_cast<uint2*>(&T.Qt[(r0 + i) * TL::PK + c4]) = qw;
-        *reinterpret_cast<uint2*>(&T.Kt[(r0 + i) * TL::PK + c4]) = kw;
+        *reinterpret_cast<uint2*>(T.Qt + to + i * TL::PK) = qw;
+        *reinterpret_cast<uint2*>(T.Kt + to + i * TL::PK) = kw;
         load_row(FULLc, next, i);
         __builtin_amdgcn_sched_barrier(0);               // a row at a time: interleaved, the rows spill
       }
@@ -237,81 +253,140 @@ __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) e[j] = __expf(m[j] + pv[j]);
         *reinterpret_cast<f32x4*>(&sm.em[par][c4]) = e;
-        *reinterpret_cast<f32x4*>(&sm.pl[par ^ 1][c4]) = m;
-        // A channel whose sum is not finite has no midpoint (and fmaxf drops a NaN): 0 m is then a NaN and the tile is
-        // cut, so that the windows before the first such token are as they would be without it.
-        if (0.f * (m[0] + m[1] + m[2] + m[3]) != 0.f) sm.cut[par] = 1;
+        *reinterpret_cast<f32x4*>(&sm.pl[par ^ 1][c4]) = end - m;
       }
       if (top > 0.5f * KRANGE * LOG2E) sm.cut[par] = 1;  // benign race: every writer stores 1
     };
-    // The windows of a cut tile (rare): G to LDS, then per window its end, factors, and Qt and Kt from memory again.
+    // A tile that is cut, between its X and Y: its G to LDS, in the operands of the tile before it (read by nobody after
+    // X), and its rows again, in the registers that took the next tile's by now.
+    auto park = [&](int n) {
+      float* Gs = reinterpret_cast<float*>(sm.t[(n & 1) ^ 1].Qt);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) *reinterpret_cast<f32x4*>(&Gs[(r0 + i) * DK + c4]) = G[i] + low;
+      int pos = base_of(n);
+      asm volatile("" : "+s"(pos));
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        load_row(std::false_type{}, pos, i);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    // The windows of a cut tile: each the longest from a on whose per-channel spread of G stays within KRANGE (at least
+    // one token).  Every wave finds its end for itself, two channels a lane, while the window before is multiplied, so a
+    // window takes two barriers; the rows wait in registers until the last window is formed, and the next tile's rows
+    // are on their way again behind its products.  With the ends found by two waves between barriers of their own, g
+    // summed from memory and the rows read again for each window, b4 H32 S8192 took 7038 us at a decay of 3.1 a token
+    // (four windows a tile), the kernel without roles 3709, this 1677 (three windows); one drop of 80 in every eighth
+    // tile 896, 908 and 530; 1.1 a token, cut at a spread of 50 and whole at 80, 5312, 2506 and 403.
     auto windows = [&](int n) {
-      const int par = n & 1, pos = p0 + n * SEG, len = min(SEG, S - pos);
+      const int par = n & 1, len = min(SEG, S - (p0 + n * SEG));
       TL& T = sm.t[par];
-      float* Gs = reinterpret_cast<float*>(sm.t[par ^ 1].Qt);
+      const float* Gs = reinterpret_cast<const float*>(sm.t[par ^ 1].Qt);
       int pt = threadIdx.x & 255;                        // formed here: nothing of this path is held by the others
       asm volatile("" : "+v"(pt));
-      const int r0 = 8 * (pt >> 5), c4 = 4 * (pt & 31);
+      const int r0 = 8 * (pt >> 5), c4 = 4 * (pt & 31), c2 = 2 * (pt & 63);
+      int go = r0 * DK + c4;                             // (one address, rows at immediate offsets)
+      asm volatile("" : "+v"(go));
+      const float* gr = Gs + go;
+      typedef float f32x2_t __attribute__((ext_vector_type(2)));
+      auto g2 = [&](int t) { return *reinterpret_cast<const f32x2_t*>(&Gs[t * DK + c2]); };
+      f32x2_t m, e, pv = *reinterpret_cast<const f32x2_t*>(&sm.pl[par][c2]);   // pv: end - m of the window before
+      int b;
+      auto next = [&](int a) {                           // the window from a: b, m, e = e^{m - base + pv}, pv
+        constexpr int U = 8;                             // tokens whose spread is looked at together
+        f32x2_t mn = {INFINITY, INFINITY}, mx = {-INFINITY, -INFINITY}, v[U], nv[U];
+        auto fetch = [&](f32x2_t (&x)[U], int t) {
+#pragma unroll
+          for (int u = 0; u < U; ++u) x[u] = g2(min(t + u, len - 1));
+        };
+        auto widen = [&](f32x2_t& lo, f32x2_t& hi, f32x2_t x) {
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            lo[j] = fminf(lo[j], x[j]);
+            hi[j] = fmaxf(hi[j], x[j]);
+          }
+        };
+        auto over = [&](f32x2_t lo, f32x2_t hi) { return __ballot(fmaxf(hi[0] - lo[0], hi[1] - lo[1]) > KRANGE) != 0; };
+        b = len;
+        fetch(v, a);
+        for (int t = a; t < len; t += U) {
+          fetch(nv, t + U);
+          f32x2_t lo = mn, hi = mx;
+#pragma unroll
+          for (int u = 0; u < U; ++u) widen(lo, hi, v[u]);
+          if (over(lo, hi)) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+              lo = mn;
+              hi = mx;
+              widen(lo, hi, v[u]);
+              if (over(lo, hi)) {
+                b = max(min(t + u, len), a + 1);
+                break;
+              }
+              mn = lo;
+              mx = hi;
+            }
+            break;
+          }
+          mn = lo;
+          mx = hi;
+#pragma unroll
+          for (int u = 0; u < U; ++u) v[u] = nv[u];
+        }
+        const f32x2_t end = g2(b - 1);
+        f32x2_t base = {0.f, 0.f};
+        if (a) base = g2(a - 1);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          m[j] = 0.5f * (mn[j] + mx[j]);
+          e[j] = __expf(m[j] - base[j] + pv[j]);
+          pv[j] = end[j] - m[j];
+        }
+      };
+      next(0);
       for (int a = 0; a < len;) {
-        if (pt == 0) sm.wend = len;
-        if (a == 0 && pt < DK) {
-          float run = 0.f;
-          for (int t = 0; t < len; ++t) {
-            if (has_g) run += gg[(int64_t)(pos + t) * DK + pt];
-            Gs[t * DK + pt] = run;
-          }
+        const int bw = b;
+        *reinterpret_cast<f32x2_t*>(&sm.mm[pw][c2]) = m;  // each wave its own copy, read by it alone
+        if (pw == 0) {
+          *reinterpret_cast<f32x2_t*>(&sm.em[par][c2]) = e;
+          if (pt == 0) sm.wend = bw;
         }
-        lds_barrier();                                   // W1
-        // longest window from a whose per-channel G spread stays within KRANGE (at least one token)
-        if (pt < DK) {
-          float mn = INFINITY, mx = -INFINITY;
-          int bad = len;
-          for (int t = a; t < len; ++t) {
-            const float gv = Gs[t * DK + pt];
-            mn = fminf(mn, gv);
-            mx = fmaxf(mx, gv);
-            if (mx - mn > KRANGE) { bad = t; break; }
-          }
-          atomicMin(&sm.wend, bad);
-        }
-        lds_barrier();                                   // W2
-        const int b = max(sm.wend, a + 1);
-        if (pt < DK) {
-          float mn = INFINITY, mx = -INFINITY;
-          for (int t = a; t < b; ++t) {
-            const float gv = Gs[t * DK + pt];
-            mn = fminf(mn, gv);
-            mx = fmaxf(mx, gv);
-          }
-          const float base = a ? Gs[(a - 1) * DK + pt] : 0.f, end = Gs[(b - 1) * DK + pt];
-          const float m = 0.5f * (mn + mx);
-          sm.mm[pt] = m;
-          sm.em[par][pt] = __expf(m - base + sm.pl[a ? par ^ 1 : par][pt]);
-          sm.pl[par ^ 1][pt] = end - m;
-        }
-        lds_barrier();                                   // W3
+        const f32x4 m4 = *reinterpret_cast<const f32x4*>(&sm.mm[pw][c4]);
+#pragma unroll
         for (int i = 0; i < 8; ++i) {
           const int r = r0 + i;
           bf16x4 qo = {}, ko = {};
-          if (r >= a && r < b) {
-            const int64_t o = (int64_t)(pos + r) * DK + c4;
-            const bf16x4 x1 = *reinterpret_cast<const bf16x4*>(q1g + o), xk = *reinterpret_cast<const bf16x4*>(kg + o);
-            bf16x4 x2 = {};
-            if (has_q2) x2 = *reinterpret_cast<const bf16x4*>(q2g + o);
+          if (r >= a && r < bw) {
+            const f32x4 g4 = *reinterpret_cast<const f32x4*>(gr + i * DK);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-              const float d = Gs[r * DK + c4 + j] - sm.mm[c4 + j];
-              const float qe = has_q2 ? (float)x1[j] - lam * (float)x2[j] : (float)x1[j];
+              const float d = g4[j] - m4[j];
+              const float qe = has_q2 ? (float)stg.q1[i][j] - lam * (float)stg.q2[i][j] : (float)stg.q1[i][j];
               qo[j] = (bf16)(qe * __expf(d));
-              ko[j] = (bf16)((float)xk[j] * __expf(-d));
+              ko[j] = (bf16)((float)stg.k[i][j] * __expf(-d));
             }
           }
-          *reinterpret_cast<bf16x4*>(&T.Qt[r * TL::PK + c4]) = qo;
-          *reinterpret_cast<bf16x4*>(&T.Kt[r * TL::PK + c4]) = ko;
+          *reinterpret_cast<bf16x4*>(T.Qt + to + i * TL::PK) = qo;
+          *reinterpret_cast<bf16x4*>(T.Kt + to + i * TL::PK) = ko;
+          __builtin_amdgcn_sched_barrier(0);
         }
-        lds_barrier();                                   // W4: the window's operands
-        lds_barrier();                                   // W5: they have been read
-        a = b;
+        if (bw == len) {
+          int pos = base_of(n + 1);
+          asm volatile("" : "+s"(pos));                  // addresses formed here, not held through the windows
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            load_row(std::false_type{}, pos, i);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+        if (bw == len && pw == 0) *reinterpret_cast<f32x2_t*>(&sm.pl[par ^ 1][c2]) = pv;
+        lds_barrier();                                   // W1: the window's operands
+        if (bw < len) {
+          next(bw);
+          lds_barrier();                                 // W2: they have been read
+        }
+        a = bw;
       }
     };
 
@@ -326,22 +401,26 @@ __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
     cumsum(Any{}, 0);
     lds_barrier();
     for (int n = -1; n < nt; ++n) {
-      // Steps whose tile n + 1 is whole (a tile n + 2 follows) and whose tile n is not cut, in a loop without other
-      // paths: every wait for a row's registers then counts exactly the younger loads.  All loads have landed on entry.
+      // Steps whose tile n + 1 is whole (a tile n + 2 follows) and whose tile n is not cut, in a loop without other loads
+      // than those of a cut tile's rows, which are as many as they replace: every wait for a row's registers then counts
+      // the younger loads.  All loads have landed on entry.
       if (plain) {
         wait_vmem();
-        for (; n + 2 < nt && !(n >= 0 && sm.cut[n & 1]); ++n) {
+        for (; n + 2 < nt && !(n >= 0 && is_cut(n)); ++n) {
           scale(Full{}, n + 1);
           lds_barrier();                                 // X
+          const int flag = sm.cut[(n + 1) & 1];          // (read ahead of the store: its latency is this step's)
           if (n >= 0 && pt == 0) sm.cut[n & 1] = 0;
+          if (__builtin_expect(__builtin_amdgcn_readfirstlane(flag) != 0, 0)) park(n + 1);
           cumsum(Full{}, n + 2);
           lds_barrier();                                 // Y
         }
       }
-      if (n >= 0 && sm.cut[n & 1]) windows(n);
+      if (n >= 0 && is_cut(n)) windows(n);
       if (n + 1 < nt) scale(Any{}, n + 1);
       lds_barrier();                                     // X: tile n + 1 is ready; tile n's partials and A^T tiles
       if (n >= 0 && pt == 0) sm.cut[n & 1] = 0;          // read before X; set again for tile n + 2 after Y
+      if (n + 1 < nt && is_cut(n + 1)) park(n + 1);
       if (n + 2 < nt) cumsum(Any{}, n + 2);
       lds_barrier();                                     // Y
     }
@@ -472,23 +551,21 @@ __global__ __launch_bounds__(64 * KW) void kda_gated_kernel(KdaParams p) {
   lds_barrier();
   for (int n = -1; n < nt; ++n) {
     const int pos = p0 + n * SEG, len = min(SEG, S - pos);
-    const bool cut = n >= 0 && sm.cut[n & 1] != 0, whole = n >= 0 && !cut;
-    if (cut) {
-      for (int a = 0; a < len;) {
+    int a = 0;                                           // the rows from here on are left for the output below
+    if (n >= 0 && is_cut(n)) {
+      for (;;) {
         lds_barrier();                                   // W1
-        lds_barrier();                                   // W2
-        const int b = max(sm.wend, a + 1);
-        lds_barrier();                                   // W3
-        lds_barrier();                                   // W4
+        const int b = __builtin_amdgcn_readfirstlane(sm.wend);
+        if (b >= len) break;
         products(n & 1);
-        lds_barrier();                                   // W5
+        lds_barrier();                                   // W2
         output(pos, a, b);
         a = b;
       }
     }
-    if (whole) products(n & 1);
+    if (n >= 0) products(n & 1);
     lds_barrier();                                       // X
-    if (whole) output(pos, 0, len);
+    if (n >= 0) output(pos, a, len);
     lds_barrier();                                       // Y
   }
 

@@ -1,8 +1,8 @@
 """Gated scan at the edges of its tiles and factorisation windows, against the float64 recurrence.
 
-A tile is one window where |G - end / 2| stays within 25 on every channel and is cut otherwise, so the gates here sit
-on both sides of that line and change sign: gates of growth as well as decay, a drop in one token of one channel,
-and one tile of several that is cut.  Tolerance: bf16 operands and output, as every bf16 scan (1e-2 of the 2-norm).
+A tile is one window where G stays within 40 of its midpoint on every channel and is cut otherwise.  The gates here
+change sign (growth as well as decay), come near half of that line, and drop in one token of one channel, so that one
+tile of several is cut; test_gpu_kda_gated_cut.py has the line itself.  Tolerance: bf16 operands and output, as every bf16 scan (1e-2 of the 2-norm).
 """
 
 import pytest
@@ -19,7 +19,7 @@ def gate(kind, B, H, S, g):
     n = torch.randn(B, H, S, 128, generator=g)
     if kind == "mild":
         return -0.05 * n.abs()
-    if kind == "near":                       # a full tile's end near -50, the last uncut value
+    if kind == "near":                       # a full tile's end near -50
         return -0.74 - 0.05 * n.abs()
     if kind == "signs":                      # rises and falls within a tile; the end is near 0, the middle is not
         t = torch.arange(S) % 64
