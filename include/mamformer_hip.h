@@ -56,8 +56,8 @@ enum {
   MH_D_PER_CHANNEL = 4,    /* D has nheads*headdim entries instead of nheads */
   MH_A_PER_STATE = 8,      /* decode only: A has dstate entries, one per state column (dA[p, n] = exp(A[n] dt)) */
   MH_DT_PER_CHANNEL = 16,  /* decode only: dt (and dt_bias) have nheads*headdim entries, one per channel */
-  MH_A_LOG = 32            /* mh_ssd_ref_scan_*: A holds log-rates, the rates are -exp(clamp(A, -5, 5)) and the
-                              backward's dA is the gradient of A as given */
+  MH_A_LOG = 32            /* mh_ssd_ref_scan_* only: A holds log-rates, the rates are -exp(clamp(A, -5, 5)) and the
+                              backward's dA is the gradient of A as given (elsewhere MH_ERR_UNSUPPORTED) */
 };
 
 /* ------------------------------------------------------------------------

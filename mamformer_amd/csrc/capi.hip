@@ -126,6 +126,8 @@ int ssd_validate(const mh_ssd_args* a, int64_t* chunk_len_out) {
   if (a->flags & (MH_A_PER_STATE | MH_DT_PER_CHANNEL))
     return fail(MH_ERR_UNSUPPORTED, "ssd: MH_A_PER_STATE / MH_DT_PER_CHANNEL are decode-step flags (the chunked "
                                     "scan factorises a per-head decay)");
+  if (a->flags & MH_A_LOG)
+    return fail(MH_ERR_UNSUPPORTED, "ssd: MH_A_LOG belongs to mh_ssd_ref_scan_* (A holds the rates here)");
   if (!a->A) return fail(MH_ERR_NULL, "ssd: A is required");
   if (a->seqlen > 0 && (!a->x || !a->dt || !a->B || !a->C || !a->y))
     return fail(MH_ERR_NULL, "ssd: x, dt, A, B, C, y are required");
@@ -179,6 +181,8 @@ int ssu_validate(const mh_ssu_args* a) {
                          (long long)a->dstate);
   }
   if ((a->flags & MH_DT_LIMIT) && !(a->dt_min <= a->dt_max)) return fail(MH_ERR_SHAPE, "state_update: dt_min > dt_max");
+  if (a->flags & MH_A_LOG)
+    return fail(MH_ERR_UNSUPPORTED, "state_update: MH_A_LOG belongs to mh_ssd_ref_scan_* (A holds the rates here)");
   if (!a->state_in || !a->state_out || !a->x || !a->dt || !a->A || !a->B || !a->C || !a->y)
     return fail(MH_ERR_NULL, "state_update: state_in, state_out, x, dt, A, B, C, y are required");
   if (!aligned16(a->state_in) || !aligned16(a->state_out))
