@@ -379,7 +379,8 @@ typedef struct {
 int mh_kda_recurrent_step(const mh_kda_step_args* a, void* stream);
 
 /* The same into other buffers: a->state and a->z are read only, the updated state
- * and z go to state_out and z_out (each NULL: not kept; the input itself: in place). */
+ * and z go to state_out and z_out (each NULL: not kept; the input itself: in place; a
+ * buffer that overlaps state, z or the other one: MH_ERR_STRIDE). */
 int mh_kda_recurrent_step_to(const mh_kda_step_args* a, float* state_out, float* z_out, void* stream);
 
 /* ------------------------------------------------------------------------

@@ -29,6 +29,12 @@ int elem_size(int32_t dtype) { return dtype == MH_F32 ? 4 : (dtype == MH_BF16 ? 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 bool stride_ok(int64_t s, int es) { return s >= 0 && ((s * es) % 16) == 0; }
 
+// Whether [p, p + np) and [q, q + nq) (bytes) share any.
+bool overlap(const void* p, size_t np, const void* q, size_t nq) {
+  const uintptr_t a = (uintptr_t)p, b = (uintptr_t)q;
+  return a < b + nq && b < a + np;
+}
+
 int hip_status(hipError_t e, const char* what) {
   if (e == hipSuccess) return MH_OK;
   return fail(MH_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
@@ -755,9 +761,8 @@ int layer_step_validate(const mh_layer_step_args* a) {
       !aligned16(a->out_w) || !aligned16(a->state_in) || !aligned16(a->state_out))
     return fail(MH_ERR_ALIGN, "layer_step: u, the weight matrices and the states must be 16-byte aligned");
   if (a->state_in != a->state_out) {
-    const uintptr_t bytes = (uintptr_t)(a->batch * a->nheads * a->headdim * a->dstate * 4);
-    const uintptr_t i0 = (uintptr_t)a->state_in, o0 = (uintptr_t)a->state_out;
-    if (i0 < o0 + bytes && o0 < i0 + bytes)
+    const size_t bytes = (size_t)(a->batch * a->nheads * a->headdim * a->dstate * 4);
+    if (overlap(a->state_in, bytes, a->state_out, bytes))
       return fail(MH_ERR_STRIDE, "layer_step: state_in and state_out overlap without being identical");
   }
   return MH_OK;
@@ -1240,6 +1245,13 @@ int mh_kda_recurrent_step_to(const mh_kda_step_args* a, float* state_out, float*
   int rc = kda_step_validate(a);
   if (rc) return rc;
   if (state_out && !aligned16(state_out)) return fail(MH_ERR_ALIGN, "kda_step: state_out must be 16-byte aligned");
+  // a workgroup per (batch, head) reads its rows and writes them: in place, or where no other one reads or writes
+  const size_t ns = (size_t)(a->batch * a->nheads * a->dk * a->dv) * 4, nz = (size_t)(a->batch * a->nheads * a->dk) * 4;
+  const bool new_s = state_out && state_out != a->state, new_z = z_out && z_out != a->z;
+  if ((new_s && (overlap(state_out, ns, a->state, ns) || overlap(state_out, ns, a->z, nz))) ||
+      (new_z && (overlap(z_out, nz, a->z, nz) || overlap(z_out, nz, a->state, ns))) ||
+      ((new_s || new_z) && state_out && z_out && overlap(state_out, ns, z_out, nz)))
+    return fail(MH_ERR_STRIDE, "kda_step: state_out and z_out must each be its input or overlap no other buffer");
   mh::KdaStepParams p;
   memset(&p, 0, sizeof(p));
   p.batch = (int)a->batch; p.nheads = (int)a->nheads; p.dk = (int)a->dk; p.dv = (int)a->dv; p.dtype = a->dtype;

@@ -5,7 +5,7 @@ import ctypes as ct
 import pytest
 
 from mamformer_amd import _lib
-from tests.test_abi import _good_bwd, _good_ssd, _good_ssu, _rc
+from tests.test_abi import _good_bwd, _good_ssd, _good_ssu, _good_step, _rc
 
 
 def _ref(a):
@@ -42,3 +42,21 @@ def test_state_update_refuses_log_rates(flags):
     u.flags = flags | _lib.MH_A_LOG
     assert _rc("mh_ssd_state_update", ct.byref(u), None) == -6
     assert b"MH_A_LOG" in _lib.lib().mh_last_error()
+
+
+STATE = 2 * 4 * 128 * 128 * 4                          # bytes of _good_step's state
+Z = 2 * 4 * 128 * 4
+
+
+@pytest.mark.parametrize("state_out,z_out", [
+    ("s+16", None), ("s-16", None), (f"s+{STATE - 16}", None), ("z", None), (f"z-{STATE - 16}", None),
+    (None, "z+4"), (None, f"z-{Z - 4}"), (None, "s"), (None, f"s+{STATE - 4}"), ("s", "s+64"), ("z", "z"),
+    ("n", "n"), ("n", f"n+{STATE - 4}"), ("s", f"z+{Z - 4}"),
+])
+def test_kda_step_refuses_overlapping_outputs(state_out, z_out):
+    a = _good_step()
+    at = {"s": 1 << 24, "z": 1 << 25, "n": 1 << 26}     # state, z, a buffer of its own
+    a.state, a.z = at["s"], at["z"]
+    p = [None if e is None else eval(e, {}, at) for e in (state_out, z_out)]
+    assert _rc("mh_kda_recurrent_step_to", ct.byref(a), *p, None) == -4
+    assert b"overlap" in _lib.lib().mh_last_error()
