@@ -392,7 +392,8 @@ int mh_kda_recurrent_step_to(const mh_kda_step_args* a, float* state_out, float*
  *   conv_w (d_inner, width); A_log, dt_bias, D (nheads,) fp32; conv_state (batch, conv_state_len,
  *   d_inner) bf16 with a contiguous last dimension, conv_state_len <= width - 1;
  *   state_in / state_out (batch, nheads, headdim, dstate) fp32, distinct or identical.
- *   Outputs: out (batch, d_model), conv_out (batch, min(conv_state_len + 1, width - 1), d_inner).
+ *   Outputs: out (batch, d_model), conv_out (batch, min(conv_state_len + 1, width - 1), d_inner), which is
+ *   conv_state itself in the same layout (conv_state_len == width - 1, contiguous) or overlaps it nowhere.
  *   Supported: batch <= 64, d_model and d_inner multiples of 32, 2 <= width <= 8, dstate as
  *   mh_ssd_state_update.
  * ---------------------------------------------------------------------- */

@@ -765,6 +765,15 @@ int layer_step_validate(const mh_layer_step_args* a) {
     if (overlap(a->state_in, bytes, a->state_out, bytes))
       return fail(MH_ERR_STRIDE, "layer_step: state_in and state_out overlap without being identical");
   }
+  if (a->conv_state_len > 0) {
+    // a workgroup reads and writes the cached rows of its own channels: the same buffer in the same layout, or another
+    const int64_t S = a->conv_state_len, di = a->nheads * a->headdim, So = std::min(S + 1, a->width - 1);
+    const bool same = a->conv_out == a->conv_state && So == S && (S == 1 || a->conv_state_stride_l == di) &&
+                      (a->batch == 1 || a->conv_state_stride_b == S * di);
+    const int64_t in = (a->batch - 1) * a->conv_state_stride_b + (S - 1) * a->conv_state_stride_l + di;
+    if (!same && overlap(a->conv_state, (size_t)(2 * in), a->conv_out, (size_t)(2 * a->batch * So * di)))
+      return fail(MH_ERR_STRIDE, "layer_step: conv_out overlaps conv_state in another layout");
+  }
   return MH_OK;
 }
 

@@ -60,3 +60,44 @@ def test_kda_step_refuses_overlapping_outputs(state_out, z_out):
     p = [None if e is None else eval(e, {}, at) for e in (state_out, z_out)]
     assert _rc("mh_kda_recurrent_step_to", ct.byref(a), *p, None) == -4
     assert b"overlap" in _lib.lib().mh_last_error()
+
+
+def _good_layer_step(width=4, rows=3):
+    b, D, H, P, N = 2, 64, 1, 64, 128
+    fake = 4096
+    a = _lib.LayerStepArgs()
+    a.batch, a.d_model, a.nheads, a.headdim, a.dstate, a.ngroups, a.dt_rank, a.width = b, D, H, P, N, 1, 2, width
+    for f in ("u", "in_w", "conv_w", "dt_w0", "dt_w1", "B_w", "C_w", "out_w", "A_log", "dt_bias", "D", "out"):
+        setattr(a, f, fake)
+    a.u_stride_b = D
+    a.state_in, a.state_out = 1 << 20, 1 << 22
+    a.conv_state, a.conv_out = 1 << 23, 1 << 24
+    a.conv_state_len, a.conv_state_stride_l, a.conv_state_stride_b = rows, H * P, rows * H * P
+    return a
+
+
+def _layer_rc(a):
+    return _rc("mh_mamba2_layer_step_workspace_bytes", ct.byref(a), ct.byref(ct.c_size_t()))
+
+
+def test_layer_step_refuses_overlapping_conv_states():
+    a = _good_layer_step()
+    assert _layer_rc(a) == 0
+    a.conv_out = a.conv_state                           # the same rows in the same places
+    assert _layer_rc(a) == 0
+    span = 2 * 3 * 64 * 2
+    for off in (2, -2, span - 2, 2 - span):
+        a.conv_out = a.conv_state + off
+        assert _layer_rc(a) == -4 and b"conv_out" in _lib.lib().mh_last_error(), off
+    for off in (span, -span):
+        a.conv_out = a.conv_state + off
+        assert _layer_rc(a) == 0, off
+    a = _good_layer_step(rows=2)                        # a row more comes out: rows move
+    a.conv_out = a.conv_state
+    assert _layer_rc(a) == -4
+    a = _good_layer_step()                              # x's half of wider rows
+    a.conv_state_stride_l, a.conv_state_stride_b = 128, 3 * 128
+    a.conv_out = a.conv_state
+    assert _layer_rc(a) == -4
+    a.batch, a.conv_state_len, a.width = 1, 1, 2        # one row of one sequence: its strides say nothing
+    assert _layer_rc(a) == 0
