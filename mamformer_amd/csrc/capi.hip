@@ -1118,8 +1118,7 @@ int mh_ssd_ref_scan_bwd(const mh_ssd_ref_bwd_args* a, void* stream) {
   p.dD = a->fwd.D ? a->dD : nullptr;
   p.d_dt_bias = a->fwd.dt_bias ? a->d_dt_bias : nullptr;
   p.dh0 = a->d_initial_state;
-  mh::ssd_rf_bwd_layout(p, a->workspace);
-  return hip_status(mh::launch_ssd_rf_bwd(p, reinterpret_cast<hipStream_t>(stream)), "ssd_ref_scan_bwd");
+  return hip_status(mh::launch_ssd_rf_bwd(p, a->workspace, reinterpret_cast<hipStream_t>(stream)), "ssd_ref_scan_bwd");
 }
 
 int mh_ssd_h_states_bwd_workspace_bytes(const mh_ssd_hs_bwd_args* a, size_t* bytes) {

@@ -138,11 +138,16 @@ struct RfParams {
   float* dD;                 // like D, or null
   float* d_dt_bias;          // (d_inner,) or null
   float* dh0;                // (b, d_inner, N) or null
+  // A large backward takes some batch rows (`batch` is then their number) and a span of the pieces at a time.
   float* ckpt;               // workspace: (b, pieces, d_inner, N) the state entering every 16-token piece
-  float* lam_ckpt;           // workspace: the same shape, the adjoint handed into every piece from its right
-  float* dB_part; float* dC_part;   // workspace: (b, channel blocks, L, N) sums over a block's channels
-  float* dA_part;            // workspace: (b, pieces, channel blocks, N)
-  float* dD_part; float* dbias_part;  // workspace: (b, pieces, d_inner) sums over the tokens of a piece
+  int span0, span;           // the span: its first piece, its pieces (all of them: 0, pieces)
+  int sweep0;                // first direction of the sweep's grid (0: states, 1: adjoints)
+  int first, last;           // the first, the last to be taken: dA, dD and d dt_bias start there and are whole there
+  float* lam_ckpt;           // workspace: (b, span, d_inner, N) the adjoint handed into every piece from its right
+  float* carry;              // workspace: (b, d_inner, N) the adjoint handed into the span from its right (span < pieces)
+  float* dB_part; float* dC_part;   // workspace: (b, channel blocks, the span's tokens, N) sums over a block's channels
+  float* dA_part;            // workspace: (b, span, channel blocks, N)
+  float* dD_part; float* dbias_part;  // workspace: (b, span, d_inner) sums over the tokens of a piece
   float* dD_sum;             // workspace: (d_inner) a channel's dD where D is per head
   int A_log;                 // A holds log-rates: the rates are -exp(clamp(A, -5, 5)), dA the gradient of A itself
 };
@@ -151,8 +156,7 @@ size_t ssd_rf_workspace_bytes(int batch, int seqlen, int d_inner, int dstate, bo
 hipError_t launch_ssd_rf(const RfParams& p, hipStream_t st);
 // Backward of the reference-form scan: checkpoints (a forward pass), the gradients, fixed-order reductions.
 size_t ssd_rf_bwd_workspace_bytes(int batch, int seqlen, int d_inner, int dstate);
-void ssd_rf_bwd_layout(RfParams& p, void* workspace);
-hipError_t launch_ssd_rf_bwd(const RfParams& p, hipStream_t st);
+hipError_t launch_ssd_rf_bwd(const RfParams& p, void* workspace, hipStream_t st);
 
 // h_states of the prefill (ssd_hstates.hip): mean over (h, p) of the state after every token.
 struct HsParams {

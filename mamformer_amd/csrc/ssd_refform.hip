@@ -639,8 +639,9 @@ __device__ __forceinline__ float rf_dt_chain(const RfParams& p, float raw, float
   return g;
 }
 
-// The adjoint walk, last block first, in the scan's layout.  p carries dy in x's place, C in B's and dhs in C's
-// (rf_sweep_kernel); dymul is 0 where dy is missing (a finite stand-in is read); HASG: dhs is given, times gmul.
+// The adjoint walk through the span, last block first, in the scan's layout.  p carries dy in x's place, C in B's and
+// dhs in C's (rf_sweep_kernel); dymul is 0 where dy is missing (a finite stand-in is read); HASG: dhs is given, times
+// gmul.
 template <typename T, int N, bool HASG>
 __device__ __forceinline__ void rf_adj_walk(const RfParams& p, RfSmem<N, rf_tb<N>(), rf_cpb<N>()>& sm, float dymul,
                                             float gmul) {
@@ -652,27 +653,29 @@ __device__ __forceinline__ void rf_adj_walk(const RfParams& p, RfSmem<N, rf_tb<N
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int cl = (64 / LPC) * w + lane / LPC, g = lane % LPC;
   const int c = c0 + cl, n0 = g * NS, L = p.seqlen;
-  const int nblk = (L + TB - 1) / TB, nsb = (L + RK - 1) / RK;
+  const int first = p.span0 * RK / TB, nblk = (min(L, (p.span0 + p.span) * RK) + TB - 1) / TB;   // the span's blocks
+  const int64_t state = ((int64_t)b * p.d_inner + c) * N + n0;
+  const float* from = (p.span0 + p.span) * RK < L ? p.carry : p.d_final;
   float k2[NS], lamc[NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
     k2[s] = rf_rate(p, n0 + s) * LOG2E;
-    lamc[s] = p.d_final ? p.d_final[((int64_t)b * p.d_inner + c) * N + n0 + s] : 0.f;
+    lamc[s] = from ? from[state + s] : 0.f;
   }
   RfRegs<T, N, TB, CPB> r;
   const float bias = p.dt_bias ? p.dt_bias[c0 + tid % CPB] : 0.f;
   rf_load<T, N, TB, CPB, false, HASG>(p, r, b, c0, (nblk - 1) * TB);
   rf_store<T, N, TB, CPB, false>(p, r, sm.st[(nblk - 1) & 1], (nblk - 1) * TB, bias);
-  if (nblk > 1) rf_load<T, N, TB, CPB, false, HASG>(p, r, b, c0, (nblk - 2) * TB);
+  if (nblk > first + 1) rf_load<T, N, TB, CPB, false, HASG>(p, r, b, c0, (nblk - 2) * TB);
   __syncthreads();
-  float* ck = p.lam_ckpt + ((int64_t)b * nsb * p.d_inner + c) * N + n0;
-  for (int k = nblk - 1; k >= 0; --k) {
+  float* ck = p.lam_ckpt + ((int64_t)b * p.span * p.d_inner + c) * N + n0;
+  for (int k = nblk - 1; k >= first; --k) {
     const RfStage<N, TB, CPB>& s = sm.st[k & 1];
 #pragma unroll 16
     for (int t = TB - 1; t >= 0; --t) {
       const int tt = k * TB + t;                           // (past the end: dt = 0, dy = 0, no dhs)
       if (t % RK == RK - 1 && tt - (RK - 1) < L) {
-        float* o = ck + (int64_t)(tt / RK) * p.d_inner * N;
+        float* o = ck + (int64_t)(tt / RK - p.span0) * p.d_inner * N;
 #pragma unroll
         for (int s2 = 0; s2 < NS; ++s2) o[s2] = lamc[s2];
       }
@@ -686,21 +689,21 @@ __device__ __forceinline__ void rf_adj_walk(const RfParams& p, RfSmem<N, rf_tb<N
         lamc[s2] = __builtin_amdgcn_exp2f(o.dt * k2[s2]) * lam;
       }
     }
-    if (k > 0) rf_store<T, N, TB, CPB, false>(p, r, sm.st[(k - 1) & 1], (k - 1) * TB, bias);
-    if (k > 1) rf_load<T, N, TB, CPB, false, HASG>(p, r, b, c0, (k - 2) * TB);
+    if (k > first) rf_store<T, N, TB, CPB, false>(p, r, sm.st[(k - 1) & 1], (k - 1) * TB, bias);
+    if (k > first + 1) rf_load<T, N, TB, CPB, false, HASG>(p, r, b, c0, (k - 2) * TB);
     lds_barrier();
   }
-  if (p.dh0) {
-    float* o = p.dh0 + ((int64_t)b * p.d_inner + c) * N + n0;
+  float* to = first > 0 ? p.carry : p.dh0;               // (each lane its own, read above)
+  if (to) {
 #pragma unroll
-    for (int s = 0; s < NS; ++s) o[s] = lamc[s];
+    for (int s = 0; s < NS; ++s) to[state + s] = lamc[s];
   }
 }
 
 template <typename T, int N, bool HASG>
 __global__ __launch_bounds__(RF_NT) void rf_sweep_kernel(RfParams p) {
   __shared__ RfSmem<N, rf_tb<N>(), rf_cpb<N>()> sm;
-  if (blockIdx.y == 0) {
+  if (blockIdx.y + p.sweep0 == 0) {
     rf_scan_walk<T, N, false, true>(p, sm);
     return;
   }
@@ -787,7 +790,7 @@ __global__ __launch_bounds__(RF_NT, 2) void rf_grad_kernel(RfParams p) {
   const int L = p.seqlen, di = p.d_inner;
   const int nsb = (L + RK - 1) / RK, ncb = (di + CH - 1) / CH;
   const int bj = blockIdx.x / ncb, cb = blockIdx.x - bj * ncb;
-  const int b = bj / nsb, j = bj - b * nsb;
+  const int b = bj / p.span, j = p.span0 + bj - b * p.span;   // bj: the (row, piece of the span)
   const int t0 = j * RK, c0 = cb * CH;
   const int tid = threadIdx.x, l = tid & 63, w = wave_id(), gl = l % LN;
   const int n0 = 4 * gl;
@@ -834,26 +837,26 @@ __global__ __launch_bounds__(RF_NT, 2) void rf_grad_kernel(RfParams p) {
     dA[i] = 0.f;
   }
   __syncthreads();
-  const int64_t prow = ((int64_t)b * nsb + j) * di;
+  const int64_t prow = ((int64_t)b * nsb + j) * di, srow = (int64_t)bj * di;   // rows by the sequence's, the span's pieces
   if (tid < CH && c0 + tid < di) {
     float dD = 0.f;
 #pragma unroll
     for (int t = 0; t < RK; ++t) dD = fmaf(sm.sv[t][tid].z, sm.sv[t][tid].w, dD);
-    p.dD_part[prow + c0 + tid] = dD;
+    p.dD_part[srow + c0 + tid] = dD;
   }
   __syncthreads();                                         // dx takes the place of dt below
 
   auto chan = [&](int s) { return (4 * s + w) * LC + l / LN; };      // channel within the block
-  auto ckpt = [&](const float* base, int q) {
-    return *reinterpret_cast<const float4*>(base + (prow + min(c0 + q, di - 1)) * N + n0);
+  auto ckpt = [&](const float* base, int64_t row, int q) {
+    return *reinterpret_cast<const float4*>(base + (row + min(c0 + q, di - 1)) * N + n0);
   };
   auto half = [&](auto OFFc) {
     constexpr int OFF = decltype(OFFc)::value;             // the half's first token
     float acc[2 * HK * 4];                                 // dB then dC: [token][state] sums over this lane's channels
 #pragma unroll
     for (int i = 0; i < 2 * HK * 4; ++i) acc[i] = 0.f;
-    float4 hn = ckpt(p.ckpt, chan(0)), ln;
-    if constexpr (OFF > 0) ln = ckpt(p.lam_ckpt, chan(0));
+    float4 hn = ckpt(p.ckpt, prow, chan(0)), ln;
+    if constexpr (OFF > 0) ln = ckpt(p.lam_ckpt, srow, chan(0));
     int s = 0;
 #pragma unroll 1
     do {                                                   // (no branch inside: a second copy of the sums at every join)
@@ -863,8 +866,8 @@ __global__ __launch_bounds__(RF_NT, 2) void rf_grad_kernel(RfParams p) {
       float h[4] = {hn.x * on, hn.y * on, hn.z * on, hn.w * on};
       float lamc[4] = {ln.x * on, ln.y * on, ln.z * on, ln.w * on};
       const int qn = chan(min(s + 1, NSTEP - 1));
-      hn = ckpt(p.ckpt, qn);
-      if constexpr (OFF > 0) ln = ckpt(p.lam_ckpt, qn);
+      hn = ckpt(p.ckpt, prow, qn);
+      if constexpr (OFF > 0) ln = ckpt(p.lam_ckpt, srow, qn);
       const float Dc = sm.D[q];
       // the B and C rows are the same every step: laundered here, so that they are read from LDS again instead of
       // held in 128 registers for the whole loop
@@ -970,9 +973,10 @@ __global__ __launch_bounds__(RF_NT, 2) void rf_grad_kernel(RfParams p) {
       __syncthreads();
     }
     const float* rf = reinterpret_cast<const float*>(red);
+    const int s0 = p.span0 * RK, Ls = min(L - s0, p.span * RK);   // the span's tokens
     for (int e = tid; e < 2 * HK * N; e += RF_NT) {
       const int t = t0 + OFF + (e / N) % HK, n = e % N;
-      if (t < L) (e < HK * N ? p.dB_part : p.dC_part)[(((int64_t)b * ncb + cb) * L + t) * N + n] = rf[e];
+      if (t < L) (e < HK * N ? p.dB_part : p.dC_part)[(((int64_t)b * ncb + cb) * Ls + t - s0) * N + n] = rf[e];
     }
     __syncthreads();                                       // red is written again
   };
@@ -990,12 +994,12 @@ __global__ __launch_bounds__(RF_NT, 2) void rf_grad_kernel(RfParams p) {
   }
   __syncthreads();
   if (tid < N)
-    p.dA_part[(((int64_t)b * nsb + j) * ncb + cb) * N + tid] = dAw[tid] + dAw[N + tid] + dAw[2 * N + tid] + dAw[3 * N + tid];
+    p.dA_part[((int64_t)bj * ncb + cb) * N + tid] = dAw[tid] + dAw[N + tid] + dAw[2 * N + tid] + dAw[3 * N + tid];
   if (tid < CH && c0 + tid < di) {
     float db = 0.f;
 #pragma unroll
     for (int t = 0; t < RK; ++t) db += sm.sv[t][tid].y;
-    p.dbias_part[prow + c0 + tid] = db;
+    p.dbias_part[srow + c0 + tid] = db;
   }
 #pragma unroll
   for (int k = 0; k < RK * CH / RF_NT; ++k) {
@@ -1009,10 +1013,11 @@ __global__ __launch_bounds__(RF_NT, 2) void rf_grad_kernel(RfParams p) {
   }
 }
 
-// dB, dC (b, L, N) = the channel blocks' partials added in order.
+// dB, dC (b, L, N), the span's tokens = the channel blocks' partials added in order.
 template <typename T>
 __global__ __launch_bounds__(256) void rf_bwd_reduce_kernel(RfParams p, int ncb) {
-  const int64_t per = (int64_t)p.seqlen * p.dstate / 4;
+  const int s0 = p.span0 * RF_RK;
+  const int64_t per = (int64_t)min(p.seqlen - s0, p.span * RF_RK) * p.dstate / 4;
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= (int64_t)p.batch * per) return;
   const int64_t b = i / per, r = i % per;
@@ -1024,10 +1029,11 @@ __global__ __launch_bounds__(256) void rf_bwd_reduce_kernel(RfParams p, int ncb)
     sb += pb[(b * ncb + k) * per + r];
     sc += pc[(b * ncb + k) * per + r];
   }
+  const int64_t o = (b * p.seqlen + s0) * p.dstate + 4 * r;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    reinterpret_cast<T*>(p.dB)[4 * i + j] = from_f32<T>(sb[j]);
-    reinterpret_cast<T*>(p.dC)[4 * i + j] = from_f32<T>(sc[j]);
+    reinterpret_cast<T*>(p.dB)[o + j] = from_f32<T>(sb[j]);
+    reinterpret_cast<T*>(p.dC)[o + j] = from_f32<T>(sc[j]);
   }
 }
 
@@ -1049,20 +1055,20 @@ __device__ __forceinline__ float rf_column_sum(const float* part, int64_t rows, 
   return a;
 }
 
-// dA (N): partials per (batch, piece, channel block); dD per channel and d dt_bias (d_inner): per (batch, piece).  One
-// workgroup per 16 columns, dA's first; with D per head the channel sums go to dD_sum and rf_bwd_head_kernel adds a
-// head's channels.
+// dA (N): partials per (batch, piece, channel block); dD per channel and d dt_bias (d_inner): per (batch, piece), of the
+// span, onto those of the spans before (to the right).  One workgroup per 16 columns, dA's first; with D per head the
+// channel sums go to dD_sum and rf_bwd_head_kernel adds a head's channels.
 __global__ __launch_bounds__(1024) void rf_bwd_param_kernel(RfParams p, int ncb, int na) {
   __shared__ float red[64][17];
   const int di = p.d_inner, N = p.dstate, q = threadIdx.x & 15;
-  const int nsb = (p.seqlen + RF_RK - 1) / RF_RK;
-  const int64_t rows = (int64_t)p.batch * nsb;
+  const int64_t rows = (int64_t)p.batch * p.span;
   if ((int)blockIdx.x < na) {
     const int i = blockIdx.x * 16 + q;
-    const float a = rf_column_sum(p.dA_part, rows * ncb, N, i, i < N, red);
+    float a = rf_column_sum(p.dA_part, rows * ncb, N, i, i < N, red);
     if (threadIdx.x < 16 && i < N) {
+      if (!p.first) a += p.dA[i];
       const float r = p.A[i];                              // A_log's gradient: through exp, inside the clamp
-      p.dA[i] = !p.A_log ? a : r >= -5.f && r <= 5.f ? a * rf_rate(p, i) : 0.f;
+      p.dA[i] = !p.last || !p.A_log ? a : r >= -5.f && r <= 5.f ? a * rf_rate(p, i) : 0.f;
     }
     return;
   }
@@ -1070,8 +1076,9 @@ __global__ __launch_bounds__(1024) void rf_bwd_param_kernel(RfParams p, int ncb,
   const float d = rf_column_sum(p.dD_part, rows, di, i, i < di, red);
   const float s = rf_column_sum(p.dbias_part, rows, di, i, i < di, red);
   if (threadIdx.x < 16 && i < di) {
-    if (p.d_dt_bias) p.d_dt_bias[i] = s;
-    if (p.dD) (p.D_per_channel ? p.dD : p.dD_sum)[i] = d;
+    if (p.d_dt_bias) p.d_dt_bias[i] = p.first ? s : p.d_dt_bias[i] + s;
+    float* o = p.D_per_channel ? p.dD : p.dD_sum;
+    if (p.dD) o[i] = p.first ? d : o[i] + d;
   }
 }
 
@@ -1100,26 +1107,34 @@ hipError_t launch_rf_bwd_t(const RfParams& p, hipStream_t st) {
     hipLaunchKernelGGL(rf_bwd_empty_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, p);
     return hipGetLastError();
   }
-  const dim3 sgrid((unsigned)(p.batch * (p.d_inner / rf_cpb<N>())), 2);
-  if (p.dhs) hipLaunchKernelGGL((rf_sweep_kernel<T, N, true>), sgrid, dim3(RF_NT), 0, st, p);
-  else hipLaunchKernelGGL((rf_sweep_kernel<T, N, false>), sgrid, dim3(RF_NT), 0, st, p);
+  const unsigned walks = (unsigned)(p.batch * (p.d_inner / rf_cpb<N>()));
+  const bool whole = p.span == (p.seqlen + RF_RK - 1) / RF_RK;
+  if (!whole && p.span0 + p.span >= (p.seqlen + RF_RK - 1) / RF_RK) {   // the first span of these rows: their states
+    hipLaunchKernelGGL((rf_sweep_kernel<T, N, false>), dim3(walks, 1), dim3(RF_NT), 0, st, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  RfParams q = p;
+  q.sweep0 = whole ? 0 : 1;
+  const dim3 sgrid(walks, whole ? 2 : 1);
+  if (p.dhs) hipLaunchKernelGGL((rf_sweep_kernel<T, N, true>), sgrid, dim3(RF_NT), 0, st, q);
+  else hipLaunchKernelGGL((rf_sweep_kernel<T, N, false>), sgrid, dim3(RF_NT), 0, st, q);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const int ncb = (p.d_inner + RF_CH - 1) / RF_CH;
-  const int nsb = (p.seqlen + RF_RK - 1) / RF_RK;
-  const dim3 grid((unsigned)((int64_t)p.batch * nsb * ncb));
+  const dim3 grid((unsigned)((int64_t)p.batch * p.span * ncb));
   if (p.dhs) hipLaunchKernelGGL((rf_grad_kernel<T, N, true>), grid, dim3(RF_NT), 0, st, p);
   else hipLaunchKernelGGL((rf_grad_kernel<T, N, false>), grid, dim3(RF_NT), 0, st, p);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const int64_t tot = (int64_t)p.batch * p.seqlen * N / 4;
+  const int64_t tot = (int64_t)p.batch * std::min(p.seqlen - p.span0 * RF_RK, p.span * RF_RK) * N / 4;
   hipLaunchKernelGGL((rf_bwd_reduce_kernel<T>), dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st, p, ncb);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   const int na = (N + 15) / 16;
   hipLaunchKernelGGL(rf_bwd_param_kernel, dim3((unsigned)(na + (p.d_inner + 15) / 16)), dim3(1024), 0, st, p, ncb, na);
   e = hipGetLastError();
-  if (e != hipSuccess || !p.dD || p.D_per_channel) return e;
+  if (e != hipSuccess || !p.dD || p.D_per_channel || !p.last) return e;
   hipLaunchKernelGGL(rf_bwd_head_kernel, dim3((unsigned)((p.d_inner / p.headdim + 255) / 256)), dim3(256), 0, st, p);
   return hipGetLastError();
 }
@@ -1153,43 +1168,105 @@ hipError_t launch_ssd_rf(const RfParams& p, hipStream_t st) {
   return launch_rf_n<float>(p, st);
 }
 
-// Backward workspace, all fp32: the states and adjoints entering every piece (b, pieces, d_inner, N) each, the dB and
-// dC partials (b, channel blocks, L, N), the dA partials (b, pieces, channel blocks, N), the dD / d dt_bias partials
-// (b, pieces, d_inner) and the channels' dD sums (d_inner).
-struct RfBwdWorkspace {
-  size_t ck, part, da, dd, ds;
-  RfBwdWorkspace(size_t batch, size_t seqlen, size_t d_inner, size_t dstate) {
-    const size_t nsb = (seqlen + RF_RK - 1) / RF_RK, ncb = (d_inner + RF_CH - 1) / RF_CH;
-    ck = align256(batch * nsb * d_inner * dstate * 4);
-    part = align256(batch * ncb * seqlen * dstate * 4);
-    da = align256(batch * nsb * ncb * dstate * 4);
-    dd = align256(batch * nsb * d_inner * 4);
-    ds = align256(d_inner * 4);
+// Backward workspace, all fp32 (the parts of RfParams).  Whole, the adjoints are as many as the states and the partials half
+// of that: 2.6 times the states' bytes, where a walk backward through the states needs little besides them (b1 L16384
+// d_inner 4096 N128: 5.7 GB, states 2.1).  Beyond RF_WHOLE_BYTES the call therefore takes a span of the pieces after
+// another, or where there are too few pieces some batch rows after others, so that all of it fits RF_WHOLE_BYTES or 9/8
+// of the states, whichever is more.  Spans first: every row's walks still run side by side.  Forward and backward, whole
+// and in spans or rows: that size 12.60 and 12.72 ms, b1 L65536 d_inner 2048 N64 14.6 and 16.6, b512 L256 25.0 and 24.3.
+constexpr size_t RF_WHOLE_BYTES = (size_t)2 << 30;
+struct RfBwdPlan {
+  int rows, span;                                          // batch rows and pieces at a time
+  size_t ck, lam, carry, part, da, dd, ds;
+
+  RfBwdPlan(int batch, int seqlen, int d_inner, int dstate) {
+    const int nsb = (seqlen + RF_RK - 1) / RF_RK;
+    if (sizes(batch, nsb, seqlen, d_inner, dstate) <= RF_WHOLE_BYTES) return;
+    const size_t most = std::max(RF_WHOLE_BYTES, ck / 8 * 9);
+    const int step = dstate <= 128 ? 32 / RF_RK : 1;       // a walk's blocks (rf_tb) are whole
+    int least = nsb;
+    for (int n = 2; n <= 32 && n <= nsb; ++n) {
+      const int sp = ((nsb + n - 1) / n + step - 1) / step * step;
+      if (sp >= nsb) continue;
+      least = sp;
+      if (sizes(batch, sp, seqlen, d_inner, dstate) <= most) return;
+    }
+    for (int n = 2; n <= batch && n <= 4; ++n)
+      if (sizes((batch + n - 1) / n, nsb, seqlen, d_inner, dstate) <= most) return;
+    sizes(batch, least, seqlen, d_inner, dstate);          // (a short sequence of one row or two: as near as its blocks allow)
   }
+
+  size_t sizes(int r, int s, int seqlen, int d_inner, int dstate) {
+    rows = r;
+    span = s;
+    const size_t b = r, sp = s, di = d_inner, N = dstate, nsb = ((size_t)seqlen + RF_RK - 1) / RF_RK;
+    const size_t ncb = (di + RF_CH - 1) / RF_CH, tokens = std::min<size_t>(seqlen, sp * RF_RK);
+    ck = align256(b * nsb * di * N * 4);
+    lam = align256(b * sp * di * N * 4);
+    carry = sp < nsb ? align256(b * di * N * 4) : 0;
+    part = align256(b * ncb * tokens * N * 4);
+    da = align256(b * sp * ncb * N * 4);
+    dd = align256(b * sp * di * 4);
+    ds = align256(di * 4);
+    return bytes();
+  }
+  size_t bytes() const { return ck + lam + carry + 2 * part + da + 2 * dd + ds; }
 };
 
 size_t ssd_rf_bwd_workspace_bytes(int batch, int seqlen, int d_inner, int dstate) {
-  const RfBwdWorkspace s(batch, seqlen, d_inner, dstate);
-  return 2 * s.ck + 2 * s.part + s.da + 2 * s.dd + s.ds;
+  return RfBwdPlan(batch, seqlen, d_inner, dstate).bytes();
 }
 
-void ssd_rf_bwd_layout(RfParams& p, void* workspace) {
-  const RfBwdWorkspace s(p.batch, p.seqlen, p.d_inner, p.dstate);
+hipError_t launch_ssd_rf_bwd(const RfParams& p, void* workspace, hipStream_t st) {
+  const RfBwdPlan s(p.batch, p.seqlen, p.d_inner, p.dstate);
+  RfParams q = p;
   char* w = reinterpret_cast<char*>(workspace);
   auto take = [&](size_t n) { char* r = w; w += n; return reinterpret_cast<float*>(r); };
-  p.ckpt = take(s.ck);
-  p.lam_ckpt = take(s.ck);
-  p.dB_part = take(s.part);
-  p.dC_part = take(s.part);
-  p.dA_part = take(s.da);
-  p.dD_part = take(s.dd);
-  p.dbias_part = take(s.dd);
-  p.dD_sum = take(s.ds);
-}
+  q.ckpt = take(s.ck);
+  q.lam_ckpt = take(s.lam);
+  q.carry = take(s.carry);
+  q.dB_part = take(s.part);
+  q.dC_part = take(s.part);
+  q.dA_part = take(s.da);
+  q.dD_part = take(s.dd);
+  q.dbias_part = take(s.dd);
+  q.dD_sum = take(s.ds);
+  auto launch = [&](const RfParams& r) { return r.dtype == DT_BF16 ? launch_rf_bwd_n<bf16>(r, st) : launch_rf_bwd_n<float>(r, st); };
+  q.first = q.last = 1;
+  if (p.seqlen == 0) return launch(q);
 
-hipError_t launch_ssd_rf_bwd(const RfParams& p, hipStream_t st) {
-  if (p.dtype == DT_BF16) return launch_rf_bwd_n<bf16>(p, st);
-  return launch_rf_bwd_n<float>(p, st);
+  const int nsb = (p.seqlen + RF_RK - 1) / RF_RK;
+  const int64_t es = p.dtype == DT_BF16 ? 2 : 4, di = p.d_inner, N = p.dstate;
+  auto at = [](auto* base, int64_t bytes) {                // null stays null
+    using P = decltype(base);
+    return base ? reinterpret_cast<P>(reinterpret_cast<uintptr_t>(base) + bytes) : base;
+  };
+  for (int64_t b0 = 0; b0 < p.batch; b0 += s.rows) {
+    RfParams r = q;
+    r.batch = (int)std::min<int64_t>(s.rows, p.batch - b0);
+    r.x = at(p.x, b0 * p.x_sb * es);
+    r.dt = at(p.dt, b0 * p.dt_sb * 4);
+    r.B = at(p.B, b0 * p.B_sb * es);
+    r.C = at(p.C, b0 * p.C_sb * es);
+    r.init_state = at(p.init_state, b0 * di * N * 4);
+    r.dy = at(p.dy, b0 * p.seqlen * di * es);
+    r.dhs = at(p.dhs, b0 * p.seqlen * N * es);
+    r.d_final = at(p.d_final, b0 * di * N * 4);
+    r.dx = at(p.dx, b0 * p.seqlen * di * es);
+    r.ddt = at(p.ddt, b0 * p.seqlen * di * 4);
+    r.dB = at(p.dB, b0 * p.seqlen * N * es);
+    r.dC = at(p.dC, b0 * p.seqlen * N * es);
+    r.dh0 = at(p.dh0, b0 * di * N * 4);
+    for (int j = (nsb - 1) / s.span * s.span; j >= 0; j -= s.span) {   // the last span first: adjoints run backward
+      r.span0 = j;
+      r.span = std::min(s.span, nsb - j);
+      r.first = b0 == 0 && j + s.span >= nsb;
+      r.last = b0 + s.rows >= p.batch && j == 0;
+      const hipError_t e = launch(r);
+      if (e != hipSuccess) return e;
+    }
+  }
+  return hipSuccess;
 }
 
 }  // namespace mh
