@@ -85,14 +85,6 @@ __device__ __forceinline__ Frag<TM> acc_to_frag(const f32x16& acc, int c) {
   for (int j = 0; j < 8; ++j) f.set(j, acc[8 * c + j]);
   return f;
 }
-// Same with a per-element scale.
-template <typename TM>
-__device__ __forceinline__ Frag<TM> acc_to_frag_scaled(const f32x16& acc, int c, float s) {
-  Frag<TM> f;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) f.set(j, acc[8 * c + j] * s);
-  return f;
-}
 
 // ---------------------------------------------------------------- wave helpers
 __device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
@@ -191,16 +183,6 @@ __device__ __forceinline__ float sum_quad(float v) {
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-  return v;
-}
-__device__ __forceinline__ float wave_min(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fminf(v, __shfl_xor(v, off, 64));
   return v;
 }
 

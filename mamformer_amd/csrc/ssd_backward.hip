@@ -203,15 +203,6 @@ __device__ __forceinline__ void tr_frags_inflight(const T* tile, int r0, int q0,
   }
 }
 
-// x^T-style transpose of a 32-column half tile (XHalf layout): D[r][q] = tile[r0 + r][q], lane = column q.
-template <typename T>
-__device__ __forceinline__ f32x16 xhalf_transpose(const T* tile, int r0, const Frag<T> (&id)[2], int half, int l32) {
-  f32x16 acc = zero16();
-#pragma unroll
-  for (int c = 0; c < 2; ++c) acc = mma(xrow_frag<T, T>(tile, r0 + l32, 16 * c + 8 * half), id[c], acc);
-  return acc;
-}
-
 // d(processed dt) / d(raw dt): sigmoid below softplus' threshold (identity above), times the clamp's pass mask.
 __device__ __forceinline__ float dt_chain(const SsdParams& p, float raw, float bias) {
   const float u = raw + bias;
@@ -1023,7 +1014,7 @@ __global__ __launch_bounds__(128 * (N / 32)) void ssd_bwd_grad_kernel(SsdBwdPara
       }
       store_dx();
     }
-    if (w == NW - 1) {                  // (a wave without an XD tile of the next head)
+    if (w == NW - 1) {                  // (N = 128: a wave without an XD tile of the next head; at N = 64 one with a single tile)
       const float colG = l < 32 ? sm.colg[st][0][l] + sm.colg[st][1][l] : sm.colg[st][2][l - 32];
       const float rowG = l < 32 ? sm.rowg[st][0][l] : sm.rowg[st][1][l - 32] + sm.rowg[st][2][l - 32];
       float bint = 0.f, u = 0.f, lh = 0.f;

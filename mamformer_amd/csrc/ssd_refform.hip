@@ -113,38 +113,7 @@ __device__ __forceinline__ float rf_reduce_scatter32(float (&v)[32], int l) {
   return v[0];
 }
 
-// 16 values over the 32 lanes of a channel: lanes 2 m and 2 m + 1 of the channel end with the sum of v[m].
-__device__ __forceinline__ float rf_reduce_scatter32_16(float (&v)[16], int l) {
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[k]), __float_as_uint(v[k + 8]), false, false);
-    v[k] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  }
-  rf_rs_step<8, 8>(v, l);
-  rf_rs_step<4, 4>(v, l);
-  rf_rs_step<2, 2>(v, l);
-  return v[0] + xor1(v[0]);
-}
-
-// 32 values over all 64 lanes of the wave: lanes 2 m and 2 m + 1 end with the sum of v[m].
-__device__ __forceinline__ float rf_reduce_scatter64_32(float (&v)[32], int l) {
-#pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[k]), __float_as_uint(v[k + 16]), false, false);
-    v[k] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  }
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[k]), __float_as_uint(v[k + 8]), false, false);
-    v[k] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  }
-  rf_rs_step<8, 8>(v, l);
-  rf_rs_step<4, 4>(v, l);
-  rf_rs_step<2, 2>(v, l);
-  return v[0] + xor1(v[0]);
-}
-
-// The same over all 64 lanes of the wave: lane l ends with the sum of v[l] (v_permlane32_swap first).
+// 64 values over all 64 lanes of the wave: lane l ends with the sum of v[l] (v_permlane32_swap first).
 __device__ __forceinline__ float rf_reduce_scatter64(float (&v)[64], int l) {
 #pragma unroll
   for (int k = 0; k < 32; ++k) {
@@ -309,7 +278,7 @@ __device__ __forceinline__ void rf_store(const RfParams& p, const RfRegs<T, N, T
   }
 }
 
-// One token's operands, read from LDS a token ahead of their use.
+// One token's operands, read from LDS ahead of their use (one token or two).
 template <int NS>
 struct RfTok {
   float dt, x, b[NS], c[NS];
