@@ -370,9 +370,10 @@ int ssd_bwd_validate(const mh_ssd_bwd_args* a) {
 
 // Heads of one group per workgroup of the gradient kernel: a power of two dividing H / G.  A workgroup takes f us for
 // its segment's B, C and masked tiles and s per head, one per CU at a time, and each partial of dB and dC that is added
-// afterwards 0.25 us.  Fixed at 16, as it was, small calls left most CUs idle (bf16 backward, us: b1 L1000 H32 16
-// heads 138, 2 heads 48; b2 L400 H32 131, 39; b1 L64 H8 67 with 8, 21 with 1), and b2 L4096 H64 took two rounds of 16
-// where one of 32 is enough (353, 307).  fp32 b1 L1000 H32: 653, 2 heads 199.
+// afterwards 0.25 us.  With 16 heads always, small calls leave most CUs idle (bf16 backward, us: b1 L1000 H32 16 heads
+// 118, 2 heads 47; b2 L400 H32 113, 39; b1 L64 H8 56 with 8, 21 with 1), and b2 L4096 H64 takes two rounds of 16 where one
+// of 32 is enough (301, 291).  fp32 b1 L1000 H32: 640, 2 heads 199.  f and s were fitted to a slower form of the bf16
+// kernel; the pick is within 3% of the best power of two at 13 sizes from b1 L64 H8 to b2 L4096 H128 all the same.
 int ssd_bwd_heads_per_wg(const mh_ssd_args* f) {
   const int64_t hpg = f->nheads / f->ngroups, nseg = (f->seqlen + 63) / 64;
   const double fix = f->dtype == MH_F32 ? 17.0 : 8.0, per = f->dtype == MH_F32 ? 32.0 : 5.2;
