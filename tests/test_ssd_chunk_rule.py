@@ -46,19 +46,20 @@ def test_chunk_rule_range_and_scratch():
     for b, L, H, N, G in sizes:
         for code, dtype in ((_lib.MH_BF16, torch.bfloat16), (_lib.MH_F32, torch.float32)):
             c = mh.ssd_chunk_len(b, L, H, 64, N, G, dtype)
-            assert c % 64 == 0 and (64 if dtype == torch.float32 else 192) <= c <= 16384
+            assert c % 64 == 0 and (64 if dtype == torch.float32 else 256) <= c <= 16384
             one = one_round(b, L, H, N, G, dtype == torch.float32)
             if workspace(b, L, H, N, G, code, one) <= _lib.NOALLOC_SCRATCH_BYTES:
                 assert workspace(b, L, H, N, G, code, 0) <= _lib.NOALLOC_SCRATCH_BYTES, (b, L, H, N, G, dtype)
 
 
-# around the shortest chunks: one segment, a chunk and one token, two chunks, and more than 8 chunks (bf16: the states'
-# pass; fp32: one-segment chunks)
+# around the shortest chunks: one segment, a chunk and one token, two chunks, and more than 8 chunks (bf16, of 256 tokens:
+# the states' pass; fp32: one-segment chunks)
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype,b,L,H,N,G", [
     (torch.float32, 1, 63, 8, 128, 1), (torch.float32, 2, 129, 8, 64, 2), (torch.float32, 1, 1025, 32, 128, 1),
     (torch.float32, 3, 705, 64, 64, 8), (torch.bfloat16, 1, 193, 48, 64, 1), (torch.bfloat16, 2, 385, 16, 128, 2),
-    (torch.bfloat16, 1, 1729, 8, 128, 1),
+    (torch.bfloat16, 1, 1729, 8, 128, 1), (torch.bfloat16, 1, 257, 48, 64, 1), (torch.bfloat16, 2, 513, 16, 128, 2),
+    (torch.bfloat16, 1, 2305, 8, 128, 1),
 ])
 def test_chosen_chunk_vs_oracle(dtype, b, L, H, N, G):
     cfg = W.SSDConfig("c", b, L, H, 64, N, G, 256, dtype, L, init_state=True)
